@@ -161,13 +161,13 @@ int vtx_stencil_segments(vtx_solver* s, int32_t* count);
  * exception (see below). */
 typedef struct vtx_tuning {
     int32_t use_graph;         /* replay frames from a hipGraph */
-    int32_t neighbor_order;    /* neighbour search thread order: 0 particle index, 1 hash-sorted,
-                                  2 vertex patches for grid cloths (sorted for other meshes) */
+    int32_t neighbor_order;    /* 0 to 2, no effect: once the neighbour search's thread order, which
+                                  is now one for all (waves over runs of particles of one cell) */
     int32_t lra_batch;         /* dense attachment distances loaded per batch: 4, 16 or 64 */
     int32_t xcd_remap;         /* hand each XCD a contiguous run of tiles */
     float frame_ms;            /* vtx_autotune: the chosen variant's frame time (0 from the cache) */
-    int32_t gather_block;      /* threads per workgroup of the neighbour search and contact pass:
-                                  64, 128 or 256 (each 256-particle tile split across workgroups) */
+    int32_t gather_block;      /* threads per workgroup of the contact pass: 64, 128 or 256 (each
+                                  256-particle tile split across workgroups) */
     int32_t streams;           /* k = 1..4: the segments split into k particle-balanced groups
                                   whose frames run concurrently on k streams */
     int32_t lra_split;         /* 1: grid cloths with 32 or more dense attachment slots run their

@@ -1495,7 +1495,7 @@ void Engine::hash_build(const DevState& d, int in, hipStream_t s) {
         stage_end(s);
     }
     stage_begin("k_neighbors", "Solver_HashCache", s);
-    VTX_HIP(launch_neighbors(d, in, tun_.nbr_order, tun_.gather_block, s));
+    VTX_HIP(launch_neighbors(d, s));
     stage_end(s);
     sorted_src_ = src;
 }
@@ -1760,21 +1760,19 @@ Tuning Engine::autotune(int frames, float frame_dt, bool use_cache, double* fram
         bms = trial(best);
         // one knob at a time, every other value of it against the best so far; the hash grid
         // (opted-in segments only) goes before the knobs of the hash and neighbour phases
-        static const int order[] = {0, 8, 1, 2, 3, 4, 5, 6, 7};
+        static const int order[] = {0, 8, 2, 3, 4, 5, 6, 7};
         for (int knob : order) {
             if (knob == 8 && !any_grid_tunable_) continue;
-            if (knob == 1 && !any_selfcol_) continue;
             if (knob == 2 && !any_lra_dense_) continue;
             if (knob == 4 && !need_collide_) continue;
             if (knob == 5 && table_seg_.size() < 2) continue;
             if (knob == 6 && !any_lra_split_) continue;
             if (knob == 7 && !any_hash_lds_) continue;
-            const int nval = knob == 5 || knob == 8 ? 4 : knob == 1 || knob == 2 || knob == 4 ? 3 : 2;
+            const int nval = knob == 5 || knob == 8 ? 4 : knob == 2 || knob == 4 ? 3 : 2;
             const Tuning base = best;
             for (int v = 0; v < nval; v++) {
                 Tuning t = base;
                 if (knob == 0) t.graph = v != 0;
-                if (knob == 1) t.nbr_order = v;
                 if (knob == 2) t.lra_batch = v == 0 ? 4 : v == 1 ? 16 : 64;
                 if (knob == 3) t.remap = v != 0;
                 if (knob == 4) t.gather_block = 64 << v;
@@ -1783,7 +1781,7 @@ Tuning Engine::autotune(int frames, float frame_dt, bool use_cache, double* fram
                 if (knob == 7) t.hash_lds = v != 0;
                 if (knob == 8) t.hash_grid = v;
                 if (knob == 8 ? t.hash_grid == base.hash_grid
-                    : knob == 0 ? t.graph == base.graph : knob == 1 ? t.nbr_order == base.nbr_order
+                    : knob == 0 ? t.graph == base.graph
                                 : knob == 2 ? t.lra_batch == base.lra_batch
                                 : knob == 3 ? t.remap == base.remap
                                 : knob == 4 ? t.gather_block == base.gather_block

@@ -129,14 +129,14 @@ struct Segment {
 };
 
 // Launch variants the tuner chooses among. Every combination gives bit-identical results: they
-// change which workgroup takes which tile, the order threads take particles in, how many loads
-// are in flight and whether launches are replayed from a graph, never the arithmetic.
+// change which workgroup takes which tile, how many loads are in flight and whether launches are
+// replayed from a graph, never the arithmetic.
 struct Tuning {
     bool graph = true;        // replay frames from a hipGraph
-    int nbr_order = 2;        // neighbour search thread order: 0 particle, 1 sorted, 2 grid patches
+    int nbr_order = 2;        // kept for callers (vtx_tuning.neighbor_order), no effect
     int lra_batch = 16;       // dense attachment distances loaded per batch: 4, 16 or 64
     bool remap = true;        // XCD-aware workgroup -> tile remap
-    int gather_block = 256;   // threads per workgroup of the neighbour search and contact pass
+    int gather_block = 256;   // threads per workgroup of the contact pass
     int streams = 1;          // k > 1: segments split into k particle-balanced groups whose frames
                               // run on k streams, overlapping latency- and VALU-bound stages
     bool lra_split = true;    // grid segments with >= VTX_LRA_SPLIT_MIN dense slots: four threads

@@ -440,263 +440,205 @@ __global__ __launch_bounds__(VTX_HASH_LDS_BT) void k_hash_small(DevState d, cons
 // CacheNeighbors_Kernel (Velvet/SpatialHashGPU.cu:79-130). Cells are visited x-, y-, z-nested;
 // inside a cell in sorted order, at most max_nbr entries per cell and in total; the list ends
 // with ~0u unless full. Squared distances are fmaf(dz,dz,fmaf(dy,dy,dx*dx)).
-// Thread -> particle mapping (ORDER), all giving the same table:
-//   NBR_PARTICLE: index order over the segment's particle tiles;
-//   NBR_SORTED:   hash-sorted order, so the lanes of one cell walk identical candidate ranges and
-//                 their loads merge; after the sweep, lanes re-dealt by candidate total;
-//   NBR_PATCH:    16 x 16 vertex patches of a grid cloth (its stencil tiles): a wave is 4 rows x
-//                 16 columns, so lanes share cells and candidates, and the 16 lanes of a patch
-//                 row hold consecutive particles, whose chunks are consecutive in the table.
-// A first sweep over the 27 cells finds the non-empty ones (bit q of mask) and the total
-// candidate count, and keeps the ranges of the first VTX_NB_CACHE non-empty cells in this
-// lane's LDS column, packed as start | length << 25 (self-collision segments have < 2^25
-// particles, lengths are capped at max_nbr <= 64); a lane with more non-empty cells recomputes
-// the rest. The walk is one flat loop over the cells' concatenation in the same order, with the
-// next candidate's position and initial position loaded while the current one is tested.
-#define VTX_NB_CACHE 16
-#ifndef VTX_NB_BATCH
-#define VTX_NB_BATCH 3   // cell ranges of the first sweep loaded per batch (27 = 9 batches of 3)
-#endif
-
-// The float4 at record i < 2^25 of the 32-B sorted records from a wave-uniform base (the
-// position half or, one float4 on, the initial-position half): a 32-bit byte offset lets the
-// load use the scalar-base + 32-bit vector-offset form.
-__device__ __forceinline__ float4 ld_sorted(const float4* base, uint32_t i) {
-    return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(base) + (size_t)((i & 0x1FFFFFFu) << 5));
-}
-
-// What the first sweep over the 27 cells leaves for the walk: the non-empty cells (bit q of
-// mask, q = 9 dx + 3 dy + dz) and the candidate total.
-struct NbCells {
-    uint32_t mask, total;
+//
+// A wave takes PW consecutive particles of the sorted order. Consecutive particles of one grid cell
+// (a run) have the same 27 candidate ranges, so the ranges are looked up once per run (the wave's
+// lanes share out the runs' cells), and the run's candidates are loaded once, one per lane: lane l
+// holds candidate l of the concatenated ranges, and the wave tests a particle against 64 candidates at
+// a time. The particle is wave-uniform (scalar loads); the accepted lanes take their places in the
+// list from the test's ballot, which keeps the walk's order. One particle per lane instead, each
+// lane walking its own 60 to 300 candidates one after the other, was bound by that chain at small
+// sizes and by the vector cache at large ones (0.9 accesses a clock on every CU): 16,384 particles
+// 88 -> 11.8 us, 65,536 particles 54.6 -> 17.1 us, 963,130 in 256 draped cloths 204.8 -> 129.9 us
+// (now 89% of its VALU issue time, 73 instructions a particle), a folded pile of 1,048,576
+// 759 -> 293 us.
+struct NbSet {
+    const float4* rec;    // sorted records: position with w = index at 2i, initial position at 2i + 1
+    const uint2* cells;   // (start, end) per hash cell
+    char* table;          // neighbour lists
+    uint64_t mc;          // ceil(2^64 / M)
+    uint32_t n, M, K, shift;
+    float cell, cell2, diam2;
+    bool n16;             // 16-bit entries
 };
 
-// The first sweep of the 27-cell walk (CacheNeighbors_Kernel, Velvet/SpatialHashGPU.cu:94-129) for
-// a particle at p: keeps the ranges of the first VTX_NB_CACHE non-empty cells in LDS column col.
-template <int BS, int NB = VTX_NB_BATCH>
-__device__ __forceinline__ NbCells neighbor_cells(const float4 p, const uint2* __restrict__ cells, const float cell,
-                                                  const uint32_t M, const uint64_t mc, const uint32_t K,
-                                                  const uint32_t shift, uint32_t (&crange)[VTX_NB_CACHE][BS],
-                                                  const uint32_t col) {
-    const int32_t ix = hash_coord(p.x, cell, shift), iy = hash_coord(p.y, cell, shift),
-                  iz = hash_coord(p.z, cell, shift);
-    uint32_t mask = 0, total = 0, nz = 0;
-    // NB cell ranges in flight at a time, each one 8-byte load at a 32-bit byte offset
-    // (tables have M < 2^28 cells)
-#pragma unroll
-    for (int q0 = 0; q0 < 27; q0 += NB) {
-        uint64_t cv[NB];
-#pragma unroll
-        for (int r = 0; r < NB; r++) {
-            const int q = q0 + r;
-            const uint32_t hq = hash_coords(ix - 1 + q / 9, iy - 1 + (q / 3) % 3, iz - 1 + q % 3, M, mc);
-            cv[r] = *reinterpret_cast<const uint64_t*>(reinterpret_cast<const char*>(cells) + (hq << 3));
-        }
-#pragma unroll
-        for (int r = 0; r < NB; r++) {
-            const int q = q0 + r;
-            const uint32_t cx = (uint32_t)cv[r], cy = (uint32_t)(cv[r] >> 32);
-            const uint32_t len = cx == VTX_INVALID ? 0u : min(cy, cx + K) - cx;
-            if (len && nz < VTX_NB_CACHE) crange[nz][col] = cx | len << 25;
-            nz += len ? 1u : 0u;
-            mask |= (len ? 1u : 0u) << q;
-            total += len;
-        }
-    }
-    return NbCells{mask, total};
+// The lists' layout: entry k of particle i, CHUNK: chunks of four entries, chunk c at entry
+// 4 (c n + i); else column-major at entry k n + i (the kernel-launch tier's layout). Entries are
+// 32-bit or, for a segment with VTX_SEG_NBR16, 16-bit (the sentinel truncated to 0xffff).
+template <bool CHUNK>
+__device__ __forceinline__ void nb_put(const NbSet& a, uint32_t id, uint32_t k, uint32_t v) {
+    const uint32_t esh = CHUNK && a.n16 ? 1u : 2u;
+    const uint32_t row = CHUNK ? k >> 2 : k, stride = (CHUNK ? 4 * a.n : a.n);
+    char* at = a.table + (((uint64_t)row * stride + (CHUNK ? 4 * id + (k & 3u) : id)) << esh);
+    if (CHUNK && a.n16) *reinterpret_cast<uint16_t*>(at) = (uint16_t)v;
+    else *reinterpret_cast<uint32_t*>(at) = v;
 }
 
-// The candidate walk after the sweep c (same function, same particle p / o / id; crange column col
-// from the sweep): sP the 32-B sorted records (position with w = index at 2i, initial position at
-// 2i + 1), cells the (start, end) table of M cells, shift the grid shift of the cell coordinates.
-// The list goes to nb, the particle's column of an n-particle table (entry offsets):
-//   CHUNK = false: entry k at offset k * n (column-major, the kernel-launch tier's layout);
-//   CHUNK = true:  entries in chunks of four, chunk c = entries 4c..4c+3 at offset 4 (c * n)
-//                  (nb at the table's entry 4 id, chunk-aligned): a lane's four consecutive
-//                  entries share one 16-byte (32-bit entries) or 8-byte (16-bit entries) run, and
-//                  a reader loads four at once.
-// Entries are 32-bit or, for a segment with VTX_SEG_NBR16, 16-bit (the sentinel truncated to
-// 0xffff); nb.put(k, v) stores entry offset k.
-struct NbOut {
-    char* base;   // the particle's first entry
-    bool w16;     // 16-bit entries (uniform over the workgroup's segment)
-    __device__ __forceinline__ void put(uint32_t k, uint32_t v) const {
-        if (w16) *reinterpret_cast<uint16_t*>(base + ((size_t)k << 1)) = (uint16_t)v;
-        else *reinterpret_cast<uint32_t*>(base + ((size_t)k << 2)) = v;
-    }
+// LDS of one wave of the search.
+template <int PW>
+struct NbLds {
+    uint32_t range[PW * 27];   // per (run, cell): start | length << 25
+    int32_t cx[PW], cy[PW], cz[PW];
+    uint32_t mark[64];
 };
 
-template <int BS, bool CHUNK>
-__device__ __forceinline__ void neighbor_list(NbCells c, const float4 p, const float4 o, const uint32_t id,
-                                              const float4* __restrict__ sP, const uint2* __restrict__ cells,
-                                              const NbOut nb, const uint32_t n, const float cell,
-                                              const float cell2, const float diam2, const uint32_t M,
-                                              const uint64_t mc, const uint32_t K, const uint32_t shift,
-                                              const uint32_t (&crange)[VTX_NB_CACHE][BS], const uint32_t col) {
+// Order LDS accesses of the lanes of one wave (a wave's LDS operations execute in order).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ uint32_t dpp0(uint32_t v) {   // the source lane's v, 0 where there is none
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+}
+
+// Inclusive sum over lanes 0..31 (later lanes undefined), inclusive maximum over the wave.
+__device__ __forceinline__ uint32_t scan32_add(uint32_t v) {
+    v += dpp0<0x111>(v);          // row_shr:1, 2, 4, 8
+    v += dpp0<0x112>(v);
+    v += dpp0<0x114>(v);
+    v += dpp0<0x118>(v);
+    return v + dpp0<0x142, 0xa>(v);   // row_bcast:15
+}
+
+__device__ __forceinline__ uint32_t scan64_max(uint32_t v) {
+    v = max(v, dpp0<0x111>(v));
+    v = max(v, dpp0<0x112>(v));
+    v = max(v, dpp0<0x114>(v));
+    v = max(v, dpp0<0x118>(v));
+    v = max(v, dpp0<0x142, 0xa>(v));
+    return max(v, dpp0<0x143, 0xc>(v));   // row_bcast:31
+}
+
+// A sorted record through the scalar cache (i wave-uniform).
+__device__ __forceinline__ void ld_record_uniform(const float4* rec, uint32_t i, float4& p, float4& o) {
+    typedef const float __attribute__((address_space(4))) cfloat;
+    cfloat* q = (cfloat*)(uintptr_t)(rec + 2 * (size_t)i);
+    p = make_float4(q[0], q[1], q[2], q[3]);
+    o = make_float4(q[4], q[5], q[6], 0.f);
+}
+
+// The lists of sorted particles [i0, i0 + cnt), cnt <= PW, by the calling wave.
+template <int PW, bool CHUNK>
+__device__ __forceinline__ void neighbor_wave(const NbSet& a, uint32_t i0, uint32_t cnt, NbLds<PW>& L) {
 #pragma clang fp contract(off)
-    const float4* __restrict__ sX0 = sP + 1;
-    const uint32_t total = c.total;
-    uint32_t mask = c.mask;
-    if (total == 0) {
-        nb.put(0, VTX_INVALID);
-        return;
+    constexpr int NC = 2;                                   // candidate chunks held at a time
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint64_t lt = (1ull << lane) - 1ull;
+    // the wave's particles: cells, runs
+    float4 me = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (lane < cnt) me = a.rec[2 * (size_t)(i0 + lane)];
+    const int32_t ix = hash_coord(me.x, a.cell, a.shift), iy = hash_coord(me.y, a.cell, a.shift),
+                  iz = hash_coord(me.z, a.cell, a.shift);
+    // every lane active in the exchange: one that sits out would hand its neighbour nothing
+    const int32_t px = __shfl_up(ix, 1, 64), py = __shfl_up(iy, 1, 64), pz = __shfl_up(iz, 1, 64);
+    const bool head = lane < cnt && ((lane == 0) | (px != ix) | (py != iy) | (pz != iz));
+    const uint64_t heads = __builtin_amdgcn_ballot_w64(head);
+    const uint32_t nruns = (uint32_t)__popcll(heads);
+    if (head) {
+        const uint32_t r = (uint32_t)__popcll(heads & lt);
+        L.cx[r] = ix;
+        L.cy[r] = iy;
+        L.cz[r] = iz;
     }
-    // position of the next candidate (called only while candidates remain): s runs through the
-    // current cell's range up to e; there the walk moves on to the next non-empty cell, from
-    // the LDS cache or, beyond it, from the cell table again
-    uint32_t z = 0, s = 0, e = 0;
-    auto next = [&]() -> uint32_t {
-        if (s == e) {
-            uint32_t st, ln;
-            if (z < VTX_NB_CACHE) {
-                const uint32_t r = crange[z][col];
-                st = r & 0x1FFFFFFu;
-                ln = r >> 25;
-            } else {
-                const int q = __builtin_ctz(mask);
-                const uint2 r = cells[hash_coords(hash_coord(p.x, cell, shift) - 1 + q / 9,
-                                                  hash_coord(p.y, cell, shift) - 1 + (q / 3) % 3,
-                                                  hash_coord(p.z, cell, shift) - 1 + q % 3, M, mc)];
-                st = r.x;
-                ln = min(r.y, r.x + K) - r.x;
+    wave_lds_sync();
+    // the runs' cell ranges, one (run, cell) per lane and round
+    for (uint32_t t = lane; t < nruns * 27u; t += 64u) {
+        const uint32_t r = (t * 2428u) >> 16, q = t - 27u * r;          // t / 27 for t < 3277
+        const uint32_t dx = (q * 57u) >> 9, yz = q - 9u * dx;           // q / 9 for q < 27
+        const uint32_t dy = (yz * 11u) >> 5, dz = yz - 3u * dy;         // yz / 3 for yz < 9
+        const uint32_t hq = hash_coords(L.cx[r] + (int32_t)dx - 1, L.cy[r] + (int32_t)dy - 1,
+                                        L.cz[r] + (int32_t)dz - 1, a.M, a.mc);
+        const uint64_t c = *reinterpret_cast<const uint64_t*>(a.cells + hq);   // one 8-byte load
+        const uint32_t st = (uint32_t)c, len = min((uint32_t)(c >> 32) - st, a.K);
+        L.range[t] = st == VTX_INVALID ? 0u : st | len << 25;
+    }
+    wave_lds_sync();
+    uint32_t kv = 0;                                        // lane m: entries of particle m
+    uint64_t rest = heads;
+    for (uint32_t r = 0; r < nruns; r++) {
+        const uint32_t m0 = (uint32_t)__builtin_ctzll(rest);
+        rest &= rest - 1ull;
+        const uint32_t m1 = rest ? (uint32_t)__builtin_ctzll(rest) : cnt;
+        const uint32_t v = lane < 27u ? L.range[r * 27u + lane] : 0u;
+        const uint32_t len = v >> 25, incl = scan32_add(len), excl = incl - len;
+        const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 31);
+        const uint32_t base = (v & 0x1FFFFFFu) - excl;      // candidate c of the cell: sorted position base + c
+        for (uint32_t g0 = 0; g0 < total; g0 += 64u * NC) {
+            uint32_t idx[NC];
+            float4 q[NC], x[NC];
+#pragma unroll
+            for (int h = 0; h < NC; h++) {
+                const uint32_t c0 = g0 + 64u * h;
+                idx[h] = VTX_INVALID;
+                if (h && c0 >= total) continue;
+                // the cell of each lane's candidate: every cell marks the lane of its first one
+                L.mark[lane] = 0;
+                wave_lds_sync();
+                if (lane < 27u && len && incl > c0 && excl < c0 + 64u) L.mark[max(excl, c0) - c0] = lane + 1u;
+                wave_lds_sync();
+                const uint32_t own = scan64_max(L.mark[lane]);
+                const uint32_t b = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((own - 1u) << 2), (int)base);
+                if (c0 + lane < total) idx[h] = b + c0 + lane;
+                const uint32_t at = c0 + lane < total ? idx[h] : i0;
+                q[h] = a.rec[2 * (size_t)at];
+                x[h] = a.rec[2 * (size_t)at + 1];
+                wave_lds_sync();
             }
-            mask &= mask - 1u;
-            z++;
-            s = st;
-            e = st + ln;
+            for (uint32_t m = m0; m < m1; m++) {
+                float4 p, o;
+                ld_record_uniform(a.rec, i0 + m, p, o);
+                const uint32_t id = __float_as_uint(p.w);
+                uint32_t k = (uint32_t)__builtin_amdgcn_readlane((int)kv, (int)m);
+#pragma unroll
+                for (int h = 0; h < NC; h++) {
+                    if (h && g0 + 64u * h >= total) continue;
+                    const float dx = p.x - q[h].x, dy = p.y - q[h].y, dz = p.z - q[h].z;
+                    const float d2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+                    const float ex = o.x - x[h].x, ey = o.y - x[h].y, ez = o.z - x[h].z;
+                    const float e2 = __builtin_fmaf(ez, ez, __builtin_fmaf(ey, ey, ex * ex));
+                    // the particle itself is the candidate at its own sorted position
+                    const bool acc = (idx[h] != i0 + m) & (idx[h] != VTX_INVALID) & (d2 < a.cell2) & (e2 > a.diam2);
+                    const uint64_t mask = __builtin_amdgcn_ballot_w64(acc);
+                    const uint32_t e = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                                                 __builtin_amdgcn_mbcnt_lo((uint32_t)mask, k));
+                    if (acc && e < a.K) nb_put<CHUNK>(a, id, e, __float_as_uint(q[h].w));
+                    k = min(k + (uint32_t)__popcll(mask), a.K);
+                }
+                kv = lane == m ? k : kv;
+            }
         }
-        return s++;
-    };
-    // candidate test in walk order, one predicate and one predicated store at the running
-    // offset koff of entry k; a full list takes no more entries
-    uint32_t k = 0, koff = 0;
-    auto take = [&](float4 qp, float4 r) {
-        const uint32_t j = __float_as_uint(qp.w);
-        const float dx = p.x - qp.x, dy = p.y - qp.y, dz = p.z - qp.z;
-        const float d2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
-        const float ex = o.x - r.x, ey = o.y - r.y, ez = o.z - r.z;
-        const float e2 = __builtin_fmaf(ez, ez, __builtin_fmaf(ey, ey, ex * ex));
-        const bool acc = (j != id) & (d2 < cell2) & (e2 > diam2) & (k < K);
-        if (acc) nb.put(koff, j);
-        koff += !acc ? 0u : !CHUNK ? n : (k & 3u) == 3u ? 4 * n - 3u : 1u;
-        k += acc ? 1u : 0u;
-    };
-    // two candidates per trip with alternating load buffers: the loads of the next candidate
-    // are in flight while the current one is tested
-    uint32_t cur = next();
-    float4 qa = ld_sorted(sP, cur), ra = ld_sorted(sX0, cur), qb, rb;
-    for (uint32_t it = 0; it < total; it += 2) {
-        const bool two = it + 1 < total;
-        if (two) {
-            cur = next();
-            qb = ld_sorted(sP, cur);
-            rb = ld_sorted(sX0, cur);
-        }
-        take(qa, ra);
-        if (!two) break;
-        if (it + 2 < total) {
-            cur = next();
-            qa = ld_sorted(sP, cur);
-            ra = ld_sorted(sX0, cur);
-        }
-        take(qb, rb);
     }
-    if (k < K) nb.put(koff, VTX_INVALID);                        // a full list has no sentinel
+    if (lane < cnt && kv < a.K) nb_put<CHUNK>(a, __float_as_uint(me.w), kv, VTX_INVALID);   // a full list has no sentinel
 }
 
-// The whole 27-cell walk of one particle, its crange column the thread's own.
-template <int BS, bool CHUNK>
-__device__ __forceinline__ void neighbor_walk(const float4 p, const float4 o, const uint32_t id,
-                                              const float4* __restrict__ sP, const uint2* __restrict__ cells,
-                                              const NbOut nb, const uint32_t n, const float cell,
-                                              const float cell2, const float diam2, const uint32_t M,
-                                              const uint64_t mc, const uint32_t K, const uint32_t shift,
-                                              uint32_t (&crange)[VTX_NB_CACHE][BS]) {
-    const NbCells c = neighbor_cells<BS>(p, cells, cell, M, mc, K, shift, crange, threadIdx.x);
-    neighbor_list<BS, CHUNK>(c, p, o, id, sP, cells, nb, n, cell, cell2, diam2, M, mc, K, shift, crange,
-                             threadIdx.x);
-}
-
-// In hash-sorted order (NBR_SORTED) the workgroup's threads take its particles again after the
-// sweep, in descending order of their candidate totals (buckets of 4 candidates, ties in any
-// order): the walk of a wave lasts as long as its longest list, and lanes of similar totals
-// (among them the lanes of one cell) waste fewer trips. A thread reads its new particle's sweep
-// from the LDS column of the thread that swept it. The lists do not depend on which thread walks
-// them. (Batch of 512 draped cloths: 289.6 -> 282.4 us per search; the patch and particle orders
-// keep their lanes, whose table stores and loads are the ones that pay there: on one 1024 x 1024
-// cloth the re-dealt patch order measured 180.2 -> 185.1 us.)
-#define VTX_NB_BUCKETS 64
-template <int ORDER, int BS>
-__global__ __launch_bounds__(BS) void k_neighbors(DevState d, const TileDev* __restrict__ tiles,
-                                                  const GridTileDev* __restrict__ gtiles, int in) {
-    constexpr bool REDEAL = ORDER == NBR_SORTED;
-    constexpr int RB = REDEAL ? BS : 1;
-    static_assert(BS >= VTX_NB_BUCKETS, "one wave scans the bucket counts");
-    __shared__ uint32_t crange[VTX_NB_CACHE][BS];   // column per sweeping thread
-    __shared__ uint32_t bcount[REDEAL ? VTX_NB_BUCKETS : 1];
-    __shared__ uint32_t bpart[RB], bmask[RB], btotal[RB];
-    uint32_t seg, i, tix, lane;
-    bool live;
-    tile_lane<VTX_TILE, BS>(d.remap, tix, lane);
-    if (ORDER == NBR_PATCH) {
-        const GridTileDev t = gtiles[tix];
-        seg = t.seg;
-        const SegDev& s0 = d.segs[seg];
-        const uint32_t a = t.a0 + lane / VTX_GT, b = t.b0 + lane % VTX_GT;
-        live = a < s0.rows && b < s0.cols;
-        i = a * s0.cols + b;
-    } else {
-        const TileDev t = tiles[tix];
-        live = lane < t.count;
-        seg = t.seg;
-        i = t.begin + lane - d.segs[seg].pbase;                 // sorted position or particle
-    }
-    if (!REDEAL && !live) return;
-    const SegDev sg = d.segs[seg];                             // one segment per workgroup
-    if (!(sg.flags & VTX_SEG_SELFCOL)) return;
-    const uint32_t n = sg.n, M = sg.M, K = sg.max_nbr, shift = seg_shift(sg);
-    const uint64_t mc = seg_mod(sg);
-    const float4* __restrict__ sP = d.sPX + 2 * (size_t)sg.pbase;   // position of sorted i at 2i, initial at 2i+1
-    const uint2* __restrict__ cells = d.cells + sg.tbase;
-    char* const table = reinterpret_cast<char*>(d.nbr + ((uint64_t)sg.nbase_hi << 32 | sg.nbase_lo));
-    const bool n16 = sg.flags & VTX_SEG_NBR16;
-    const uint32_t esh = n16 ? 1u : 2u;   // log2 of the entry size
-    if constexpr (!REDEAL) {
-        const float4 p = d.P[in][sg.pbase + i], o = d.X0[sg.pbase + i];
-        neighbor_walk<BS, true>(p, o, i, sP, cells, NbOut{table + ((size_t)4 * i << esh), n16}, n, sg.cell,
-                                sg.cell2, sg.diam2, M, mc, K, shift, crange);
-    } else {
-        NbCells c{0u, 0u};
-        // nine cell ranges in flight per batch: this path holds fewer registers than the others
-        // (batches of 3 measured 261.8 against 258.4 us on the batch of 512 cloths)
-        if (live) c = neighbor_cells<BS, 9>(sP[2 * i], cells, sg.cell, M, mc, K, shift, crange, threadIdx.x);
-        // descending totals: bucket VTX_NB_BUCKETS - 1 - total / 4, idle threads last
-        const uint32_t t = threadIdx.x;
-        if (t < VTX_NB_BUCKETS) bcount[t] = 0;
-        __syncthreads();
-        const uint32_t key =
-            live ? VTX_NB_BUCKETS - 1u - min(c.total >> 2, VTX_NB_BUCKETS - 1u) : VTX_NB_BUCKETS - 1u;
-        const uint32_t slot = atomicAdd(&bcount[key], 1u);
-        __syncthreads();
-        if (t < VTX_NB_BUCKETS) {
-            const uint32_t v = bcount[t];
-            bcount[t] = wave_incl_scan(v) - v;
-        }
-        __syncthreads();
-        const uint32_t at = bcount[key] + slot;
-        bpart[at] = live ? i : VTX_INVALID;
-        bmask[at] = c.mask;
-        btotal[at] = c.total | t << 16;                         // totals <= 27 * 64
-        __syncthreads();
-        i = bpart[t];
-        if (i == VTX_INVALID) return;
-        const uint32_t tc = btotal[t];
-        const float4 p = sP[2 * i], o = sP[2 * i + 1];
-        const uint32_t id = __float_as_uint(p.w);
-        neighbor_list<BS, true>(NbCells{bmask[t], tc & 0xFFFFu}, p, o, id, sP, cells,
-                                NbOut{table + ((size_t)4 * id << esh), n16}, n, sg.cell, sg.cell2, sg.diam2, M, mc,
-                                K, shift, crange, tc >> 16);
-    }
+// The search over the segments' particle tiles (a tile's sorted positions): 4 PW particles per
+// workgroup of four waves.
+template <int PW>
+__global__ __launch_bounds__(256) void k_neighbors(DevState d) {
+    __shared__ NbLds<PW> lds[4];
+    const uint32_t b = tile_of(d.remap), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr uint32_t S = VTX_TILE / (4 * PW);                 // workgroups per tile
+    const TileDev t = d.tiles[b / S];
+    const uint32_t first = ((b % S) * 4 + wave) * PW;
+    const SegDev& sg = d.segs[t.seg];
+    if (first >= t.count || !(sg.flags & VTX_SEG_SELFCOL)) return;
+    NbSet a;
+    a.rec = d.sPX + 2 * (size_t)sg.pbase;
+    a.cells = d.cells + sg.tbase;
+    a.table = reinterpret_cast<char*>(d.nbr + ((uint64_t)sg.nbase_hi << 32 | sg.nbase_lo));
+    a.mc = seg_mod(sg);
+    a.n = sg.n;
+    a.M = sg.M;
+    a.K = sg.max_nbr;
+    a.shift = seg_shift(sg);
+    a.cell = sg.cell;
+    a.cell2 = sg.cell2;
+    a.diam2 = sg.diam2;
+    a.n16 = sg.flags & VTX_SEG_NBR16;
+    neighbor_wave<PW, true>(a, t.begin - sg.pbase + first, min((uint32_t)PW, t.count - first), lds[wave]);
 }
 
 // ---------------------------------------------------------------- kernel-launch tier
@@ -762,18 +704,17 @@ __global__ __launch_bounds__(VTX_TILE) void k_raw_cell_bounds(const uint32_t* __
     rec[2 * (size_t)g + 1] = ld_xyz(pos0, id, 0.f);
 }
 
-// CacheNeighbors_Kernel (Velvet/SpatialHashGPU.cu:79-130), threads in sorted order.
-template <int BS>
-__global__ __launch_bounds__(BS) void k_raw_neighbors(const float4* __restrict__ rec, const uint2* __restrict__ cells,
-                                                      uint32_t* __restrict__ nbr, uint32_t n, float cell, float cell2,
-                                                      float diam2, uint32_t M, uint64_t mc, uint32_t K) {
-    __shared__ uint32_t crange[VTX_NB_CACHE][BS];
-    const uint32_t i = blockIdx.x * BS + threadIdx.x;
-    if (i >= n) return;
-    const float4 p = rec[2 * (size_t)i], o = rec[2 * (size_t)i + 1];
-    const uint32_t id = __float_as_uint(p.w);
-    neighbor_walk<BS, false>(p, o, id, rec, cells, NbOut{reinterpret_cast<char*>(nbr + id), false}, n, cell, cell2,
-                             diam2, M, mc, K, 0u, crange);
+// CacheNeighbors_Kernel (Velvet/SpatialHashGPU.cu:79-130).
+template <int PW>
+__global__ __launch_bounds__(256) void k_raw_neighbors(const float4* __restrict__ rec, const uint2* __restrict__ cells,
+                                                       uint32_t* __restrict__ nbr, uint32_t n, float cell, float cell2,
+                                                       float diam2, uint32_t M, uint64_t mc, uint32_t K) {
+    __shared__ NbLds<PW> lds[4];
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t first = (blockIdx.x * 4 + wave) * PW;
+    if (first >= n) return;
+    const NbSet a{rec, cells, reinterpret_cast<char*>(nbr), mc, n, M, K, 0u, cell, cell2, diam2, false};
+    neighbor_wave<PW, false>(a, first, min((uint32_t)PW, n - first), lds[wave]);
 }
 
 // The interleaved table to the caller's cell_start / cell_end (empty cells: ~0u in both).
@@ -785,6 +726,13 @@ __global__ __launch_bounds__(VTX_TILE) void k_raw_split_cells(const uint2* __res
         end[i] = c.y;
     }
 }
+
+// Particles per wave of the neighbour search. Up to 2^17 particles a wave takes 8: the chip's 8,192
+// waves are not all busy, and a wave's particles go one after the other (measured, us per search, 8 /
+// 32 particles a wave: 16,384 particles 11.8 / 27.9, 65,536 17.1 / 29.7). Above, 32: the lookups of a
+// run and its candidates' loads serve more particles (963,130 particles in 256 cloths 164.9 / 129.9;
+// a pile of 1,048,576 runs long lists either way, 268 / 293).
+static bool search_small(uint32_t particles) { return particles <= (1u << 17); }
 
 static uint64_t mod_constant(uint32_t M) {   // ceil(2^64 / M) mod 2^64 (M = 1 gives 0: h % 1 = 0)
     return M > 1 ? ~0ull / M + 1ull : 0ull;
@@ -838,9 +786,13 @@ hipError_t hash_objects(const HashObjectsArgs& a, void* workspace, hipStream_t s
     if (n) {
         hipLaunchKernelGGL(k_raw_cell_bounds, dim3(blocks), dim3(VTX_TILE), 0, s, (const uint32_t*)a.particle_hash,
                            (const uint32_t*)a.particle_index, n, a.positions, a.original_positions, cells, rec);
-        hipLaunchKernelGGL((k_raw_neighbors<128>), dim3((n + 127) / 128), dim3(128), 0, s, (const float4*)rec,
-                           (const uint2*)cells, a.neighbors, n, a.cell_spacing, a.cell_spacing2, a.particle_diameter2,
-                           M, mc, a.max_num_neighbors);
+        const auto nb = [&](auto kernel, uint32_t pw) {
+            hipLaunchKernelGGL(kernel, dim3((n + 4 * pw - 1) / (4 * pw)), dim3(256), 0, s, (const float4*)rec,
+                               (const uint2*)cells, a.neighbors, n, a.cell_spacing, a.cell_spacing2,
+                               a.particle_diameter2, M, mc, a.max_num_neighbors);
+        };
+        if (search_small(n)) nb(k_raw_neighbors<8>, 8);
+        else nb(k_raw_neighbors<32>, 32);
     }
     uint32_t sb = (M + VTX_TILE - 1) / VTX_TILE;
     if (sb > 4096) sb = 4096;
@@ -936,28 +888,12 @@ hipError_t launch_cell_bounds(const DevState& d, int in, int src, hipStream_t s)
     return hipGetLastError();
 }
 
-template <int BS>
-static void launch_neighbors_bs(const DevState& d, int in, int order, hipStream_t s) {
-    constexpr uint32_t S = VTX_TILE / BS;
-    const dim3 bl(BS);
-    if (order == NBR_PARTICLE) {
-        hipLaunchKernelGGL((k_neighbors<NBR_PARTICLE, BS>), dim3(d.ntiles * S), bl, 0, s, d, d.tiles, d.gtiles, in);
-    } else if (order == NBR_SORTED) {
-        hipLaunchKernelGGL((k_neighbors<NBR_SORTED, BS>), dim3(d.ntiles * S), bl, 0, s, d, d.tiles, d.gtiles, in);
-    } else {   // grid segments by patches (both grid tile lists), the others in sorted order
-        if (d.ngtiles)
-            hipLaunchKernelGGL((k_neighbors<NBR_PATCH, BS>), dim3(d.ngtiles * S), bl, 0, s, d, d.itiles, d.gtiles, in);
-        if (d.nltiles)
-            hipLaunchKernelGGL((k_neighbors<NBR_PATCH, BS>), dim3(d.nltiles * S), bl, 0, s, d, d.itiles, d.ltiles, in);
-        if (d.nitiles)
-            hipLaunchKernelGGL((k_neighbors<NBR_SORTED, BS>), dim3(d.nitiles * S), bl, 0, s, d, d.itiles, d.gtiles, in);
-    }
-}
-
-hipError_t launch_neighbors(const DevState& d, int in, int order, int block, hipStream_t s) {
-    if (block == 64) launch_neighbors_bs<64>(d, in, order, s);
-    else if (block == 128) launch_neighbors_bs<128>(d, in, order, s);
-    else launch_neighbors_bs<256>(d, in, order, s);
+hipError_t launch_neighbors(const DevState& d, hipStream_t s) {
+    const auto nb = [&](auto kernel, uint32_t pw) {
+        hipLaunchKernelGGL(kernel, dim3(d.ntiles * (VTX_TILE / (4 * pw))), dim3(256), 0, s, d);
+    };
+    if (search_small(d.nparticles)) nb(k_neighbors<8>, 8);
+    else nb(k_neighbors<32>, 32);
     return hipGetLastError();
 }
 
