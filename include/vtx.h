@@ -316,8 +316,9 @@ int vtx_hash_objects_noalloc(uint32_t* particle_hash, uint32_t* particle_index, 
 /* Per-stage GPU time under the reference's ScopedTimerGPU labels (Velvet/Timer.hpp:242-260,
  * Velvet/GUI.cpp:32-51). With timing on, frames are launched without the graph and every launch
  * group is bracketed by a HIP event pair on the solver's stream; vtx_read_timing returns JSON
- * {label: {"ms": total, "launches": count, "kernel": name}} accumulated since timing was switched
- * on, plus "total". A label is the reference's stage label ("Solver_HashCache", ...), or several
+ * {label: {"ms": total, "launches": count, "passes": count, "kernel": name}} accumulated since
+ * timing was switched on, plus "total". "passes" counts the Jacobi passes of the launches (a small
+ * cloth runs several per launch; equal to "launches" for other stages). A label is the reference's stage label ("Solver_HashCache", ...), or several
  * joined by '+' where one kernel runs those stages fused ("Solver_CollideParticles+
  * Solver_ApplyDeltas+Solver_CollideSDFs" for k_collide); "kernel" names the kernel(s). */
 int vtx_set_timing(vtx_solver* s, int32_t on);

@@ -1179,13 +1179,38 @@ static uint32_t ceil_log2(uint32_t v) {
     return b;
 }
 
+// Whether a segment's Jacobi passes can run fused (k_iterate_fused): a grid cloth whose attachments are
+// none, or dense ones of at most VTX_LRA_PARTS slots.
+static bool fusable(const Segment& sg) {
+    return sg.prep.grid && (sg.at_pid.empty() || (sg.prep.lra_dense && sg.slots.size() / 3 <= VTX_LRA_PARTS));
+}
+
+// Tile side of the fused passes for the live set, 0: one pass per launch. Small tiles share a small
+// cloth's work among more CUs but work more of the halo out again, so the side grows with the live set
+// until the tiles of 16 take three quarters of the 256 CUs; beyond, one pass per launch fills the chip.
+// Measured, us per frame of 4 substeps x 10 passes, one pass per launch / side 8 / 12 / 16: 40 x 40 335 /
+// 115 / 134 / 163; 128 x 128 333 / 119 / 139 / 165, and with three solvers' frames overlapping 119 / 94 /
+// 60 / 59; 200 x 200 339 / 296 / 243 / 170, overlapping 123 / 223 / 127 / 98; 256 x 256 338 / 386 / 247 /
+// 172, but overlapping 124 / 358 / 208 / 142; 300 x 300 367 / 564 / 353 / 302, overlapping 142 / - / - / 198.
+uint32_t Engine::fuse_side() const {
+    uint64_t n8 = 0, n12 = 0, n16 = 0;
+    for (auto& sp : segs_)
+        if (sp && sp->active && sp->uploaded && sp->n() && fusable(*sp)) {
+            const uint64_t r = sp->dev.rows, c = sp->dev.cols;
+            n8 += ((r + 7) / 8) * ((c + 7) / 8);
+            n12 += ((r + 11) / 12) * ((c + 11) / 12);
+            n16 += ((r + 15) / 16) * ((c + 15) / 16);
+        }
+    return n8 <= 128 ? 8u : n12 <= 256 ? 12u : n16 <= 196 ? 16u : 0u;
+}
+
 // Segment, tile and sort tables of the active segments.
 void Engine::rebuild_tables() {
     sync_stream();
     invalidate_graph();
     std::vector<SegDev> hseg;
     std::vector<TileDev> htile, hitile;
-    std::vector<GridTileDev> hgtile, hltile;
+    std::vector<GridTileDev> hgtile, hltile, hftile, hmtile;
     std::vector<uint32_t> hsmall;                // table indices of segments hashed in LDS
     std::vector<SortTileDev> hst;
     table_seg_.clear();
@@ -1210,7 +1235,8 @@ void Engine::rebuild_tables() {
     // G groups of about total/G particles each (a prefix of the segment table per group); timing
     // mode keeps one group so that per-launch figures cover the whole workload
     const uint32_t G = timing_ ? 1u : std::max(1u, std::min<uint32_t>((uint32_t)tun_.streams, nlive));
-    struct Cut { size_t t, i, g, l, s, m; uint32_t h, p; };
+    const uint32_t fside = fuse_side();
+    struct Cut { size_t t, i, g, l, s, m, f, n; uint32_t h, p; };
     std::vector<Cut> cuts;                     // where groups 1..G-1 begin
     uint64_t cum = 0;
     for (size_t si = 0; si < segs_.size(); si++) {
@@ -1228,7 +1254,7 @@ void Engine::rebuild_tables() {
                     VTX_EINVAL, "active segments of one solver must share substeps, iterations and interleave");
         if (cuts.size() + 1 < G && cum > 0 && cum * G >= total_n * (cuts.size() + 1)) {
             cuts.push_back(Cut{htile.size(), hitile.size(), hgtile.size(), hltile.size(), hst.size(), hsmall.size(),
-                               hbase, (uint32_t)cum});
+                               hftile.size(), hmtile.size(), hbase, (uint32_t)cum});
             compact = 0;                       // each group sorts on its own
         }
         cum += sg.n();
@@ -1271,11 +1297,20 @@ void Engine::rebuild_tables() {
             htile.push_back(t);
             if (!sg.prep.grid) hitile.push_back(t);
         }
+        const bool fused = fside && fusable(sg);
         for (GridTileDev gt : sg.prep.gtiles) {
             gt.seg = ti;
             gt.at_off += (uint32_t)sg.rg.at;
-            (lsplit && tun_.lra_split ? hltile : hgtile).push_back(gt);
+            (fused ? hmtile : lsplit && tun_.lra_split ? hltile : hgtile).push_back(gt);
         }
+        for (uint32_t a = 0; fused && a < d.rows; a += fside)
+            for (uint32_t b = 0; b < d.cols; b += fside) {
+                GridTileDev ft{};
+                ft.seg = ti;
+                ft.a0 = a;
+                ft.b0 = b;
+                hftile.push_back(ft);
+            }
         const uint32_t nst = in_lds ? 0u : (d.n + VTX_SORT_TILE - 1) / VTX_SORT_TILE;
         for (uint32_t k = 0; k < nst; k++) {
             SortTileDev st{};
@@ -1317,6 +1352,9 @@ void Engine::rebuild_tables() {
     d.ngtiles = (uint32_t)hgtile.size();
     d.nltiles = (uint32_t)hltile.size();
     d.nhsegs = (uint32_t)hsmall.size();
+    d.nftiles = (uint32_t)hftile.size();
+    d.nmtiles = (uint32_t)hmtile.size();
+    d.fside = fside;
     d.nstiles = (uint32_t)hst.size();
     d.nhist = hbase;
     d.ncells = (uint32_t)acell_.cap;
@@ -1330,7 +1368,8 @@ void Engine::rebuild_tables() {
     }
     TableSet ts;
     const size_t k_seg = ts.add(hseg), k_tile = ts.add(htile), k_itile = ts.add(hitile), k_gtile = ts.add(hgtile),
-                 k_ltile = ts.add(hltile), k_st = ts.add(hst), k_hs = ts.add(hsmall);
+                 k_ltile = ts.add(hltile), k_st = ts.add(hst), k_hs = ts.add(hsmall),
+                 k_ft = ts.add(hftile), k_mt = ts.add(hmtile);
     upload_tables(ts);
     d.segs = (const SegDev*)(tab_dev_ + ts.off[k_seg]);
     d.tiles = (const TileDev*)(tab_dev_ + ts.off[k_tile]);
@@ -1339,6 +1378,8 @@ void Engine::rebuild_tables() {
     d.ltiles = (const GridTileDev*)(tab_dev_ + ts.off[k_ltile]);
     d.stiles = (const SortTileDev*)(tab_dev_ + ts.off[k_st]);
     d.hsegs = (const uint32_t*)(tab_dev_ + ts.off[k_hs]);
+    d.ftiles = (const GridTileDev*)(tab_dev_ + ts.off[k_ft]);
+    d.mtiles = (const GridTileDev*)(tab_dev_ + ts.off[k_mt]);
     d.X = pl_.X;
     d.V = pl_.V;
     d.P[0] = pl_.P0;
@@ -1371,9 +1412,9 @@ void Engine::rebuild_tables() {
     d.hbase0 = 0;
     ds_ = d;
     groups_.clear();
-    cuts.push_back(Cut{htile.size(), hitile.size(), hgtile.size(), hltile.size(), hst.size(), hsmall.size(), hbase,
-                       d.nparticles});
-    Cut lo{0, 0, 0, 0, 0, 0, 0, 0};
+    cuts.push_back(Cut{htile.size(), hitile.size(), hgtile.size(), hltile.size(), hst.size(), hsmall.size(),
+                       hftile.size(), hmtile.size(), hbase, d.nparticles});
+    Cut lo{};
     for (size_t k = 0; k < cuts.size(); k++) {
         const Cut& hi = cuts[k];
         DevState g = d;
@@ -1384,6 +1425,10 @@ void Engine::rebuild_tables() {
         g.stiles = d.stiles + lo.s;
         g.hsegs = d.hsegs + lo.m;
         g.nhsegs = (uint32_t)(hi.m - lo.m);
+        g.ftiles = d.ftiles + lo.f;
+        g.mtiles = d.mtiles + lo.n;
+        g.nftiles = (uint32_t)(hi.f - lo.f);
+        g.nmtiles = (uint32_t)(hi.n - lo.n);
         g.ntiles = (uint32_t)(hi.t - lo.t);
         g.nitiles = (uint32_t)(hi.i - lo.i);
         g.ngtiles = (uint32_t)(hi.g - lo.g);
@@ -1451,7 +1496,7 @@ int32_t Engine::stencil_segments() {
 }
 
 // ---------------------------------------------------------------------------- frames
-void Engine::stage_begin(const char* kernel, const char* label, hipStream_t s) {
+void Engine::stage_begin(const char* kernel, const char* label, hipStream_t s, int passes) {
     if (!timing_) return;
     if (stage_used_ == stages_.size()) {
         StageTime st;
@@ -1461,6 +1506,7 @@ void Engine::stage_begin(const char* kernel, const char* label, hipStream_t s) {
     }
     stages_[stage_used_].kernel = kernel;
     stages_[stage_used_].label = label;
+    stages_[stage_used_].passes = passes;
     VTX_HIP(hipEventRecord(stages_[stage_used_].a, s));
 }
 
@@ -1528,21 +1574,36 @@ void Engine::record_group(const DevState& d, float frame_dt, hipStream_t s, hipE
             stage_end(s);
             cur ^= 1;
         }
-        for (int it = 0; it < iterations_; it++) {
-            const int epi = it == iterations_ - 1 ? epi_last : EPILOGUE_NONE;
-            stage_begin("k_iterate",
-                        epi == EPILOGUE_NONE
-                            ? "Solver_SolveStretch+Solver_SolveAttach+Solver_SolveBending+Solver_ApplyDeltas"
-                        : epi == EPILOGUE_FINALIZE
-                            ? "Solver_SolveStretch+Solver_SolveAttach+Solver_SolveBending+Solver_ApplyDeltas+"
-                              "Solver_Finalize"
-                            : "Solver_SolveStretch+Solver_SolveAttach+Solver_SolveBending+Solver_ApplyDeltas+"
-                              "Solver_Finalize+Solver_Predict",
-                        s);
+        static const char* const label[] = {
+            "Solver_SolveStretch+Solver_SolveAttach+Solver_SolveBending+Solver_ApplyDeltas",
+            "Solver_SolveStretch+Solver_SolveAttach+Solver_SolveBending+Solver_ApplyDeltas+Solver_Finalize",
+            "Solver_SolveStretch+Solver_SolveAttach+Solver_SolveBending+Solver_ApplyDeltas+Solver_Finalize+"
+            "Solver_Predict"};
+        const bool single = d.nitiles || d.ngtiles || d.nltiles;   // segments that run one pass per launch
+        int fcur = cur, left = iterations_;
+        if (d.nftiles && iterations_) {
+            const int most = fuse_passes(d.fside);
+            int launches = (iterations_ + most - 1) / most;
+            // every segment leaves the substep in the same ping-pong buffer
+            if (single && (launches ^ iterations_) & 1) launches++;
+            for (; launches > 0; launches--) {
+                const int passes = (left + launches - 1) / launches;
+                left -= passes;
+                const int epi = left ? (int)EPILOGUE_NONE : epi_last;
+                stage_begin("k_iterate", label[epi], s, passes);
+                VTX_HIP(launch_iterate_fused(d, fcur, passes, h, epi, s));
+                stage_end(s);
+                fcur ^= 1;
+            }
+        }
+        for (int it = 0; single && it < iterations_; it++) {
+            const int epi = it == iterations_ - 1 ? epi_last : (int)EPILOGUE_NONE;
+            stage_begin("k_iterate", label[epi], s);
             VTX_HIP(launch_iterate(d, cur, h, epi, true, tun_.lra_batch, s));
             stage_end(s);
             cur ^= 1;
         }
+        if (iterations_ && !single) cur = fcur;
     }
     stage_begin("k_normals", "Solver_UpdateNormals", s);
     VTX_HIP(launch_normals(d, s));
@@ -1602,6 +1663,7 @@ void Engine::simulate(float frame_dt) {
             VTX_HIP(hipEventElapsedTime(&ms, stages_[k].a, stages_[k].b));
             timing_ms_[stages_[k].label] += ms;
             timing_n_[stages_[k].label] += 1;
+            timing_passes_[stages_[k].label] += stages_[k].passes;
             timing_kernel_[stages_[k].label] = stages_[k].kernel;
             timing_ms_["total"] += ms;
             timing_n_["total"] += 1;
@@ -1841,7 +1903,8 @@ std::string Engine::timing_report() {
         o << (first ? "" : ", ") << "\"" << kv.first << "\": {\"ms\": " << kv.second
           << ", \"launches\": " << timing_n_[kv.first];
         auto k = timing_kernel_.find(kv.first);
-        if (k != timing_kernel_.end()) o << ", \"kernel\": \"" << k->second << "\"";
+        if (k != timing_kernel_.end())
+            o << ", \"passes\": " << timing_passes_[kv.first] << ", \"kernel\": \"" << k->second << "\"";
         o << "}";
         first = false;
     }

@@ -154,6 +154,7 @@ struct StageTime {
     const char* kernel;
     const char* label;
     hipEvent_t a, b;
+    int passes;   // Jacobi passes of the launch (1 for other kernels)
 };
 
 // Stretch (every unique edge) and bending (every edge of exactly two triangles, rest angle from
@@ -262,12 +263,13 @@ private:
     bool pools_fit(const Ranges& need);
     void release(Segment& sg);
     void rebuild_tables();
+    uint32_t fuse_side() const;
     void upload_tables(const TableSet& t);
     void grow_pools(const Ranges& need);
     void record_frame(float frame_dt, hipStream_t s, bool lazy);
     void hash_build(const DevState& d, int in, hipStream_t s);
     void record_group(const DevState& d, float frame_dt, hipStream_t s, hipEvent_t after_hash = nullptr);
-    void stage_begin(const char* kernel, const char* label, hipStream_t s);
+    void stage_begin(const char* kernel, const char* label, hipStream_t s, int passes = 1);
     void stage_end(hipStream_t s);
     void check_seg(int32_t s) const;
     void free_tables();
@@ -330,7 +332,7 @@ private:
     std::vector<StageTime> stages_;
     size_t stage_used_ = 0;
     std::map<std::string, double> timing_ms_;
-    std::map<std::string, long> timing_n_;
+    std::map<std::string, long> timing_n_, timing_passes_;
     std::map<std::string, std::string> timing_kernel_;
 };
 

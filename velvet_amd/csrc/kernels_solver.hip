@@ -39,8 +39,8 @@ __device__ __forceinline__ float facos(float x) {
     p = fmaf(p, ax, 0.0889789874f);
     p = fmaf(p, ax, -0.2145988016f);
     p = fmaf(p, ax, 1.5707963050f);
-    const float r = fsqrt(1.0f - ax) * p;
-    return x < 0.f ? 3.14159265358979f - r : r;
+    const float q = fsqrt(1.0f - ax);
+    return x < 0.f ? fmaf(-q, p, 3.14159265358979f) : q * p;
 }
 
 // ComputeFriction (Velvet/VtClothSolverGPU.cu:272-287). tl == 0 gives mt * inf = inf, clamped
@@ -247,10 +247,10 @@ enum { EPI_NONE = 0, EPI_FINALIZE = 1, EPI_FINALIZE_PREDICT = 2 };
 // nws = -w * stiffness, the endpoint's factor of every one of its terms.
 __device__ __forceinline__ void stretch_term(V3 p, float w, float nws, float4 q, float rest, V3& delta, int& cnt) {
     const V3 diff = p - xyz(q);
-    const float dist = fsqrt(dot(diff, diff));
+    const float dist = fsqrt(dot_fma(diff, diff));
     const float wsum = w + q.w;
     if (dist != rest && wsum > 0.f) {
-        delta += ((dist - rest) * nws * frcp(wsum * (dist + VTX_EPSILON))) * diff;
+        delta = madd(delta, diff, (dist - rest) * nws * frcp(wsum * (dist + VTX_EPSILON)));
         cnt++;
     }
 }
@@ -264,7 +264,7 @@ __device__ __forceinline__ void attach_term(V3 p, float w, float4 slot, float di
                                             int& cnt) {
     const float target = dist0 * lrs;
     const V3 diff = p - xyz(slot);
-    const float f = __builtin_fmaf(target, frsq(dot(diff, diff)), -1.0f);
+    const float f = __builtin_fmaf(target, frsq(dot_fma(diff, diff)), -1.0f);
     // the reference returns early for a pinned particle with a positive target
     const bool act = !(w == 0.f && target > 0.f) && f < 0.f;
     const float k = act ? f : 0.f;
@@ -373,34 +373,44 @@ struct BendGrad {
     float k0, k1;
 };
 
+//
+// The multiply-adds are spelled out, so that every kernel that evaluates a constraint rounds it alike
+// (the sign test at the end decides the whole correction of a flat pair, so a last bit can show). The
+// stencil path (GRID) and the general path differ in the order of some sums.
+template <bool GRID>
 __device__ __forceinline__ bool bend_eval(float4 q0, float4 q1, float4 q2, float4 q3, float rest, float xpbd,
                                           float& lam, BendGrad& g) {
+#pragma clang fp contract(off)
+    const auto dot_ge = [](V3 u, V3 v) {
+        return GRID ? dot_fma(u, v) : __builtin_fmaf(u.z, v.z, __builtin_fmaf(u.y, v.y, u.x * v.x));
+    };
     const V3 p0 = xyz(q0), p1 = xyz(q1), p2 = xyz(q2), p3 = xyz(q3);
     const V3 e = p3 - p2;
-    const float ee = dot(e, e);
+    const float ee = dot_fma(e, e);
     if (ee < VTX_EPSILON * VTX_EPSILON) return false;   // |e| < eps
     const float inv_elen = frsq(ee);                      // |e| and 1/|e| from one rsq
     const float elen = ee * inv_elen;
     const V3 a = p2 - p0, b = p3 - p1;
-    g.c1 = cross(a, e);
-    g.c2 = cross(e, b);
-    const float g11 = dot(g.c1, g.c1), g22 = dot(g.c2, g.c2), g12 = dot(g.c1, g.c2);
+    g.c1 = cross_fma(a, e);
+    g.c2 = cross_fma(e, b);
+    const float g11 = dot_fma(g.c1, g.c1), g22 = dot_fma(g.c2, g.c2), g12 = dot_fma(g.c1, g.c2);
     const float r1 = frsq(g11), r2 = frsq(g22);
     const float r1s = r1 * r1, r2s = r2 * r2;
     g.k0 = elen * r1s;
     g.k1 = elen * r2s;
-    const float s1 = ((-dot(a, e) - ee) * inv_elen) * r1s, s2 = (-dot(b, e) * inv_elen) * r2s;
-    g.d2 = s1 * g.c1 + s2 * g.c2;
+    const float s1 = ((-dot_ge(a, e) - ee) * inv_elen) * r1s, s2 = (-dot_ge(b, e) * inv_elen) * r2s;
+    g.d2 = GRID ? madd(s2 * g.c2, g.c1, s1) : madd(s1 * g.c1, g.c2, s2);
     const float cd = fminf(fmaxf(g12 * (r1 * r2), -1.0f), 1.0f);
     const float phi = facos(cd);
     // |d0|^2 = |e|^2 r1^2, |d1|^2 = |e|^2 r2^2, and d3 = t1 c1 + t2 c2 from the Gram entries:
     // |d3|^2 = t1 (t1 g11 + 2 t2 g12) + t2^2 g22
-    const float t1 = -(g.k0 + s1), t2 = -(g.k1 + s2), t2g = t2 * g12;
+    const float t1 = -__builtin_fmaf(elen, r1s, s1), t2 = -__builtin_fmaf(elen, r2s, s2), t2g = t2 * g12;
     const float d3s = __builtin_fmaf(t1, __builtin_fmaf(t1, g11, t2g + t2g), t2 * (t2 * g22));
-    float l = ee * (q0.w * r1s + q1.w * r2s) + q2.w * dot(g.d2, g.d2) + q3.w * d3s;
+    const float w01 = GRID ? __builtin_fmaf(q0.w, r1s, q1.w * r2s) : __builtin_fmaf(q1.w, r2s, q0.w * r1s);
+    float l = __builtin_fmaf(q3.w, d3s, __builtin_fmaf(ee, w01, q2.w * dot_fma(g.d2, g.d2)));
     if (l < VTX_EPSILON) return false;
     l = (phi - rest) * frcp(l + xpbd);
-    if (dot(a, g.c2) > 0.0f) l = -l;      // (n1 x n2).e > 0
+    if (dot_ge(a, g.c2) > 0.0f) l = -l;      // (n1 x n2).e > 0
     lam = l;
     return true;
 }
@@ -416,16 +426,16 @@ __device__ __forceinline__ void epilogue(const DevState& d, const SegDev& sg, ui
         const float4 x4 = d.X[g];
         const V3 x = xyz(x4);
         V3 raw = (p - x) * frcp(h);
-        const float rl = flen(raw);
+        const float rl = fsqrt(dot_fma(raw, raw));
         if (rl > sg.max_speed) {
             raw = raw * (frcp(rl) * sg.max_speed);
-            p = x + raw * h;
+            p = madd(x, raw, h);
         }
-        V3 v = raw * (1.0f - sg.damping * h);
+        V3 v = raw * __builtin_fmaf(-sg.damping, h, 1.0f);
         d.X[g] = f4(p, x4.w);
         if (EPI == EPI_FINALIZE_PREDICT) {
-            v = v + v3(sg.gx, sg.gy, sg.gz) * h;
-            d.P[in ^ 1][g] = f4(p + v * h, x4.w);
+            v = madd(v, v3(sg.gx, sg.gy, sg.gz), h);
+            d.P[in ^ 1][g] = f4(madd(p, v, h), x4.w);
         } else {
             d.V[g] = f4(v, 0.f);
         }
@@ -470,14 +480,14 @@ __global__ __launch_bounds__(VTX_TILE) void k_iterate(DevState d, const TileDev*
             const uint32_t pb = sg.pbase;
             float lam;
             BendGrad bg;
-            if (!bend_eval(P[pb + ix.x], P[pb + ix.y], P[pb + ix.z], P[pb + ix.w], d.brest[bid], xpbd_bend, lam, bg))
+            if (!bend_eval<false>(P[pb + ix.x], P[pb + ix.y], P[pb + ix.z], P[pb + ix.w], d.brest[bid], xpbd_bend, lam, bg))
                 continue;
             const V3 dk = role == 0 ? bg.k0 * bg.c1 : role == 1 ? bg.k1 * bg.c2 : role == 2 ? bg.d2
-                                                                              : -(bg.k0 * bg.c1 + bg.k1 * bg.c2 + bg.d2);
-            delta += (-w * lam) * dk;
+                                                                              : -(madd(bg.k0 * bg.c1, bg.c2, bg.k1) + bg.d2);
+            delta = madd(delta, dk, -w * lam);
             cnt++;
         }
-        if (cnt > 0) p += delta * (frcp((float)cnt) * sg.omega);
+        if (cnt > 0) p = madd(p, delta, frcp((float)cnt) * sg.omega);
     }
     epilogue<EPI>(d, sg, g, in, p, w, h);
 }
@@ -516,6 +526,16 @@ __device__ __forceinline__ void slot_rect(int a0, int b0, int rows, int cols, in
     w = min(RB1, cols - 2 - b0) - rb0 + 1;
 }
 
+// Offsets of a slot's vertices from its owner cell in a staged tile of row pitch PITCH: the canonical
+// vertex order per type (vtx_device.hpp).
+template <int TYPE, int PITCH>
+struct SlotAt {
+    static constexpr int i0 = TYPE == 0 ? 0 : TYPE == 1 ? -PITCH + 1 : PITCH - 1;
+    static constexpr int i1 = TYPE == 0 ? PITCH + 1 : TYPE == 1 ? PITCH : 1;
+    static constexpr int i2 = TYPE == 0 ? 1 : TYPE == 1 ? 0 : PITCH;
+    static constexpr int i3 = TYPE == 0 ? PITCH : TYPE == 1 ? 1 : 0;
+};
+
 // Evaluate the bending slot owned at tile-relative cell (ra, rb) of one type (a cell of
 // slot_rect's rectangle) into LDS at its row-major index j in the type's range; act (cleared
 // before) marks the slots that contribute. The slot keeps g_k = -lam d_k for roles 0..2 (planes
@@ -534,12 +554,8 @@ __device__ __forceinline__ void eval_slot(const DevState& d, const SegDev& sg, c
     bool on = ((sg.flags >> (3 + TYPE)) & 1u) || ((d.gflags[sg.pbase + (uint32_t)(a * cols + b)] >> TYPE) & 1u);
     if (on) {
         const int o = (ra + VTX_GH) * VTX_GP + (rb + VTX_GH);    // owner in staged coordinates
-        // canonical vertex order per type (vtx_device.hpp)
-        constexpr int i0 = TYPE == 0 ? 0 : TYPE == 1 ? -VTX_GP + 1 : VTX_GP - 1;
-        constexpr int i1 = TYPE == 0 ? VTX_GP + 1 : TYPE == 1 ? VTX_GP : 1;
-        constexpr int i2 = TYPE == 0 ? 1 : TYPE == 1 ? 0 : VTX_GP;
-        constexpr int i3 = TYPE == 0 ? VTX_GP : TYPE == 1 ? 1 : 0;
-        const float4 q0 = sp[o + i0], q1 = sp[o + i1], q2 = sp[o + i2], q3 = sp[o + i3];
+        using A = SlotAt<TYPE, VTX_GP>;
+        const float4 q0 = sp[o + A::i0], q1 = sp[o + A::i1], q2 = sp[o + A::i2], q3 = sp[o + A::i3];
         float rest = 0.f;
         if (!(sg.flags & VTX_SEG_BEND_REST0)) {
             const float4 r4 = SREST ? srest[(ra + 1) * VTX_RC + (rb + 1)] : d.brest4[sg.pbase + (uint32_t)(a * cols + b)];
@@ -547,7 +563,7 @@ __device__ __forceinline__ void eval_slot(const DevState& d, const SegDev& sg, c
         }
         float lam;
         BendGrad bg;
-        on = bend_eval(q0, q1, q2, q3, rest, xpbd, lam, bg);
+        on = bend_eval<true>(q0, q1, q2, q3, rest, xpbd, lam, bg);
         if (on) {
             const V3 g0 = (-lam * bg.k0) * bg.c1, g1 = (-lam * bg.k1) * bg.c2, g2 = -lam * bg.d2;
             corr[0][j] = g0.x; corr[1][j] = g0.y; corr[2][j] = g0.z;
@@ -737,9 +753,199 @@ __global__ __launch_bounds__(VTX_TILE * SPLIT) void k_iterate_grid(DevState d, c
     bend_type_pass<2, BT, PRE>(d, sg, sp, srest, corr, act + VTX_NSX + VTX_NSR, a0, b0, rows, cols, xpbd_bend, inside, ty,
                           tx, bend, cnt);
     if (!inside) return;
-    delta += w * bend;
-    if (cnt > 0) p += delta * (frcp((float)cnt) * sg.omega);
+    delta = madd(delta, bend, w);
+    if (cnt > 0) p = madd(p, delta, frcp((float)cnt) * sg.omega);
     epilogue<EPI>(d, sg, g, in, p, w, h);
+}
+
+// Several Jacobi passes of a T x T tile in one launch. A small or medium cloth gives a pass too little
+// work for the chip: a pass is then its launch, the staging load and three barrier-separated slot
+// phases, about 8 us whatever the size up to 200 x 200 vertices. Here a workgroup stages its tile with
+// a halo of 2 vertices per pass and runs the passes on it in LDS, each on the region that the passes
+// after it still need (2 vertices less on every side), so the halo's vertices are worked out again by
+// the tiles that own them. Every vertex adds the terms of k_iterate_grid in the same order: the same
+// result, bit for bit. The staged side is VTX_FS = 24 for every T: at most 4 passes for T = 8, 3 for
+// T = 12, 2 for T = 16. A pass is bound by its chain of LDS reads and dependent arithmetic, so the
+// three slot types are evaluated side by side (two barriers a pass), a slot leaves one 16-B word per
+// role, and the sums run without branches. Per launch (40 x 40, T = 8): 4.4, 6.3, 9.0, 11.1 us for
+// 1 to 4 passes, against 8.0 us for one pass of k_iterate_grid; of the 11.1 us, 6.1 us are VALU issue.
+// Attachments: none, or dense ones of at most VTX_LRA_PARTS slots.
+template <int T, int R = VTX_FS - 4>
+struct FuseTile {
+    static constexpr int HS = (VTX_FS - T) / 2;                          // staged halo
+    static constexpr int LO = HS + (T - R) / 2;                          // staged row / column of region (0, 0)
+    // slots around the region by type (X, R, D): owner rows and columns from -1
+    static constexpr int NX = (R + 1) * (R + 1), NR = (R + 2) * (R + 1);
+    static constexpr int NS = NX + 2 * NR;
+    static constexpr int UX = (NX + 63) / 64, UR = (NR + 63) / 64, UNITS = UX + 2 * UR;   // waves' shares
+};
+
+// One slot of type TYPE (index e of the type's range around the region) into corr[role][slot]: g_r and
+// the pass's mark in w. A slot that contributes nothing keeps an older mark.
+template <int T, int R, int TYPE>
+__device__ __forceinline__ void fuse_slot(const DevState& d, const SegDev& sg, const float4* sp,
+                                          float4 (*corr)[FuseTile<T>::NS], uint32_t mark, int a0, int b0, int e,
+                                          float xpbd) {
+#pragma clang fp contract(off)   // role 3: the products round before they are added, as in k_iterate_grid's gather
+    using F = FuseTile<T, R>;
+    constexpr int W = R + (TYPE == 2 ? 2 : 1);
+    const int ra = e / W, rb = e % W;                      // owner cell + (1, 1), relative to the region
+    const int a = a0 + F::LO - F::HS + ra - 1, b = b0 + F::LO - F::HS + rb - 1;
+    const int rows = (int)sg.rows, cols = (int)sg.cols;
+    if (e >= (TYPE == 0 ? F::NX : F::NR) || a < (TYPE == 1 ? 1 : 0) || a > rows - 2 || b < (TYPE == 2 ? 1 : 0) ||
+        b > cols - 2)
+        return;
+    const uint32_t cell = sg.pbase + (uint32_t)(a * cols + b);
+    if (!((sg.flags >> (3 + TYPE)) & 1u) && !((d.gflags[cell] >> TYPE) & 1u)) return;
+    const int o = (ra + F::LO - 1) * VTX_FS + rb + F::LO - 1;
+    using A = SlotAt<TYPE, VTX_FS>;
+    const float4 q0 = sp[o + A::i0], q1 = sp[o + A::i1], q2 = sp[o + A::i2], q3 = sp[o + A::i3];
+    float rest = 0.f;
+    if (!(sg.flags & VTX_SEG_BEND_REST0)) rest = reinterpret_cast<const float*>(d.brest4 + cell)[TYPE];
+    float lam;
+    BendGrad bg;
+    if (!bend_eval<true>(q0, q1, q2, q3, rest, xpbd, lam, bg)) return;
+    const V3 g0 = (-lam * bg.k0) * bg.c1, g1 = (-lam * bg.k1) * bg.c2, g2 = -lam * bg.d2;
+    const int j = (TYPE == 0 ? 0 : TYPE == 1 ? F::NX : F::NX + F::NR) + e;
+    corr[0][j] = f4(g0, __uint_as_float(mark));
+    corr[1][j] = f4(g1, __uint_as_float(mark));
+    corr[2][j] = f4(g2, __uint_as_float(mark));
+    corr[3][j] = make_float4(-((g0.x + g1.x) + g2.x), -((g0.y + g1.y) + g2.y), -((g0.z + g1.z) + g2.z),
+                             __uint_as_float(mark));
+}
+
+// The four memberships of region vertex (y, x) in one slot type, added in role order. All LDS reads are
+// issued before the first use; a slot that contributes nothing adds +0, which changes no sum.
+template <int T, int R, int TYPE>
+__device__ __forceinline__ void fuse_gather(const float4 (*corr)[FuseTile<T>::NS], uint32_t mark, int y, int x, V3& bend,
+                                            int& cnt) {
+    using F = FuseTile<T, R>;
+    // role r of the slot owned at (y + dy_r, x + dx_r), per type (bend_type_pass)
+    constexpr int dy[3][4] = {{0, -1, 0, -1}, {1, -1, 0, 0}, {-1, 0, -1, 0}};
+    constexpr int dx[3][4] = {{0, -1, -1, 0}, {-1, 0, 0, -1}, {1, -1, 0, 0}};
+    constexpr int W = R + (TYPE == 2 ? 2 : 1);
+    const int o = (TYPE == 0 ? 0 : TYPE == 1 ? F::NX : F::NX + F::NR) + (y + 1) * W + x + 1;
+    float4 g[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) g[r] = corr[r][o + dy[TYPE][r] * W + dx[TYPE][r]];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const bool on = __float_as_uint(g[r].w) == mark;
+        bend += v3(on ? g[r].x : 0.f, on ? g[r].y : 0.f, on ? g[r].z : 0.f);
+        cnt += on ? 1 : 0;
+    }
+}
+
+// One pass on the region of side R centred on the tile; EPI applies to the last one (R == T).
+template <int EPI, int T, int R>
+__device__ __forceinline__ void fuse_pass(const DevState& d, const SegDev& sg, float4* sp, const float4* sr,
+                                          const float (*sl)[VTX_FS * VTX_FS], float4 (*corr)[FuseTile<T>::NS],
+                                          uint32_t nslots, int a0, int b0, int in, float h, float xpbd) {
+    using F = FuseTile<T, R>;
+    constexpr uint32_t mark = (VTX_FS - R) / 4;            // one per region size
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    // bending slots, 64 of one type per wave and round; the last waves first, as the first ones hold
+    // the vertices
+    const int wave = (int)__builtin_amdgcn_readfirstlane((uint32_t)tid >> 6);
+#pragma unroll
+    for (int u0 = 0; u0 < F::UNITS; u0 += 16) {
+        const int u = u0 + 15 - wave;
+        if (u < F::UX) {
+            if (!(sg.flags & VTX_SEG_NONE_X)) fuse_slot<T, R, 0>(d, sg, sp, corr, mark, a0, b0, u * 64 + lane, xpbd);
+        } else if (u < F::UX + F::UR) {
+            if (!(sg.flags & VTX_SEG_NONE_R))
+                fuse_slot<T, R, 1>(d, sg, sp, corr, mark, a0, b0, (u - F::UX) * 64 + lane, xpbd);
+        } else if (u < F::UNITS) {
+            if (!(sg.flags & VTX_SEG_NONE_D))
+                fuse_slot<T, R, 2>(d, sg, sp, corr, mark, a0, b0, (u - F::UX - F::UR) * 64 + lane, xpbd);
+        }
+    }
+    const int y = tid / R, x = tid % R;
+    const int a = a0 + F::LO - F::HS + y, b = b0 + F::LO - F::HS + x;
+    const bool inside = tid < R * R && a >= 0 && a < (int)sg.rows && b >= 0 && b < (int)sg.cols;
+    const int sc = (y + F::LO) * VTX_FS + x + F::LO;
+    V3 p = v3(0.f, 0.f, 0.f), delta = p;
+    float w = 0.f;
+    int cnt = 0;
+    if (inside) {
+        const float4 p4 = sp[sc];
+        p = xyz(p4);
+        w = p4.w;
+        const float k = -w * sg.stiffness;
+        const float4 r_own = sr[sc], r_left = sr[sc - 1], r_up = sr[sc - VTX_FS];
+        const float rest[8] = {r_own.x, r_left.x, r_own.y, r_up.y, r_own.z, sr[sc - VTX_FS - 1].z, r_left.w, r_up.w};
+        constexpr int at[8] = {1, -1, VTX_FS, -VTX_FS, VTX_FS + 1, -VTX_FS - 1, VTX_FS - 1, -VTX_FS + 1};
+        float4 q[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) q[e] = sp[sc + at[e]];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {   // stretch_term with selects; an absent constraint has a NaN rest length
+            const V3 diff = p - xyz(q[e]);
+            const float dist = fsqrt(dot_fma(diff, diff)), wsum = w + q[e].w;
+            const bool on = rest[e] == rest[e] && dist != rest[e] && wsum > 0.f;
+            const V3 sum = madd(delta, diff, (dist - rest[e]) * k * frcp(wsum * (dist + VTX_EPSILON)));
+            delta = v3(on ? sum.x : delta.x, on ? sum.y : delta.y, on ? sum.z : delta.z);
+            cnt += on ? 1 : 0;
+        }
+        for (uint32_t s = 0; s < nslots; s++) {                 // every slot is a part of its own
+            V3 part = v3(0.f, 0.f, 0.f);
+            attach_term(p, w, d.slots[sg.sbase + s], sl[s][sc], sg.lrs, part, cnt);
+            delta += part;
+        }
+    }
+    __syncthreads();
+    if (inside) {
+        V3 bend = v3(0.f, 0.f, 0.f);
+        fuse_gather<T, R, 0>(corr, mark, y, x, bend, cnt);
+        fuse_gather<T, R, 1>(corr, mark, y, x, bend, cnt);
+        fuse_gather<T, R, 2>(corr, mark, y, x, bend, cnt);
+        delta = madd(delta, bend, w);
+        if (cnt > 0) p = madd(p, delta, frcp((float)cnt) * sg.omega);
+        if (R > T) sp[sc] = f4(p, w);
+        else epilogue<EPI>(d, sg, sg.pbase + (uint32_t)(a * (int)sg.cols + b), in, p, w, h);
+    }
+    if (R > T) __syncthreads();
+}
+
+template <int EPI, int T>
+__global__ __launch_bounds__(1024) void k_iterate_fused(DevState d, const GridTileDev* __restrict__ tiles, int in,
+                                                        int passes, float h) {
+    using F = FuseTile<T>;
+    __shared__ float4 sp[VTX_FS * VTX_FS];                    // positions
+    __shared__ float4 sr[VTX_FS * VTX_FS];                    // owned stretch rest lengths, NaN off the cloth
+    __shared__ float sl[VTX_LRA_PARTS][VTX_FS * VTX_FS];      // attachment distances
+    __shared__ float4 corr[4][F::NS];                         // per role: g, mark of the pass that wrote it
+    const GridTileDev t = tiles[tile_of(d.remap)];
+    const SegDev sg = d.segs[t.seg];
+    const int rows = (int)sg.rows, cols = (int)sg.cols, a0 = (int)t.a0, b0 = (int)t.b0;
+    const int tid = (int)threadIdx.x;
+    const uint32_t nslots = sg.flags & VTX_SEG_LRA_DENSE ? sg.scount : 0u;
+    {
+        const int ra = tid / VTX_FS - F::HS, rb = tid % VTX_FS - F::HS, a = a0 + ra, b = b0 + rb, H = 2 * passes;
+        float4 p = make_float4(0.f, 0.f, 0.f, 0.f), r = nan4();
+        const bool in_cloth = tid < VTX_FS * VTX_FS && ra >= -H && ra < T + H && rb >= -H && rb < T + H && a >= 0 &&
+                              a < rows && b >= 0 && b < cols;
+        const uint32_t v = in_cloth ? (uint32_t)(a * cols + b) : 0u;
+        if (in_cloth) {
+            p = d.P[in][sg.pbase + v];
+            r = d.rest4[sg.pbase + v];
+        }
+        for (int e = tid; e < 4 * F::NS; e += 1024) corr[0][e].w = 0.f;   // while the loads are in flight
+        if (in_cloth)
+            for (uint32_t s = 0; s < nslots; s++) sl[s][tid] = d.lra[sg.lbase + (size_t)s * sg.n + v];
+        if (tid < VTX_FS * VTX_FS) {
+            sp[tid] = p;
+            sr[tid] = r;
+        }
+    }
+    __syncthreads();
+    const float xpbd = sg.bend_compliance * frcp(h) * frcp(h);   // compliance / h^2 (cu:173)
+    if constexpr (T <= 8)
+        if (passes > 3) fuse_pass<EPI, T, T + 12>(d, sg, sp, sr, sl, corr, nslots, a0, b0, in, h, xpbd);
+    if constexpr (T <= 12)
+        if (passes > 2) fuse_pass<EPI, T, T + 8>(d, sg, sp, sr, sl, corr, nslots, a0, b0, in, h, xpbd);
+    if (passes > 1) fuse_pass<EPI, T, T + 4>(d, sg, sp, sr, sl, corr, nslots, a0, b0, in, h, xpbd);
+    fuse_pass<EPI, T, T>(d, sg, sp, sr, sl, corr, nslots, a0, b0, in, h, xpbd);
 }
 
 // ComputeTriangleNormals + ComputeVertexNormals (Velvet/VtClothSolverGPU.cu:419-450) as a
@@ -884,6 +1090,23 @@ hipError_t launch_iterate(const DevState& d, int in, float h, int epilogue, bool
     return last_launch();
 }
 
+template <int T>
+static void launch_fused(const DevState& d, int in, int passes, float h, int epilogue, hipStream_t s) {
+    const dim3 gr(d.nftiles), bl(1024);
+    if (epilogue == EPI_NONE) hipLaunchKernelGGL((k_iterate_fused<EPI_NONE, T>), gr, bl, 0, s, d, d.ftiles, in, passes, h);
+    else if (epilogue == EPI_FINALIZE) hipLaunchKernelGGL((k_iterate_fused<EPI_FINALIZE, T>), gr, bl, 0, s, d, d.ftiles, in, passes, h);
+    else hipLaunchKernelGGL((k_iterate_fused<EPI_FINALIZE_PREDICT, T>), gr, bl, 0, s, d, d.ftiles, in, passes, h);
+}
+
+hipError_t launch_iterate_fused(const DevState& d, int in, int passes, float h, int epilogue, hipStream_t s) {
+    if (!d.nftiles) return hipSuccess;
+    if (passes < 1 || passes > fuse_passes(d.fside)) return hipErrorInvalidValue;   // the staged halo
+    if (d.fside == 8) launch_fused<8>(d, in, passes, h, epilogue, s);
+    else if (d.fside == 12) launch_fused<12>(d, in, passes, h, epilogue, s);
+    else launch_fused<16>(d, in, passes, h, epilogue, s);
+    return last_launch();
+}
+
 hipError_t launch_check_finite(const DevState& d, uint32_t* flags, uint32_t nseg, hipStream_t s) {
     hipLaunchKernelGGL(k_clear_flags, dim3((nseg + 255) / 256), dim3(256), 0, s, flags, nseg);
     if (d.ntiles) hipLaunchKernelGGL(k_check_finite, dim3(d.ntiles), dim3(VTX_TILE), 0, s, d, flags);
@@ -894,6 +1117,7 @@ hipError_t launch_normals(const DevState& d, hipStream_t s) {
     if (d.nitiles) hipLaunchKernelGGL(k_normals, dim3(d.nitiles), dim3(VTX_TILE), 0, s, d, d.itiles);
     if (d.ngtiles) hipLaunchKernelGGL(k_normals_grid, dim3(d.ngtiles), dim3(VTX_TILE), 0, s, d, d.gtiles);
     if (d.nltiles) hipLaunchKernelGGL(k_normals_grid, dim3(d.nltiles), dim3(VTX_TILE), 0, s, d, d.ltiles);
+    if (d.nmtiles) hipLaunchKernelGGL(k_normals_grid, dim3(d.nmtiles), dim3(VTX_TILE), 0, s, d, d.mtiles);
     return last_launch();
 }
 

@@ -14,6 +14,9 @@ hipError_t launch_collide(const DevState& d, int in, float h, int block, hipStre
 // lra_batch: dense attachment distances loaded per batch (4, 16 or 64; same results)
 hipError_t launch_iterate(const DevState& d, int in, float h, int epilogue, bool constraints, int lra_batch,
                           hipStream_t s);
+// Fused passes of the grid segments in d.ftiles: most passes per launch for tiles of side 8, 12, 16
+inline int fuse_passes(uint32_t side) { return (VTX_FS - (int)side) / 4; }
+hipError_t launch_iterate_fused(const DevState& d, int in, int passes, float h, int epilogue, hipStream_t s);
 hipError_t launch_normals(const DevState& d, hipStream_t s);
 hipError_t launch_check_finite(const DevState& d, uint32_t* flags, uint32_t nseg, hipStream_t s);
 

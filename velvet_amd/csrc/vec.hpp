@@ -21,6 +21,18 @@ __device__ __forceinline__ V3 operator/(V3 a, float s) { return V3{a.x / s, a.y 
 __device__ __forceinline__ V3& operator+=(V3& a, V3 b) { a = a + b; return a; }
 __device__ __forceinline__ V3& operator-=(V3& a, V3 b) { a = a - b; return a; }
 __device__ __forceinline__ float dot(V3 a, V3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
+// The same with every multiply-add spelled out, so that a function rounds alike in each kernel that
+// inlines it (the compiler's choice of the products to fuse depends on the code around them).
+__device__ __forceinline__ float dot_fma(V3 a, V3 b) {
+    return __builtin_fmaf(a.z, b.z, __builtin_fmaf(a.x, b.x, a.y * b.y));
+}
+__device__ __forceinline__ V3 cross_fma(V3 a, V3 b) {
+    return V3{__builtin_fmaf(a.y, b.z, -(a.z * b.y)), __builtin_fmaf(a.z, b.x, -(a.x * b.z)),
+              __builtin_fmaf(a.x, b.y, -(a.y * b.x))};
+}
+__device__ __forceinline__ V3 madd(V3 c, V3 a, float s) {   // c + a s
+    return V3{__builtin_fmaf(a.x, s, c.x), __builtin_fmaf(a.y, s, c.y), __builtin_fmaf(a.z, s, c.z)};
+}
 __device__ __forceinline__ float length(V3 a) { return sqrtf(dot(a, a)); }
 __device__ __forceinline__ V3 cross(V3 a, V3 b) {
     return V3{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};

@@ -67,6 +67,7 @@
 #define VTX_GT 16
 #define VTX_GH 2
 #define VTX_GP (VTX_GT + 2 * VTX_GH)      // 20: staged positions per side
+#define VTX_FS 24                         // staged side of a fused tile (k_iterate_fused)
 // Bending slot types of a grid cell (a, b), each with its canonical vertex order
 // (p0, p1, p2, p3) as (row, col) offsets from the cell:
 //   X: diagonal (a+1,b)-(a,b+1)    (0,0) (1,1) (0,1) (1,0)   -- Velvet/VtClothObjectGPU.hpp:121-130
@@ -154,12 +155,15 @@ struct DevState {
     const TileDev* itiles;    // particle tiles of segments on the general (ELL) Jacobi path
     const GridTileDev* gtiles;
     const GridTileDev* ltiles;   // grid tiles whose dense attachments run on four lanes per particle
+    const GridTileDev* ftiles;   // fside x fside tiles of the grid segments whose passes are fused
+    const GridTileDev* mtiles;   // the same segments' VTX_GT x VTX_GT tiles (normals)
     const uint32_t* hsegs;       // segments whose hash is built in LDS (VTX_SEG_HASH_LDS)
     const float4* rest4;      // grid: stretch rest lengths owned by a vertex (R, D, X-diag, anti-diag)
     const uint32_t* gflags;   // grid: bending slots present at a cell (VTX_BX | VTX_BR | VTX_BD)
     const float4* brest4;     // grid: bending rest angles of a cell (X, R, D)
     uint32_t ntiles, nstiles, nhist, ncells;
-    uint32_t hbase0, nltiles, nhsegs, pad3;  // first histogram entry of this table set
+    uint32_t hbase0, nltiles, nhsegs;        // hbase0: first histogram entry of this table set
+    uint32_t nftiles, nmtiles, fside;
     uint32_t nparticles, nitiles, ngtiles, remap;   // remap: workgroups -> tiles through xcd_tile
 };
 
