@@ -759,7 +759,7 @@ void Engine::prepare_segment(Segment& sg) {
         s_tr[i + 1] += s_tr[i];
     }
     std::vector<uint2> l_st(s_st[n]), l_at(s_at[n]);
-    std::vector<uint32_t> l_bd(s_bd[n]), l_tr(s_tr[n]);
+    std::vector<uint32_t> l_bd(s_bd[n]), l_tr(s_tr[n]), ub;   // ub: first bend record of each tile
     if (!pr.grid) {
         std::vector<uint32_t> f(s_st.begin(), s_st.end() - 1);
         for (size_t c = 0; c < S; c++) {
@@ -768,13 +768,33 @@ void Engine::prepare_segment(Segment& sg) {
             l_st[f[a]++] = make_uint2(b, r);
             l_st[f[b]++] = make_uint2(a, r);
         }
+        // bend records per tile, in registration order: a bend goes to every tile that holds one of its
+        // particles, and a particle's entries name its tile's records
+        const size_t ntile = (n + VTX_TILE - 1) / VTX_TILE;
+        std::vector<uint32_t> cnt(ntile + 1, 0), seen(ntile, VTX_INVALID);
+        for (size_t c = 0; c < B; c++)
+            for (uint32_t r = 0; r < 4; r++) {
+                const uint32_t t = sg.bd[4 * c + r] / VTX_TILE;
+                if (seen[t] == (uint32_t)c) continue;
+                seen[t] = (uint32_t)c;
+                cnt[t + 1]++;
+            }
+        for (size_t t = 0; t < ntile; t++) cnt[t + 1] += cnt[t];
+        ub = cnt;
+        pr.brec.resize(cnt[ntile]);
+        pr.brest.resize(cnt[ntile]);
+        std::fill(seen.begin(), seen.end(), VTX_INVALID);
         std::vector<uint32_t> fb(s_bd.begin(), s_bd.end() - 1);
         for (size_t c = 0; c < B; c++)
-            for (uint32_t r = 0; r < 4; r++) l_bd[fb[sg.bd[4 * c + r]]++] = (uint32_t)c | (r << 30);
-        for (size_t c = 0; c < B; c++) {
-            pr.brec.push_back(make_uint4(sg.bd[4 * c], sg.bd[4 * c + 1], sg.bd[4 * c + 2], sg.bd[4 * c + 3]));
-            pr.brest.push_back(sg.bd_rest[c]);
-        }
+            for (uint32_t r = 0; r < 4; r++) {
+                const uint32_t v = sg.bd[4 * c + r], t = v / VTX_TILE;
+                if (seen[t] != (uint32_t)c) {
+                    seen[t] = (uint32_t)c;
+                    pr.brec[cnt[t]] = make_uint4(sg.bd[4 * c], sg.bd[4 * c + 1], sg.bd[4 * c + 2], sg.bd[4 * c + 3]);
+                    pr.brest[cnt[t]++] = sg.bd_rest[c];
+                }
+                l_bd[fb[v]++] = (cnt[t] - 1 - ub[t]) | (r << 30);
+            }
     }
     // dense long-range attachments: entry c = slot * n + particle for every slot and particle
     pr.lra_dense = n > 0 && L > 0 && A == (size_t)L * n;
@@ -804,6 +824,8 @@ void Engine::prepare_segment(Segment& sg) {
             pack_tile(pr.est, s_st, l_st, first, t.count, make_uint2(VTX_INVALID, 0u), &t.st_off, &t.st_k);
             pack_tile(pr.eat, s_at, l_at, first, t.count, make_uint2(VTX_INVALID, 0u), &t.at_off, &t.at_k);
             pack_tile(pr.ebd, s_bd, l_bd, first, t.count, VTX_INVALID, &t.bd_off, &t.bd_k);
+            t.ub_off = ub[first / VTX_TILE];
+            t.ub_n = ub[first / VTX_TILE + 1] - t.ub_off;
         }
         if (!pr.grid) pack_tile(pr.etr, s_tr, l_tr, first, t.count, VTX_INVALID, &t.tr_off, &t.tr_k);
         pr.tiles.push_back(t);
@@ -1030,7 +1052,6 @@ void Engine::upload(Segment& sg, hipStream_t s) {
         d.scount = (uint32_t)pr.slots.size();
         d.cbase = (uint32_t)r.col;
         d.ccount = (uint32_t)pr.cols.size();
-        d.bbase = (uint32_t)r.brec;
         d.trbase = (uint32_t)r.trec;
         d.flags = (selfcol ? VTX_SEG_SELFCOL : 0u) | (pr.grid ? pr.grid_flags : 0u) |
                   (pr.lra_dense ? VTX_SEG_LRA_DENSE : 0u) | (selfcol && n <= VTX_NBR16_N ? VTX_SEG_NBR16 : 0u);
@@ -1294,6 +1315,7 @@ void Engine::rebuild_tables() {
             t.at_off += (uint32_t)sg.rg.at;
             t.bd_off += (uint32_t)sg.rg.bd;
             t.tr_off += (uint32_t)sg.rg.tr;
+            t.ub_off += (uint32_t)sg.rg.brec;
             htile.push_back(t);
             if (!sg.prep.grid) hitile.push_back(t);
         }

@@ -89,13 +89,14 @@ struct alignas(16) SegDev {
     float gx, gy, gz, pad0;
     uint32_t mod_lo, mod_hi;               // ceil(2^64 / M): exact remainder by multiplication
     uint32_t rows, cols;                   // grid segments: vertex grid shape
-    uint32_t bbase, trbase, lbase, pad2;   // bend-record / triangle-record / dense-LRA bases
+    uint32_t trbase, lbase, pad1, pad2;    // triangle-record / dense-LRA bases
 };
 
 struct alignas(16) TileDev {
     uint32_t seg, begin, count, pad0;      // begin = global index of the tile's first particle
     uint32_t st_off, st_k, at_off, at_k;   // stretch / attach ELL offsets (entries) and widths
     uint32_t bd_off, bd_k, tr_off, tr_k;   // bend / triangle ELL offsets and widths
+    uint32_t ub_off, ub_n, pad1, pad2;     // the tile's bend records: offset and count
 };
 
 struct alignas(16) SortTileDev {
@@ -136,8 +137,8 @@ struct DevState {
     // ELL entries and records hold segment-local indices; kernels add the segment's bases
     const uint2* st;          // stretch ELL: (other particle, rest bits)
     const uint2* at;          // attach ELL: (slot, distance bits)
-    const uint32_t* bd;       // bend ELL: bend id | role << 30
-    const uint4* brec;        // bend records: 4 particle indices
+    const uint32_t* bd;       // bend ELL: record of the tile | role << 30, ascending per particle
+    const uint4* brec;        // bend records: 4 particle indices; per tile, every bend that touches it
     const float* brest;       // bend rest angles
     const uint32_t* tr;       // triangle ELL: triangle id
     const uint4* trec;        // triangle records: 3 particle indices
