@@ -163,15 +163,16 @@ typedef struct vtx_tuning {
     int32_t use_graph;         /* replay frames from a hipGraph */
     int32_t neighbor_order;    /* 0 to 2, no effect: once the neighbour search's thread order, which
                                   is now one for all (waves over runs of particles of one cell) */
-    int32_t lra_batch;         /* dense attachment distances loaded per batch: 4, 16 or 64 */
+    int32_t lra_batch;         /* dense attachment distances a grid cloth with 32 or more slots loads per
+                                  batch: 4 or 16 (64, accepted as before, runs as 16) */
     int32_t xcd_remap;         /* hand each XCD a contiguous run of tiles */
     float frame_ms;            /* vtx_autotune: the chosen variant's frame time (0 from the cache) */
     int32_t gather_block;      /* threads per workgroup of the contact pass: 64, 128 or 256 (each
                                   256-particle tile split across workgroups) */
     int32_t streams;           /* k = 1..4: the segments split into k particle-balanced groups
                                   whose frames run concurrently on k streams */
-    int32_t lra_split;         /* 1: grid cloths with 32 or more dense attachment slots run their
-                                  Jacobi pass with four threads per particle; 0: one thread */
+    int32_t lra_split;         /* no effect: once four or one threads per particle in the Jacobi pass of
+                                  grid cloths with 32 or more dense attachment slots; now always four */
     int32_t hash_lds;          /* 1: self-colliding segments of at most 16384 particles (table of
                                   at most 2^16 cells) build their spatial hash in one workgroup;
                                   0: every segment takes the device-wide sort */

@@ -698,6 +698,40 @@ static void fill_state(const Segment& sg, Prepared& pr) {
         pr.slots[k] = make_float4(sg.slots[3 * k], sg.slots[3 * k + 1], sg.slots[3 * k + 2], 0.f);
 }
 
+// Tiled dense attachments (VTX_SEG_LRA_TILED): float4 of one tile, and whether a grid segment has them.
+// Whole tiles and groups of four are stored, so a cloth of few columns or rows would take up to 16 times
+// the memory: beyond twice (and 4 MB) the distances stay slot-major.
+static size_t tiled_stride(size_t L) {
+    return VTX_LRA_PARTS * (((L + VTX_LRA_PARTS - 1) / VTX_LRA_PARTS + 3) / 4) * VTX_TILE;
+}
+
+static bool tiles_distances(const Prepared& pr, size_t n, size_t L) {
+    if (!pr.grid || L < VTX_LRA_SPLIT_MIN) return false;
+    const size_t tiles = (size_t)((pr.grows + VTX_GT - 1) / VTX_GT) * ((pr.gcols + VTX_GT - 1) / VTX_GT);
+    const size_t stored = 4 * tiled_stride(L) * tiles;
+    return stored <= 2 * L * n || stored <= (1u << 20);
+}
+
+// Dense attachments of a grid segment in its tiles' order, as target distances.
+static void tile_distances(const Segment& sg, Prepared& pr) {
+    const size_t n = sg.n(), L = sg.slots.size() / 3, qs = (L + VTX_LRA_PARTS - 1) / VTX_LRA_PARTS;
+    const float lrs = sg.prm.long_range_stretchiness;
+    const size_t groups = (qs + 3) / 4, per_tile = tiled_stride(L);
+    pr.lra.resize(4 * per_tile * pr.gtiles.size());
+    for (size_t ti = 0; ti < pr.gtiles.size(); ti++) {
+        GridTileDev& t = pr.gtiles[ti];
+        t.at_off = (uint32_t)(ti * per_tile);
+        const uint32_t h = std::min<uint32_t>(VTX_GT, pr.grows - t.a0), w = std::min<uint32_t>(VTX_GT, pr.gcols - t.b0);
+        for (size_t s = 0; s < L; s++) {
+            const size_t q = s / qs, k = s % qs;
+            float* out = pr.lra.data() + 4 * (ti * per_tile + (q * groups + k / 4) * VTX_TILE) + k % 4;
+            const float* in = sg.at_dist.data() + s * n + (size_t)t.a0 * pr.gcols + t.b0;
+            for (uint32_t a = 0; a < h; a++, in += pr.gcols, out += 4 * VTX_GT)
+                for (uint32_t b = 0; b < w; b++) out[4 * b] = in[b] * lrs;
+        }
+    }
+}
+
 // Host packing of one segment into its position-independent device layout.
 void Engine::prepare(int32_t si) { prepare_segment(seg(si)); }
 
@@ -801,7 +835,8 @@ void Engine::prepare_segment(Segment& sg) {
     for (size_t c = 0; c < A && pr.lra_dense; c++)
         pr.lra_dense = (size_t)sg.at_pid[c] == c % n && (size_t)sg.at_slot[c] == c / n;
     if (pr.lra_dense) {
-        pr.lra = sg.at_dist;   // already slot-major
+        pr.lra_tiled = tiles_distances(pr, n, L);
+        if (!pr.lra_tiled) pr.lra = sg.at_dist;   // already slot-major
         std::fill(s_at.begin(), s_at.end(), 0u);
         l_at.clear();
     } else {
@@ -844,6 +879,7 @@ void Engine::prepare_segment(Segment& sg) {
                 pack_lanes(pr.eat, s_at, l_at, lanes, make_uint2(VTX_INVALID, 0u), &gt.at_off, &gt.at_k);
                 pr.gtiles.push_back(gt);
             }
+        if (pr.lra_tiled) tile_distances(sg, pr);
     }
     sg.prep = std::move(pr);
     sg.prepared = true;
@@ -866,7 +902,7 @@ static Ranges needs_of(const Segment& sg) {
     r.n_trec = pr.trec.size();
     r.n_slot = pr.slots.size();
     r.n_col = pr.cols.size();
-    r.n_lra = pr.lra.size();
+    r.n_lra = (pr.lra.size() + 3) & ~size_t(3);   // ranges of whole float4
     return r;
 }
 
@@ -1031,7 +1067,7 @@ void Engine::upload(Segment& sg, hipStream_t s) {
     take(aslot_, need.n_slot, &r.slot);
     take(acol_, need.n_col, &r.col);
     take(alra_, need.n_lra, &r.lra);
-    VTX_REQUIRE(r.lra + r.n_lra < (1ull << 32), VTX_ECAPACITY, "dense attachment pool exceeds 2^32 entries");
+    VTX_REQUIRE(r.lra + r.n_lra < (1ull << 34), VTX_ECAPACITY, "dense attachment pool exceeds 2^34 entries");
     sg.rg = r;
     // a failed copy gives the ranges back, so that a later attempt starts clean
     try {
@@ -1054,8 +1090,8 @@ void Engine::upload(Segment& sg, hipStream_t s) {
         d.ccount = (uint32_t)pr.cols.size();
         d.trbase = (uint32_t)r.trec;
         d.flags = (selfcol ? VTX_SEG_SELFCOL : 0u) | (pr.grid ? pr.grid_flags : 0u) |
-                  (pr.lra_dense ? VTX_SEG_LRA_DENSE : 0u) | (selfcol && n <= VTX_NBR16_N ? VTX_SEG_NBR16 : 0u);
-        d.lbase = (uint32_t)r.lra;
+                  (pr.lra_dense ? VTX_SEG_LRA_DENSE : 0u) | (pr.lra_tiled ? VTX_SEG_LRA_TILED : 0u) | (selfcol && n <= VTX_NBR16_N ? VTX_SEG_NBR16 : 0u);
+        d.lbase = (uint32_t)(r.lra / 4);
         d.max_nbr = (uint32_t)p.max_num_neighbors;
         // binary32 products exactly as the reference forms them (Velvet/SpatialHashGPU.hpp:21,44,47)
         d.diameter = p.particle_diameter;
@@ -1306,8 +1342,7 @@ void Engine::rebuild_tables() {
         }
         if ((d.flags & VTX_SEG_SELFCOL) || d.ccount) need_collide_ = true;
         if (d.flags & VTX_SEG_LRA_DENSE) any_lra_dense_ = true;
-        const bool lsplit = sg.prep.grid && (d.flags & VTX_SEG_LRA_DENSE) && d.scount >= VTX_LRA_SPLIT_MIN;
-        any_lra_split_ = any_lra_split_ || lsplit;
+        any_lra_split_ = any_lra_split_ || sg.prep.lra_tiled;
         for (TileDev t : sg.prep.tiles) {
             t.seg = ti;
             t.begin += d.pbase;
@@ -1322,8 +1357,8 @@ void Engine::rebuild_tables() {
         const bool fused = fside && fusable(sg);
         for (GridTileDev gt : sg.prep.gtiles) {
             gt.seg = ti;
-            gt.at_off += (uint32_t)sg.rg.at;
-            (fused ? hmtile : lsplit && tun_.lra_split ? hltile : hgtile).push_back(gt);
+            gt.at_off += (uint32_t)(sg.prep.lra_tiled ? sg.rg.lra / 4 : sg.rg.at);
+            (fused ? hmtile : sg.prep.lra_tiled ? hltile : hgtile).push_back(gt);
         }
         for (uint32_t a = 0; fused && a < d.rows; a += fside)
             for (uint32_t b = 0; b < d.cols; b += fside) {
@@ -1739,7 +1774,7 @@ void Engine::set_tuning(const Tuning& t) {
                 "gather_block must be 64, 128 or 256");
     VTX_REQUIRE(t.streams >= 1 && t.streams <= VTX_MAX_STREAMS, VTX_EINVAL, "streams must be 1 to 4");
     VTX_REQUIRE(t.hash_grid >= 0 && t.hash_grid <= 3, VTX_EINVAL, "hash_grid must be 0 to 3");
-    if (t.streams != tun_.streams || t.lra_split != tun_.lra_split || t.hash_lds != tun_.hash_lds ||
+    if (t.streams != tun_.streams || t.hash_lds != tun_.hash_lds ||
         t.hash_grid != tun_.hash_grid)
         tables_dirty_ = true;
     tun_ = t;
@@ -1844,24 +1879,22 @@ Tuning Engine::autotune(int frames, float frame_dt, bool use_cache, double* fram
         bms = trial(best);
         // one knob at a time, every other value of it against the best so far; the hash grid
         // (opted-in segments only) goes before the knobs of the hash and neighbour phases
-        static const int order[] = {0, 8, 2, 3, 4, 5, 6, 7};
+        static const int order[] = {0, 8, 2, 3, 4, 5, 7};
         for (int knob : order) {
             if (knob == 8 && !any_grid_tunable_) continue;
-            if (knob == 2 && !any_lra_dense_) continue;
+            if (knob == 2 && !any_lra_split_) continue;
             if (knob == 4 && !need_collide_) continue;
             if (knob == 5 && table_seg_.size() < 2) continue;
-            if (knob == 6 && !any_lra_split_) continue;
             if (knob == 7 && !any_hash_lds_) continue;
-            const int nval = knob == 5 || knob == 8 ? 4 : knob == 2 || knob == 4 ? 3 : 2;
+            const int nval = knob == 5 || knob == 8 ? 4 : knob == 4 ? 3 : 2;
             const Tuning base = best;
             for (int v = 0; v < nval; v++) {
                 Tuning t = base;
                 if (knob == 0) t.graph = v != 0;
-                if (knob == 2) t.lra_batch = v == 0 ? 4 : v == 1 ? 16 : 64;
+                if (knob == 2) t.lra_batch = v == 0 ? 4 : 16;
                 if (knob == 3) t.remap = v != 0;
                 if (knob == 4) t.gather_block = 64 << v;
                 if (knob == 5) t.streams = v + 1;
-                if (knob == 6) t.lra_split = v != 0;
                 if (knob == 7) t.hash_lds = v != 0;
                 if (knob == 8) t.hash_grid = v;
                 if (knob == 8 ? t.hash_grid == base.hash_grid
@@ -1870,7 +1903,7 @@ Tuning Engine::autotune(int frames, float frame_dt, bool use_cache, double* fram
                                 : knob == 3 ? t.remap == base.remap
                                 : knob == 4 ? t.gather_block == base.gather_block
                                 : knob == 5 ? t.streams == base.streams
-                                : knob == 6 ? t.lra_split == base.lra_split : t.hash_lds == base.hash_lds)
+                                            : t.hash_lds == base.hash_lds)
                     continue;
                 const double ms = trial(t);
                 if (ms < 0.99 * bms) {

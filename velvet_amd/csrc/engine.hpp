@@ -58,8 +58,8 @@ struct Prepared {
     std::vector<float4> slots, rest4, brest4;
     std::vector<uint32_t> gflags;
     std::vector<ColliderDev> cols;
-    std::vector<float> lra;                     // dense attachments: distances, slot-major
-    bool lra_dense = false;
+    std::vector<float> lra;                     // dense attachments: distances, slot-major or tiled
+    bool lra_dense = false, lra_tiled = false;
     std::vector<TileDev> tiles;                 // ELL offsets relative to the segment's ranges
     std::vector<GridTileDev> gtiles;
 };
@@ -134,13 +134,12 @@ struct Segment {
 struct Tuning {
     bool graph = true;        // replay frames from a hipGraph
     int nbr_order = 2;        // kept for callers (vtx_tuning.neighbor_order), no effect
-    int lra_batch = 16;       // dense attachment distances loaded per batch: 4, 16 or 64
+    int lra_batch = 16;       // distances of 32 or more dense slots loaded per batch: 4 or 16 (64 runs as 16)
     bool remap = true;        // XCD-aware workgroup -> tile remap
     int gather_block = 256;   // threads per workgroup of the contact pass
     int streams = 1;          // k > 1: segments split into k particle-balanced groups whose frames
                               // run on k streams, overlapping latency- and VALU-bound stages
-    bool lra_split = true;    // grid segments with >= VTX_LRA_SPLIT_MIN dense slots: four threads
-                              // per particle in the Jacobi pass
+    bool lra_split = true;    // kept for callers (vtx_tuning.lra_split), no effect
     bool hash_lds = true;     // small self-colliding segments build their hash in one workgroup
     int hash_grid = 0;        // hash-grid resolution of segments with tune_hash_grid: 0 the
                               // reference grid; 1..3 origin shifted, table 1x / 2x / 4x. The only
@@ -321,7 +320,7 @@ private:
     uint64_t frames_ = 0;                    // frames simulated
     Tuning tun_;
     bool any_lra_dense_ = false;
-    bool any_lra_split_ = false;   // a stencil segment has >= VTX_LRA_SPLIT_MIN dense slots
+    bool any_lra_split_ = false;   // a stencil segment has tiled dense attachments
     bool any_hash_lds_ = false;    // a self-colliding segment is small enough for k_hash_small
     bool any_grid_tunable_ = false;   // a live self-colliding segment has tune_hash_grid
     bool use_stencil_ = true;

@@ -260,9 +260,7 @@ __device__ __forceinline__ void stretch_term(V3 p, float w, float nws, float4 q,
 // diff * (t / |diff| - 1); "|diff| > t" is the same test as "t / |diff| - 1 < 0", so one
 // reciprocal square root serves both. Branch-free (selects): the slot position is used on every
 // path, so its loads can be issued ahead of the term instead of inside a conditional block.
-__device__ __forceinline__ void attach_term(V3 p, float w, float4 slot, float dist0, float lrs, V3& delta,
-                                            int& cnt) {
-    const float target = dist0 * lrs;
+__device__ __forceinline__ void attach_to(V3 p, float w, float4 slot, float target, V3& delta, int& cnt) {
     const V3 diff = p - xyz(slot);
     const float f = __builtin_fmaf(target, frsq(dot_fma(diff, diff)), -1.0f);
     // the reference returns early for a pinned particle with a positive target
@@ -274,6 +272,11 @@ __device__ __forceinline__ void attach_term(V3 p, float w, float4 slot, float di
     cnt += act ? 1 : 0;
 }
 
+__device__ __forceinline__ void attach_term(V3 p, float w, float4 slot, float dist0, float lrs, V3& delta,
+                                            int& cnt) {
+    attach_to(p, w, slot, dist0 * lrs, delta, cnt);
+}
+
 // Slot range [s0, s1) of part q of a segment's attachments (see VTX_LRA_PARTS).
 __device__ __forceinline__ void lra_part_range(const SegDev& sg, uint32_t q, uint32_t& s0, uint32_t& s1) {
     const uint32_t qs = (sg.scount + VTX_LRA_PARTS - 1) / VTX_LRA_PARTS;
@@ -282,43 +285,97 @@ __device__ __forceinline__ void lra_part_range(const SegDev& sg, uint32_t q, uin
 }
 
 // Dense attachments of one particle to slots [s0, s1), summed from zero in slot order.
-// Distances are fetched LB slots at a time so that several loads are in flight per lane (a large
-// cloth may give only one wave per SIMD); every LB gives the same sum.
-template <int LB>
+// Distances are fetched four slots at a time so that several loads are in flight per lane.
 __device__ __forceinline__ void attach_dense(const DevState& d, const SegDev& sg, uint32_t local, uint32_t s0,
                                              uint32_t s1, V3 p, float w, V3& part, int& cnt) {
-    const float* __restrict__ lra = d.lra + sg.lbase + local;
+    const float* __restrict__ lra = d.lra + 4 * (size_t)sg.lbase + local;
     const float4* __restrict__ slot = d.slots + sg.sbase;
     const size_t n = sg.n;
     uint32_t s = s0;
-    for (; s + LB <= s1; s += LB) {
-        float r[LB];
+    for (; s + 4 <= s1; s += 4) {
+        float r[4];
+        float4 q[4];                                        // wave-uniform
 #pragma unroll
-        for (int u = 0; u < LB; u++) r[u] = lra[(size_t)(s + u) * n];
-        // slot positions (wave-uniform) four at a time, so that few are live at once
+        for (int u = 0; u < 4; u++) r[u] = lra[(size_t)(s + u) * n];
 #pragma unroll
-        for (int g = 0; g < LB; g += 4) {
-            float4 q[4];
+        for (int u = 0; u < 4; u++) q[u] = slot[s + u];
 #pragma unroll
-            for (int u = 0; u < 4; u++) q[u] = slot[s + g + u];
-#pragma unroll
-            for (int u = 0; u < 4; u++) attach_term(p, w, q[u], r[g + u], sg.lrs, part, cnt);
-            __builtin_amdgcn_sched_barrier(0);
-        }
+        for (int u = 0; u < 4; u++) attach_term(p, w, q[u], r[u], sg.lrs, part, cnt);
     }
     for (; s < s1; s++) attach_term(p, w, slot[s], lra[(size_t)s * n], sg.lrs, part, cnt);
+}
+
+// The same from a tile's target distances (VTX_SEG_LRA_TILED): dist = the part's first group of this
+// lane, one float4 per group of four slots, VTX_TILE apart. B groups are in flight while the B before
+// them are summed, and a group's slot positions (wave-uniform) while the group before it is; `first`
+// holds the first B groups, loaded by the caller as early as it can.
+template <int B>
+struct TiledBatch {
+    float4 r[B];
+    __device__ __forceinline__ void load(const float4* __restrict__ dist, uint32_t g, uint32_t groups) {
+#pragma unroll
+        for (int u = 0; u < B; u++) r[u] = dist[(size_t)min(g + u, groups - 1u) * VTX_TILE];
+    }
+};
+
+struct SlotGroup {
+    float4 q[4];
+    __device__ __forceinline__ void load(const float4* __restrict__ slot) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) q[k] = slot[k];
+    }
+};
+
+template <int B>
+__device__ __forceinline__ void attach_tiled(const DevState& d, const SegDev& sg, const float4* __restrict__ dist,
+                                             TiledBatch<B> cur, uint32_t s0, uint32_t s1, V3 p, float w, V3& part,
+                                             int& cnt) {
+    const float4* __restrict__ slot = d.slots + sg.sbase + s0;
+    const uint32_t groups = (s1 - s0 + 3) / 4, full = (s1 - s0) / 4;
+    if (full) {
+        SlotGroup now;
+        now.load(slot);
+        for (uint32_t g = 0; g < full; g += B) {
+            TiledBatch<B> next;
+            next.load(dist, g + B, groups);
+#pragma unroll
+            for (int u = 0; u < B; u++) {
+                if (g + u >= full) break;
+                SlotGroup then;
+                then.load(slot + 4 * min(g + u + 1, full - 1u));
+                attach_to(p, w, now.q[0], cur.r[u].x, part, cnt);
+                attach_to(p, w, now.q[1], cur.r[u].y, part, cnt);
+                attach_to(p, w, now.q[2], cur.r[u].z, part, cnt);
+                attach_to(p, w, now.q[3], cur.r[u].w, part, cnt);
+                now = then;
+            }
+            cur = next;
+        }
+    }
+    if (full < groups) {                                    // one to three slots left
+        const float4 r = dist[(size_t)full * VTX_TILE];
+        attach_to(p, w, slot[4 * full], r.x, part, cnt);
+        if (s0 + 4 * full + 1 < s1) attach_to(p, w, slot[4 * full + 1], r.y, part, cnt);
+        if (s0 + 4 * full + 2 < s1) attach_to(p, w, slot[4 * full + 2], r.z, part, cnt);
+    }
+}
+
+// First group of part q of a tile's lane.
+__device__ __forceinline__ const float4* tiled_part(const DevState& d, const SegDev& sg, uint32_t at_off, uint32_t q,
+                                                    uint32_t lane) {
+    const uint32_t qs = (sg.scount + VTX_LRA_PARTS - 1) / VTX_LRA_PARTS;
+    return reinterpret_cast<const float4*>(d.lra) + at_off + (size_t)q * ((qs + 3) / 4) * VTX_TILE + lane;
 }
 
 // All attachments of one particle, added to delta part by part (VTX_LRA_PARTS): dense
 // (slot-major distances, the slot position is the same for every lane) or from the tile's attach
 // ELL in registration order, where a part ends wherever the slot's part changes -- so attachments
 // registered particle-major in slot order sum exactly as the dense form does.
-template <int LB>
 __device__ __forceinline__ void attach_terms(const DevState& d, const SegDev& sg, uint32_t at_off, uint32_t at_k,
                                              uint32_t lane, uint32_t local, V3 p, float w, V3& delta, int& cnt) {
     if (sg.flags & VTX_SEG_LRA_DENSE) {
         if (sg.scount <= VTX_LRA_PARTS) {   // every slot is a part of its own
-            const float* __restrict__ lra = d.lra + sg.lbase + local;
+            const float* __restrict__ lra = d.lra + 4 * (size_t)sg.lbase + local;
             const float4* __restrict__ slot = d.slots + sg.sbase;
             for (uint32_t s = 0; s < sg.scount; s++) {
                 V3 part = v3(0.f, 0.f, 0.f);
@@ -332,7 +389,7 @@ __device__ __forceinline__ void attach_terms(const DevState& d, const SegDev& sg
             uint32_t s0, s1;
             lra_part_range(sg, q, s0, s1);
             V3 part = v3(0.f, 0.f, 0.f);
-            attach_dense<LB>(d, sg, local, s0, s1, p, w, part, cnt);
+            attach_dense(d, sg, local, s0, s1, p, w, part, cnt);
             delta += part;
         }
         return;
@@ -569,7 +626,7 @@ __global__ __launch_bounds__(VTX_MT, RPT == 1 ? 6 : 3) void k_iterate(DevState d
                 if (k0 + k < t.st_k && c[k].x != VTX_INVALID)
                     stretch_term(p, w, nws, q[k], __uint_as_float(c[k].y), delta, cnt);
         }
-        attach_terms<4>(d, sg, t.at_off, t.at_k, tid, g - sg.pbase, p, w, delta, cnt);
+        attach_terms(d, sg, t.at_off, t.at_k, tid, g - sg.pbase, p, w, delta, cnt);
     }
 #pragma unroll
     for (uint32_t k = 0; k < ER; k++) ent[k * VTX_MT + tid] = er[k];
@@ -600,7 +657,6 @@ __global__ __launch_bounds__(VTX_MT, RPT == 1 ? 6 : 3) void k_iterate(DevState d
 #define VTX_NSR (18 * 17)
 #define VTX_NSD (17 * 18)
 #define VTX_NSMAX VTX_NSR
-#define VTX_RC 18              // owner cells of any type per tile side: -1..16
 
 template <int TYPE>
 __device__ __forceinline__ int slot_index(int ra, int rb) {
@@ -634,12 +690,10 @@ struct SlotAt {
 // slot_rect's rectangle) into LDS at its row-major index j in the type's range; act (cleared
 // before) marks the slots that contribute. The slot keeps g_k = -lam d_k for roles 0..2 (planes
 // 3k..3k+2); role 3's is -(g_0 + g_1 + g_2), as the four gradients of a dihedral angle sum to
-// zero, and each vertex scales the sum of its terms by its own inverse mass. SREST: the rest
-// angles come from srest, the tile's owner cells (rows and columns -1..16, row-major by 18) staged
-// in LDS with the positions, instead of from brest4.
-template <int TYPE, bool SREST>
+// zero, and each vertex scales the sum of its terms by its own inverse mass.
+template <int TYPE>
 __device__ __forceinline__ void eval_slot(const DevState& d, const SegDev& sg, const float4* sp,
-                                          const float4* srest, float (*corr)[VTX_NSMAX], uint8_t* act, int a0,
+                                          float (*corr)[VTX_NSMAX], uint8_t* act, int a0,
                                           int b0, int cols, int ra, int rb, float xpbd) {
     constexpr int W = TYPE == 2 ? 18 : 17;                                  // owner columns of the range
     const uint32_t j = (uint32_t)((ra + 1) * W + (rb + 1));                 // row-major storage index
@@ -652,7 +706,7 @@ __device__ __forceinline__ void eval_slot(const DevState& d, const SegDev& sg, c
         const float4 q0 = sp[o + A::i0], q1 = sp[o + A::i1], q2 = sp[o + A::i2], q3 = sp[o + A::i3];
         float rest = 0.f;
         if (!(sg.flags & VTX_SEG_BEND_REST0)) {
-            const float4 r4 = SREST ? srest[(ra + 1) * VTX_RC + (rb + 1)] : d.brest4[sg.pbase + (uint32_t)(a * cols + b)];
+            const float4 r4 = d.brest4[sg.pbase + (uint32_t)(a * cols + b)];
             rest = TYPE == 0 ? r4.x : TYPE == 1 ? r4.y : r4.z;
         }
         float lam;
@@ -672,9 +726,9 @@ __device__ __forceinline__ void eval_slot(const DevState& d, const SegDev& sg, c
 // t: row t / w, column t % w), so a tile cut by the cloth's edge runs no lanes on cells that
 // cannot hold a slot; then every tile vertex adds its four memberships of this type in role
 // order to bend (gradients times -lam; the vertex's inverse mass is applied to the sum).
-template <int TYPE, int BT, bool SREST>
+template <int TYPE>
 __device__ __forceinline__ void bend_type_pass(const DevState& d, const SegDev& sg, const float4* sp,
-                                               const float4* srest, float (*corr)[VTX_NSMAX], uint8_t* act,
+                                               float (*corr)[VTX_NSMAX], uint8_t* act,
                                                int a0, int b0,
                                                int rows, int cols, float xpbd, bool inside, int ty, int tx,
                                                V3& bend, int& cnt) {
@@ -684,13 +738,14 @@ __device__ __forceinline__ void bend_type_pass(const DevState& d, const SegDev& 
         slot_rect<TYPE>(a0, b0, rows, cols, ra0, rb0, h, w);
         if (h > 0 && w > 0) {
             const uint32_t n = (uint32_t)(h * w), m = (65536u + (uint32_t)w - 1u) / (uint32_t)w;   // t / w = t m >> 16 (t < 1024, w <= 18)
+            constexpr uint32_t BT = VTX_TILE;
             static_assert(2 * BT >= VTX_NSMAX, "a slot type fits two rounds of the workgroup");
 #pragma unroll
-            for (uint32_t r = 0; r < (BT >= VTX_NSMAX ? 1u : 2u); r++) {
+            for (uint32_t r = 0; r < 2u; r++) {
                 const uint32_t t = tid + r * BT;
                 if (t < n) {
                     const uint32_t q = (t * m) >> 16;
-                    eval_slot<TYPE, SREST>(d, sg, sp, srest, corr, act, a0, b0, cols, ra0 + (int)q, rb0 + (int)(t - q * (uint32_t)w), xpbd);
+                    eval_slot<TYPE>(d, sg, sp, corr, act, a0, b0, cols, ra0 + (int)q, rb0 + (int)(t - q * (uint32_t)w), xpbd);
                 }
             }
         }
@@ -732,39 +787,23 @@ __device__ __forceinline__ float4 nan4() {
     return make_float4(q, q, q, q);
 }
 
-// SPLIT = 1: one thread per vertex. SPLIT = VTX_LRA_PARTS: a workgroup of four threads per
-// vertex for segments with many dense attachments (a 256 x 256 cloth with 256 slots gives one
-// tile per CU, and a single wave per SIMD would walk 256 slots per vertex): thread q of a vertex
-// sums attachment part q, the first thread adds the parts in order, and all threads share the
-// bending slots (one round per type). Both forms add the same terms in the same order.
-// The split form (one workgroup per CU on a large cloth, so little hides a load's latency) also
-// stages the tile's bending rest angles in LDS with the positions instead of loading one per slot
-// evaluation.
-template <int EPI, int LB, int SPLIT>
-__global__ __launch_bounds__(VTX_TILE * SPLIT) void k_iterate_grid(DevState d, const GridTileDev* __restrict__ tiles,
+template <int EPI>
+__global__ __launch_bounds__(VTX_TILE) void k_iterate_grid(DevState d, const GridTileDev* __restrict__ tiles,
                                                                    int in, float h) {
-    constexpr int BT = VTX_TILE * SPLIT;
     __shared__ float4 sp[VTX_GP * VTX_GP];
     __shared__ float corr[9][VTX_NSMAX];           // plane r*3+c: component c of role r's g_r
     __shared__ uint32_t actw[(VTX_NSX + VTX_NSR + VTX_NSD + 3) / 4];   // per type: slot contributes
-    constexpr bool PRE = SPLIT > 1;
-    __shared__ float4 srest_s[PRE ? VTX_RC * VTX_RC : 1];
     uint8_t* const act = reinterpret_cast<uint8_t*>(actw);
     const GridTileDev t = tiles[tile_of(d.remap)];
     const SegDev sg = d.segs[t.seg];
     const int rows = (int)sg.rows, cols = (int)sg.cols;
     const int a0 = (int)t.a0, b0 = (int)t.b0;
     const uint32_t tid = threadIdx.x;
-    const uint32_t lane = SPLIT == 1 ? tid : tid % VTX_TILE;
-    // part of the split form: wave-uniform (VTX_TILE is a multiple of the wave), so the slot
-    // positions below are scalar loads
-    const uint32_t qpart = SPLIT == 1 ? 0u : __builtin_amdgcn_readfirstlane(tid / VTX_TILE);
     const float4* __restrict__ P = d.P[in];
-    const int ty = (int)(lane / VTX_GT), tx = (int)(lane % VTX_GT);
+    const int ty = (int)(tid / VTX_GT), tx = (int)(tid % VTX_GT);
     const int a = a0 + ty, b = b0 + tx;
-    const bool in_cloth = a < rows && b < cols;
-    const bool inside = in_cloth && qpart == 0;        // the thread that owns the vertex
-    const uint32_t g = in_cloth ? sg.pbase + (uint32_t)(a * cols + b) : 0u;
+    const bool inside = a < rows && b < cols;
+    const uint32_t g = inside ? sg.pbase + (uint32_t)(a * cols + b) : 0u;
     // stretch rest lengths: R own/left, D own/up, X-diagonal own/up-left, anti-diagonal of left/up,
     // issued before the staging loads and always (from the vertex itself where a neighbour is
     // missing): a load that a lane may skip leaves the outstanding count unknown to the compiler,
@@ -778,20 +817,12 @@ __global__ __launch_bounds__(VTX_TILE * SPLIT) void k_iterate_grid(DevState d, c
     if (!(a > 0 && b > 0)) r_ul = nan4();
 
     // clear the slot marks; stage positions of rows [a0-2, a0+18) x cols [b0-2, b0+18)
-    for (uint32_t e = tid; e < (VTX_NSX + VTX_NSR + VTX_NSD + 3) / 4; e += BT) actw[e] = 0u;
-    for (uint32_t e = tid; e < VTX_GP * VTX_GP; e += BT) {
+    for (uint32_t e = tid; e < (VTX_NSX + VTX_NSR + VTX_NSD + 3) / 4; e += VTX_TILE) actw[e] = 0u;
+    for (uint32_t e = tid; e < VTX_GP * VTX_GP; e += VTX_TILE) {
         const int sa = a0 - VTX_GH + (int)(e / VTX_GP), sb = b0 - VTX_GH + (int)(e % VTX_GP);
         float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
         if (sa >= 0 && sa < rows && sb >= 0 && sb < cols) v = P[sg.pbase + (uint32_t)(sa * cols + sb)];
         sp[e] = v;
-    }
-    if (PRE && !(sg.flags & VTX_SEG_BEND_REST0)) {   // rest angles of owner cells rows/cols -1..16
-        for (uint32_t e = tid; e < VTX_RC * VTX_RC; e += BT) {
-            const int sa = a0 - 1 + (int)(e / VTX_RC), sb = b0 - 1 + (int)(e % VTX_RC);
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (sa >= 0 && sa < rows && sb >= 0 && sb < cols) v = d.brest4[sg.pbase + (uint32_t)(sa * cols + sb)];
-            srest_s[e] = v;
-        }
     }
 
     __syncthreads();
@@ -813,38 +844,15 @@ __global__ __launch_bounds__(VTX_TILE * SPLIT) void k_iterate_grid(DevState d, c
         if (r_ul.z == r_ul.z) stretch_term(p, w, k, sp[sc - VTX_GP - 1], r_ul.z, delta, cnt);
         if (r_left.w == r_left.w) stretch_term(p, w, k, sp[sc + VTX_GP - 1], r_left.w, delta, cnt);
         if (r_up.w == r_up.w) stretch_term(p, w, k, sp[sc - VTX_GP + 1], r_up.w, delta, cnt);
-        if constexpr (SPLIT == 1) attach_terms<LB>(d, sg, t.at_off, t.at_k, tid, (uint32_t)(a * cols + b), p, w, delta, cnt);
-    }
-    if constexpr (SPLIT > 1) {   // only dense segments come here (VTX_SEG_LRA_DENSE)
-        __shared__ float4 lpart[SPLIT - 1][VTX_TILE];
-        V3 part = v3(0.f, 0.f, 0.f);
-        int pc = 0;
-        if (in_cloth) {
-            uint32_t s0, s1;
-            lra_part_range(sg, qpart, s0, s1);
-            attach_dense<LB>(d, sg, g - sg.pbase, s0, s1, p, w, part, pc);
-            if (qpart > 0) lpart[qpart - 1][lane] = f4(part, __int_as_float(pc));
-        }
-        __syncthreads();
-        if (inside) {
-            delta += part;
-            cnt += pc;
-#pragma unroll
-            for (int q = 0; q < SPLIT - 1; q++) {
-                const float4 e = lpart[q][lane];
-                delta += xyz(e);
-                cnt += __float_as_int(e.w);
-            }
-        }
+        attach_terms(d, sg, t.at_off, t.at_k, tid, (uint32_t)(a * cols + b), p, w, delta, cnt);
     }
     // bending: X roles 0..3, R roles 0..3, D roles 0..3
     const float xpbd_bend = sg.bend_compliance * frcp(h) * frcp(h);   // compliance / h^2 (cu:173)
     V3 bend = v3(0.f, 0.f, 0.f);
-    const float4* const srest = srest_s;   // read by the split form (PRE) only, when staged
-    bend_type_pass<0, BT, PRE>(d, sg, sp, srest, corr, act, a0, b0, rows, cols, xpbd_bend, inside, ty, tx, bend, cnt);
-    bend_type_pass<1, BT, PRE>(d, sg, sp, srest, corr, act + VTX_NSX, a0, b0, rows, cols, xpbd_bend, inside, ty, tx, bend,
+    bend_type_pass<0>(d, sg, sp, corr, act, a0, b0, rows, cols, xpbd_bend, inside, ty, tx, bend, cnt);
+    bend_type_pass<1>(d, sg, sp, corr, act + VTX_NSX, a0, b0, rows, cols, xpbd_bend, inside, ty, tx, bend,
                           cnt);
-    bend_type_pass<2, BT, PRE>(d, sg, sp, srest, corr, act + VTX_NSX + VTX_NSR, a0, b0, rows, cols, xpbd_bend, inside, ty,
+    bend_type_pass<2>(d, sg, sp, corr, act + VTX_NSX + VTX_NSR, a0, b0, rows, cols, xpbd_bend, inside, ty,
                           tx, bend, cnt);
     if (!inside) return;
     delta = madd(delta, bend, w);
@@ -874,11 +882,11 @@ struct FuseTile {
     static constexpr int UX = (NX + 63) / 64, UR = (NR + 63) / 64, UNITS = UX + 2 * UR;   // waves' shares
 };
 
-// One slot of type TYPE (index e of the type's range around the region) into corr[role][slot]: g_r and
-// the pass's mark in w. A slot that contributes nothing keeps an older mark.
-template <int T, int R, int TYPE>
-__device__ __forceinline__ void fuse_slot(const DevState& d, const SegDev& sg, const float4* sp,
-                                          float4 (*corr)[FuseTile<T>::NS], uint32_t mark, int a0, int b0, int e,
+// One slot of type TYPE (index e of the type's range around the region) into corr[role][slot], NR roles:
+// g_r and the pass's mark in w. A slot that contributes nothing keeps an older mark.
+template <int T, int R, int TYPE, int NR, int NS>
+__device__ __forceinline__ void fuse_slot(const DevState& d, const SegDev& sg, const float4* sp, float4 (&corr)[NR][NS],
+                                          uint32_t mark, int a0, int b0, int e,
                                           float xpbd) {
 #pragma clang fp contract(off)   // role 3: the products round before they are added, as in k_iterate_grid's gather
     using F = FuseTile<T, R>;
@@ -904,15 +912,15 @@ __device__ __forceinline__ void fuse_slot(const DevState& d, const SegDev& sg, c
     corr[0][j] = f4(g0, __uint_as_float(mark));
     corr[1][j] = f4(g1, __uint_as_float(mark));
     corr[2][j] = f4(g2, __uint_as_float(mark));
-    corr[3][j] = make_float4(-((g0.x + g1.x) + g2.x), -((g0.y + g1.y) + g2.y), -((g0.z + g1.z) + g2.z),
-                             __uint_as_float(mark));
+    if constexpr (NR > 3)
+        corr[3][j] = make_float4(-((g0.x + g1.x) + g2.x), -((g0.y + g1.y) + g2.y), -((g0.z + g1.z) + g2.z),
+                                 __uint_as_float(mark));
 }
 
 // The four memberships of region vertex (y, x) in one slot type, added in role order. All LDS reads are
 // issued before the first use; a slot that contributes nothing adds +0, which changes no sum.
-template <int T, int R, int TYPE>
-__device__ __forceinline__ void fuse_gather(const float4 (*corr)[FuseTile<T>::NS], uint32_t mark, int y, int x, V3& bend,
-                                            int& cnt) {
+template <int T, int R, int TYPE, int NR, int NS>
+__device__ __forceinline__ void fuse_gather(const float4 (&corr)[NR][NS], uint32_t mark, int y, int x, V3& bend, int& cnt) {
     using F = FuseTile<T, R>;
     // role r of the slot owned at (y + dy_r, x + dx_r), per type (bend_type_pass)
     constexpr int dy[3][4] = {{0, -1, 0, -1}, {1, -1, 0, 0}, {-1, 0, -1, 0}};
@@ -921,7 +929,15 @@ __device__ __forceinline__ void fuse_gather(const float4 (*corr)[FuseTile<T>::NS
     const int o = (TYPE == 0 ? 0 : TYPE == 1 ? F::NX : F::NX + F::NR) + (y + 1) * W + x + 1;
     float4 g[4];
 #pragma unroll
-    for (int r = 0; r < 4; r++) g[r] = corr[r][o + dy[TYPE][r] * W + dx[TYPE][r]];
+    for (int r = 0; r < 4; r++) {
+        const int j = o + dy[TYPE][r] * W + dx[TYPE][r];
+        if (r < NR) {
+            g[r] = corr[r][j];
+        } else {
+            const float4 u = corr[0][j], v = corr[1][j], q = corr[2][j];
+            g[r] = make_float4(-((u.x + v.x) + q.x), -((u.y + v.y) + q.y), -((u.z + v.z) + q.z), u.w);
+        }
+    }
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         const bool on = __float_as_uint(g[r].w) == mark;
@@ -930,10 +946,38 @@ __device__ __forceinline__ void fuse_gather(const float4 (*corr)[FuseTile<T>::NS
     }
 }
 
+// The eight stretch terms of the vertex at staged index sc, in the order of k_iterate_grid, with selects
+// (an absent constraint has a NaN rest length); STEP neighbours are read at a time.
+template <int STEP>
+__device__ __forceinline__ void fuse_stretch(const SegDev& sg, const float4* sp, const float4* sr, int sc, V3 p, float w,
+                                             V3& delta, int& cnt) {
+    const float k = -w * sg.stiffness;
+    const float4 r_own = sr[sc], r_left = sr[sc - 1], r_up = sr[sc - VTX_FS];
+    const float rest[8] = {r_own.x, r_left.x, r_own.y, r_up.y, r_own.z, sr[sc - VTX_FS - 1].z, r_left.w, r_up.w};
+    constexpr int at[8] = {1, -1, VTX_FS, -VTX_FS, VTX_FS + 1, -VTX_FS - 1, VTX_FS - 1, -VTX_FS + 1};
+#pragma unroll
+    for (int e0 = 0; e0 < 8; e0 += STEP) {
+        float4 q[STEP];
+#pragma unroll
+        for (int e = 0; e < STEP; e++) q[e] = sp[sc + at[e0 + e]];
+#pragma unroll
+        for (int e = 0; e < STEP; e++) {   // stretch_term
+            const float r = rest[e0 + e];
+            const V3 diff = p - xyz(q[e]);
+            const float dist = fsqrt(dot_fma(diff, diff)), wsum = w + q[e].w;
+            const bool on = r == r && dist != r && wsum > 0.f;
+            const V3 sum = madd(delta, diff, (dist - r) * k * frcp(wsum * (dist + VTX_EPSILON)));
+            delta = v3(on ? sum.x : delta.x, on ? sum.y : delta.y, on ? sum.z : delta.z);
+            cnt += on ? 1 : 0;
+        }
+        if (STEP < 8) __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
 // One pass on the region of side R centred on the tile; EPI applies to the last one (R == T).
 template <int EPI, int T, int R>
 __device__ __forceinline__ void fuse_pass(const DevState& d, const SegDev& sg, float4* sp, const float4* sr,
-                                          const float (*sl)[VTX_FS * VTX_FS], float4 (*corr)[FuseTile<T>::NS],
+                                          const float (*sl)[VTX_FS * VTX_FS], float4 (&corr)[4][FuseTile<T>::NS],
                                           uint32_t nslots, int a0, int b0, int in, float h, float xpbd) {
     using F = FuseTile<T, R>;
     constexpr uint32_t mark = (VTX_FS - R) / 4;            // one per region size
@@ -965,22 +1009,7 @@ __device__ __forceinline__ void fuse_pass(const DevState& d, const SegDev& sg, f
         const float4 p4 = sp[sc];
         p = xyz(p4);
         w = p4.w;
-        const float k = -w * sg.stiffness;
-        const float4 r_own = sr[sc], r_left = sr[sc - 1], r_up = sr[sc - VTX_FS];
-        const float rest[8] = {r_own.x, r_left.x, r_own.y, r_up.y, r_own.z, sr[sc - VTX_FS - 1].z, r_left.w, r_up.w};
-        constexpr int at[8] = {1, -1, VTX_FS, -VTX_FS, VTX_FS + 1, -VTX_FS - 1, VTX_FS - 1, -VTX_FS + 1};
-        float4 q[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++) q[e] = sp[sc + at[e]];
-#pragma unroll
-        for (int e = 0; e < 8; e++) {   // stretch_term with selects; an absent constraint has a NaN rest length
-            const V3 diff = p - xyz(q[e]);
-            const float dist = fsqrt(dot_fma(diff, diff)), wsum = w + q[e].w;
-            const bool on = rest[e] == rest[e] && dist != rest[e] && wsum > 0.f;
-            const V3 sum = madd(delta, diff, (dist - rest[e]) * k * frcp(wsum * (dist + VTX_EPSILON)));
-            delta = v3(on ? sum.x : delta.x, on ? sum.y : delta.y, on ? sum.z : delta.z);
-            cnt += on ? 1 : 0;
-        }
+        fuse_stretch<8>(sg, sp, sr, sc, p, w, delta, cnt);
         for (uint32_t s = 0; s < nslots; s++) {                 // every slot is a part of its own
             V3 part = v3(0.f, 0.f, 0.f);
             attach_term(p, w, d.slots[sg.sbase + s], sl[s][sc], sg.lrs, part, cnt);
@@ -1026,7 +1055,7 @@ __global__ __launch_bounds__(1024) void k_iterate_fused(DevState d, const GridTi
         }
         for (int e = tid; e < 4 * F::NS; e += 1024) corr[0][e].w = 0.f;   // while the loads are in flight
         if (in_cloth)
-            for (uint32_t s = 0; s < nslots; s++) sl[s][tid] = d.lra[sg.lbase + (size_t)s * sg.n + v];
+            for (uint32_t s = 0; s < nslots; s++) sl[s][tid] = d.lra[4 * (size_t)sg.lbase + (size_t)s * sg.n + v];
         if (tid < VTX_FS * VTX_FS) {
             sp[tid] = p;
             sr[tid] = r;
@@ -1040,6 +1069,104 @@ __global__ __launch_bounds__(1024) void k_iterate_fused(DevState d, const GridTi
         if (passes > 2) fuse_pass<EPI, T, T + 8>(d, sg, sp, sr, sl, corr, nslots, a0, b0, in, h, xpbd);
     if (passes > 1) fuse_pass<EPI, T, T + 4>(d, sg, sp, sr, sl, corr, nslots, a0, b0, in, h, xpbd);
     fuse_pass<EPI, T, T>(d, sg, sp, sr, sl, corr, nslots, a0, b0, in, h, xpbd);
+}
+
+// One pass of a 16 x 16 tile of a cloth with many dense attachments (VTX_SEG_LRA_TILED, at least
+// VTX_LRA_SPLIT_MIN slots), four threads per vertex: thread q of a vertex sums attachment part q, the
+// first adds the parts in order after its stretch terms, and the other waves evaluate the bending slots.
+// A 256 x 256 cloth gives one tile per CU: the distances come as one 16-B load per four slots,
+// contiguous over the tile (the slot-major order gives 64-B runs), started before the positions are
+// staged, and there is one barrier between the terms and the sums. At 256 slots the pass is bound by the
+// 67 MB of distances, which no L2 keeps from one launch to the next: 19.6 -> 17.9 us alone (67 MB at the
+// 5.2 TB/s that overlapping passes reach are 12.9 us), 862 -> 652 us a frame with three solvers' passes
+// overlapping, for which the registers and LDS leave room for two workgroups per CU (with all four roles
+// in LDS and one workgroup per CU 16.7 us alone, but 743 us a frame overlapping).
+template <int EPI, int B>
+__global__ __launch_bounds__(1024, 8) void k_iterate_split(DevState d, const GridTileDev* __restrict__ tiles, int in, float h) {
+    constexpr int T = VTX_GT;
+    using F = FuseTile<T, T>;
+    __shared__ float4 sp[VTX_FS * VTX_FS];
+    __shared__ float4 sr[VTX_FS * VTX_FS];
+    __shared__ float4 corr[3][F::NS];                         // role 3 from the others: two workgroups per CU
+    __shared__ float4 lpart[VTX_LRA_PARTS - 1][VTX_TILE];
+    static_assert(VTX_LRA_PARTS * VTX_TILE == 1024, "a thread per vertex and part");
+    const GridTileDev t = tiles[tile_of(d.remap)];
+    const SegDev sg = d.segs[t.seg];
+    const int rows = (int)sg.rows, cols = (int)sg.cols, a0 = (int)t.a0, b0 = (int)t.b0;
+    const int tid = (int)threadIdx.x, lane = tid % VTX_TILE;
+    const uint32_t qpart = __builtin_amdgcn_readfirstlane((uint32_t)tid / VTX_TILE);   // wave-uniform
+    uint32_t s0, s1;
+    lra_part_range(sg, qpart, s0, s1);
+    const float4* __restrict__ dist = tiled_part(d, sg, t.at_off, qpart, (uint32_t)lane);
+    TiledBatch<B> first = {};
+    if (s0 < s1) first.load(dist, 0, (s1 - s0 + 3) / 4);
+    {   // positions and rest lengths of the tile and two vertices around it
+        const int ra = tid / VTX_FS - F::HS, rb = tid % VTX_FS - F::HS, a = a0 + ra, b = b0 + rb;
+        const bool in_cloth = tid < VTX_FS * VTX_FS && ra >= -2 && ra < T + 2 && rb >= -2 && rb < T + 2 && a >= 0 &&
+                              a < rows && b >= 0 && b < cols;
+        float4 p = make_float4(0.f, 0.f, 0.f, 0.f), r = nan4();
+        if (in_cloth) {
+            const uint32_t v = sg.pbase + (uint32_t)(a * cols + b);
+            p = d.P[in][v];
+            r = d.rest4[v];
+        }
+        for (int e = tid; e < 3 * F::NS; e += 1024) corr[0][e].w = 0.f;   // no slot marked
+        if (tid < VTX_FS * VTX_FS) {
+            sp[tid] = p;
+            sr[tid] = r;
+        }
+    }
+    __syncthreads();
+    const float xpbd = sg.bend_compliance * frcp(h) * frcp(h);   // compliance / h^2 (cu:173)
+    constexpr uint32_t mark = 1;
+    const int y = lane / T, x = lane % T, a = a0 + y, b = b0 + x;
+    const int sc = (y + F::LO) * VTX_FS + x + F::LO;
+    const bool in_cloth = a < rows && b < cols, inside = in_cloth && qpart == 0;
+    const float4 p4 = sp[sc];
+    V3 p = xyz(p4), delta = v3(0.f, 0.f, 0.f), part = delta;
+    const float w = p4.w;
+    int cnt = 0, pc = 0;
+    if (inside) fuse_stretch<2>(sg, sp, sr, sc, p, w, delta, cnt);
+    if (in_cloth) {
+        if (s0 < s1) attach_tiled<B>(d, sg, dist, first, s0, s1, p, w, part, pc);
+        if (qpart > 0) lpart[qpart - 1][lane] = f4(part, __int_as_float(pc));
+    }
+    // bending slots, 64 of one type per wave and round, on the waves of parts 1..3
+    const int wave = (int)__builtin_amdgcn_readfirstlane((uint32_t)tid >> 6), nw = 12;
+    if (qpart > 0)
+#pragma unroll
+        for (int u0 = 0; u0 < F::UNITS; u0 += nw) {
+            const int u = u0 + 15 - wave;
+            if (u < F::UX) {
+                if (!(sg.flags & VTX_SEG_NONE_X)) fuse_slot<T, T, 0>(d, sg, sp, corr, mark, a0, b0, u * 64 + tid % 64, xpbd);
+            } else if (u < F::UX + F::UR) {
+                if (!(sg.flags & VTX_SEG_NONE_R))
+                    fuse_slot<T, T, 1>(d, sg, sp, corr, mark, a0, b0, (u - F::UX) * 64 + tid % 64, xpbd);
+            } else if (u < F::UNITS) {
+                if (!(sg.flags & VTX_SEG_NONE_D))
+                    fuse_slot<T, T, 2>(d, sg, sp, corr, mark, a0, b0, (u - F::UX - F::UR) * 64 + tid % 64, xpbd);
+            }
+        }
+    __syncthreads();
+    if (!inside) return;
+    delta += part;
+    cnt += pc;
+#pragma unroll
+    for (int q = 0; q < VTX_LRA_PARTS - 1; q++) {
+        const float4 e = lpart[q][lane];
+        delta += xyz(e);
+        cnt += __float_as_int(e.w);
+    }
+    __builtin_amdgcn_sched_barrier(0);                      // few words live at a time: 64 registers a thread
+    V3 bend = v3(0.f, 0.f, 0.f);
+    fuse_gather<T, T, 0>(corr, mark, y, x, bend, cnt);
+    __builtin_amdgcn_sched_barrier(0);
+    fuse_gather<T, T, 1>(corr, mark, y, x, bend, cnt);
+    __builtin_amdgcn_sched_barrier(0);
+    fuse_gather<T, T, 2>(corr, mark, y, x, bend, cnt);
+    delta = madd(delta, bend, w);
+    if (cnt > 0) p = madd(p, delta, frcp((float)cnt) * sg.omega);
+    epilogue<EPI>(d, sg, sg.pbase + (uint32_t)(a * cols + b), in, p, w, h);
 }
 
 // ComputeTriangleNormals + ComputeVertexNormals (Velvet/VtClothSolverGPU.cu:419-450) as a
@@ -1144,14 +1271,22 @@ hipError_t launch_collide(const DevState& d, int in, float h, int block, hipStre
     return last_launch();
 }
 
-template <int LB, int SPLIT>
-static void launch_iterate_grid(const DevState& d, const GridTileDev* tiles, uint32_t ntiles, int in, float h,
-                                int epilogue, hipStream_t s) {
-    if (!ntiles) return;
-    const dim3 gg(ntiles), bl(VTX_TILE * SPLIT);
-    if (epilogue == EPI_NONE) hipLaunchKernelGGL((k_iterate_grid<EPI_NONE, LB, SPLIT>), gg, bl, 0, s, d, tiles, in, h);
-    else if (epilogue == EPI_FINALIZE) hipLaunchKernelGGL((k_iterate_grid<EPI_FINALIZE, LB, SPLIT>), gg, bl, 0, s, d, tiles, in, h);
-    else hipLaunchKernelGGL((k_iterate_grid<EPI_FINALIZE_PREDICT, LB, SPLIT>), gg, bl, 0, s, d, tiles, in, h);
+static void launch_iterate_grid(const DevState& d, int in, float h, int epilogue, hipStream_t s) {
+    if (!d.ngtiles) return;
+    const dim3 gr(d.ngtiles), bl(VTX_TILE);
+    if (epilogue == EPI_NONE) hipLaunchKernelGGL(k_iterate_grid<EPI_NONE>, gr, bl, 0, s, d, d.gtiles, in, h);
+    else if (epilogue == EPI_FINALIZE) hipLaunchKernelGGL(k_iterate_grid<EPI_FINALIZE>, gr, bl, 0, s, d, d.gtiles, in, h);
+    else hipLaunchKernelGGL(k_iterate_grid<EPI_FINALIZE_PREDICT>, gr, bl, 0, s, d, d.gtiles, in, h);
+}
+
+// B: groups of four distances in flight per thread
+template <int B>
+static void launch_iterate_split(const DevState& d, int in, float h, int epilogue, hipStream_t s) {
+    if (!d.nltiles) return;
+    const dim3 gr(d.nltiles), bl(VTX_TILE * VTX_LRA_PARTS);
+    if (epilogue == EPI_NONE) hipLaunchKernelGGL((k_iterate_split<EPI_NONE, B>), gr, bl, 0, s, d, d.ltiles, in, h);
+    else if (epilogue == EPI_FINALIZE) hipLaunchKernelGGL((k_iterate_split<EPI_FINALIZE, B>), gr, bl, 0, s, d, d.ltiles, in, h);
+    else hipLaunchKernelGGL((k_iterate_split<EPI_FINALIZE_PREDICT, B>), gr, bl, 0, s, d, d.ltiles, in, h);
 }
 
 template <int RPT>
@@ -1161,18 +1296,6 @@ static void launch_iterate_mesh(const DevState& d, int in, float h, int epilogue
     if (epilogue == EPI_NONE) hipLaunchKernelGGL((k_iterate<EPI_NONE, RPT>), gr, bl, 0, s, d, d.itiles, in, h);
     else if (epilogue == EPI_FINALIZE) hipLaunchKernelGGL((k_iterate<EPI_FINALIZE, RPT>), gr, bl, 0, s, d, d.itiles, in, h);
     else hipLaunchKernelGGL((k_iterate<EPI_FINALIZE_PREDICT, RPT>), gr, bl, 0, s, d, d.itiles, in, h);
-}
-
-template <int LB>
-static void launch_iterate_lb(const DevState& d, int in, float h, int epilogue, hipStream_t s) {
-    launch_iterate_grid<LB, 1>(d, d.gtiles, d.ngtiles, in, h, epilogue, s);
-    // four threads per particle leave 128 registers per thread: batches of 64 would spill
-    launch_iterate_grid<(LB > 16 ? 16 : LB), VTX_LRA_PARTS>(d, d.ltiles, d.nltiles, in, h, epilogue, s);
-    // a tile's records in one round while every tile has a CU of its own (8.5 against 11.5 us for 90
-    // tiles of 1,334 records), else in rounds of half the LDS and twice the workgroups per CU (625 tiles
-    // 28.5 against 33.4 us)
-    if (d.nitiles <= 256) launch_iterate_mesh<2>(d, in, h, epilogue, s);
-    else launch_iterate_mesh<1>(d, in, h, epilogue, s);
 }
 
 hipError_t launch_iterate(const DevState& d, int in, float h, int epilogue, bool constraints, int lra_batch,
@@ -1185,9 +1308,15 @@ hipError_t launch_iterate(const DevState& d, int in, float h, int epilogue, bool
         else hipLaunchKernelGGL(k_epilogue<EPI_FINALIZE_PREDICT>, gr, bl, 0, s, d, in, h);
         return last_launch();
     }
-    if (lra_batch >= 64) launch_iterate_lb<64>(d, in, h, epilogue, s);
-    else if (lra_batch >= 16) launch_iterate_lb<16>(d, in, h, epilogue, s);
-    else launch_iterate_lb<4>(d, in, h, epilogue, s);
+    launch_iterate_grid(d, in, h, epilogue, s);
+    // four threads per vertex leave 128 registers a thread: a batch of 64 distances runs as 16
+    if (lra_batch >= 16) launch_iterate_split<4>(d, in, h, epilogue, s);
+    else launch_iterate_split<1>(d, in, h, epilogue, s);
+    // a tile's records in one round while every tile has a CU of its own (8.5 against 11.5 us for 90
+    // tiles of 1,334 records), else in rounds of half the LDS and twice the workgroups per CU (625 tiles
+    // 28.5 against 33.4 us)
+    if (d.nitiles <= 256) launch_iterate_mesh<2>(d, in, h, epilogue, s);
+    else launch_iterate_mesh<1>(d, in, h, epilogue, s);
     return last_launch();
 }
 

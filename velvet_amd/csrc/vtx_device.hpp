@@ -33,8 +33,13 @@
 #define VTX_SEG_NONE_R 128u
 #define VTX_SEG_NONE_D 256u
 // Attachments are "every particle to every slot, in slot order" (Velvet/VtClothObjectGPU.hpp:134-148):
-// only the distances are stored, slot-major: lra[lbase + slot * n + particle].
+// only the distances are stored, slot-major: lra[4 lbase + slot * n + particle].
 #define VTX_SEG_LRA_DENSE 512u
+// Dense attachments of a grid segment with at least VTX_LRA_SPLIT_MIN slots are stored tile by tile in
+// the order its passes read them (unless whole tiles would store far more than there are): per 16 x 16
+// tile (GridTileDev::at_off, in float4), part and group of four slots, one float4 of target distances
+// (times the stretchiness) per lane of the tile.
+#define VTX_SEG_LRA_TILED 8192u
 // The segment's spatial hash is built by one workgroup in LDS (k_hash_small): self-collision,
 // at most VTX_HASH_LDS_N particles and a table of at most 2^16 cells. The device-wide hash
 // kernels skip it.
@@ -55,8 +60,8 @@
 #define VTX_NBR16_N 65535u
 // A particle's attachment terms are summed in four parts by slot index -- slots
 // [q*Qs, (q+1)*Qs) with Qs = ceil(scount / 4) -- each part from zero in slot order, and the parts
-// are added to the particle's delta in order q = 0..3. One lane can run all four parts, or four
-// lanes one part each (stencil segments with at least VTX_LRA_SPLIT_MIN dense slots), with the
+// are added to the particle's delta in order q = 0..3. One lane runs all four parts, or four
+// lanes one part each (grid segments with at least VTX_LRA_SPLIT_MIN dense slots), with the
 // same result.
 #define VTX_LRA_PARTS 4
 // Most streams a frame's segment groups run on (vtx_tuning.streams).
@@ -89,7 +94,7 @@ struct alignas(16) SegDev {
     float gx, gy, gz, pad0;
     uint32_t mod_lo, mod_hi;               // ceil(2^64 / M): exact remainder by multiplication
     uint32_t rows, cols;                   // grid segments: vertex grid shape
-    uint32_t trbase, lbase, pad1, pad2;    // triangle-record / dense-LRA bases
+    uint32_t trbase, lbase, pad1, pad2;    // triangle-record base, dense-LRA base (in float4)
 };
 
 struct alignas(16) TileDev {
@@ -107,7 +112,7 @@ struct alignas(16) SortTileDev {
 
 struct alignas(16) GridTileDev {
     uint32_t seg, a0, b0, pad0;            // segment, first row / column of the tile
-    uint32_t at_off, at_k, pad1, pad2;     // attach ELL of the tile's lanes
+    uint32_t at_off, at_k, pad1, pad2;     // attach ELL of the tile's lanes, or its tiled dense distances
 };
 
 // Collider with its transforms as 3x4 row-major affine matrices:
