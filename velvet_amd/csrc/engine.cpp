@@ -1109,11 +1109,7 @@ void Engine::upload(Segment& sg, hipStream_t s) {
         d.gx = p.gravity[0];
         d.gy = p.gravity[1];
         d.gz = p.gravity[2];
-        if (selfcol) {
-            const uint64_t c = UINT64_MAX / d.M + 1;   // ceil(2^64 / M); wraps to 0 for M = 1
-            d.mod_lo = (uint32_t)(c & 0xFFFFFFFFu);
-            d.mod_hi = (uint32_t)(c >> 32);
-        }
+        if (selfcol) d.mod = mod_constant(d.M);
         d.rows = pr.grows;
         d.cols = pr.gcols;
         sg.dev = d;
@@ -1268,7 +1264,7 @@ void Engine::rebuild_tables() {
     std::vector<SegDev> hseg;
     std::vector<TileDev> htile, hitile;
     std::vector<GridTileDev> hgtile, hltile, hftile, hmtile;
-    std::vector<uint32_t> hsmall;                // table indices of segments hashed in LDS
+    std::vector<HashPartDev> hpart;                  // cell ranges of the segments k_hash_part builds
     std::vector<SortTileDev> hst;
     table_seg_.clear();
     any_selfcol_ = false;
@@ -1284,11 +1280,14 @@ void Engine::rebuild_tables() {
     // each group sorts on its own, so its scan positions restart at zero
     uint64_t total_n = 0;
     uint32_t nlive = 0;
+    bool hkeyed = false;                       // k_hash_keys runs ahead of k_hash_part
     for (auto& sp : segs_)
         if (sp && sp->active && sp->uploaded && sp->n()) {
             total_n += sp->n();
             nlive++;
+            hkeyed = hkeyed || (sp->selfcol() && sp->n() > VTX_HASH_PART_KEYS);
         }
+    hkeyed = hkeyed || total_n > VTX_HASH_PART_TOTAL;
     // G groups of about total/G particles each (a prefix of the segment table per group); timing
     // mode keeps one group so that per-launch figures cover the whole workload
     const uint32_t G = timing_ ? 1u : std::max(1u, std::min<uint32_t>((uint32_t)tun_.streams, nlive));
@@ -1310,7 +1309,7 @@ void Engine::rebuild_tables() {
         VTX_REQUIRE(p.num_substeps == substeps_ && p.num_iterations == iterations_ && p.interleaved_hash == interleave_,
                     VTX_EINVAL, "active segments of one solver must share substeps, iterations and interleave");
         if (cuts.size() + 1 < G && cum > 0 && cum * G >= total_n * (cuts.size() + 1)) {
-            cuts.push_back(Cut{htile.size(), hitile.size(), hgtile.size(), hltile.size(), hst.size(), hsmall.size(),
+            cuts.push_back(Cut{htile.size(), hitile.size(), hgtile.size(), hltile.size(), hst.size(), hpart.size(),
                                hftile.size(), hmtile.size(), hbase, (uint32_t)cum});
             compact = 0;                       // each group sorts on its own
         }
@@ -1321,18 +1320,23 @@ void Engine::rebuild_tables() {
             const bool shifted = sg.prm.tune_hash_grid && tun_.hash_grid > 0;
             any_grid_tunable_ = any_grid_tunable_ || sg.prm.tune_hash_grid;
             sg.dev.M = sg.grid_table_size(shifted ? tun_.hash_grid : 0);
-            const uint64_t c = UINT64_MAX / sg.dev.M + 1;   // ceil(2^64 / M); wraps to 0 for M = 1
-            sg.dev.mod_lo = (uint32_t)(c & 0xFFFFFFFFu);
-            sg.dev.mod_hi = (uint32_t)(c >> 32);
+            sg.dev.mod = mod_constant(sg.dev.M);
             sg.dev.flags = (sg.dev.flags & ~VTX_SEG_HASH_SHIFT) | (shifted ? VTX_SEG_HASH_SHIFT : 0u);
         }
-        const bool hlds = (sg.dev.flags & VTX_SEG_SELFCOL) && sg.dev.n <= VTX_HASH_LDS_N && sg.dev.M <= (1u << 16);
+        const bool hlds = (sg.dev.flags & VTX_SEG_SELFCOL) && sg.dev.n <= VTX_HASH_PART_N && sg.dev.M <= VTX_HASH_PART_M;
         any_hash_lds_ = any_hash_lds_ || hlds;
         const bool in_lds = hlds && tun_.hash_lds;
         hseg.push_back(sg.dev);
         if (in_lds) {
-            hseg.back().flags |= VTX_SEG_HASH_LDS;
-            hsmall.push_back(ti);
+            hseg.back().flags |= VTX_SEG_HASH_PART;
+            const SegDev& d = hseg.back();
+            const uint32_t share = total_n > VTX_HASH_PART_FULL ? VTX_HASH_PART_SHARE_FULL : VTX_HASH_PART_SHARE;
+            const uint32_t width = hash_part_width(d.n, d.M, share);
+            const bool keyed = hkeyed && d.n > share;   // each of several ranges would work every key out
+            if (keyed) hseg.back().flags |= VTX_SEG_HASH_KEYED;
+            for (uint32_t lo = 0; lo < d.M; lo += width)
+                hpart.push_back(HashPartDev{d.pbase, d.n, d.tbase, d.M, lo, std::min(width, d.M - lo), d.mod,
+                                            (d.flags & VTX_SEG_HASH_SHIFT) ? VTX_HASH_SHIFT : 0u, keyed, d.cell, {0u, 0u}});
         }
         const SegDev& d = sg.dev;
         live_particles_ += d.n;
@@ -1408,24 +1412,18 @@ void Engine::rebuild_tables() {
     d.nitiles = (uint32_t)hitile.size();
     d.ngtiles = (uint32_t)hgtile.size();
     d.nltiles = (uint32_t)hltile.size();
-    d.nhsegs = (uint32_t)hsmall.size();
+    d.nhparts = (uint32_t)hpart.size();
     d.nftiles = (uint32_t)hftile.size();
     d.nmtiles = (uint32_t)hmtile.size();
     d.fside = fside;
+    d.hkeyed = hkeyed;
+    d.hfull = total_n > VTX_HASH_PART_FULL;
     d.nstiles = (uint32_t)hst.size();
     d.nhist = hbase;
     d.ncells = (uint32_t)acell_.cap;
-    {   // largest small segments first, within each group's range, so the longest builds start first
-        std::vector<size_t> edge{0};
-        for (const Cut& c : cuts) edge.push_back(c.m);
-        edge.push_back(hsmall.size());
-        for (size_t k = 0; k + 1 < edge.size(); k++)
-            std::stable_sort(hsmall.begin() + (ptrdiff_t)edge[k], hsmall.begin() + (ptrdiff_t)edge[k + 1],
-                             [&](uint32_t a, uint32_t b) { return hseg[a].n > hseg[b].n; });
-    }
     TableSet ts;
     const size_t k_seg = ts.add(hseg), k_tile = ts.add(htile), k_itile = ts.add(hitile), k_gtile = ts.add(hgtile),
-                 k_ltile = ts.add(hltile), k_st = ts.add(hst), k_hs = ts.add(hsmall),
+                 k_ltile = ts.add(hltile), k_st = ts.add(hst), k_hs = ts.add(hpart),
                  k_ft = ts.add(hftile), k_mt = ts.add(hmtile);
     upload_tables(ts);
     d.segs = (const SegDev*)(tab_dev_ + ts.off[k_seg]);
@@ -1434,7 +1432,7 @@ void Engine::rebuild_tables() {
     d.gtiles = (const GridTileDev*)(tab_dev_ + ts.off[k_gtile]);
     d.ltiles = (const GridTileDev*)(tab_dev_ + ts.off[k_ltile]);
     d.stiles = (const SortTileDev*)(tab_dev_ + ts.off[k_st]);
-    d.hsegs = (const uint32_t*)(tab_dev_ + ts.off[k_hs]);
+    d.hparts = (const HashPartDev*)(tab_dev_ + ts.off[k_hs]);
     d.ftiles = (const GridTileDev*)(tab_dev_ + ts.off[k_ft]);
     d.mtiles = (const GridTileDev*)(tab_dev_ + ts.off[k_mt]);
     d.X = pl_.X;
@@ -1469,7 +1467,7 @@ void Engine::rebuild_tables() {
     d.hbase0 = 0;
     ds_ = d;
     groups_.clear();
-    cuts.push_back(Cut{htile.size(), hitile.size(), hgtile.size(), hltile.size(), hst.size(), hsmall.size(),
+    cuts.push_back(Cut{htile.size(), hitile.size(), hgtile.size(), hltile.size(), hst.size(), hpart.size(),
                        hftile.size(), hmtile.size(), hbase, d.nparticles});
     Cut lo{};
     for (size_t k = 0; k < cuts.size(); k++) {
@@ -1480,8 +1478,8 @@ void Engine::rebuild_tables() {
         g.gtiles = d.gtiles + lo.g;
         g.ltiles = d.ltiles + lo.l;
         g.stiles = d.stiles + lo.s;
-        g.hsegs = d.hsegs + lo.m;
-        g.nhsegs = (uint32_t)(hi.m - lo.m);
+        g.hparts = d.hparts + lo.m;
+        g.nhparts = (uint32_t)(hi.m - lo.m);
         g.ftiles = d.ftiles + lo.f;
         g.mtiles = d.mtiles + lo.n;
         g.nftiles = (uint32_t)(hi.f - lo.f);
@@ -1575,16 +1573,20 @@ void Engine::stage_end(hipStream_t s) {
 
 // SpatialHashGPU::Hash -> HashObjects (Velvet/SpatialHashGPU.hpp:41-52, Velvet/SpatialHashGPU.cu:159-196).
 void Engine::hash_build(const DevState& d, int in, hipStream_t s) {
-    // small segments: the whole build in one workgroup each, into the buffer the device-wide
-    // sort of the other segments ends in
-    stage_begin("k_hash_small", "Solver_HashParticle+Solver_HashSort+Solver_HashBuildCell", s);
-    VTX_HIP(launch_hash_small(d, in, passes_ & 1, s));
-    stage_end(s);
-    int src = passes_ & 1;
-    if (d.nstiles) {   // segments on the device-wide path (every segment has sort tiles but those above)
+    // segments of k_hash_part build into the buffer the device-wide sort of the others ends in
+    const int dst = passes_ & 1;
+    int src = dst;
+    if (d.nstiles || d.hkeyed) {
         stage_begin("k_hash_keys", "Solver_HashParticle", s);
-        VTX_HIP(launch_hash_keys(d, in, s));
+        VTX_HIP(launch_hash_keys(d, in, dst, s));
         stage_end(s);
+    }
+    if (d.nhparts) {
+        stage_begin("k_hash_part", "Solver_HashParticle+Solver_HashSort+Solver_HashBuildCell", s);
+        VTX_HIP(launch_hash_parts(d, in, dst, s));
+        stage_end(s);
+    }
+    if (d.nstiles) {   // segments on the device-wide path (every segment has sort tiles but those above)
         stage_begin("k_sort_hist+k_scan_reduce+k_scan_apply+k_sort_scatter", "Solver_HashSort", s);
         src = 0;
         for (int pass = 0; pass < passes_; pass++) {

@@ -140,7 +140,7 @@ struct Tuning {
     int streams = 1;          // k > 1: segments split into k particle-balanced groups whose frames
                               // run on k streams, overlapping latency- and VALU-bound stages
     bool lra_split = true;    // kept for callers (vtx_tuning.lra_split), no effect
-    bool hash_lds = true;     // small self-colliding segments build their hash in one workgroup
+    bool hash_lds = true;     // self-colliding segments up to 2^17 particles build their hash by cell ranges
     int hash_grid = 0;        // hash-grid resolution of segments with tune_hash_grid: 0 the
                               // reference grid; 1..3 origin shifted, table 1x / 2x / 4x. The only
                               // field that changes results (list order, bucket sharing)
@@ -321,7 +321,7 @@ private:
     Tuning tun_;
     bool any_lra_dense_ = false;
     bool any_lra_split_ = false;   // a stencil segment has tiled dense attachments
-    bool any_hash_lds_ = false;    // a self-colliding segment is small enough for k_hash_small
+    bool any_hash_lds_ = false;    // a self-colliding segment is small enough for k_hash_part
     bool any_grid_tunable_ = false;   // a live self-colliding segment has tune_hash_grid
     bool use_stencil_ = true;
     hipGraphExec_t gexec_ = nullptr;

@@ -1,7 +1,8 @@
 // Spatial-hash build for gfx950: cell hash, stable LSD radix sort, cell start/end and the
 // cached neighbour table (Velvet/SpatialHashGPU.cu:13-196).
 //
-// All segments are sorted in one pass sequence. Keys are the per-segment hash (< M of that
+// Segments of up to 2^17 particles are built by cell ranges (k_hash_part). The others are sorted in one
+// device-wide pass sequence. Keys are the per-segment hash (< M of that
 // segment), values the local particle index. Sort tiles never straddle segments and the
 // digit histograms are laid out (segment, digit, tile), so one exclusive scan over the whole
 // histogram gives every (segment, digit, tile) its global output offset: the segments come
@@ -13,6 +14,7 @@
 #include <hip/hip_runtime.h>
 
 #include <mutex>
+#include <type_traits>
 
 #include "launch.hpp"
 #include "vec.hpp"
@@ -22,18 +24,16 @@ namespace vtx {
 
 
 // HashCoords (Velvet/SpatialHashGPU.cu:18-22): 32-bit wrap-around products, then
-// abs(h % M). |h % M| == |h| mod M for C's truncating remainder, and the unsigned remainder is
-// taken by multiplication with c = ceil(2^64 / M): ((c * a) mod 2^64) * M >> 64 == a mod M for
-// all 32-bit a and M (Lemire, Kaser, Kurz, "Faster remainder by direct computation", 2019).
-__device__ __forceinline__ uint32_t hash_coords(int32_t x, int32_t y, int32_t z, uint32_t M, uint64_t c) {
+// abs(h % M). |h % M| == |h| mod M for C's truncating remainder, and the unsigned remainder of
+// a <= 2^31 takes one product with m = floor(2^32 / M) (mod_constant): a/M - a m / 2^32 < a / 2^32 <= 1/2,
+// so the quotient's floor is right or one too small, and one subtraction mends it.
+__device__ __forceinline__ uint32_t hash_coords(int32_t x, int32_t y, int32_t z, uint32_t M, uint32_t m) {
     const int32_t h = (int32_t)(((uint32_t)x * 92837111u) ^ ((uint32_t)y * 689287499u) ^
                                 ((uint32_t)z * 283923481u));
-    const uint32_t a = h < 0 ? (uint32_t)(-(int64_t)h) : (uint32_t)h;
-    const uint64_t low = c * (uint64_t)a;
-    return (uint32_t)__umul64hi(low, (uint64_t)M);
+    const uint32_t a = h < 0 ? 0u - (uint32_t)h : (uint32_t)h;
+    const uint32_t r = a - __umulhi(a, m) * M;
+    return min(r, r - M);
 }
-
-__device__ __forceinline__ uint64_t seg_mod(const SegDev& sg) { return (uint64_t)sg.mod_hi << 32 | sg.mod_lo; }
 
 // ComputeIntCoord (Velvet/SpatialHashGPU.cu:13-16): floor of a correctly rounded binary32
 // quotient (the library is built with -fhip-fp32-correctly-rounded-divide-sqrt).
@@ -41,10 +41,33 @@ __device__ __forceinline__ int32_t int_coord(float v, float cell) {
     return (int32_t)floorf(__fdiv_rn(v, cell));
 }
 
-// Cell coordinate as hashed: ComputeIntCoord plus the segment's grid shift (0 on the reference
-// grid, VTX_HASH_SHIFT on a tuned one), with 32-bit wrap-around.
-__device__ __forceinline__ int32_t hash_coord(float v, float cell, uint32_t shift) {
-    return (int32_t)((uint32_t)int_coord(v, cell) + shift);
+// The cell of a position, as hashed: ComputeIntCoord plus the grid shift (0 on the reference grid,
+// VTX_HASH_SHIFT on a tuned one) with 32-bit wrap-around. t = v times the cell's reciprocal (1 ulp) is
+// within 2^-22 |t| of the quotient, so where t is more than 2^-20 |t| away from an integer its floor is
+// the rounded quotient's; the division runs for the rest (large, on a cell's face, not finite). A key
+// takes 50 VALU issue slots instead of 85.
+__device__ __forceinline__ void cell_coords(float4 p, float cell, uint32_t shift, int32_t& x, int32_t& y, int32_t& z) {
+    const float inv = __builtin_amdgcn_rcpf(cell);
+    const float tx = p.x * inv, ty = p.y * inv, tz = p.z * inv;
+    const float fx = floorf(tx), fy = floorf(ty), fz = floorf(tz);
+    const float gx = fabsf(tx - fx - 0.5f), gy = fabsf(ty - fy - 0.5f), gz = fabsf(tz - fz - 0.5f);
+    constexpr float E = 9.5367431640625e-07f;   // 2^-20
+    const bool clear = (gx < 0.5f - E * fabsf(tx)) & (gy < 0.5f - E * fabsf(ty)) & (gz < 0.5f - E * fabsf(tz));
+    int32_t cx = (int32_t)fx, cy = (int32_t)fy, cz = (int32_t)fz;
+    if (!clear) {
+        cx = int_coord(p.x, cell);
+        cy = int_coord(p.y, cell);
+        cz = int_coord(p.z, cell);
+    }
+    x = (int32_t)((uint32_t)cx + shift);
+    y = (int32_t)((uint32_t)cy + shift);
+    z = (int32_t)((uint32_t)cz + shift);
+}
+
+__device__ __forceinline__ uint32_t position_key(float4 p, float cell, uint32_t shift, uint32_t M, uint32_t m) {
+    int32_t x, y, z;
+    cell_coords(p, cell, shift, x, y, z);
+    return hash_coords(x, y, z, M, m);
 }
 
 __device__ __forceinline__ uint32_t seg_shift(const SegDev& sg) {
@@ -52,21 +75,22 @@ __device__ __forceinline__ uint32_t seg_shift(const SegDev& sg) {
 }
 
 // ComputeParticleHash_Kernel (Velvet/SpatialHashGPU.cu:34-42) over predicted positions.
-__global__ __launch_bounds__(VTX_TILE) void k_hash_keys(DevState d, int in) {
+// Segments that k_hash_part builds get theirs where it reads them: dst = the side its results go to.
+__global__ __launch_bounds__(VTX_TILE) void k_hash_keys(DevState d, int in, int dst) {
     const TileDev t = d.tiles[tile_of(d.remap)];
     if (threadIdx.x >= t.count) return;
     const SegDev sg = d.segs[t.seg];
     const uint32_t g = t.begin + threadIdx.x;
-    if (sg.flags & VTX_SEG_HASH_LDS) return;
-    d.vals[0][g] = g - sg.pbase;
+    const bool part = sg.flags & VTX_SEG_HASH_PART;
+    if (part && !(sg.flags & VTX_SEG_HASH_KEYED)) return;
+    if (!part) d.vals[0][g] = g - sg.pbase;
     if (!(sg.flags & VTX_SEG_SELFCOL)) {
         d.keys[0][g] = 0;      // segment without self-collision: sorted as one cell, unused
         return;
     }
     const float4 p = d.P[in][g];
     const uint32_t sh = seg_shift(sg);
-    d.keys[0][g] = hash_coords(hash_coord(p.x, sg.cell, sh), hash_coord(p.y, sg.cell, sh),
-                               hash_coord(p.z, sg.cell, sh), sg.M, seg_mod(sg));
+    d.keys[part ? dst ^ 1 : 0][g] = position_key(p, sg.cell, sh, sg.M, sg.mod);
 }
 
 // Digit histogram of one sort tile (count keys from `keys`): the count of digit g goes to
@@ -230,7 +254,7 @@ __global__ __launch_bounds__(VTX_TILE) void k_clear_cells(DevState d) {
     const TileDev t = d.tiles[tile_of(d.remap)];
     if (threadIdx.x >= t.count) return;
     const SegDev sg = d.segs[t.seg];
-    if (!(sg.flags & VTX_SEG_SELFCOL) || (sg.flags & VTX_SEG_HASH_LDS)) return;
+    if (!(sg.flags & VTX_SEG_SELFCOL) || (sg.flags & VTX_SEG_HASH_PART)) return;
     uint2* __restrict__ cells = d.cells + sg.tbase;
     for (uint32_t i = t.begin - sg.pbase + threadIdx.x; i < sg.M; i += sg.n) cells[i] = make_uint2(VTX_INVALID, VTX_INVALID);
 }
@@ -243,7 +267,7 @@ __global__ __launch_bounds__(VTX_TILE) void k_cell_bounds(DevState d, int in, in
     const TileDev t = d.tiles[tile_of(d.remap)];
     if (threadIdx.x >= t.count) return;
     const SegDev sg = d.segs[t.seg];
-    if (!(sg.flags & VTX_SEG_SELFCOL) || (sg.flags & VTX_SEG_HASH_LDS)) return;
+    if (!(sg.flags & VTX_SEG_SELFCOL) || (sg.flags & VTX_SEG_HASH_PART)) return;
     const uint32_t g = t.begin + threadIdx.x;
     const uint32_t local = g - sg.pbase;
     const uint32_t* __restrict__ sk = d.keys[src];
@@ -271,7 +295,7 @@ __global__ __launch_bounds__(VTX_TILE) void k_sorted_records(DevState d, int in,
     const TileDev t = d.tiles[tile_of(d.remap)];
     if (threadIdx.x >= t.count) return;
     const SegDev sg = d.segs[t.seg];
-    if (!(sg.flags & VTX_SEG_SELFCOL) || (sg.flags & VTX_SEG_HASH_LDS)) return;
+    if (!(sg.flags & VTX_SEG_SELFCOL) || (sg.flags & VTX_SEG_HASH_PART)) return;
     const uint32_t g = t.begin + threadIdx.x;
     const size_t o = 2 * (size_t)(sg.pbase + d.keys[src ^ 1][g]);
     const float4 q = d.P[in][g];
@@ -279,162 +303,246 @@ __global__ __launch_bounds__(VTX_TILE) void k_sorted_records(DevState d, int in,
     d.sPX[o + 1] = d.X0[g];
 }
 
-// The whole spatial-hash build of one small segment in one workgroup of VTX_HASH_LDS_BT threads:
-// keys of the predicted positions (k_hash_keys), a stable LSD radix sort in LDS on key << 16 |
-// local index (8 bits per pass; each wave counts its own contiguous chunk with LDS atomics and
-// then scatters it, 64 keys at a time ranked by wave ballots over the pass's digit bits, so only
-// three workgroup barriers per pass), the cell table (k_clear_cells + k_cell_bounds) and the
-// sorted records. The sort runs on one CU and is bound by its VALU issue (a wave64 instruction
-// takes four cycles of a 16-lane SIMD), hence the atomic counts: the ballot match is needed only
-// for the ranks of the stable scatter. The records are written from particle order through the
-// inverse permutation (kept in the free sort buffer): the positions and initial positions are
-// read coalesced and each 32-B record is one scattered write, where the sorted-order form gathers
-// two scattered 16-B reads per particle (batch of 512 cloths: 99.6 -> 79.2 us per build).
-// Same keys, same stable order, so the same table and records as the device-wide path, in one
-// launch for every small segment instead of a dozen over all of them.
-// NMAX: particles per segment at most (16384: 144 KB of LDS, one workgroup per CU). Global
-// loads are issued eight elements at a time so that their latencies overlap.
-#define VTX_HASH_LDS_BT 1024
-template <uint32_t NMAX>
-__global__ __launch_bounds__(VTX_HASH_LDS_BT) void k_hash_small(DevState d, const uint32_t* __restrict__ list, int in,
-                                                                int dst) {
-    constexpr uint32_t NW = VTX_HASH_LDS_BT / 64;
-    __shared__ uint32_t buf[2][NMAX];                // key << 16 | local index
-    __shared__ uint32_t wcnt[NW][256];               // per wave: digit counts, then running offsets
-    __shared__ uint32_t wsum[4];
-    const SegDev sg = d.segs[list[blockIdx.x]];
-    const uint32_t n = sg.n, M = sg.M, tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    uint2* __restrict__ cells = d.cells + sg.tbase;
-    for (uint32_t i = tid; i < M; i += VTX_HASH_LDS_BT) cells[i] = make_uint2(VTX_INVALID, VTX_INVALID);
-    const uint64_t mc = seg_mod(sg);
-    const uint32_t sh = seg_shift(sg);
-    const float4* __restrict__ P = d.P[in] + sg.pbase;
-    // the predicted positions stay in registers (NMAX / STEP rounds of U per thread) until the
-    // sorted records are written: the workgroup runs alone on its CU, so the 48 extra VGPRs cost
-    // no occupancy, and the records then read only the initial positions (75.0 against 78.7 us for
-    // the batch of 512 cloths)
-    constexpr uint32_t U = 8, STEP = U * VTX_HASH_LDS_BT, NS = (NMAX + STEP - 1) / STEP;
-    float kx[NS][U], ky[NS][U], kz[NS][U];
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ uint32_t dpp0(uint32_t v) {   // the source lane's v, 0 where there is none
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+}
+
+// Inclusive sum over lanes 0..31 (lanes 32..63: over themselves), inclusive sum and maximum over the wave.
+__device__ __forceinline__ uint32_t scan32_add(uint32_t v) {
+    v += dpp0<0x111>(v);          // row_shr:1, 2, 4, 8
+    v += dpp0<0x112>(v);
+    v += dpp0<0x114>(v);
+    v += dpp0<0x118>(v);
+    return v + dpp0<0x142, 0xa>(v);   // row_bcast:15
+}
+
+__device__ __forceinline__ uint32_t scan64_add(uint32_t v) {
+    v = scan32_add(v);
+    return v + dpp0<0x143, 0xc>(v);   // row_bcast:31
+}
+
+__device__ __forceinline__ uint32_t scan64_max(uint32_t v) {
+    v = max(v, dpp0<0x111>(v));
+    v = max(v, dpp0<0x112>(v));
+    v = max(v, dpp0<0x114>(v));
+    v = max(v, dpp0<0x118>(v));
+    v = max(v, dpp0<0x142, 0xa>(v));
+    return max(v, dpp0<0x143, 0xc>(v));   // row_bcast:31
+}
+
+// The whole spatial-hash build of one segment of at most VTX_HASH_PART_N particles in one launch (after
+// k_hash_keys, see VTX_HASH_PART_KEYS): the table's cells are cut into ranges, and a workgroup builds one
+// range on its own. It runs over the keys of all particles, counts those in its range per cell in LDS and
+// those below the range (the range's first sorted position), scans the counts, puts the range's particles
+// into their cells in any order and finds each one's place inside its cell by counting the cell's smaller
+// indices: a stable sort by key, so the same table and records as the device-wide path. A cell of more
+// than VTX_HASH_HEAVY particles is placed by one more run over the keys in index order instead, so that
+// no input costs quadratic time.
+// Bound by latency: a launch's 2.6 us, then the chain range record, keys, LDS counts, scan, placement,
+// gathered records, and from 2^15 particles on the two runs over the keys. No workgroup waits for another,
+// where the dozen launches of a device-wide sort did and one workgroup per segment with a radix sort in
+// LDS took one CU for the whole of it: 4,608 particles 20 -> 8.5 us (one workgroup), 16,384 55 -> 14.4
+// (one workgroup; k_hash_keys included, as below), 22,500 49 -> 16 (device-wide), 65,536 73 -> 25,
+// 131,044 in a frame of four builds 492 -> 354, 16 cloths of 65,536 1338 -> 1122 a frame of four builds.
+struct HashPartLds {
+    uint32_t cnt[VTX_HASH_PART_CELLS];      // per cell of the range: count, start, end (exclusive)
+    uint32_t list[VTX_HASH_PART_LIST + 3];  // the range's particles by cell: cell << 20 | index
+    uint32_t heavy[VTX_HASH_PART_N / VTX_HASH_HEAVY];
+    uint32_t wsum[16], nheavy, below;
+};
+
+// S: the particles (key(i), written(g, key, i) for sorted position g, cell(k, begin, end)).
+template <uint32_t BT, bool KEYED, class S>
+__device__ __forceinline__ void hash_part(const S& s, uint32_t n, uint32_t lo, uint32_t C, uint32_t* __restrict__ spill,
+                                          HashPartLds& L) {
+    constexpr uint32_t NW = BT / 64, U = 8, Q = VTX_HASH_PART_CELLS / (4 * BT);
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 #pragma unroll
-    for (uint32_t s0 = 0; s0 < NS; s0++) {
-        const uint32_t i0 = tid + s0 * STEP;
+    for (uint32_t q = 0; q < Q; q++) reinterpret_cast<uint4*>(L.cnt)[q * BT + tid] = make_uint4(0u, 0u, 0u, 0u);
+    if (tid == 0) L.nheavy = L.below = 0u;
+    __syncthreads();
+    // counts
+    uint32_t kk[U], below = 0;
+    const uint32_t rounds = KEYED ? n : 1u;
+    for (uint32_t i0 = 0; i0 < rounds; i0 += U * BT) {
+        s.template load<BT, U>(i0 + tid, kk);
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++) {
+            if (i0 + u * BT >= n) break;
+            const bool valid = i0 + u * BT + tid < n;
+            below += valid && kk[u] < lo;
+            kk[u] = valid ? kk[u] - lo : VTX_INVALID;
+            if (kk[u] < C) atomicAdd(&L.cnt[kk[u]], 1u);
+        }
+    }
+    below = scan64_add(below);
+    if (lane == 63 && below) atomicAdd(&L.below, below);
+    __syncthreads();
+    // exclusive scan, consecutive cells per thread
+    uint4 c4[Q];
+    uint32_t sum = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < Q; q++) {
+        const uint4 c = c4[q] = reinterpret_cast<const uint4*>(L.cnt)[Q * tid + q];
+        sum += c.x + c.y + c.z + c.w;
+        if (max(max(c.x, c.y), max(c.z, c.w)) > VTX_HASH_HEAVY) {
+            const uint32_t k = 4 * (Q * tid + q);
+            if (c.x > VTX_HASH_HEAVY) L.heavy[atomicAdd(&L.nheavy, 1u)] = k;
+            if (c.y > VTX_HASH_HEAVY) L.heavy[atomicAdd(&L.nheavy, 1u)] = k + 1;
+            if (c.z > VTX_HASH_HEAVY) L.heavy[atomicAdd(&L.nheavy, 1u)] = k + 2;
+            if (c.w > VTX_HASH_HEAVY) L.heavy[atomicAdd(&L.nheavy, 1u)] = k + 3;
+        }
+    }
+    const uint32_t incl = scan64_add(sum);
+    if (lane == 63) L.wsum[wave] = incl;
+    __syncthreads();
+    static_assert(NW <= 16, "the waves' sums are scanned in rows of 16 lanes");
+    uint32_t ws = (lane & 15u) < NW ? L.wsum[lane & 15u] : 0u;
+    ws += dpp0<0x111>(ws);
+    ws += dpp0<0x112>(ws);
+    ws += dpp0<0x114>(ws);
+    ws += dpp0<0x118>(ws);
+    const uint32_t own = (uint32_t)__builtin_amdgcn_readlane((int)ws, 15);
+    uint32_t off = incl - sum + (wave ? (uint32_t)__builtin_amdgcn_readlane((int)ws, (int)wave - 1) : 0u);
+#pragma unroll
+    for (uint32_t q = 0; q < Q; q++) {
+        const uint4 c = c4[q];
+        reinterpret_cast<uint4*>(L.cnt)[Q * tid + q] = make_uint4(off, off + c.x, off + c.x + c.y, off + c.x + c.y + c.z);
+        off += c.x + c.y + c.z + c.w;
+    }
+    const uint32_t base = L.below, nheavy = L.nheavy;
+    __syncthreads();
+    // the range's particles into their cells, in any order; more than fit go through global scratch
+    const auto rest = [&](uint32_t* __restrict__ list, auto clamp) {
+        for (uint32_t i0 = 0; i0 < rounds; i0 += U * BT) {
+            if (KEYED && n > U * BT) s.template load<BT, U>(i0 + tid, kk);
+#pragma unroll
+            for (uint32_t u = 0; u < U; u++) {
+                if (i0 + u * BT >= n) break;
+                const uint32_t i = i0 + u * BT + tid;
+                const uint32_t k = KEYED && n > U * BT ? (i < n ? kk[u] - lo : VTX_INVALID) : kk[u];
+                if (k < C) list[atomicAdd(&L.cnt[k], 1u)] = k << 20 | i;
+            }
+        }
+        __syncthreads();
+        for (uint32_t g = tid; g < own; g += BT) {
+            const uint32_t e = list[g], k = e >> 20;
+            const uint32_t begin = k ? L.cnt[k - 1] : 0u, end = L.cnt[k];
+            if (end - begin > VTX_HASH_HEAVY) continue;
+            uint32_t at = begin;
+            for (uint32_t j = begin; j < end; j += 4) {   // what follows the cell in the list is larger than e
+                uint32_t o[4];
+#pragma unroll
+                for (uint32_t u = 0; u < 4; u++) o[u] = list[clamp.value ? min(j + u, own - 1u) : j + u];
+#pragma unroll
+                for (uint32_t u = 0; u < 4; u++) at += (!clamp.value || j + u < own) && o[u] < e;
+            }
+            s.put(base + at, lo + k, e & 0xFFFFFu);
+        }
+    };
+    if (own <= VTX_HASH_PART_LIST) {
+        if (tid < 3) L.list[own + tid] = VTX_INVALID;
+        rest(L.list, std::false_type{});
+    } else {
+        rest(spill + base, std::true_type{});
+    }
+    for (uint32_t k = tid; k < C; k += BT) {
+        const uint32_t begin = k ? L.cnt[k - 1] : 0u, end = L.cnt[k];
+        s.cell(lo + k, end > begin ? base + begin : VTX_INVALID, end > begin ? base + end : VTX_INVALID);
+    }
+    // heavy cells: wave w takes the w-th part of the particles; its matches before the others' counts
+    for (uint32_t h = 0; h < nheavy; h++) {
+        const uint32_t k = L.heavy[h], chunk = (n + NW - 1) / NW;
+        const uint32_t b = min(wave * chunk, n), e = min(b + chunk, n);
+        uint32_t count = 0;
+        for (uint32_t i0 = b; i0 < e; i0 += 64) {
+            const uint32_t i = i0 + lane;
+            count += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(i < e && s.key(min(i, n - 1u)) == lo + k));
+        }
+        __syncthreads();
+        if (lane == 0) L.wsum[wave] = count;
+        __syncthreads();
+        uint32_t at = base + (k ? L.cnt[k - 1] : 0u);
+        for (uint32_t w = 0; w < wave; w++) at += L.wsum[w];
+        for (uint32_t i0 = b; i0 < e; i0 += 64) {
+            const uint32_t i = i0 + lane;
+            const bool hit = i < e && s.key(min(i, n - 1u)) == lo + k;
+            const uint64_t mask = __builtin_amdgcn_ballot_w64(hit);
+            if (hit) s.put(at + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull)), lo + k, i);
+            at += (uint32_t)__popcll(mask);
+        }
+    }
+}
+
+// A segment's particles: float4 positions, keys from k_hash_keys or worked out here.
+template <bool KEYED>
+struct SegmentHash {
+    const float4 *P, *X0;
+    const uint32_t* keys;
+    uint2* cells;
+    float4* rec;
+    uint32_t *ko, *vo;
+    uint32_t mod;
+    float size;
+    uint32_t n, M, shift;
+    __device__ __forceinline__ uint32_t of(float4 p) const {
+        return position_key(p, size, shift, M, mod);
+    }
+    __device__ __forceinline__ uint32_t key(uint32_t i) const { return KEYED ? keys[i] : of(P[i]); }
+    template <uint32_t BT, uint32_t U>
+    __device__ __forceinline__ void load(uint32_t i, uint32_t (&k)[U]) const {
+        if (KEYED) {
+#pragma unroll
+            for (uint32_t u = 0; u < U; u++) k[u] = keys[min(i + u * BT, n - 1u)];
+            return;
+        }
         float4 p[U];
 #pragma unroll
         for (uint32_t u = 0; u < U; u++) {
-            const uint32_t i = i0 + u * VTX_HASH_LDS_BT;
-            p[u] = i < n ? P[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+            p[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (i + u * BT < n) p[u] = P[i + u * BT];
         }
 #pragma unroll
         for (uint32_t u = 0; u < U; u++) {
-            const uint32_t i = i0 + u * VTX_HASH_LDS_BT;
-            kx[s0][u] = p[u].x;
-            ky[s0][u] = p[u].y;
-            kz[s0][u] = p[u].z;
-            if (i < n)
-                buf[0][i] = hash_coords(hash_coord(p[u].x, sg.cell, sh), hash_coord(p[u].y, sg.cell, sh),
-                                        hash_coord(p[u].z, sg.cell, sh), M, mc) << 16 | i;
+            k[u] = VTX_INVALID;
+            if (u * BT < n) k[u] = of(p[u]);
         }
     }
-    __syncthreads();
-    const uint32_t bits = M > 1 ? 32u - (uint32_t)__clz(M - 1u) : 0u;
-    const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    // wave w owns the contiguous chunk [c0, c1) of the array: the chunks in wave order and the
-    // keys in each chunk in order make the sort stable
-    const uint32_t chunk = (n + NW - 1) / NW;
-    const uint32_t c0 = min(wave * chunk, n), c1 = min(c0 + chunk, n);
-    uint32_t* __restrict__ hw = wcnt[wave];
-    uint32_t cur = 0;
-    for (uint32_t shift = 16; shift < 16 + bits; shift += 8) {
-        const int nb = (int)min(8u, 16u + bits - shift);   // digit bits of this pass (the key has `bits`)
-        // 1. per-wave digit counts (LDS atomics on the wave's own counters: order does not matter)
-        for (uint32_t k = lane; k < 256; k += 64) hw[k] = 0;
-        __builtin_amdgcn_wave_barrier();
-        for (uint32_t i = c0 + lane; i < c1; i += 64) atomicAdd(&hw[(buf[cur][i] >> shift) & 255u], 1u);
-        __syncthreads();
-        // 2. each digit's start: digits in order, then waves in order (first 256 threads)
-        uint32_t tot = 0, incl = 0;
-        if (tid < 256) {
-            for (uint32_t w = 0; w < NW; w++) tot += wcnt[w][tid];
-            incl = wave_incl_scan(tot);
-            if (lane == 63) wsum[wave] = incl;
-        }
-        __syncthreads();
-        if (tid < 256) {
-            uint32_t run = incl - tot;
-            for (uint32_t w = 0; w < wave; w++) run += wsum[w];
-            for (uint32_t w = 0; w < NW; w++) {
-                const uint32_t c = wcnt[w][tid];
-                wcnt[w][tid] = run;
-                run += c;
-            }
-        }
-        __syncthreads();
-        // 3. each wave scatters its chunk in order
-        for (uint32_t r0 = c0; r0 < c1; r0 += 64) {
-            const uint32_t i = r0 + lane;
-            const bool valid = i < c1;
-            const uint32_t e = valid ? buf[cur][i] : 0u;
-            const uint32_t dg = (e >> shift) & 255u;
-            // lanes with this lane's digit: per digit bit, the ballot of the bit or its complement
-            // (invalid lanes hold digit 0 and are cleared by the first mask)
-            uint64_t peers = __builtin_amdgcn_ballot_w64(valid);
-#pragma unroll
-            for (int b = 0; b < 8; b++) {
-                if (b >= nb) break;                 // bits above the key are zero in every digit
-                const uint32_t m = (uint32_t)((int32_t)(dg << (31 - b)) >> 31);   // bit b as 0 / ~0
-                const uint64_t bal = __builtin_amdgcn_ballot_w64(m != 0u);
-                peers &= ~(bal ^ ((uint64_t)m << 32 | m));   // lanes whose bit b equals this lane's
-            }
-            const uint32_t rank = (uint32_t)__popcll(peers & lt);
-            const uint32_t at = hw[dg];
-            if (valid) buf[cur ^ 1][at + rank] = e;
-            __builtin_amdgcn_wave_barrier();
-            if (valid && rank == 0) hw[dg] = at + (uint32_t)__popcll(peers);
-            __builtin_amdgcn_wave_barrier();
-        }
-        __syncthreads();
-        cur ^= 1;
+    __device__ __forceinline__ void put(uint32_t g, uint32_t k, uint32_t i) const {
+        const float4 p = P[i], x = X0[i];
+        ko[g] = k;
+        vo[g] = i;
+        rec[2 * (size_t)g] = make_float4(p.x, p.y, p.z, __uint_as_float(i));
+        rec[2 * (size_t)g + 1] = x;
     }
-    // sorted keys and values, cell start / end (as k_cell_bounds); the inverse permutation
-    uint32_t* __restrict__ ko = d.keys[dst] + sg.pbase;
-    uint32_t* __restrict__ vo = d.vals[dst] + sg.pbase;
-    uint32_t* __restrict__ inv = buf[cur ^ 1];
-    for (uint32_t g = tid; g < n; g += VTX_HASH_LDS_BT) {
-        const uint32_t e = buf[cur][g], key = e >> 16, id = e & 0xFFFFu;
-        inv[id] = g;
-        ko[g] = key;
-        vo[g] = id;
-        if (g == 0) {
-            cells[key].x = 0;
-        } else {
-            const uint32_t prev = buf[cur][g - 1] >> 16;
-            if (key != prev) {
-                cells[key].x = g;
-                cells[prev].y = g;
-            }
-        }
-        if (g == n - 1) cells[key].y = n;
-    }
-    __syncthreads();
-    // sorted records written from particle order: coalesced reads, scattered 32-B records
-#pragma unroll
-    for (uint32_t s0 = 0; s0 < NS; s0++) {
-        const uint32_t i0 = tid + s0 * STEP;
-        float4 x0[U];
-#pragma unroll
-        for (uint32_t u = 0; u < U; u++) {
-            const uint32_t i = i0 + u * VTX_HASH_LDS_BT;
-            x0[u] = i < n ? d.X0[sg.pbase + i] : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < U; u++) {
-            const uint32_t i = i0 + u * VTX_HASH_LDS_BT;
-            if (i >= n) continue;
-            const size_t o = 2 * (size_t)(sg.pbase + inv[i]);
-            d.sPX[o] = make_float4(kx[s0][u], ky[s0][u], kz[s0][u], __uint_as_float(i));
-            d.sPX[o + 1] = x0[u];
-        }
-    }
+    __device__ __forceinline__ void cell(uint32_t k, uint32_t begin, uint32_t end) const { cells[k] = make_uint2(begin, end); }
+};
+
+template <uint32_t BT, bool KEYED>
+__device__ __forceinline__ void hash_part_segment(const DevState& d, const HashPartDev& t, int in, int dst, HashPartLds& L) {
+    SegmentHash<KEYED> s;
+    s.P = d.P[in] + t.pbase;
+    s.X0 = d.X0 + t.pbase;
+    s.keys = d.keys[dst ^ 1] + t.pbase;
+    s.cells = d.cells + t.tbase;
+    s.rec = d.sPX + 2 * (size_t)t.pbase;
+    s.ko = d.keys[dst] + t.pbase;
+    s.vo = d.vals[dst] + t.pbase;
+    s.mod = t.mod;
+    s.size = t.cell;
+    s.n = t.n;
+    s.M = t.M;
+    s.shift = t.shift;
+    hash_part<BT, KEYED>(s, t.n, t.lo, t.cells, d.vals[dst ^ 1] + t.pbase, L);
+}
+
+template <uint32_t BT>
+__global__ __launch_bounds__(BT, 8) void k_hash_part(DevState d, int in, int dst) {
+    __shared__ HashPartLds lds;
+    const HashPartDev t = d.hparts[tile_of(d.remap)];   // the ranges of a segment on one XCD: they read the same particles
+    if (t.keyed) hash_part_segment<BT, true>(d, t, in, dst, lds);
+    else hash_part_segment<BT, false>(d, t, in, dst, lds);
 }
 
 // CacheNeighbors_Kernel (Velvet/SpatialHashGPU.cu:79-130). Cells are visited x-, y-, z-nested;
@@ -456,7 +564,7 @@ struct NbSet {
     const float4* rec;    // sorted records: position with w = index at 2i, initial position at 2i + 1
     const uint2* cells;   // (start, end) per hash cell
     char* table;          // neighbour lists
-    uint64_t mc;          // ceil(2^64 / M)
+    uint32_t mod;         // mod_constant(M)
     uint32_t n, M, K, shift;
     float cell, cell2, diam2;
     bool n16;             // 16-bit entries
@@ -489,29 +597,6 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <int CTRL, int ROWS = 0xf>
-__device__ __forceinline__ uint32_t dpp0(uint32_t v) {   // the source lane's v, 0 where there is none
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
-}
-
-// Inclusive sum over lanes 0..31 (later lanes undefined), inclusive maximum over the wave.
-__device__ __forceinline__ uint32_t scan32_add(uint32_t v) {
-    v += dpp0<0x111>(v);          // row_shr:1, 2, 4, 8
-    v += dpp0<0x112>(v);
-    v += dpp0<0x114>(v);
-    v += dpp0<0x118>(v);
-    return v + dpp0<0x142, 0xa>(v);   // row_bcast:15
-}
-
-__device__ __forceinline__ uint32_t scan64_max(uint32_t v) {
-    v = max(v, dpp0<0x111>(v));
-    v = max(v, dpp0<0x112>(v));
-    v = max(v, dpp0<0x114>(v));
-    v = max(v, dpp0<0x118>(v));
-    v = max(v, dpp0<0x142, 0xa>(v));
-    return max(v, dpp0<0x143, 0xc>(v));   // row_bcast:31
-}
-
 // A sorted record through the scalar cache (i wave-uniform).
 __device__ __forceinline__ void ld_record_uniform(const float4* rec, uint32_t i, float4& p, float4& o) {
     typedef const float __attribute__((address_space(4))) cfloat;
@@ -530,8 +615,8 @@ __device__ __forceinline__ void neighbor_wave(const NbSet& a, uint32_t i0, uint3
     // the wave's particles: cells, runs
     float4 me = make_float4(0.f, 0.f, 0.f, 0.f);
     if (lane < cnt) me = a.rec[2 * (size_t)(i0 + lane)];
-    const int32_t ix = hash_coord(me.x, a.cell, a.shift), iy = hash_coord(me.y, a.cell, a.shift),
-                  iz = hash_coord(me.z, a.cell, a.shift);
+    int32_t ix, iy, iz;
+    cell_coords(me, a.cell, a.shift, ix, iy, iz);
     // every lane active in the exchange: one that sits out would hand its neighbour nothing
     const int32_t px = __shfl_up(ix, 1, 64), py = __shfl_up(iy, 1, 64), pz = __shfl_up(iz, 1, 64);
     const bool head = lane < cnt && ((lane == 0) | (px != ix) | (py != iy) | (pz != iz));
@@ -550,7 +635,7 @@ __device__ __forceinline__ void neighbor_wave(const NbSet& a, uint32_t i0, uint3
         const uint32_t dx = (q * 57u) >> 9, yz = q - 9u * dx;           // q / 9 for q < 27
         const uint32_t dy = (yz * 11u) >> 5, dz = yz - 3u * dy;         // yz / 3 for yz < 9
         const uint32_t hq = hash_coords(L.cx[r] + (int32_t)dx - 1, L.cy[r] + (int32_t)dy - 1,
-                                        L.cz[r] + (int32_t)dz - 1, a.M, a.mc);
+                                        L.cz[r] + (int32_t)dz - 1, a.M, a.mod);
         const uint64_t c = *reinterpret_cast<const uint64_t*>(a.cells + hq);   // one 8-byte load
         const uint32_t st = (uint32_t)c, len = min((uint32_t)(c >> 32) - st, a.K);
         L.range[t] = st == VTX_INVALID ? 0u : st | len << 25;
@@ -629,7 +714,7 @@ __global__ __launch_bounds__(256) void k_neighbors(DevState d) {
     a.rec = d.sPX + 2 * (size_t)sg.pbase;
     a.cells = d.cells + sg.tbase;
     a.table = reinterpret_cast<char*>(d.nbr + ((uint64_t)sg.nbase_hi << 32 | sg.nbase_lo));
-    a.mc = seg_mod(sg);
+    a.mod = sg.mod;
     a.n = sg.n;
     a.M = sg.M;
     a.K = sg.max_nbr;
@@ -654,12 +739,12 @@ __device__ __forceinline__ float4 ld_xyz(const float* __restrict__ a, uint32_t i
 
 // ComputeParticleHash_Kernel (Velvet/SpatialHashGPU.cu:34-42).
 __global__ __launch_bounds__(VTX_TILE) void k_raw_keys(const float* __restrict__ pos, uint32_t n, float cell,
-                                                       uint32_t M, uint64_t mc, uint32_t* __restrict__ keys,
+                                                       uint32_t M, uint32_t mod, uint32_t* __restrict__ keys,
                                                        uint32_t* __restrict__ vals) {
     const uint32_t i = blockIdx.x * VTX_TILE + threadIdx.x;
     if (i >= n) return;
     const float4 p = ld_xyz(pos, i, 0.f);
-    keys[i] = hash_coords(int_coord(p.x, cell), int_coord(p.y, cell), int_coord(p.z, cell), M, mc);
+    keys[i] = position_key(p, cell, 0u, M, mod);
     vals[i] = i;
 }
 
@@ -704,16 +789,72 @@ __global__ __launch_bounds__(VTX_TILE) void k_raw_cell_bounds(const uint32_t* __
     rec[2 * (size_t)g + 1] = ld_xyz(pos0, id, 0.f);
 }
 
+// The same table, arrays and records by cell ranges (hash_part), straight from the positions or from the
+// keys of k_raw_keys; the caller's cell arrays are written here too.
+template <bool KEYED>
+struct RawHash {
+    const float *pos, *pos0;
+    const uint32_t* keys;
+    uint2* cells;
+    float4* rec;
+    uint32_t *ko, *vo, *start, *end;
+    uint32_t mod;
+    float size;
+    uint32_t n, M;
+    __device__ __forceinline__ uint32_t of(float4 p) const {
+        return position_key(p, size, 0u, M, mod);
+    }
+    __device__ __forceinline__ uint32_t key(uint32_t i) const { return KEYED ? keys[i] : of(ld_xyz(pos, i, 0.f)); }
+    template <uint32_t BT, uint32_t U>
+    __device__ __forceinline__ void load(uint32_t i, uint32_t (&k)[U]) const {
+        if (KEYED) {
+#pragma unroll
+            for (uint32_t u = 0; u < U; u++) k[u] = keys[min(i + u * BT, n - 1u)];
+            return;
+        }
+        float4 p[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++) {
+            p[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (i + u * BT < n) p[u] = ld_xyz(pos, i + u * BT, 0.f);
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++) {
+            k[u] = VTX_INVALID;
+            if (u * BT < n) k[u] = of(p[u]);
+        }
+    }
+    __device__ __forceinline__ void put(uint32_t g, uint32_t k, uint32_t i) const {
+        const float4 p = ld_xyz(pos, i, __uint_as_float(i)), x = ld_xyz(pos0, i, 0.f);
+        ko[g] = k;
+        vo[g] = i;
+        rec[2 * (size_t)g] = p;
+        rec[2 * (size_t)g + 1] = x;
+    }
+    __device__ __forceinline__ void cell(uint32_t k, uint32_t b, uint32_t e) const {
+        cells[k] = make_uint2(b, e);
+        start[k] = b;
+        end[k] = e;
+    }
+};
+
+template <bool KEYED>
+__global__ __launch_bounds__(VTX_HASH_PART_BT, 8) void k_raw_hash_part(RawHash<KEYED> s, uint32_t width, uint32_t* spill) {
+    __shared__ HashPartLds lds;
+    const uint32_t lo = blockIdx.x * width;
+    hash_part<VTX_HASH_PART_BT, KEYED>(s, s.n, lo, min(width, s.M - lo), spill, lds);
+}
+
 // CacheNeighbors_Kernel (Velvet/SpatialHashGPU.cu:79-130).
 template <int PW>
 __global__ __launch_bounds__(256) void k_raw_neighbors(const float4* __restrict__ rec, const uint2* __restrict__ cells,
                                                        uint32_t* __restrict__ nbr, uint32_t n, float cell, float cell2,
-                                                       float diam2, uint32_t M, uint64_t mc, uint32_t K) {
+                                                       float diam2, uint32_t M, uint32_t mod, uint32_t K) {
     __shared__ NbLds<PW> lds[4];
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t first = (blockIdx.x * 4 + wave) * PW;
     if (first >= n) return;
-    const NbSet a{rec, cells, reinterpret_cast<char*>(nbr), mc, n, M, K, 0u, cell, cell2, diam2, false};
+    const NbSet a{rec, cells, reinterpret_cast<char*>(nbr), mod, n, M, K, 0u, cell, cell2, diam2, false};
     neighbor_wave<PW, false>(a, first, min((uint32_t)PW, n - first), lds[wave]);
 }
 
@@ -733,10 +874,6 @@ __global__ __launch_bounds__(VTX_TILE) void k_raw_split_cells(const uint2* __res
 // run and its candidates' loads serve more particles (963,130 particles in 256 cloths 164.9 / 129.9;
 // a pile of 1,048,576 runs long lists either way, 268 / 293).
 static bool search_small(uint32_t particles) { return particles <= (1u << 17); }
-
-static uint64_t mod_constant(uint32_t M) {   // ceil(2^64 / M) mod 2^64 (M = 1 gives 0: h % 1 = 0)
-    return M > 1 ? ~0ull / M + 1ull : 0ull;
-}
 
 size_t hash_workspace_bytes(uint32_t n, uint32_t M) {
     const size_t tiles = (n + VTX_SORT_TILE - 1) / VTX_SORT_TILE;
@@ -761,6 +898,36 @@ hipError_t hash_objects(const HashObjectsArgs& a, void* workspace, hipStream_t s
     w += up(4 * (size_t)256 * tiles);
     uint32_t* part = reinterpret_cast<uint32_t*>(w);
 
+    const uint32_t blocks = (n + VTX_TILE - 1) / VTX_TILE;
+    const uint32_t mod = mod_constant(M);
+    const auto search = [&] {
+        const auto nb = [&](auto kernel, uint32_t pw) {
+            hipLaunchKernelGGL(kernel, dim3((n + 4 * pw - 1) / (4 * pw)), dim3(256), 0, s, (const float4*)rec,
+                               (const uint2*)cells, a.neighbors, n, a.cell_spacing, a.cell_spacing2,
+                               a.particle_diameter2, M, mod, a.max_num_neighbors);
+        };
+        if (search_small(n)) nb(k_raw_neighbors<8>, 8);
+        else nb(k_raw_neighbors<32>, 32);
+    };
+    if (n && n <= VTX_HASH_PART_N && M <= VTX_HASH_PART_M) {   // one or two launches instead of up to sixteen
+        const uint32_t width = hash_part_width(n, M, VTX_HASH_PART_SHARE), parts = (M + width - 1) / width;
+        const auto build = [&](auto keyed) {
+            constexpr bool K = decltype(keyed)::value;
+            const RawHash<K> h{a.positions, a.original_positions, kalt, cells, rec, a.particle_hash, a.particle_index,
+                               a.cell_start, a.cell_end, mod, a.cell_spacing, n, M};
+            hipLaunchKernelGGL((k_raw_hash_part<K>), dim3(parts), dim3(VTX_HASH_PART_BT), 0, s, h, width, valt);
+        };
+        if (n > VTX_HASH_PART_KEYS) {
+            hipLaunchKernelGGL(k_raw_keys, dim3(blocks), dim3(VTX_TILE), 0, s, a.positions, n, a.cell_spacing, M, mod,
+                               kalt, valt);
+            build(std::true_type{});
+        } else {
+            build(std::false_type{});
+        }
+        search();
+        return hipGetLastError();
+    }
+
     // stable LSD radix sort on ceil(log2 M) bits (Velvet/SpatialHashGPU.cu:179), 8 per pass;
     // the keys start on the side that makes the last pass end in the caller's arrays
     const uint32_t bits = M > 1 ? 32u - (uint32_t)__builtin_clz(M - 1u) : 0u;
@@ -768,9 +935,7 @@ hipError_t hash_objects(const HashObjectsArgs& a, void* workspace, hipStream_t s
     uint32_t* k[2] = {a.particle_hash, kalt};
     uint32_t* v[2] = {a.particle_index, valt};
     int src = passes & 1;
-    const uint32_t blocks = (n + VTX_TILE - 1) / VTX_TILE;
-    const uint64_t mc = mod_constant(M);
-    if (n) hipLaunchKernelGGL(k_raw_keys, dim3(blocks), dim3(VTX_TILE), 0, s, a.positions, n, a.cell_spacing, M, mc,
+    if (n) hipLaunchKernelGGL(k_raw_keys, dim3(blocks), dim3(VTX_TILE), 0, s, a.positions, n, a.cell_spacing, M, mod,
                               k[src], v[src]);
     for (int pass = 0; pass < passes && n; pass++) {
         hipLaunchKernelGGL(k_raw_sort_hist, dim3(tiles), dim3(VTX_TILE), 0, s, (const uint32_t*)k[src], n, 8 * pass,
@@ -786,13 +951,7 @@ hipError_t hash_objects(const HashObjectsArgs& a, void* workspace, hipStream_t s
     if (n) {
         hipLaunchKernelGGL(k_raw_cell_bounds, dim3(blocks), dim3(VTX_TILE), 0, s, (const uint32_t*)a.particle_hash,
                            (const uint32_t*)a.particle_index, n, a.positions, a.original_positions, cells, rec);
-        const auto nb = [&](auto kernel, uint32_t pw) {
-            hipLaunchKernelGGL(kernel, dim3((n + 4 * pw - 1) / (4 * pw)), dim3(256), 0, s, (const float4*)rec,
-                               (const uint2*)cells, a.neighbors, n, a.cell_spacing, a.cell_spacing2,
-                               a.particle_diameter2, M, mc, a.max_num_neighbors);
-        };
-        if (search_small(n)) nb(k_raw_neighbors<8>, 8);
-        else nb(k_raw_neighbors<32>, 32);
+        search();
     }
     uint32_t sb = (M + VTX_TILE - 1) / VTX_TILE;
     if (sb > 4096) sb = 4096;
@@ -839,8 +998,8 @@ hipError_t hash_objects_noalloc(const HashObjectsArgs& a, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------- host launchers
-hipError_t launch_hash_keys(const DevState& d, int in, hipStream_t s) {
-    hipLaunchKernelGGL(k_hash_keys, dim3(d.ntiles), dim3(VTX_TILE), 0, s, d, in);
+hipError_t launch_hash_keys(const DevState& d, int in, int dst, hipStream_t s) {
+    hipLaunchKernelGGL(k_hash_keys, dim3(d.ntiles), dim3(VTX_TILE), 0, s, d, in, dst);
     return hipGetLastError();
 }
 
@@ -868,12 +1027,14 @@ hipError_t launch_fill_u32(uint32_t* a, uint32_t n, uint32_t v, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_hash_small(const DevState& d, int in, int dst, hipStream_t s) {
-    // one launch, largest segments first: workgroups of small segments fill the CUs that the
-    // large ones leave
-    if (d.nhsegs)
-        hipLaunchKernelGGL((k_hash_small<VTX_HASH_LDS_N>), dim3(d.nhsegs), dim3(VTX_HASH_LDS_BT), 0, s, d, d.hsegs, in,
-                           dst);
+hipError_t launch_hash_parts(const DevState& d, int in, int dst, hipStream_t s) {
+    // a full chip: 512 threads a range hold half of the wave slots while they wait (512 cloths of 963,130
+    // particles with three solvers overlapping, us a frame pair, 1024 / 512 threads: 3205 / 3175); a lone
+    // cloth's ranges take 1024 (the chip is empty, more loads in flight)
+    if (d.nhparts && d.hfull)
+        hipLaunchKernelGGL(k_hash_part<VTX_HASH_PART_BT / 2>, dim3(d.nhparts), dim3(VTX_HASH_PART_BT / 2), 0, s, d, in, dst);
+    else if (d.nhparts)
+        hipLaunchKernelGGL(k_hash_part<VTX_HASH_PART_BT>, dim3(d.nhparts), dim3(VTX_HASH_PART_BT), 0, s, d, in, dst);
     return hipGetLastError();
 }
 

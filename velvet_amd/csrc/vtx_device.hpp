@@ -40,11 +40,36 @@
 // tile (GridTileDev::at_off, in float4), part and group of four slots, one float4 of target distances
 // (times the stretchiness) per lane of the tile.
 #define VTX_SEG_LRA_TILED 8192u
-// The segment's spatial hash is built by one workgroup in LDS (k_hash_small): self-collision,
-// at most VTX_HASH_LDS_N particles and a table of at most 2^16 cells. The device-wide hash
-// kernels skip it.
-#define VTX_SEG_HASH_LDS 1024u
-#define VTX_HASH_LDS_N 16384
+// The segment's spatial hash is built by k_hash_part: self-collision, at most VTX_HASH_PART_N particles
+// and VTX_HASH_PART_M cells. The device-wide hash kernels skip it.
+#define VTX_SEG_HASH_PART 1024u
+#define VTX_HASH_PART_N 131072u
+#define VTX_HASH_PART_M 524288u
+// ... from the keys that k_hash_keys works out first: when a segment is larger than VTX_HASH_PART_KEYS
+// (eight keys a thread in registers) or VTX_HASH_PART_TOTAL particles are live, so that the launch (3 us)
+// costs less than every range working out all keys of its segment (16,384 particles: 5 us a range).
+#define VTX_SEG_HASH_KEYED 16384u
+#define VTX_HASH_PART_KEYS 8192u
+#define VTX_HASH_PART_TOTAL 65536u
+#define VTX_HASH_PART_BT 1024u       // threads of a workgroup
+#define VTX_HASH_PART_CELLS 4096u    // cells of a range at most
+#define VTX_HASH_PART_LIST 4096u     // particles of a range held in LDS
+#define VTX_HASH_HEAVY 128u
+// floor(2^32 / M), for the remainder by M (hash_coords).
+static inline uint32_t mod_constant(uint32_t M) { return M > 1 ? (uint32_t)((1ull << 32) / M) : ~0u; }
+
+// Cells of a range, for a table of M cells and n particles with `share` meant for a range: few, so that
+// many CUs take part (us per build, 1024 / 2048 a range: 4,608 particles 8.5 / 10.1, 22,500 12.5 / 15.7),
+// unless the live set fills the chip anyway and each range's run over all keys of its segment and its
+// fixed part count (963,130 particles in 512 cloths 63 / 46).
+#define VTX_HASH_PART_SHARE 1024u
+#define VTX_HASH_PART_SHARE_FULL 2048u
+#define VTX_HASH_PART_FULL 262144u   // live particles
+static inline uint32_t hash_part_width(uint32_t n, uint32_t M, uint32_t share) {
+    uint32_t parts = (n + share - 1) / share;
+    if (parts < (M + VTX_HASH_PART_CELLS - 1) / VTX_HASH_PART_CELLS) parts = (M + VTX_HASH_PART_CELLS - 1) / VTX_HASH_PART_CELLS;
+    return (M + parts - 1) / parts;
+}
 // The segment hashes its cell coordinates after adding VTX_HASH_SHIFT to each (32-bit
 // wrap-around): a tuned hash grid. HashCoords gives cells (x, y, z) and (-x, y, -z) one bucket
 // (with odd x and z the two products' two's-complement negations cancel in the XOR, and abs()
@@ -92,7 +117,7 @@ struct alignas(16) SegDev {
     float max_speed, damping, omega, lrs;
     float bend_compliance, margin, friction, stiffness;
     float gx, gy, gz, pad0;
-    uint32_t mod_lo, mod_hi;               // ceil(2^64 / M): exact remainder by multiplication
+    uint32_t mod, mod_pad;                 // mod_constant(M)
     uint32_t rows, cols;                   // grid segments: vertex grid shape
     uint32_t trbase, lbase, pad1, pad2;    // triangle-record base, dense-LRA base (in float4)
 };
@@ -130,6 +155,13 @@ struct alignas(16) ColliderDev {
 };
 
 // Pointers and sizes every kernel may need; passed by value (kernel-argument segment).
+// A range of a segment's hash cells (k_hash_part), with what its workgroup needs of the segment.
+struct HashPartDev {
+    uint32_t pbase, n, tbase, M, lo, cells, mod, shift, keyed;
+    float cell;
+    uint32_t pad[2];
+};
+
 struct DevState {
     const SegDev* segs;
     const TileDev* tiles;
@@ -163,13 +195,13 @@ struct DevState {
     const GridTileDev* ltiles;   // grid tiles whose dense attachments run on four lanes per particle
     const GridTileDev* ftiles;   // fside x fside tiles of the grid segments whose passes are fused
     const GridTileDev* mtiles;   // the same segments' VTX_GT x VTX_GT tiles (normals)
-    const uint32_t* hsegs;       // segments whose hash is built in LDS (VTX_SEG_HASH_LDS)
+    const HashPartDev* hparts;   // cell ranges of the segments k_hash_part builds
     const float4* rest4;      // grid: stretch rest lengths owned by a vertex (R, D, X-diag, anti-diag)
     const uint32_t* gflags;   // grid: bending slots present at a cell (VTX_BX | VTX_BR | VTX_BD)
     const float4* brest4;     // grid: bending rest angles of a cell (X, R, D)
     uint32_t ntiles, nstiles, nhist, ncells;
-    uint32_t hbase0, nltiles, nhsegs;        // hbase0: first histogram entry of this table set
-    uint32_t nftiles, nmtiles, fside;
+    uint32_t hbase0, nltiles, nhparts;       // hbase0: first histogram entry of this table set
+    uint32_t nftiles, nmtiles, fside, hkeyed, hfull;   // hfull: more than VTX_HASH_PART_FULL live particles; hkeyed: k_hash_part's segments have VTX_SEG_HASH_KEYED
     uint32_t nparticles, nitiles, ngtiles, remap;   // remap: workgroups -> tiles through xcd_tile
 };
 
