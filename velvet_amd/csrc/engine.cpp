@@ -596,6 +596,13 @@ int32_t Engine::add_attach_slot(int32_t s, const float* pos) {
     return (int32_t)(sg.slots.size() / 3 - 1);
 }
 
+// Updates between frames travel in a launch's arguments; into a caller's capture they would be frozen.
+void Engine::refuse_capture() {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    VTX_HIP(hipStreamIsCapturing(stream_, &st));
+    VTX_REQUIRE(st == hipStreamCaptureStatusNone, VTX_EHIP, "the stream is being captured");
+}
+
 void Engine::set_attach_slot_position(int32_t s, int32_t slot, const float* pos) {
     join();
     Segment& sg = seg(s);
@@ -605,8 +612,8 @@ void Engine::set_attach_slot_position(int32_t s, int32_t slot, const float* pos)
     const float4 v = make_float4(pos[0], pos[1], pos[2], 0.f);
     if (sg.prepared) sg.prep.slots[(size_t)slot] = v;
     if (sg.uploaded) {   // the graph reads the slot table: no re-record
-        VTX_HIP(hipMemcpyAsync(pl_.slots + sg.rg.slot + slot, &v, sizeof(float4), hipMemcpyHostToDevice, stream_));
-        sync_stream();
+        refuse_capture();
+        VTX_HIP(launch_set_slot(pl_.slots + sg.rg.slot + slot, v, stream_));
     }
 }
 
@@ -669,9 +676,8 @@ void Engine::set_colliders(int32_t s, const vtx_collider* cols, uint32_t n) {
         sg.cols.assign(cols, cols + n);
         for (uint32_t c = 0; c < n; c++) sg.prep.cols[c] = pack_collider(cols[c]);
         if (sg.uploaded && n) {
-            VTX_HIP(hipMemcpyAsync(pl_.cols + sg.rg.col, sg.prep.cols.data(), sizeof(ColliderDev) * n,
-                                   hipMemcpyHostToDevice, stream_));
-            sync_stream();
+            refuse_capture();
+            VTX_HIP(launch_set_colliders(pl_.cols + sg.rg.col, sg.prep.cols.data(), n, stream_));
         }
         return;
     }

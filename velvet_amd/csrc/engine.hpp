@@ -256,6 +256,7 @@ private:
     void pull_state(Segment& sg);
     void touch(int32_t s);                   // a structural change of segment s
     void invalidate_graph();
+    void refuse_capture();
     void sync_stream();                      // join(), then wait for the solver's stream
     void ensure_committed();
     void upload(Segment& sg, hipStream_t s);

@@ -1257,6 +1257,37 @@ __global__ __launch_bounds__(VTX_TILE) void k_check_finite(DevState d, uint32_t*
 // ---------------------------------------------------------------- host launchers
 static inline hipError_t last_launch() { return hipGetLastError(); }
 
+// Collider and slot updates between two frames: the values are the launch's arguments, so nothing waits
+// for the frame in flight and no host buffer has to outlive the call (a copy from host memory did both).
+struct ColliderArgs {
+    ColliderDev c[8];
+};
+
+__global__ __launch_bounds__(64) void k_set_colliders(ColliderDev* __restrict__ dst, ColliderArgs a, uint32_t n) {
+    const uint32_t words = n * (uint32_t)(sizeof(ColliderDev) / 4);
+    for (uint32_t i = threadIdx.x; i < words; i += 64)
+        reinterpret_cast<uint32_t*>(dst)[i] = reinterpret_cast<const uint32_t*>(a.c)[i];
+}
+
+__global__ __launch_bounds__(64) void k_set_slot(float4* __restrict__ dst, float4 v) {
+    if (threadIdx.x == 0) *dst = v;
+}
+
+hipError_t launch_set_colliders(ColliderDev* dst, const ColliderDev* src, uint32_t n, hipStream_t s) {
+    for (uint32_t c0 = 0; c0 < n; c0 += 8) {
+        ColliderArgs a{};
+        const uint32_t k = n - c0 < 8 ? n - c0 : 8u;
+        for (uint32_t c = 0; c < k; c++) a.c[c] = src[c0 + c];
+        hipLaunchKernelGGL(k_set_colliders, dim3(1), dim3(64), 0, s, dst + c0, a, k);
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_set_slot(float4* dst, float4 v, hipStream_t s) {
+    hipLaunchKernelGGL(k_set_slot, dim3(1), dim3(64), 0, s, dst, v);
+    return hipGetLastError();
+}
+
 hipError_t launch_frame_begin(const DevState& d, float frame_dt, float h, hipStream_t s) {
     if (!d.ntiles) return hipSuccess;
     hipLaunchKernelGGL(k_frame_begin, dim3(d.ntiles), dim3(VTX_TILE), 0, s, d, frame_dt, h);

@@ -20,6 +20,10 @@ hipError_t launch_iterate_fused(const DevState& d, int in, int passes, float h, 
 hipError_t launch_normals(const DevState& d, hipStream_t s);
 hipError_t launch_check_finite(const DevState& d, uint32_t* flags, uint32_t nseg, hipStream_t s);
 
+// Host values into device tables in stream order, carried in the launch's arguments.
+hipError_t launch_set_colliders(ColliderDev* dst, const ColliderDev* src, uint32_t n, hipStream_t s);
+hipError_t launch_set_slot(float4* dst, float4 v, hipStream_t s);
+
 hipError_t launch_hash_keys(const DevState& d, int in, int dst, hipStream_t s);
 hipError_t launch_sort_pass(const DevState& d, int src, int shift, hipStream_t s);
 hipError_t launch_scan(uint32_t* a, uint32_t n, uint32_t* part, hipStream_t s);

@@ -9,6 +9,7 @@ VtClothObjectGPU::Start does (Velvet/VtClothObjectGPU.hpp:43-58).
 from __future__ import annotations
 
 import ctypes as C
+import math
 from typing import Iterable, List, Optional, Sequence
 
 import numpy as np
@@ -47,18 +48,28 @@ def to_vtx_params(p: S.Params) -> VtxParams:
     return v
 
 
+def _transform(position, rotation, scale):
+    """Sixteen floats of T * R * S, column by column: what scenes.transform_matrix gives, without its
+    matrix products where the rotation is zero (a collider update of every frame)."""
+    if len(position) == 3 and rotation[0] == 0 and rotation[1] == 0 and rotation[2] == 0:
+        (x, y, z), a, b, c = map(float, position), float(scale[0]), float(scale[1]), float(scale[2])
+        if math.isfinite(x + y + z + a + b + c):
+            return [a, 0.0, 0.0, 0.0, 0.0, b, 0.0, 0.0, 0.0, 0.0, c, 0.0, x, y, z, 1.0]
+    return S.transform_matrix(position, rotation, scale).T.ravel().tolist()
+
+
 def to_vtx_colliders(cols: Sequence[S.Collider], frame_dt=None):
     arr = (VtxCollider * max(1, len(cols)))()
-    for i, c in enumerate(cols):
-        cur, last = S.collider_matrices(c)
-        arr[i].type = int(c.type)
+    for a, c in zip(arr, cols):
+        a.type = int(c.type)
         for k in range(3):
-            arr[i].position[k] = float(c.position[k])
-            arr[i].scale[k] = float(c.scale[k])
-        for k in range(16):
-            arr[i].cur[k] = float(cur[k])
-            arr[i].last[k] = float(last[k])
-        arr[i].delta_time = float(S.FRAME_DT if frame_dt is None else frame_dt)
+            a.position[k] = float(c.position[k])
+            a.scale[k] = float(c.scale[k])
+        a.cur[:] = _transform(c.position, c.rotation, c.scale)
+        a.last[:] = _transform(c.position if c.last_position is None else c.last_position,
+                               c.rotation if c.last_rotation is None else c.last_rotation,
+                               c.scale if c.last_scale is None else c.last_scale)
+        a.delta_time = float(S.FRAME_DT if frame_dt is None else frame_dt)
     return arr
 
 
