@@ -753,7 +753,7 @@ void Engine::prepare_segment(Segment& sg) {
     for (auto& c : sg.cols) pr.cols.push_back(pack_collider(c));
 
     GridLayout G;
-    pr.grid = use_stencil_ && detect_grid(sg, G);
+    pr.grid = use_stencil_ && detect_grid(sg, G) && G.rows < (1 << 22) && G.cols < (1 << 22);   // 24-bit products of the tiles
     if (pr.grid) {
         pr.grows = G.rows;
         pr.gcols = G.cols;
@@ -877,6 +877,10 @@ void Engine::prepare_segment(Segment& sg) {
                 GridTileDev gt{};
                 gt.a0 = a0;
                 gt.b0 = b0;
+                const auto recip = [](int w) { return w > 0 ? (uint32_t)((32768 + w - 1) / w) : 0u; };
+                const int right = (int)pr.gcols - 2 - (int)b0;
+                gt.recip = recip(std::min(15, right) - std::max(-1, -(int)b0) + 1) |
+                           recip(std::min(16, right) - std::max(-1, 1 - (int)b0) + 1) << 16;
                 std::vector<int64_t> lanes(VTX_TILE, -1);
                 for (uint32_t l = 0; l < VTX_TILE; l++) {
                     const uint32_t a = a0 + l / VTX_GT, b = b0 + l % VTX_GT;

@@ -650,18 +650,19 @@ __global__ __launch_bounds__(VTX_MT, RPT == 1 ? 6 : 3) void k_iterate(DevState d
 // the tile is evaluated once (not once per member vertex), its four corrections are kept in
 // LDS, and each vertex gathers its 8 stretch terms, its attachments and its 12 bending terms in
 // a fixed order. The three slot types are evaluated one after another through the same LDS
-// area (X, then R, then D), which keeps the workgroup at ~18 KB of LDS (8 workgroups per CU).
+// area (X, then R, then D), which keeps the workgroup at ~18 KB of LDS (8 workgroups per CU). A large live
+// set is bound by VALU issue (1024 x 1024: 99% of the 24 us in which the CUs are busy, of 28.2 us a pass;
+// the LDS is busy half of the time): of 869 instructions a wave, 430 are the slots' arithmetic, 180 the
+// stretch terms. Cell indices by 24-bit products with the division shared between types, and staging
+// without divisions took it from 28.7 to 28.2 us (512 cloths of 963,130 particles 3174 -> 3129 us a frame
+// pair). Vectors of four per role instead of the planes take 21 KB, one workgroup less per CU: 31.5 us.
 // Slot owner ranges relative to the tile origin (a0, b0): X rows/cols [-1, 15] (17 x 17),
 // R rows [-1, 16] cols [-1, 15] (18 x 17), D rows [-1, 15] cols [-1, 16] (17 x 18).
 #define VTX_NSX (17 * 17)
 #define VTX_NSR (18 * 17)
 #define VTX_NSD (17 * 18)
 #define VTX_NSMAX VTX_NSR
-
-template <int TYPE>
-__device__ __forceinline__ int slot_index(int ra, int rb) {
-    return TYPE == 2 ? (ra + 1) * 18 + (rb + 1) : (ra + 1) * 17 + (rb + 1);
-}
+#define VTX_NSP 320   // plane pitch: whole banks, so two planes go in one LDS instruction
 
 // Owner cells of one slot type that can hold a slot in a tile, tile-relative: rows
 // [ra0, ra0 + h), columns [rb0, rb0 + w). The type's owner range of the tile (X: rows and columns
@@ -686,100 +687,83 @@ struct SlotAt {
     static constexpr int i3 = TYPE == 0 ? PITCH : TYPE == 1 ? 1 : 0;
 };
 
-// Evaluate the bending slot owned at tile-relative cell (ra, rb) of one type (a cell of
-// slot_rect's rectangle) into LDS at its row-major index j in the type's range; act (cleared
-// before) marks the slots that contribute. The slot keeps g_k = -lam d_k for roles 0..2 (planes
-// 3k..3k+2); role 3's is -(g_0 + g_1 + g_2), as the four gradients of a dihedral angle sum to
-// zero, and each vertex scales the sum of its terms by its own inverse mass.
+// The cells of a type's rectangle are dealt to the threads densely (thread t: row t / w, column t % w), so
+// a tile cut by the cloth's edge runs no lanes on cells that cannot hold a slot. X and R have the same
+// columns, so one division serves both. recip: GridTileDev::recip (t < 324, w <= 18).
+struct SlotCell {
+    uint32_t t, q, c;
+    __device__ __forceinline__ SlotCell(uint32_t t_, uint32_t w, uint32_t recip) : t(t_) {
+        q = __umul24(t, recip) >> 15;
+        c = t - __umul24(q, w);
+    }
+};
+
+// Evaluate one cell's bending slot of a type into LDS at its row-major index in the type's range, in
+// planes 3k..3k+2 of corr: g_k = -lam d_k for roles 0..2, the type's mark in act. Role 3's is
+// -(g_0 + g_1 + g_2), as the four gradients of a dihedral angle sum to zero, and each vertex scales the
+// sum of its terms by its own inverse mass. A slot that contributes nothing keeps an older mark.
+// ra0, rb0: slot_rect's; base: the rectangle's first cell.
 template <int TYPE>
 __device__ __forceinline__ void eval_slot(const DevState& d, const SegDev& sg, const float4* sp,
-                                          float (*corr)[VTX_NSMAX], uint8_t* act, int a0,
-                                          int b0, int cols, int ra, int rb, float xpbd) {
-    constexpr int W = TYPE == 2 ? 18 : 17;                                  // owner columns of the range
-    const uint32_t j = (uint32_t)((ra + 1) * W + (rb + 1));                 // row-major storage index
-    const int a = a0 + ra, b = b0 + rb;
+                                          float (*corr)[VTX_NSP], uint8_t* act, uint32_t base, int cols, int ra0, int rb0,
+                                          SlotCell s, float xpbd) {
+    constexpr uint32_t W = TYPE == 2 ? 18 : 17;                             // owner columns of the range
     // in the rectangle every slot of a FULL type is present; otherwise the cell's flags tell
-    bool on = ((sg.flags >> (3 + TYPE)) & 1u) || ((d.gflags[sg.pbase + (uint32_t)(a * cols + b)] >> TYPE) & 1u);
-    if (on) {
-        const int o = (ra + VTX_GH) * VTX_GP + (rb + VTX_GH);    // owner in staged coordinates
-        using A = SlotAt<TYPE, VTX_GP>;
-        const float4 q0 = sp[o + A::i0], q1 = sp[o + A::i1], q2 = sp[o + A::i2], q3 = sp[o + A::i3];
-        float rest = 0.f;
-        if (!(sg.flags & VTX_SEG_BEND_REST0)) {
-            const float4 r4 = d.brest4[sg.pbase + (uint32_t)(a * cols + b)];
-            rest = TYPE == 0 ? r4.x : TYPE == 1 ? r4.y : r4.z;
-        }
-        float lam;
-        BendGrad bg;
-        on = bend_eval<true>(q0, q1, q2, q3, rest, xpbd, lam, bg);
-        if (on) {
-            const V3 g0 = (-lam * bg.k0) * bg.c1, g1 = (-lam * bg.k1) * bg.c2, g2 = -lam * bg.d2;
-            corr[0][j] = g0.x; corr[1][j] = g0.y; corr[2][j] = g0.z;
-            corr[3][j] = g1.x; corr[4][j] = g1.y; corr[5][j] = g1.z;
-            corr[6][j] = g2.x; corr[7][j] = g2.y; corr[8][j] = g2.z;
-            act[j] = 1;
-        }
-    }
+    const uint32_t cell = __umul24(s.q, (uint32_t)cols) + s.c;              // from the rectangle's first
+    if (!((sg.flags >> (3 + TYPE)) & 1u) && !(((d.gflags + base)[cell] >> TYPE) & 1u)) return;
+    const uint32_t o = __umul24(s.q, VTX_GP) + s.c + (uint32_t)((ra0 + VTX_GH) * VTX_GP + rb0 + VTX_GH);   // staged owner
+    using A = SlotAt<TYPE, VTX_GP>;
+    const float4 q0 = sp[o + A::i0], q1 = sp[o + A::i1], q2 = sp[o + A::i2], q3 = sp[o + A::i3];
+    float rest = 0.f;
+    if (!(sg.flags & VTX_SEG_BEND_REST0)) rest = reinterpret_cast<const float*>(d.brest4 + base + cell)[TYPE];
+    float lam;
+    BendGrad bg;
+    if (!bend_eval<true>(q0, q1, q2, q3, rest, xpbd, lam, bg)) return;
+    const uint32_t j = __umul24(s.q, W) + s.c + (uint32_t)((ra0 + 1) * (int)W + rb0 + 1);
+    const V3 g0 = (-lam * bg.k0) * bg.c1, g1 = (-lam * bg.k1) * bg.c2, g2 = -lam * bg.d2;
+    corr[0][j] = g0.x; corr[1][j] = g0.y; corr[2][j] = g0.z;
+    corr[3][j] = g1.x; corr[4][j] = g1.y; corr[5][j] = g1.z;
+    corr[6][j] = g2.x; corr[7][j] = g2.y; corr[8][j] = g2.z;
+    act[j] = TYPE + 1;
 }
 
-// One slot type: the workgroup's threads take the cells of the type's rectangle densely (thread
-// t: row t / w, column t % w), so a tile cut by the cloth's edge runs no lanes on cells that
-// cannot hold a slot; then every tile vertex adds its four memberships of this type in role
-// order to bend (gradients times -lam; the vertex's inverse mass is applied to the sum).
+// One slot type of a tile: the evaluations, then every tile vertex adds its four memberships of this type
+// in role order to bend (gradients times -lam; the vertex's inverse mass is applied to the sum).
 template <int TYPE>
 __device__ __forceinline__ void bend_type_pass(const DevState& d, const SegDev& sg, const float4* sp,
-                                               float (*corr)[VTX_NSMAX], uint8_t* act,
-                                               int a0, int b0,
-                                               int rows, int cols, float xpbd, bool inside, int ty, int tx,
+                                               float (*corr)[VTX_NSP], uint8_t* act, int a0, int b0, int rows, int cols,
+                                               SlotCell s0, SlotCell s1, float xpbd, bool inside, int ty, int tx,
                                                V3& bend, int& cnt) {
-    const uint32_t tid = threadIdx.x;
     if (!((sg.flags >> (6 + TYPE)) & 1u)) {   // the type is present at all
         int ra0, rb0, h, w;
         slot_rect<TYPE>(a0, b0, rows, cols, ra0, rb0, h, w);
-        if (h > 0 && w > 0) {
-            const uint32_t n = (uint32_t)(h * w), m = (65536u + (uint32_t)w - 1u) / (uint32_t)w;   // t / w = t m >> 16 (t < 1024, w <= 18)
-            constexpr uint32_t BT = VTX_TILE;
-            static_assert(2 * BT >= VTX_NSMAX, "a slot type fits two rounds of the workgroup");
-#pragma unroll
-            for (uint32_t r = 0; r < 2u; r++) {
-                const uint32_t t = tid + r * BT;
-                if (t < n) {
-                    const uint32_t q = (t * m) >> 16;
-                    eval_slot<TYPE>(d, sg, sp, corr, act, a0, b0, cols, ra0 + (int)q, rb0 + (int)(t - q * (uint32_t)w), xpbd);
-                }
-            }
-        }
+        const uint32_t n = h > 0 && w > 0 ? (uint32_t)(h * w) : 0u;
+        const uint32_t base = sg.pbase + (uint32_t)((a0 + ra0) * cols + b0 + rb0);
+        static_assert(2 * VTX_TILE >= VTX_NSMAX, "a slot type fits two rounds of the workgroup");
+        if (s0.t < n) eval_slot<TYPE>(d, sg, sp, corr, act, base, cols, ra0, rb0, s0, xpbd);
+        if (s1.t < n) eval_slot<TYPE>(d, sg, sp, corr, act, base, cols, ra0, rb0, s1, xpbd);
     }
     __syncthreads();
     if (inside) {
         // role r of the slot owned at (ty + dy_r, tx + dx_r), per type:
         //   X: (0,0) (-1,-1) (0,-1) (-1,0);  R: (1,-1) (-1,0) (0,0) (0,-1);  D: (-1,1) (0,-1) (-1,0) (0,0)
-        int sidx[4];
-        if (TYPE == 0) {
-            sidx[0] = slot_index<0>(ty, tx); sidx[1] = slot_index<0>(ty - 1, tx - 1);
-            sidx[2] = slot_index<0>(ty, tx - 1); sidx[3] = slot_index<0>(ty - 1, tx);
-        } else if (TYPE == 1) {
-            sidx[0] = slot_index<1>(ty + 1, tx - 1); sidx[1] = slot_index<1>(ty - 1, tx);
-            sidx[2] = slot_index<1>(ty, tx); sidx[3] = slot_index<1>(ty, tx - 1);
-        } else {
-            sidx[0] = slot_index<2>(ty - 1, tx + 1); sidx[1] = slot_index<2>(ty, tx - 1);
-            sidx[2] = slot_index<2>(ty - 1, tx); sidx[3] = slot_index<2>(ty, tx);
-        }
+        constexpr int W = TYPE == 2 ? 18 : 17;
+        constexpr int DY[4] = {TYPE == 0 ? 0 : TYPE == 1 ? 1 : -1, TYPE == 2 ? 0 : -1, TYPE == 2 ? -1 : 0, TYPE == 0 ? -1 : 0};
+        constexpr int DX[4] = {TYPE == 0 ? 0 : TYPE == 1 ? -1 : 1, TYPE == 1 ? 0 : -1, TYPE == 0 ? -1 : 0, TYPE == 1 ? -1 : 0};
+        const int j0 = (ty + 1) * W + tx + 1;
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            const int j = sidx[r];
-            if (act[j]) {
-                if (r < 3) {
-                    bend += v3(corr[3 * r][j], corr[3 * r + 1][j], corr[3 * r + 2][j]);
-                } else {
-                    bend -= v3(corr[0][j], corr[1][j], corr[2][j]) + v3(corr[3][j], corr[4][j], corr[5][j]) +
-                            v3(corr[6][j], corr[7][j], corr[8][j]);
-                }
-                cnt++;
-            }
+            const int j = j0 + DY[r] * W + DX[r];
+            if (act[j] != TYPE + 1) continue;
+            if (r < 3)
+                bend += v3(corr[3 * r][j], corr[3 * r + 1][j], corr[3 * r + 2][j]);
+            else
+                bend -= v3(corr[0][j], corr[1][j], corr[2][j]) + v3(corr[3][j], corr[4][j], corr[5][j]) +
+                        v3(corr[6][j], corr[7][j], corr[8][j]);
+            cnt++;
         }
     }
-    __syncthreads();   // the next type reuses corr / act
+    __syncthreads();   // the next type reuses corr
 }
 
 __device__ __forceinline__ float4 nan4() {
@@ -791,8 +775,8 @@ template <int EPI>
 __global__ __launch_bounds__(VTX_TILE) void k_iterate_grid(DevState d, const GridTileDev* __restrict__ tiles,
                                                                    int in, float h) {
     __shared__ float4 sp[VTX_GP * VTX_GP];
-    __shared__ float corr[9][VTX_NSMAX];           // plane r*3+c: component c of role r's g_r
-    __shared__ uint32_t actw[(VTX_NSX + VTX_NSR + VTX_NSD + 3) / 4];   // per type: slot contributes
+    __shared__ float corr[9][VTX_NSP];           // plane r*3+c: component c of role r's g_r
+    __shared__ uint32_t actw[(VTX_NSMAX + 3) / 4];   // the type whose slot last contributed there
     uint8_t* const act = reinterpret_cast<uint8_t*>(actw);
     const GridTileDev t = tiles[tile_of(d.remap)];
     const SegDev sg = d.segs[t.seg];
@@ -803,7 +787,10 @@ __global__ __launch_bounds__(VTX_TILE) void k_iterate_grid(DevState d, const Gri
     const int ty = (int)(tid / VTX_GT), tx = (int)(tid % VTX_GT);
     const int a = a0 + ty, b = b0 + tx;
     const bool inside = a < rows && b < cols;
-    const uint32_t g = inside ? sg.pbase + (uint32_t)(a * cols + b) : 0u;
+    // offsets from the tile's first vertex stay in 32 bits (cols < 2^22)
+    const uint32_t first = sg.pbase + (uint32_t)(a0 * cols + b0);
+    const uint32_t own = inside ? __umul24((uint32_t)ty, (uint32_t)cols) + (uint32_t)tx : 0u;
+    const uint32_t g = first + own;
     // stretch rest lengths: R own/left, D own/up, X-diagonal own/up-left, anti-diagonal of left/up,
     // issued before the staging loads and always (from the vertex itself where a neighbour is
     // missing): a load that a lane may skip leaves the outstanding count unknown to the compiler,
@@ -817,12 +804,21 @@ __global__ __launch_bounds__(VTX_TILE) void k_iterate_grid(DevState d, const Gri
     if (!(a > 0 && b > 0)) r_ul = nan4();
 
     // clear the slot marks; stage positions of rows [a0-2, a0+18) x cols [b0-2, b0+18)
-    for (uint32_t e = tid; e < (VTX_NSX + VTX_NSR + VTX_NSD + 3) / 4; e += VTX_TILE) actw[e] = 0u;
+    if (tid < (VTX_NSMAX + 3) / 4) actw[tid] = 0u;
+    uint32_t sr = (tid * 3277u) >> 16, scol = tid - sr * VTX_GP;               // tid / 20 for tid < 256
+#pragma unroll
     for (uint32_t e = tid; e < VTX_GP * VTX_GP; e += VTX_TILE) {
-        const int sa = a0 - VTX_GH + (int)(e / VTX_GP), sb = b0 - VTX_GH + (int)(e % VTX_GP);
+        const int sa = a0 - VTX_GH + (int)sr, sb = b0 - VTX_GH + (int)scol;
         float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (sa >= 0 && sa < rows && sb >= 0 && sb < cols) v = P[sg.pbase + (uint32_t)(sa * cols + sb)];
+        if ((uint32_t)sa < (uint32_t)rows && (uint32_t)sb < (uint32_t)cols)
+            v = P[sg.pbase + (__umul24((uint32_t)sa, (uint32_t)cols) + (uint32_t)sb)];
         sp[e] = v;
+        sr += VTX_TILE / VTX_GP;                                                // 256 = 12 rows and 16 columns on
+        scol += VTX_TILE % VTX_GP;
+        if (scol >= VTX_GP) {
+            scol -= VTX_GP;
+            sr++;
+        }
     }
 
     __syncthreads();
@@ -849,11 +845,14 @@ __global__ __launch_bounds__(VTX_TILE) void k_iterate_grid(DevState d, const Gri
     // bending: X roles 0..3, R roles 0..3, D roles 0..3
     const float xpbd_bend = sg.bend_compliance * frcp(h) * frcp(h);   // compliance / h^2 (cu:173)
     V3 bend = v3(0.f, 0.f, 0.f);
-    bend_type_pass<0>(d, sg, sp, corr, act, a0, b0, rows, cols, xpbd_bend, inside, ty, tx, bend, cnt);
-    bend_type_pass<1>(d, sg, sp, corr, act + VTX_NSX, a0, b0, rows, cols, xpbd_bend, inside, ty, tx, bend,
-                          cnt);
-    bend_type_pass<2>(d, sg, sp, corr, act + VTX_NSX + VTX_NSR, a0, b0, rows, cols, xpbd_bend, inside, ty,
-                          tx, bend, cnt);
+    // the rectangles' columns: X and R from b0 (or 0) - 1, D from b0 (or 1) - 1 to one more (slot_rect)
+    const uint32_t wx = (uint32_t)max(min(15, cols - 2 - b0) - max(-1, -b0) + 1, 0);
+    const uint32_t wd = (uint32_t)max(min(16, cols - 2 - b0) - max(-1, 1 - b0) + 1, 0);
+    const SlotCell x0(tid, wx, t.recip & 0xFFFFu), x1(tid + VTX_TILE, wx, t.recip & 0xFFFFu);
+    bend_type_pass<0>(d, sg, sp, corr, act, a0, b0, rows, cols, x0, x1, xpbd_bend, inside, ty, tx, bend, cnt);
+    bend_type_pass<1>(d, sg, sp, corr, act, a0, b0, rows, cols, x0, x1, xpbd_bend, inside, ty, tx, bend, cnt);
+    const SlotCell d0(tid, wd, t.recip >> 16), d1(tid + VTX_TILE, wd, t.recip >> 16);
+    bend_type_pass<2>(d, sg, sp, corr, act, a0, b0, rows, cols, d0, d1, xpbd_bend, inside, ty, tx, bend, cnt);
     if (!inside) return;
     delta = madd(delta, bend, w);
     if (cnt > 0) p = madd(p, delta, frcp((float)cnt) * sg.omega);

@@ -137,7 +137,8 @@ struct alignas(16) SortTileDev {
 
 struct alignas(16) GridTileDev {
     uint32_t seg, a0, b0, pad0;            // segment, first row / column of the tile
-    uint32_t at_off, at_k, pad1, pad2;     // attach ELL of the tile's lanes, or its tiled dense distances
+    uint32_t at_off, at_k;                 // attach ELL of the tile's lanes, or its tiled dense distances
+    uint32_t recip, pad1;                  // ceil(2^15 / w), w = columns of the slot rectangles: X and R, D << 16
 };
 
 // Collider with its transforms as 3x4 row-major affine matrices:
