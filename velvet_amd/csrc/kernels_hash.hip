@@ -27,12 +27,16 @@ namespace vtx {
 // abs(h % M). |h % M| == |h| mod M for C's truncating remainder, and the unsigned remainder of
 // a <= 2^31 takes one product with m = floor(2^32 / M) (mod_constant): a/M - a m / 2^32 < a / 2^32 <= 1/2,
 // so the quotient's floor is right or one too small, and one subtraction mends it.
-__device__ __forceinline__ uint32_t hash_coords(int32_t x, int32_t y, int32_t z, uint32_t M, uint32_t m) {
-    const int32_t h = (int32_t)(((uint32_t)x * 92837111u) ^ ((uint32_t)y * 689287499u) ^
-                                ((uint32_t)z * 283923481u));
-    const uint32_t a = h < 0 ? 0u - (uint32_t)h : (uint32_t)h;
+constexpr uint32_t HX = 92837111u, HY = 689287499u, HZ = 283923481u;
+
+__device__ __forceinline__ uint32_t hash_reduce(uint32_t h, uint32_t M, uint32_t m) {
+    const uint32_t a = (int32_t)h < 0 ? 0u - h : h;
     const uint32_t r = a - __umulhi(a, m) * M;
     return min(r, r - M);
+}
+
+__device__ __forceinline__ uint32_t hash_coords(int32_t x, int32_t y, int32_t z, uint32_t M, uint32_t m) {
+    return hash_reduce(((uint32_t)x * HX) ^ ((uint32_t)y * HY) ^ ((uint32_t)z * HZ), M, m);
 }
 
 // ComputeIntCoord (Velvet/SpatialHashGPU.cu:13-16): floor of a correctly rounded binary32
@@ -557,9 +561,12 @@ __global__ __launch_bounds__(BT, 8) void k_hash_part(DevState d, int in, int dst
 // list from the test's ballot, which keeps the walk's order. One particle per lane instead, each
 // lane walking its own 60 to 300 candidates one after the other, was bound by that chain at small
 // sizes and by the vector cache at large ones (0.9 accesses a clock on every CU): 16,384 particles
-// 88 -> 11.8 us, 65,536 particles 54.6 -> 17.1 us, 963,130 in 256 draped cloths 204.8 -> 129.9 us
-// (now 89% of its VALU issue time, 73 instructions a particle), a folded pile of 1,048,576
-// 759 -> 293 us.
+// 88 -> 11.8 us, 65,536 particles 54.6 -> 16.9 us, 963,130 in 256 draped cloths 204.8 -> 106.7 us (a
+// particle tests some 150 candidates at 15 VALU instructions per 64, and 6 more where one is accepted:
+// 85% of its VALU issue time). A segment whose records outgrow the L2 is bound by fetching each cell's
+// records some 27 times, as neighbours in the sorted order are no neighbours in space: a folded pile of
+// 1,048,576 759 -> 267 us, 874 MB. Taking cells by particle index instead fetches 210 MB, but its waves
+// are uneven and it gains nothing with three solvers overlapping (2.89 -> 3.02 ms a frame pair).
 struct NbSet {
     const float4* rec;    // sorted records: position with w = index at 2i, initial position at 2i + 1
     const uint2* cells;   // (start, end) per hash cell
@@ -582,11 +589,40 @@ __device__ __forceinline__ void nb_put(const NbSet& a, uint32_t id, uint32_t k, 
     else *reinterpret_cast<uint32_t*>(at) = v;
 }
 
+// How the search stores entries: chunks of 16-bit or 32-bit entries or the column-major layout, and whether
+// a table's byte offsets fit 32 bits with 24-bit factors (n < 2^22).
+enum NbStore { NB_CHUNK16, NB_CHUNK32, NB_COLUMN };
+
+// nb_put with `row` = entries of a row (4 n or n) and at0 = the particle's first entry, both wave-uniform.
+template <NbStore ST, bool SMALL>
+__device__ __forceinline__ void nb_put_uniform(const NbSet& a, uint32_t id, uint32_t row, uint32_t at0, uint32_t k, uint32_t v) {
+    if (!SMALL) {
+        nb_put<ST != NB_COLUMN>(a, id, k, v);
+        return;
+    }
+    uint32_t off;   // the compiler takes the 32-bit product otherwise, a quarter of the rate
+    if (ST == NB_COLUMN) {
+        asm("v_mul_u32_u24 %0, %2, %1" : "=v"(off) : "v"(k), "s"(row));
+        off += at0;
+    } else {
+        asm("v_mul_u32_u24 %0, %2, %1" : "=v"(off) : "v"(k >> 2), "s"(row));
+        off += at0 | (k & 3u);
+    }
+    if (ST == NB_CHUNK16) *reinterpret_cast<uint16_t*>(a.table + (off << 1)) = (uint16_t)v;
+    else *reinterpret_cast<uint32_t*>(a.table + (off << 2)) = v;
+}
+
+// v with lane l's value replaced (x and l wave-uniform).
+__device__ __forceinline__ uint32_t write_lane(uint32_t v, uint32_t x, uint32_t l) {
+    asm("s_mov_b32 m0, %2\n\tv_writelane_b32 %0, %1, m0" : "+v"(v) : "s"(x), "s"(l) : "m0");
+    return v;
+}
+
 // LDS of one wave of the search.
 template <int PW>
 struct NbLds {
     uint32_t range[PW * 27];   // per (run, cell): start | length << 25
-    int32_t cx[PW], cy[PW], cz[PW];
+    uint32_t cx[PW], cy[PW], cz[PW];   // per run: its cell's coordinates times the hash's factors
     uint32_t mark[64];
 };
 
@@ -606,8 +642,8 @@ __device__ __forceinline__ void ld_record_uniform(const float4* rec, uint32_t i,
 }
 
 // The lists of sorted particles [i0, i0 + cnt), cnt <= PW, by the calling wave.
-template <int PW, bool CHUNK>
-__device__ __forceinline__ void neighbor_wave(const NbSet& a, uint32_t i0, uint32_t cnt, NbLds<PW>& L) {
+template <int PW, NbStore ST, bool SMALL>
+__device__ __forceinline__ void neighbor_wave_as(const NbSet& a, uint32_t i0, uint32_t cnt, NbLds<PW>& L) {
 #pragma clang fp contract(off)
     constexpr int NC = 2;                                   // candidate chunks held at a time
     const uint32_t lane = threadIdx.x & 63u;
@@ -622,26 +658,37 @@ __device__ __forceinline__ void neighbor_wave(const NbSet& a, uint32_t i0, uint3
     const bool head = lane < cnt && ((lane == 0) | (px != ix) | (py != iy) | (pz != iz));
     const uint64_t heads = __builtin_amdgcn_ballot_w64(head);
     const uint32_t nruns = (uint32_t)__popcll(heads);
-    if (head) {
+    if (head) {                                             // the cell as hashed, factor by factor
         const uint32_t r = (uint32_t)__popcll(heads & lt);
-        L.cx[r] = ix;
-        L.cy[r] = iy;
-        L.cz[r] = iz;
+        L.cx[r] = (uint32_t)ix * HX;
+        L.cy[r] = (uint32_t)iy * HY;
+        L.cz[r] = (uint32_t)iz * HZ;
     }
     wave_lds_sync();
-    // the runs' cell ranges, one (run, cell) per lane and round
-    for (uint32_t t = lane; t < nruns * 27u; t += 64u) {
-        const uint32_t r = (t * 2428u) >> 16, q = t - 27u * r;          // t / 27 for t < 3277
-        const uint32_t dx = (q * 57u) >> 9, yz = q - 9u * dx;           // q / 9 for q < 27
-        const uint32_t dy = (yz * 11u) >> 5, dz = yz - 3u * dy;         // yz / 3 for yz < 9
-        const uint32_t hq = hash_coords(L.cx[r] + (int32_t)dx - 1, L.cy[r] + (int32_t)dy - 1,
-                                        L.cz[r] + (int32_t)dz - 1, a.M, a.mod);
-        const uint64_t c = *reinterpret_cast<const uint64_t*>(a.cells + hq);   // one 8-byte load
-        const uint32_t st = (uint32_t)c, len = min((uint32_t)(c >> 32) - st, a.K);
-        L.range[t] = st == VTX_INVALID ? 0u : st | len << 25;
+    // the runs' cell ranges: a half of the wave takes one run, a lane (of 27) always the same of its cells,
+    // so that the lane's share of the hash's products is worked out once; four rounds' loads in flight
+    const uint32_t q = lane & 31u, dx = (q * 57u) >> 9, yz = q - 9u * dx, dy = (yz * 11u) >> 5, dz = yz - 3u * dy;
+    const uint32_t ox = (dx - 1u) * HX, oy = (dy - 1u) * HY, oz = (dz - 1u) * HZ;
+    for (uint32_t r0 = 0; r0 < nruns; r0 += 8u) {
+        uint64_t c[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; u++) {
+            if (r0 + 2u * u >= nruns) break;
+            const uint32_t r = min(r0 + 2u * u + (lane >> 5), nruns - 1u);
+            const uint32_t hq = hash_reduce((L.cx[r] + ox) ^ (L.cy[r] + oy) ^ (L.cz[r] + oz), a.M, a.mod);
+            c[u] = q < 27u ? *reinterpret_cast<const uint64_t*>(a.cells + hq) : 0ull;   // one 8-byte load
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; u++) {
+            if (r0 + 2u * u >= nruns) break;
+            const uint32_t r = r0 + 2u * u + (lane >> 5);
+            const uint32_t st = (uint32_t)c[u], len = min((uint32_t)(c[u] >> 32) - st, a.K);
+            if (q < 27u && r < nruns) L.range[r * 27u + q] = st == VTX_INVALID ? 0u : st | len << 25;
+        }
     }
     wave_lds_sync();
     uint32_t kv = 0;                                        // lane m: entries of particle m
+    const uint32_t row = ST == NB_COLUMN ? a.n : 4 * a.n;
     uint64_t rest = heads;
     for (uint32_t r = 0; r < nruns; r++) {
         const uint32_t m0 = (uint32_t)__builtin_ctzll(rest);
@@ -652,12 +699,11 @@ __device__ __forceinline__ void neighbor_wave(const NbSet& a, uint32_t i0, uint3
         const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 31);
         const uint32_t base = (v & 0x1FFFFFFu) - excl;      // candidate c of the cell: sorted position base + c
         for (uint32_t g0 = 0; g0 < total; g0 += 64u * NC) {
-            uint32_t idx[NC];
             float4 q[NC], x[NC];
 #pragma unroll
             for (int h = 0; h < NC; h++) {
                 const uint32_t c0 = g0 + 64u * h;
-                idx[h] = VTX_INVALID;
+                q[h] = x[h] = make_float4(0.f, 0.f, 0.f, 0.f);
                 if (h && c0 >= total) continue;
                 // the cell of each lane's candidate: every cell marks the lane of its first one
                 L.mark[lane] = 0;
@@ -666,12 +712,13 @@ __device__ __forceinline__ void neighbor_wave(const NbSet& a, uint32_t i0, uint3
                 wave_lds_sync();
                 const uint32_t own = scan64_max(L.mark[lane]);
                 const uint32_t b = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((own - 1u) << 2), (int)base);
-                if (c0 + lane < total) idx[h] = b + c0 + lane;
-                const uint32_t at = c0 + lane < total ? idx[h] : i0;
+                const uint32_t at = c0 + lane < total ? b + c0 + lane : i0;
                 q[h] = a.rec[2 * (size_t)at];
                 x[h] = a.rec[2 * (size_t)at + 1];
+                if (c0 + lane >= total) q[h].x = __builtin_nanf("");
                 wave_lds_sync();
             }
+            // lanes without a candidate are farther than any distance; the particle itself is told by its index
             for (uint32_t m = m0; m < m1; m++) {
                 float4 p, o;
                 ld_record_uniform(a.rec, i0 + m, p, o);
@@ -684,19 +731,29 @@ __device__ __forceinline__ void neighbor_wave(const NbSet& a, uint32_t i0, uint3
                     const float d2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
                     const float ex = o.x - x[h].x, ey = o.y - x[h].y, ez = o.z - x[h].z;
                     const float e2 = __builtin_fmaf(ez, ez, __builtin_fmaf(ey, ey, ex * ex));
-                    // the particle itself is the candidate at its own sorted position
-                    const bool acc = (idx[h] != i0 + m) & (idx[h] != VTX_INVALID) & (d2 < a.cell2) & (e2 > a.diam2);
-                    const uint64_t mask = __builtin_amdgcn_ballot_w64(acc);
+                    const uint64_t mask = __builtin_amdgcn_ballot_w64(d2 < a.cell2) &
+                                          __builtin_amdgcn_ballot_w64(e2 > a.diam2) &
+                                          __builtin_amdgcn_ballot_w64(__float_as_uint(q[h].w) != id);
+                    if (!mask) continue;
                     const uint32_t e = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
                                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)mask, k));
-                    if (acc && e < a.K) nb_put<CHUNK>(a, id, e, __float_as_uint(q[h].w));
+                    if (__builtin_amdgcn_inverse_ballot_w64(mask) && e < a.K)
+                        nb_put_uniform<ST, SMALL>(a, id, row, ST == NB_COLUMN ? id : 4 * id, e, __float_as_uint(q[h].w));
                     k = min(k + (uint32_t)__popcll(mask), a.K);
                 }
-                kv = lane == m ? k : kv;
+                kv = write_lane(kv, k, m);
             }
         }
     }
-    if (lane < cnt && kv < a.K) nb_put<CHUNK>(a, __float_as_uint(me.w), kv, VTX_INVALID);   // a full list has no sentinel
+    // a full list has no sentinel
+    if (lane < cnt && kv < a.K) nb_put<ST != NB_COLUMN>(a, __float_as_uint(me.w), kv, VTX_INVALID);
+}
+
+template <int PW, bool CHUNK>
+__device__ __forceinline__ void neighbor_wave(const NbSet& a, uint32_t i0, uint32_t cnt, NbLds<PW>& L) {
+    if (CHUNK && a.n16) neighbor_wave_as<PW, NB_CHUNK16, true>(a, i0, cnt, L);   // n < 2^16
+    else if (a.n < (1u << 22)) neighbor_wave_as<PW, CHUNK ? NB_CHUNK32 : NB_COLUMN, true>(a, i0, cnt, L);
+    else neighbor_wave_as<PW, CHUNK ? NB_CHUNK32 : NB_COLUMN, false>(a, i0, cnt, L);
 }
 
 // The search over the segments' particle tiles (a tile's sorted positions): 4 PW particles per
