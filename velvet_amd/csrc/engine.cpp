@@ -1426,8 +1426,8 @@ void Engine::rebuild_tables() {
     d.nftiles = (uint32_t)hftile.size();
     d.nmtiles = (uint32_t)hmtile.size();
     d.fside = fside;
-    d.hkeyed = hkeyed;
-    d.hfull = total_n > VTX_HASH_PART_FULL;
+    d.live = (any_selfcol_ ? VTX_LIVE_SELFCOL : 0u) | (hkeyed ? VTX_LIVE_KEYED : 0u) |
+             (total_n > VTX_HASH_PART_FULL ? VTX_LIVE_FULL : 0u);
     d.nstiles = (uint32_t)hst.size();
     d.nhist = hbase;
     d.ncells = (uint32_t)acell_.cap;
@@ -1586,7 +1586,7 @@ void Engine::hash_build(const DevState& d, int in, hipStream_t s) {
     // segments of k_hash_part build into the buffer the device-wide sort of the others ends in
     const int dst = passes_ & 1;
     int src = dst;
-    if (d.nstiles || d.hkeyed) {
+    if (d.nstiles || (d.live & VTX_LIVE_KEYED)) {
         stage_begin("k_hash_keys", "Solver_HashParticle", s);
         VTX_HIP(launch_hash_keys(d, in, dst, s));
         stage_end(s);

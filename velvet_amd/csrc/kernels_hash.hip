@@ -1088,7 +1088,7 @@ hipError_t launch_hash_parts(const DevState& d, int in, int dst, hipStream_t s) 
     // a full chip: 512 threads a range hold half of the wave slots while they wait (512 cloths of 963,130
     // particles with three solvers overlapping, us a frame pair, 1024 / 512 threads: 3205 / 3175); a lone
     // cloth's ranges take 1024 (the chip is empty, more loads in flight)
-    if (d.nhparts && d.hfull)
+    if (d.nhparts && (d.live & VTX_LIVE_FULL))
         hipLaunchKernelGGL(k_hash_part<VTX_HASH_PART_BT / 2>, dim3(d.nhparts), dim3(VTX_HASH_PART_BT / 2), 0, s, d, in, dst);
     else if (d.nhparts)
         hipLaunchKernelGGL(k_hash_part<VTX_HASH_PART_BT>, dim3(d.nhparts), dim3(VTX_HASH_PART_BT), 0, s, d, in, dst);

@@ -150,8 +150,9 @@ __global__ __launch_bounds__(VTX_TILE) void k_frame_begin(DevState d, float fram
 
 // CollideParticles_Kernel + ApplyDeltas (Velvet/VtClothSolverGPU.cu:329-386) followed by the
 // substep's CollideSDF (cu:289-314, hpp:87).
-template <int BS>
+template <int BS, int U>
 __global__ __launch_bounds__(BS) void k_collide(DevState d, int in, float h) {
+    constexpr bool AHEAD = U > 4;
     uint32_t tix, lane;
     tile_lane<VTX_TILE, BS>(d.remap, tix, lane);
     const TileDev t = d.tiles[tix];
@@ -174,16 +175,16 @@ __global__ __launch_bounds__(BS) void k_collide(DevState d, int in, float h) {
         V3 delta = v3(0.f, 0.f, 0.f);
         int cnt = 0;
         const V3 vel_i = p - x;
-        // neighbours four at a time (one chunk): while a group's positions load, the next chunk
-        // loads too; the four terms are then added in list order. An entry counts only if every
+        // neighbours U at a time (chunks of four): while a group's positions load, the next chunks
+        // load too; the terms are then added in list order. An entry counts only if every
         // entry before it is a particle index (the list ends at the first sentinel, later rows are
         // stale). A neighbour's start-of-substep position enters only the friction of a contact,
-        // so it is loaded for contacts alone: most listed neighbours of a resting cloth lie
-        // beyond the diameter, and the pass is bound by the cache lines its gathers touch.
+        // so it is loaded for contacts alone unless AHEAD: most listed neighbours of a resting cloth lie
+        // beyond the diameter, and a large pass is bound by the cache lines its gathers touch.
         bool live = true;
         const uint32_t K = sg.max_nbr;
-        uint32_t jn[4];
-        auto chunk = [&](uint32_t k0) {   // entries k0..k0+3, those at K or beyond as sentinels
+        uint32_t jn[U];
+        auto load = [&](uint32_t k0, uint32_t* jn) {   // entries k0..k0+3, those at K or beyond as sentinels
             uint4 c;
             if (n16) {
                 const uint2 h = nb2[(size_t)(k0 >> 2) * n];
@@ -196,30 +197,42 @@ __global__ __launch_bounds__(BS) void k_collide(DevState d, int in, float h) {
             jn[2] = k0 + 2 < K ? c.z : VTX_INVALID;
             jn[3] = k0 + 3 < K ? c.w : VTX_INVALID;
         };
-        chunk(0);
-        for (uint32_t k0 = 0; k0 < K && live; k0 += 4) {
-            bool ok[4];
-            uint32_t jg[4];
+        auto chunk = [&](uint32_t k0) {
+            load(k0, jn);
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
+            for (int u = 4; u < U; u += 4) {
+                jn[u] = jn[u + 1] = jn[u + 2] = jn[u + 3] = VTX_INVALID;
+                if (k0 + u < K) load(k0 + u, jn + u);
+            }
+        };
+        chunk(0);
+        for (uint32_t k0 = 0; k0 < K && live; k0 += U) {
+            bool ok[U];
+            uint32_t jg[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
                 live = live && jn[u] < n;
                 ok[u] = live;
                 jg[u] = sg.pbase + (ok[u] ? jn[u] : 0u);
             }
-            float4 pj4[4], xj4[4];
+            float4 pj4[U], xj4[U];
 #pragma unroll
-            for (int u = 0; u < 4; u++) pj4[u] = P[jg[u]];
-            if (live && k0 + 4 < K) chunk(k0 + 4);
-            bool hit[4];
-            float dist[4];
+            for (int u = 0; u < U; u++) pj4[u] = P[jg[u]];
+            if (AHEAD) {
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
+                for (int u = 0; u < U; u++) xj4[u] = d.X[jg[u]];
+            }
+            if (live && k0 + U < K) chunk(k0 + U);
+            bool hit[U];
+            float dist[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
                 dist[u] = flen(p - xyz(pj4[u]));
                 hit[u] = ok[u] && !(w + pj4[u].w <= 0.f) && !(dist[u] >= sg.diameter);
-                if (hit[u]) xj4[u] = d.X[jg[u]];
+                if (!AHEAD && hit[u]) xj4[u] = d.X[jg[u]];
             }
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
+            for (int u = 0; u < U; u++) {
                 if (!hit[u]) continue;
                 const float denom = w + pj4[u].w;
                 const V3 pj = xyz(pj4[u]);
@@ -1295,9 +1308,17 @@ hipError_t launch_frame_begin(const DevState& d, float frame_dt, float h, hipStr
 
 hipError_t launch_collide(const DevState& d, int in, float h, int block, hipStream_t s) {
     if (!d.ntiles) return hipSuccess;
-    if (block == 64) hipLaunchKernelGGL(k_collide<64>, dim3(d.ntiles * 4), dim3(64), 0, s, d, in, h);
-    else if (block == 128) hipLaunchKernelGGL(k_collide<128>, dim3(d.ntiles * 2), dim3(128), 0, s, d, in, h);
-    else hipLaunchKernelGGL(k_collide<256>, dim3(d.ntiles), dim3(256), 0, s, d, in, h);
+    const auto launch = [&](auto kernel, uint32_t bs) {
+        hipLaunchKernelGGL(kernel, dim3(d.ntiles * (VTX_TILE / bs)), dim3(bs), 0, s, d, in, h);
+    };
+    // few particles with neighbours: the pass is the chain of its loads, so eight neighbours and their start positions at a
+    // time, on many CUs; many: the lines it touches and the registers (102 for 72) count, so four, and start
+    // positions of contacts only. Folded cloths, us a frame of ten contact passes, 4 / 8: 4,096 particles
+    // 158 / 137, 40,000 190 / 175, 65,536 242 / 232, 131,044 302 / 313, 1,048,576 1109 / 1280.
+    if ((d.live & VTX_LIVE_SELFCOL) && d.nparticles <= VTX_COLLIDE_SMALL) launch(k_collide<64, 8>, 64);
+    else if (block == 64) launch(k_collide<64, 4>, 64);
+    else if (block == 128) launch(k_collide<128, 4>, 128);
+    else launch(k_collide<256, 4>, 256);
     return last_launch();
 }
 

@@ -55,6 +55,8 @@
 #define VTX_HASH_PART_CELLS 4096u    // cells of a range at most
 #define VTX_HASH_PART_LIST 4096u     // particles of a range held in LDS
 #define VTX_HASH_HEAVY 128u
+#define VTX_COLLIDE_SMALL 81920u   // live particles up to which the contact pass reads ahead
+
 // floor(2^32 / M), for the remainder by M (hash_coords).
 static inline uint32_t mod_constant(uint32_t M) { return M > 1 ? (uint32_t)((1ull << 32) / M) : ~0u; }
 
@@ -155,6 +157,11 @@ struct alignas(16) ColliderDev {
     float rel[12];
 };
 
+// What the live set has (DevState::live).
+#define VTX_LIVE_SELFCOL 1u   // a segment that collides with itself
+#define VTX_LIVE_KEYED 2u     // k_hash_part's segments of several ranges have VTX_SEG_HASH_KEYED
+#define VTX_LIVE_FULL 4u      // more than VTX_HASH_PART_FULL particles
+
 // Pointers and sizes every kernel may need; passed by value (kernel-argument segment).
 // A range of a segment's hash cells (k_hash_part), with what its workgroup needs of the segment.
 struct HashPartDev {
@@ -202,7 +209,7 @@ struct DevState {
     const float4* brest4;     // grid: bending rest angles of a cell (X, R, D)
     uint32_t ntiles, nstiles, nhist, ncells;
     uint32_t hbase0, nltiles, nhparts;       // hbase0: first histogram entry of this table set
-    uint32_t nftiles, nmtiles, fside, hkeyed, hfull;   // hfull: more than VTX_HASH_PART_FULL live particles; hkeyed: k_hash_part's segments have VTX_SEG_HASH_KEYED
+    uint32_t nftiles, nmtiles, fside, live;   // live: VTX_LIVE_* of the table set
     uint32_t nparticles, nitiles, ngtiles, remap;   // remap: workgroups -> tiles through xcd_tile
 };
 
