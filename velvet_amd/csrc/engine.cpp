@@ -1281,6 +1281,7 @@ void Engine::rebuild_tables() {
     any_lra_dense_ = false;
     any_lra_split_ = false;
     any_hash_lds_ = false;
+    any_large_search_ = false;
     any_grid_tunable_ = false;
     need_collide_ = false;
     live_particles_ = 0;
@@ -1335,6 +1336,7 @@ void Engine::rebuild_tables() {
         }
         const bool hlds = (sg.dev.flags & VTX_SEG_SELFCOL) && sg.dev.n <= VTX_HASH_PART_N && sg.dev.M <= VTX_HASH_PART_M;
         any_hash_lds_ = any_hash_lds_ || hlds;
+        any_large_search_ = any_large_search_ || ((sg.dev.flags & VTX_SEG_SELFCOL) && sg.dev.n > VTX_SEARCH_BY_INDEX);
         const bool in_lds = hlds && tun_.hash_lds;
         hseg.push_back(sg.dev);
         if (in_lds) {
@@ -1610,7 +1612,7 @@ void Engine::hash_build(const DevState& d, int in, hipStream_t s) {
         stage_end(s);
     }
     stage_begin("k_neighbors", "Solver_HashCache", s);
-    VTX_HIP(launch_neighbors(d, s));
+    VTX_HIP(launch_neighbors(d, in, src, tun_.nbr_order == 0, s));
     stage_end(s);
     sorted_src_ = src;
 }
@@ -1891,26 +1893,31 @@ Tuning Engine::autotune(int frames, float frame_dt, bool use_cache, double* fram
         bms = trial(best);
         // one knob at a time, every other value of it against the best so far; the hash grid
         // (opted-in segments only) goes before the knobs of the hash and neighbour phases
-        static const int order[] = {0, 8, 2, 3, 4, 5, 7};
+        static const int order[] = {0, 8, 1, 2, 3, 4, 5, 7};
         for (int knob : order) {
             if (knob == 8 && !any_grid_tunable_) continue;
+            if (knob == 1 && !any_large_search_) continue;
             if (knob == 2 && !any_lra_split_) continue;
             if (knob == 4 && !need_collide_) continue;
             if (knob == 5 && table_seg_.size() < 2) continue;
             if (knob == 7 && !any_hash_lds_) continue;
-            const int nval = knob == 5 || knob == 8 ? 4 : knob == 4 ? 3 : 2;
+            // the grid decides whether the search by index gains: tried together
+            const int nval = knob == 8 && any_large_search_ ? 8 : knob == 5 || knob == 8 ? 4 : knob == 4 ? 3 : 2;
             const Tuning base = best;
             for (int v = 0; v < nval; v++) {
                 Tuning t = base;
                 if (knob == 0) t.graph = v != 0;
+                if (knob == 1) t.nbr_order = v == 0 ? 0 : 1;
                 if (knob == 2) t.lra_batch = v == 0 ? 4 : 16;
                 if (knob == 3) t.remap = v != 0;
                 if (knob == 4) t.gather_block = 64 << v;
                 if (knob == 5) t.streams = v + 1;
                 if (knob == 7) t.hash_lds = v != 0;
-                if (knob == 8) t.hash_grid = v;
-                if (knob == 8 ? t.hash_grid == base.hash_grid
+                if (knob == 8) t.hash_grid = v & 3;
+                if (knob == 8 && v > 3) t.nbr_order = 0;
+                if (knob == 8 ? t.hash_grid == base.hash_grid && t.nbr_order == base.nbr_order
                     : knob == 0 ? t.graph == base.graph
+                    : knob == 1 ? (t.nbr_order == 0) == (base.nbr_order == 0)
                                 : knob == 2 ? t.lra_batch == base.lra_batch
                                 : knob == 3 ? t.remap == base.remap
                                 : knob == 4 ? t.gather_block == base.gather_block

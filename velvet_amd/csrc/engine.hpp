@@ -133,7 +133,7 @@ struct Segment {
 // replayed from a graph, never the arithmetic.
 struct Tuning {
     bool graph = true;        // replay frames from a hipGraph
-    int nbr_order = 2;        // kept for callers (vtx_tuning.neighbor_order), no effect
+    int nbr_order = 2;        // 0: the search takes large segments by particle index; 1, 2: in sorted order
     int lra_batch = 16;       // distances of 32 or more dense slots loaded per batch: 4 or 16 (64 runs as 16)
     bool remap = true;        // XCD-aware workgroup -> tile remap
     int gather_block = 256;   // threads per workgroup of the contact pass
@@ -323,6 +323,7 @@ private:
     bool any_lra_dense_ = false;
     bool any_lra_split_ = false;   // a stencil segment has tiled dense attachments
     bool any_hash_lds_ = false;    // a self-colliding segment is small enough for k_hash_part
+    bool any_large_search_ = false;   // a self-colliding segment is large enough for the search by index
     bool any_grid_tunable_ = false;   // a live self-colliding segment has tune_hash_grid
     bool use_stencil_ = true;
     hipGraphExec_t gexec_ = nullptr;

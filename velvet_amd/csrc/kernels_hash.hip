@@ -565,8 +565,7 @@ __global__ __launch_bounds__(BT, 8) void k_hash_part(DevState d, int in, int dst
 // particle tests some 150 candidates at 15 VALU instructions per 64, and 6 more where one is accepted:
 // 85% of its VALU issue time). A segment whose records outgrow the L2 is bound by fetching each cell's
 // records some 27 times, as neighbours in the sorted order are no neighbours in space: a folded pile of
-// 1,048,576 759 -> 267 us, 874 MB. Taking cells by particle index instead fetches 210 MB, but its waves
-// are uneven and it gains nothing with three solvers overlapping (2.89 -> 3.02 ms a frame pair).
+// 1,048,576 759 -> 267 us, 874 MB (by particle index instead: neighbor_blocks).
 struct NbSet {
     const float4* rec;    // sorted records: position with w = index at 2i, initial position at 2i + 1
     const uint2* cells;   // (start, end) per hash cell
@@ -641,8 +640,9 @@ __device__ __forceinline__ void ld_record_uniform(const float4* rec, uint32_t i,
     o = make_float4(q[4], q[5], q[6], 0.f);
 }
 
-// The lists of sorted particles [i0, i0 + cnt), cnt <= PW, by the calling wave.
-template <int PW, NbStore ST, bool SMALL>
+// The lists of cnt <= PW particles by the calling wave: the sorted positions from i0 on, or with LISTED
+// lane m's i0.
+template <int PW, NbStore ST, bool SMALL, bool LISTED>
 __device__ __forceinline__ void neighbor_wave_as(const NbSet& a, uint32_t i0, uint32_t cnt, NbLds<PW>& L) {
 #pragma clang fp contract(off)
     constexpr int NC = 2;                                   // candidate chunks held at a time
@@ -650,7 +650,7 @@ __device__ __forceinline__ void neighbor_wave_as(const NbSet& a, uint32_t i0, ui
     const uint64_t lt = (1ull << lane) - 1ull;
     // the wave's particles: cells, runs
     float4 me = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (lane < cnt) me = a.rec[2 * (size_t)(i0 + lane)];
+    if (lane < cnt) me = a.rec[2 * (size_t)(LISTED ? i0 : i0 + lane)];
     int32_t ix, iy, iz;
     cell_coords(me, a.cell, a.shift, ix, iy, iz);
     // every lane active in the exchange: one that sits out would hand its neighbour nothing
@@ -712,7 +712,7 @@ __device__ __forceinline__ void neighbor_wave_as(const NbSet& a, uint32_t i0, ui
                 wave_lds_sync();
                 const uint32_t own = scan64_max(L.mark[lane]);
                 const uint32_t b = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((own - 1u) << 2), (int)base);
-                const uint32_t at = c0 + lane < total ? b + c0 + lane : i0;
+                const uint32_t at = c0 + lane < total ? b + c0 + lane : 0u;
                 q[h] = a.rec[2 * (size_t)at];
                 x[h] = a.rec[2 * (size_t)at + 1];
                 if (c0 + lane >= total) q[h].x = __builtin_nanf("");
@@ -721,7 +721,7 @@ __device__ __forceinline__ void neighbor_wave_as(const NbSet& a, uint32_t i0, ui
             // lanes without a candidate are farther than any distance; the particle itself is told by its index
             for (uint32_t m = m0; m < m1; m++) {
                 float4 p, o;
-                ld_record_uniform(a.rec, i0 + m, p, o);
+                ld_record_uniform(a.rec, LISTED ? (uint32_t)__builtin_amdgcn_readlane((int)i0, (int)m) : i0 + m, p, o);
                 const uint32_t id = __float_as_uint(p.w);
                 uint32_t k = (uint32_t)__builtin_amdgcn_readlane((int)kv, (int)m);
 #pragma unroll
@@ -749,17 +749,54 @@ __device__ __forceinline__ void neighbor_wave_as(const NbSet& a, uint32_t i0, ui
     if (lane < cnt && kv < a.K) nb_put<ST != NB_COLUMN>(a, __float_as_uint(me.w), kv, VTX_INVALID);
 }
 
-template <int PW, bool CHUNK>
+template <int PW, bool CHUNK, bool LISTED = false>
 __device__ __forceinline__ void neighbor_wave(const NbSet& a, uint32_t i0, uint32_t cnt, NbLds<PW>& L) {
-    if (CHUNK && a.n16) neighbor_wave_as<PW, NB_CHUNK16, true>(a, i0, cnt, L);   // n < 2^16
-    else if (a.n < (1u << 22)) neighbor_wave_as<PW, CHUNK ? NB_CHUNK32 : NB_COLUMN, true>(a, i0, cnt, L);
-    else neighbor_wave_as<PW, CHUNK ? NB_CHUNK32 : NB_COLUMN, false>(a, i0, cnt, L);
+    if (CHUNK && a.n16) neighbor_wave_as<PW, NB_CHUNK16, true, LISTED>(a, i0, cnt, L);   // n < 2^16
+    else if (a.n < (1u << 22)) neighbor_wave_as<PW, CHUNK ? NB_CHUNK32 : NB_COLUMN, true, LISTED>(a, i0, cnt, L);
+    else neighbor_wave_as<PW, CHUNK ? NB_CHUNK32 : NB_COLUMN, false, LISTED>(a, i0, cnt, L);
+}
+
+// The search by particle index (neighbor_order 0), for segments whose records outgrow the L2. In sorted order
+// the waves that run at one time have no cells in common, as neighbouring hashes are no neighbours in space.
+// Here a wave takes whole blocks of cells by index: neighbours in a cloth's index order are neighbours in
+// space, and a tile's wave and those beside it (on one XCD) share cells. A block is what a bucket holds of an
+// aligned run of PW sorted positions; the one of its particles that leads it is drawn by a hash of its first
+// position, so that of several layers not the lowest does all the work. inv: particle -> sorted position.
+// A draped 1,048,576-particle cloth on grid 1: 244 -> 162 us a search, 1.74 -> 1.58 ms a frame; on the
+// reference grid, whose mirrored cells share buckets, no gain; and a pile whose frames overlap with two
+// other solvers' loses, 2.89 -> 3.03 ms, as the waves are uneven and fetches are not what bounds it. So the
+// caller (neighbor_order) or the tuner chooses.
+template <int PW>
+__device__ __forceinline__ void neighbor_blocks(const NbSet& a, const uint32_t* __restrict__ inv,
+                                                const float4* __restrict__ P, uint32_t first, uint32_t cnt, NbLds<PW>& L) {
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t begin = 0, len = 0;
+    if (lane < cnt) {
+        const uint32_t pos = inv[first + lane];
+        const uint2 c = a.cells[position_key(P[first + lane], a.cell, a.shift, a.M, a.mod)];
+        begin = max(c.x, pos & ~(PW - 1u));
+        const uint32_t n = min(c.y, (pos & ~(PW - 1u)) + PW) - begin;
+        if (pos == begin + (((begin * 2654435761u) >> 16) * n >> 16)) len = n;
+    }
+    const uint32_t incl = scan32_add(len), excl = incl - len;
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 31);
+    for (uint32_t b = 0; b < total; b += PW) {
+        L.mark[lane] = 0;
+        wave_lds_sync();
+        if (len && incl > b && excl < b + PW) L.mark[max(excl, b) - b] = lane + 1u;
+        wave_lds_sync();
+        const uint32_t own = scan64_max(L.mark[lane]);
+        const uint32_t at = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((own - 1u) << 2), (int)(begin - excl));
+        wave_lds_sync();
+        neighbor_wave<PW, true, true>(a, at + b + lane, min((uint32_t)PW, total - b), L);
+        wave_lds_sync();
+    }
 }
 
 // The search over the segments' particle tiles (a tile's sorted positions): 4 PW particles per
 // workgroup of four waves.
-template <int PW>
-__global__ __launch_bounds__(256) void k_neighbors(DevState d) {
+template <int PW, bool BY_INDEX>
+__global__ __launch_bounds__(256) void k_neighbors(DevState d, int in, const uint32_t* __restrict__ inv) {
     __shared__ NbLds<PW> lds[4];
     const uint32_t b = tile_of(d.remap), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     constexpr uint32_t S = VTX_TILE / (4 * PW);                 // workgroups per tile
@@ -780,7 +817,11 @@ __global__ __launch_bounds__(256) void k_neighbors(DevState d) {
     a.cell2 = sg.cell2;
     a.diam2 = sg.diam2;
     a.n16 = sg.flags & VTX_SEG_NBR16;
-    neighbor_wave<PW, true>(a, t.begin - sg.pbase + first, min((uint32_t)PW, t.count - first), lds[wave]);
+    const uint32_t i = t.begin - sg.pbase + first, cnt = min((uint32_t)PW, t.count - first);
+    if (BY_INDEX && sg.n > VTX_SEARCH_BY_INDEX && !(sg.flags & VTX_SEG_HASH_PART))
+        neighbor_blocks<PW>(a, inv + sg.pbase, d.P[in] + sg.pbase, i, cnt, lds[wave]);
+    else
+        neighbor_wave<PW, true>(a, i, cnt, lds[wave]);
 }
 
 // ---------------------------------------------------------------- kernel-launch tier
@@ -1106,12 +1147,14 @@ hipError_t launch_cell_bounds(const DevState& d, int in, int src, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_neighbors(const DevState& d, hipStream_t s) {
+hipError_t launch_neighbors(const DevState& d, int in, int src, bool by_index, hipStream_t s) {
     const auto nb = [&](auto kernel, uint32_t pw) {
-        hipLaunchKernelGGL(kernel, dim3(d.ntiles * (VTX_TILE / (4 * pw))), dim3(256), 0, s, d);
+        hipLaunchKernelGGL(kernel, dim3(d.ntiles * (VTX_TILE / (4 * pw))), dim3(256), 0, s, d, in,
+                           (const uint32_t*)d.keys[src ^ 1]);   // the inverse permutations k_cell_bounds leaves
     };
-    if (search_small(d.nparticles)) nb(k_neighbors<8>, 8);
-    else nb(k_neighbors<32>, 32);
+    if (search_small(d.nparticles)) nb(k_neighbors<8, false>, 8);
+    else if (by_index) nb(k_neighbors<32, true>, 32);
+    else nb(k_neighbors<32, false>, 32);
     return hipGetLastError();
 }
 

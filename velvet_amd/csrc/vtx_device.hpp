@@ -57,6 +57,8 @@
 #define VTX_HASH_HEAVY 128u
 #define VTX_COLLIDE_SMALL 81920u   // live particles up to which the contact pass reads ahead
 
+#define VTX_SEARCH_BY_INDEX 131072u   // particles of a segment whose records (32 B each) outgrow an L2
+
 // floor(2^32 / M), for the remainder by M (hash_coords).
 static inline uint32_t mod_constant(uint32_t M) { return M > 1 ? (uint32_t)((1ull << 32) / M) : ~0u; }
 
