@@ -776,7 +776,7 @@ __device__ __forceinline__ void neighbor_blocks(const NbSet& a, const uint32_t* 
         const uint2 c = a.cells[position_key(P[first + lane], a.cell, a.shift, a.M, a.mod)];
         begin = max(c.x, pos & ~(PW - 1u));
         const uint32_t n = min(c.y, (pos & ~(PW - 1u)) + PW) - begin;
-        if (pos == begin + (((begin * 2654435761u) >> 16) * n >> 16)) len = n;
+        if (c.x <= pos && pos < c.y && pos == begin + (((begin * 2654435761u) >> 16) * n >> 16)) len = n;   // len <= PW
     }
     const uint32_t incl = scan32_add(len), excl = incl - len;
     const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 31);
