@@ -597,6 +597,7 @@ int32_t Engine::add_attach_slot(int32_t s, const float* pos) {
 }
 
 // Updates between frames travel in a launch's arguments; into a caller's capture they would be frozen.
+// Asked before the host's copies change, so that a refused update is not applied by a later upload.
 void Engine::refuse_capture() {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     VTX_HIP(hipStreamIsCapturing(stream_, &st));
@@ -608,13 +609,13 @@ void Engine::set_attach_slot_position(int32_t s, int32_t slot, const float* pos)
     Segment& sg = seg(s);
     VTX_REQUIRE(pos, VTX_EINVAL, "slot position is NULL");
     VTX_REQUIRE(slot >= 0 && (size_t)slot < sg.slots.size() / 3, VTX_EINVAL, "slot index out of range");
-    std::copy(pos, pos + 3, sg.slots.begin() + 3 * slot);
     const float4 v = make_float4(pos[0], pos[1], pos[2], 0.f);
-    if (sg.prepared) sg.prep.slots[(size_t)slot] = v;
     if (sg.uploaded) {   // the graph reads the slot table: no re-record
         refuse_capture();
         VTX_HIP(launch_set_slot(pl_.slots + sg.rg.slot + slot, v, stream_));
     }
+    std::copy(pos, pos + 3, sg.slots.begin() + 3 * slot);
+    if (sg.prepared) sg.prep.slots[(size_t)slot] = v;
 }
 
 // AddAttach (Velvet/VtClothSolverGPU.hpp:170-176): distance 0 pins the particle.
@@ -673,12 +674,14 @@ void Engine::set_colliders(int32_t s, const vtx_collider* cols, uint32_t n) {
     for (uint32_t c = 0; c < n; c++)
         VTX_REQUIRE(cols[c].type >= 0 && cols[c].type <= 2, VTX_EINVAL, "unknown collider type");
     if (sg.cols.size() == n && sg.prepared) {   // same count: rewrite in place, no re-record
-        sg.cols.assign(cols, cols + n);
-        for (uint32_t c = 0; c < n; c++) sg.prep.cols[c] = pack_collider(cols[c]);
+        std::vector<ColliderDev> packed(n);
+        for (uint32_t c = 0; c < n; c++) packed[c] = pack_collider(cols[c]);
         if (sg.uploaded && n) {
             refuse_capture();
-            VTX_HIP(launch_set_colliders(pl_.cols + sg.rg.col, sg.prep.cols.data(), n, stream_));
+            VTX_HIP(launch_set_colliders(pl_.cols + sg.rg.col, packed.data(), n, stream_));
         }
+        sg.cols.assign(cols, cols + n);
+        sg.prep.cols.swap(packed);
         return;
     }
     touch(s);
