@@ -1968,6 +1968,7 @@ void Engine::set_timing(bool on) {
     timing_ = on;
     timing_ms_.clear();
     timing_n_.clear();
+    timing_passes_.clear();
     timing_kernel_.clear();
 }
 
