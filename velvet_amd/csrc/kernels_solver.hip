@@ -1065,7 +1065,9 @@ __global__ __launch_bounds__(1024) void k_iterate_fused(DevState d, const GridTi
             p = d.P[in][sg.pbase + v];
             r = d.rest4[sg.pbase + v];
         }
-        for (int e = tid; e < 4 * F::NS; e += 1024) corr[0][e].w = 0.f;   // while the loads are in flight
+        for (int e = tid; e < F::NS; e += 1024)                           // while the loads are in flight
+#pragma unroll
+            for (int r = 0; r < 4; r++) corr[r][e].w = 0.f;
         if (in_cloth)
             for (uint32_t s = 0; s < nslots; s++) sl[s][tid] = d.lra[4 * (size_t)sg.lbase + (size_t)s * sg.n + v];
         if (tid < VTX_FS * VTX_FS) {
@@ -1122,7 +1124,9 @@ __global__ __launch_bounds__(1024, 8) void k_iterate_split(DevState d, const Gri
             p = d.P[in][v];
             r = d.rest4[v];
         }
-        for (int e = tid; e < 3 * F::NS; e += 1024) corr[0][e].w = 0.f;   // no slot marked
+        for (int e = tid; e < F::NS; e += 1024)                           // no slot marked
+#pragma unroll
+            for (int r = 0; r < 3; r++) corr[r][e].w = 0.f;
         if (tid < VTX_FS * VTX_FS) {
             sp[tid] = p;
             sr[tid] = r;
