@@ -13,6 +13,7 @@
 // cub::DeviceRadixSort::SortPairs call (Velvet/SpatialHashGPU.cu:133-157).
 #include <hip/hip_runtime.h>
 
+#include <cstddef>
 #include <mutex>
 #include <type_traits>
 
@@ -349,12 +350,13 @@ __device__ __forceinline__ uint32_t scan64_max(uint32_t v) {
 // LDS took one CU for the whole of it: 4,608 particles 20 -> 8.5 us (one workgroup), 16,384 55 -> 14.4
 // (one workgroup; k_hash_keys included, as below), 22,500 49 -> 16 (device-wide), 65,536 73 -> 25,
 // 131,044 in a frame of four builds 492 -> 354, 16 cloths of 65,536 1338 -> 1122 a frame of four builds.
-struct HashPartLds {
+struct alignas(16) HashPartLds {           // cnt is read and written four words at a time
     uint32_t cnt[VTX_HASH_PART_CELLS];      // per cell of the range: count, start, end (exclusive)
     uint32_t list[VTX_HASH_PART_LIST + 3];  // the range's particles by cell: cell << 20 | index
     uint32_t heavy[VTX_HASH_PART_N / VTX_HASH_HEAVY];
     uint32_t wsum[16], nheavy, below;
 };
+static_assert(offsetof(HashPartLds, cnt) % 16 == 0, "cnt is accessed in 16-byte units");
 
 // S: the particles (key(i), written(g, key, i) for sorted position g, cell(k, begin, end)).
 template <uint32_t BT, bool KEYED, class S>
