@@ -1337,7 +1337,7 @@ void Engine::rebuild_tables() {
             sg.dev.mod = mod_constant(sg.dev.M);
             sg.dev.flags = (sg.dev.flags & ~VTX_SEG_HASH_SHIFT) | (shifted ? VTX_SEG_HASH_SHIFT : 0u);
         }
-        const bool hlds = (sg.dev.flags & VTX_SEG_SELFCOL) && sg.dev.n <= VTX_HASH_PART_N && sg.dev.M <= VTX_HASH_PART_M;
+        const bool hlds = (sg.dev.flags & VTX_SEG_SELFCOL) && hash_by_ranges(sg.dev.n, sg.dev.M);
         any_hash_lds_ = any_hash_lds_ || hlds;
         any_large_search_ = any_large_search_ || ((sg.dev.flags & VTX_SEG_SELFCOL) && sg.dev.n > VTX_SEARCH_BY_INDEX);
         const bool in_lds = hlds && tun_.hash_lds;

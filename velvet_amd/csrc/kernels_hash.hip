@@ -336,14 +336,24 @@ __device__ __forceinline__ uint32_t scan64_max(uint32_t v) {
     return max(v, dpp0<0x143, 0xc>(v));   // row_bcast:31
 }
 
+// Order LDS accesses of the lanes of one wave (a wave's LDS operations execute in order).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // The whole spatial-hash build of one segment of at most VTX_HASH_PART_N particles in one launch (after
 // k_hash_keys, see VTX_HASH_PART_KEYS): the table's cells are cut into ranges, and a workgroup builds one
 // range on its own. It runs over the keys of all particles, counts those in its range per cell in LDS and
 // those below the range (the range's first sorted position), scans the counts, puts the range's particles
 // into their cells in any order and finds each one's place inside its cell by counting the cell's smaller
-// indices: a stable sort by key, so the same table and records as the device-wide path. A cell of more
-// than VTX_HASH_HEAVY particles is placed by one more run over the keys in index order instead, so that
-// no input costs quadratic time.
+// indices: a stable sort by key, so the same table and records as the device-wide path. Counting a cell
+// of c particles costs c^2, so a range with a cell of more than VTX_HASH_HEAVY sorts its list in LDS
+// instead, or, if it holds more than the list, places such cells by two runs over the keys in index order
+// for up to 256 of them at a time (hash_part_runs), so that no input costs quadratic time: 131,072 objects
+// with their search, in cells of 100 / 140 / 300 / 2,000: 66 / 80 / 93 / 101 us, in a table of 1,000 cells
+// 95 us (device-wide sort 113 / 113 / 111 / 109, 97; two runs for each crowded cell 66 / 649 / 455 / 263, 460).
 // Bound by latency: a launch's 2.6 us, then the chain range record, keys, LDS counts, scan, placement,
 // gathered records, and from 2^15 particles on the two runs over the keys. No workgroup waits for another,
 // where the dozen launches of a device-wide sort did and one workgroup per segment with a radix sort in
@@ -358,7 +368,113 @@ struct alignas(16) HashPartLds {           // cnt is read and written four words
 };
 static_assert(offsetof(HashPartLds, cnt) % 16 == 0, "cnt is accessed in 16-byte units");
 
-// S: the particles (key(i), written(g, key, i) for sorted position g, cell(k, begin, end)).
+// Ascending bitonic sort of a[0..m), m a power of two of at least 1. Thread t exchanges a pair 2^b apart;
+// for pairs up to 64 apart a wave's threads stay within 128 words of their own, so steps of such pairs
+// follow each other without a workgroup barrier.
+template <uint32_t BT>
+__device__ __forceinline__ void sort_list(uint32_t* a, uint32_t m) {
+    for (uint32_t k = 2; k <= m; k <<= 1)
+        for (uint32_t j = k >> 1; j; j >>= 1) {
+            for (uint32_t t = threadIdx.x; t < m >> 1; t += BT) {
+                const uint32_t i = (t & ~(j - 1u)) << 1 | (t & (j - 1u));
+                const uint32_t x = a[i], y = a[i | j];
+                if ((x > y) == !(i & k)) {
+                    a[i] = y;
+                    a[i | j] = x;
+                }
+            }
+            if (j > 64u || (j == 1u && k >= 128u)) __syncthreads();   // the next step's pairs: j / 2 or k apart
+            else wave_lds_sync();
+        }
+    __syncthreads();
+}
+
+// The cells of more than VTX_HASH_HEAVY particles of a range that holds more than its list, up to 256 (512)
+// of them at a time: wave w takes the w-th part of the particles in order, counts its particles per cell,
+// then places them behind those of the waves before it, 64 at a time ranked by ballots over the cell's number.
+// U times 64 keys are in flight.
+template <uint32_t BT, uint32_t U, class S>
+__device__ __forceinline__ void hash_part_runs(const S& s, uint32_t n, uint32_t lo, uint32_t C, uint32_t base,
+                                               uint32_t nheavy, HashPartLds& L) {
+    constexpr uint32_t NW = BT / 64, HB = VTX_HASH_PART_LIST / NW;
+    constexpr int BITS = HB == 256 ? 8 : 9;
+    static_assert(HB == 1u << BITS, "a cell's number among HB");
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    __syncthreads();                                        // the cells' bounds are read
+    for (uint32_t h = tid; h < nheavy; h += BT) {           // with the cell's first place (< 2^17)
+        const uint32_t k = L.heavy[h];
+        L.heavy[h] = (k ? L.cnt[k - 1] : 0u) << 12 | k;
+    }
+    __syncthreads();
+    for (uint32_t k = tid; k < C; k += BT) L.cnt[k] = VTX_INVALID;
+    __syncthreads();
+    for (uint32_t h = tid; h < nheavy; h += BT) L.cnt[L.heavy[h] & 0xFFFu] = h;
+    uint32_t* const hw = L.list + wave * HB;
+    const uint32_t chunk = (n + NW - 1) / NW, b = min(wave * chunk, n), e = min(b + chunk, n);
+    const uint64_t lt = (1ull << lane) - 1ull;
+    for (uint32_t h0 = 0; h0 < nheavy; h0 += HB) {
+        const uint32_t nb = min(HB, nheavy - h0);
+        for (uint32_t q = lane; q < HB; q += 64) hw[q] = 0;
+        __syncthreads();
+        uint32_t kk[U], q[U];                               // keys; the cells' numbers, nb or more: none
+        const auto load = [&](uint32_t i0) {
+#pragma unroll
+            for (uint32_t u = 0; u < U; u++) kk[u] = s.key(min(i0 + 64 * u + lane, n - 1u));
+#pragma unroll
+            for (uint32_t u = 0; u < U; u++) {
+                const uint32_t k = kk[u] - lo;
+                q[u] = VTX_INVALID;
+                if (i0 + 64 * u + lane < e && k < C) q[u] = L.cnt[k] - h0;
+            }
+        };
+        for (uint32_t i0 = b; i0 < e; i0 += 64 * U) {
+            load(i0);
+#pragma unroll
+            for (uint32_t u = 0; u < U; u++)
+                if (q[u] < nb) atomicAdd(&hw[q[u]], 1u);
+        }
+        __syncthreads();
+        for (uint32_t h = tid; h < nb; h += BT) {
+            uint32_t run = base + (L.heavy[h0 + h] >> 12);
+            for (uint32_t w = 0; w < NW; w++) {
+                const uint32_t c = L.list[w * HB + h];
+                L.list[w * HB + h] = run;
+                run += c;
+            }
+        }
+        __syncthreads();
+        for (uint32_t i0 = b; i0 < e; i0 += 64 * U) {
+            load(i0);
+            uint32_t at[U];
+#pragma unroll
+            for (uint32_t u = 0; u < U; u++) {
+                const bool hit = q[u] < nb;
+                uint64_t peers = __builtin_amdgcn_ballot_w64(hit);
+                if (!peers) continue;
+#pragma unroll
+                for (int c = 0; c < BITS; c++) {
+                    const uint32_t m = (uint32_t)((int32_t)(q[u] << (31 - c)) >> 31);   // bit c as 0 / ~0
+                    peers &= ~(__builtin_amdgcn_ballot_w64(m != 0u) ^ ((uint64_t)m << 32 | m));
+                }
+                const uint32_t rank = (uint32_t)__popcll(peers & lt);
+                at[u] = hw[hit ? q[u] : 0u] + rank;
+                wave_lds_sync();
+                if (hit && rank == 0) hw[q[u]] = at[u] + (uint32_t)__popcll(peers);
+                wave_lds_sync();
+            }
+            float4 p[U], x[U];
+#pragma unroll
+            for (uint32_t u = 0; u < U; u++)
+                if (q[u] < nb) s.get(i0 + 64 * u + lane, p[u], x[u]);
+#pragma unroll
+            for (uint32_t u = 0; u < U; u++)
+                if (q[u] < nb) s.put(at[u], kk[u], i0 + 64 * u + lane, p[u], x[u]);
+        }
+        __syncthreads();
+    }
+}
+
+// S: the particles (key(i), put(g, key, i) for sorted position g, cell(k, begin, end)).
 template <uint32_t BT, bool KEYED, class S>
 __device__ __forceinline__ void hash_part(const S& s, uint32_t n, uint32_t lo, uint32_t C, uint32_t* __restrict__ spill,
                                           HashPartLds& L) {
@@ -418,6 +534,7 @@ __device__ __forceinline__ void hash_part(const S& s, uint32_t n, uint32_t lo, u
         off += c.x + c.y + c.z + c.w;
     }
     const uint32_t base = L.below, nheavy = L.nheavy;
+    const uint32_t padded = own <= 1u ? 1u : 1u << (32 - __builtin_clz(own - 1u));   // list entries to sort
     __syncthreads();
     // the range's particles into their cells, in any order; more than fit go through global scratch
     const auto rest = [&](uint32_t* __restrict__ list, auto clamp) {
@@ -432,6 +549,14 @@ __device__ __forceinline__ void hash_part(const S& s, uint32_t n, uint32_t lo, u
             }
         }
         __syncthreads();
+        if (!clamp.value && nheavy) {
+            sort_list<BT>(list, padded);
+            for (uint32_t g = tid; g < own; g += BT) {
+                const uint32_t e = list[g];
+                s.put(base + g, lo + (e >> 20), e & 0xFFFFFu);
+            }
+            return;
+        }
         for (uint32_t g = tid; g < own; g += BT) {
             const uint32_t e = list[g], k = e >> 20;
             const uint32_t begin = k ? L.cnt[k - 1] : 0u, end = L.cnt[k];
@@ -449,6 +574,8 @@ __device__ __forceinline__ void hash_part(const S& s, uint32_t n, uint32_t lo, u
     };
     if (own <= VTX_HASH_PART_LIST) {
         if (tid < 3) L.list[own + tid] = VTX_INVALID;
+        if (nheavy)
+            for (uint32_t g = own + tid; g < padded; g += BT) L.list[g] = VTX_INVALID;
         rest(L.list, std::false_type{});
     } else {
         rest(spill + base, std::true_type{});
@@ -457,28 +584,7 @@ __device__ __forceinline__ void hash_part(const S& s, uint32_t n, uint32_t lo, u
         const uint32_t begin = k ? L.cnt[k - 1] : 0u, end = L.cnt[k];
         s.cell(lo + k, end > begin ? base + begin : VTX_INVALID, end > begin ? base + end : VTX_INVALID);
     }
-    // heavy cells: wave w takes the w-th part of the particles; its matches before the others' counts
-    for (uint32_t h = 0; h < nheavy; h++) {
-        const uint32_t k = L.heavy[h], chunk = (n + NW - 1) / NW;
-        const uint32_t b = min(wave * chunk, n), e = min(b + chunk, n);
-        uint32_t count = 0;
-        for (uint32_t i0 = b; i0 < e; i0 += 64) {
-            const uint32_t i = i0 + lane;
-            count += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(i < e && s.key(min(i, n - 1u)) == lo + k));
-        }
-        __syncthreads();
-        if (lane == 0) L.wsum[wave] = count;
-        __syncthreads();
-        uint32_t at = base + (k ? L.cnt[k - 1] : 0u);
-        for (uint32_t w = 0; w < wave; w++) at += L.wsum[w];
-        for (uint32_t i0 = b; i0 < e; i0 += 64) {
-            const uint32_t i = i0 + lane;
-            const bool hit = i < e && s.key(min(i, n - 1u)) == lo + k;
-            const uint64_t mask = __builtin_amdgcn_ballot_w64(hit);
-            if (hit) s.put(at + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull)), lo + k, i);
-            at += (uint32_t)__popcll(mask);
-        }
-    }
+    if (nheavy && own > VTX_HASH_PART_LIST) hash_part_runs<BT, KEYED ? 4 : 1>(s, n, lo, C, base, nheavy, L);
 }
 
 // A segment's particles: float4 positions, keys from k_hash_keys or worked out here.
@@ -515,12 +621,20 @@ struct SegmentHash {
             if (u * BT < n) k[u] = of(p[u]);
         }
     }
-    __device__ __forceinline__ void put(uint32_t g, uint32_t k, uint32_t i) const {
-        const float4 p = P[i], x = X0[i];
+    __device__ __forceinline__ void get(uint32_t i, float4& p, float4& x) const {
+        p = P[i];
+        x = X0[i];
+    }
+    __device__ __forceinline__ void put(uint32_t g, uint32_t k, uint32_t i, float4 p, float4 x) const {
         ko[g] = k;
         vo[g] = i;
         rec[2 * (size_t)g] = make_float4(p.x, p.y, p.z, __uint_as_float(i));
         rec[2 * (size_t)g + 1] = x;
+    }
+    __device__ __forceinline__ void put(uint32_t g, uint32_t k, uint32_t i) const {
+        float4 p, x;
+        get(i, p, x);
+        put(g, k, i, p, x);
     }
     __device__ __forceinline__ void cell(uint32_t k, uint32_t begin, uint32_t end) const { cells[k] = make_uint2(begin, end); }
 };
@@ -626,13 +740,6 @@ struct NbLds {
     uint32_t cx[PW], cy[PW], cz[PW];   // per run: its cell's coordinates times the hash's factors
     uint32_t mark[64];
 };
-
-// Order LDS accesses of the lanes of one wave (a wave's LDS operations execute in order).
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // A sorted record through the scalar cache (i wave-uniform).
 __device__ __forceinline__ void ld_record_uniform(const float4* rec, uint32_t i, float4& p, float4& o) {
@@ -924,12 +1031,20 @@ struct RawHash {
             if (u * BT < n) k[u] = of(p[u]);
         }
     }
-    __device__ __forceinline__ void put(uint32_t g, uint32_t k, uint32_t i) const {
-        const float4 p = ld_xyz(pos, i, __uint_as_float(i)), x = ld_xyz(pos0, i, 0.f);
+    __device__ __forceinline__ void get(uint32_t i, float4& p, float4& x) const {
+        p = ld_xyz(pos, i, __uint_as_float(i));
+        x = ld_xyz(pos0, i, 0.f);
+    }
+    __device__ __forceinline__ void put(uint32_t g, uint32_t k, uint32_t i, float4 p, float4 x) const {
         ko[g] = k;
         vo[g] = i;
         rec[2 * (size_t)g] = p;
         rec[2 * (size_t)g + 1] = x;
+    }
+    __device__ __forceinline__ void put(uint32_t g, uint32_t k, uint32_t i) const {
+        float4 p, x;
+        get(i, p, x);
+        put(g, k, i, p, x);
     }
     __device__ __forceinline__ void cell(uint32_t k, uint32_t b, uint32_t e) const {
         cells[k] = make_uint2(b, e);
@@ -1009,7 +1124,7 @@ hipError_t hash_objects(const HashObjectsArgs& a, void* workspace, hipStream_t s
         if (search_small(n)) nb(k_raw_neighbors<8>, 8);
         else nb(k_raw_neighbors<32>, 32);
     };
-    if (n && n <= VTX_HASH_PART_N && M <= VTX_HASH_PART_M) {   // one or two launches instead of up to sixteen
+    if (n && hash_by_ranges(n, M)) {   // one or two launches instead of up to sixteen
         const uint32_t width = hash_part_width(n, M, VTX_HASH_PART_SHARE), parts = (M + width - 1) / width;
         const auto build = [&](auto keyed) {
             constexpr bool K = decltype(keyed)::value;

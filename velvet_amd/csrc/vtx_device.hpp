@@ -69,6 +69,11 @@ static inline uint32_t mod_constant(uint32_t M) { return M > 1 ? (uint32_t)((1ul
 #define VTX_HASH_PART_SHARE 1024u
 #define VTX_HASH_PART_SHARE_FULL 2048u
 #define VTX_HASH_PART_FULL 262144u   // live particles
+// Whether a segment is built by cell ranges: beyond these sizes the device-wide sort takes it, and where a
+// cell of an evenly filled table would fill half of a range's list.
+static inline bool hash_by_ranges(uint32_t n, uint32_t M) {
+    return n <= VTX_HASH_PART_N && M <= VTX_HASH_PART_M && n <= (uint64_t)M * (VTX_HASH_PART_LIST / 2);
+}
 static inline uint32_t hash_part_width(uint32_t n, uint32_t M, uint32_t share) {
     uint32_t parts = (n + share - 1) / share;
     if (parts < (M + VTX_HASH_PART_CELLS - 1) / VTX_HASH_PART_CELLS) parts = (M + VTX_HASH_PART_CELLS - 1) / VTX_HASH_PART_CELLS;
