@@ -1306,6 +1306,21 @@ void Engine::rebuild_tables() {
     // mode keeps one group so that per-launch figures cover the whole workload
     const uint32_t G = timing_ ? 1u : std::max(1u, std::min<uint32_t>((uint32_t)tun_.streams, nlive));
     const uint32_t fside = fuse_side();
+    // groups with a grid cloth that runs one pass per launch: the others' tiles ride in those launches, as
+    // fused launches would come on top of them, one after the other on the group's stream (5 substeps x 10
+    // passes, 40 x 40 beside 48 x 48 with 8 slots 477 us a frame, with fused launches 601; 200 x 200 beside
+    // 40 x 40 with 8 slots 452 / 660)
+    std::vector<uint8_t> single(G, 0);
+    {
+        uint64_t c = 0;
+        uint32_t k = 0;
+        for (auto& sp : segs_)
+            if (sp && sp->active && sp->uploaded && sp->n()) {
+                if (k + 1 < G && c > 0 && c * G >= total_n * (k + 1)) k++;   // as the cuts below
+                c += sp->n();
+                if (sp->prep.grid && !sp->prep.lra_tiled && !fusable(*sp)) single[k] = 1;
+            }
+    }
     struct Cut { size_t t, i, g, l, s, m, f, n; uint32_t h, p; };
     std::vector<Cut> cuts;                     // where groups 1..G-1 begin
     uint64_t cum = 0;
@@ -1373,7 +1388,7 @@ void Engine::rebuild_tables() {
             htile.push_back(t);
             if (!sg.prep.grid) hitile.push_back(t);
         }
-        const bool fused = fside && fusable(sg);
+        const bool fused = fside && fusable(sg) && !single[cuts.size()];
         for (GridTileDev gt : sg.prep.gtiles) {
             gt.seg = ti;
             gt.at_off += (uint32_t)(sg.prep.lra_tiled ? sg.rg.lra / 4 : sg.rg.at);
