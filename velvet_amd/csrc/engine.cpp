@@ -1417,6 +1417,15 @@ void Engine::rebuild_tables() {
         hbase += 256u * nst;
         if (!in_lds) compact += d.n;
     }
+    // tiles without bending constraints behind the others of their group, for the launch of their own: where
+    // all are, or where they fill the chip by themselves; a few go along with the others' launch
+    std::vector<uint32_t> plain(cuts.size() + 1, 0);
+    for (size_t k = 0; k <= cuts.size(); k++) {
+        const auto b = hitile.begin() + (ptrdiff_t)(k ? cuts[k - 1].i : 0);
+        const auto e = k < cuts.size() ? hitile.begin() + (ptrdiff_t)cuts[k].i : hitile.end();
+        const auto m = std::stable_partition(b, e, [](const TileDev& t) { return t.ub_n != 0; });
+        if (m == b || e - m > 256) plain[k] = (uint32_t)(e - m);
+    }
     passes_ = std::max(1, (int)((maxbits + 7) / 8));
     VTX_REQUIRE((hbase + VTX_SCAN_BLOCK - 1) / VTX_SCAN_BLOCK <= 65536u, VTX_ECAPACITY, "histogram too large");
     const size_t npart = VTX_MAX_STREAMS * ((hbase + VTX_SCAN_BLOCK - 1) / VTX_SCAN_BLOCK + 1);   // a share per group
@@ -1516,6 +1525,7 @@ void Engine::rebuild_tables() {
         g.nmtiles = (uint32_t)(hi.n - lo.n);
         g.ntiles = (uint32_t)(hi.t - lo.t);
         g.nitiles = (uint32_t)(hi.i - lo.i);
+        g.nptiles = plain[k];
         g.ngtiles = (uint32_t)(hi.g - lo.g);
         g.nltiles = (uint32_t)(hi.l - lo.l);
         g.nstiles = (uint32_t)(hi.s - lo.s);

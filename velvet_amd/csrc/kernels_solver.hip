@@ -523,6 +523,26 @@ __global__ __launch_bounds__(VTX_TILE) void k_epilogue(DevState d, int in, float
     epilogue<EPI>(d, sg, g, in, xyz(p4), p4.w, h);
 }
 
+// The stretch terms of a particle on the general path (lane of its tile, local index), eight neighbours in flight.
+__device__ __forceinline__ void stretch_terms(const DevState& d, const SegDev& sg, const TileDev& t,
+                                              const float4* __restrict__ P, uint32_t lane, uint32_t local, V3 p, float w,
+                                              V3& delta, int& cnt) {
+    constexpr uint32_t NS = 8;
+    const float nws = -w * sg.stiffness;
+    for (uint32_t k0 = 0; k0 < t.st_k; k0 += NS) {
+        uint2 c[NS];
+        float4 q[NS];
+#pragma unroll
+        for (uint32_t k = 0; k < NS; k++) c[k] = (d.st + t.st_off + min(k0 + k, t.st_k - 1u) * VTX_TILE)[lane];
+#pragma unroll
+        for (uint32_t k = 0; k < NS; k++) q[k] = P[c[k].x == VTX_INVALID ? local : c[k].x];
+#pragma unroll
+        for (uint32_t k = 0; k < NS; k++)
+            if (k0 + k < t.st_k && c[k].x != VTX_INVALID)
+                stretch_term(p, w, nws, q[k], __uint_as_float(c[k].y), delta, cnt);
+    }
+}
+
 // One Jacobi pass on the general path: SolveStretch (cu:65-102) + SolveAttachment
 // (cu:205-235) + SolveBending (cu:117-189) gathered per particle over its incident
 // constraints (sliced ELL), then ApplyDeltas (cu:253-264) and the epilogue.
@@ -541,7 +561,6 @@ __global__ __launch_bounds__(VTX_MT, RPT == 1 ? 6 : 3) void k_iterate(DevState d
     constexpr uint32_t UB = RPT * VTX_MT;               // records of a round
     __shared__ float4 grad[4][UB];
     __shared__ uint32_t act[UB];
-    constexpr uint32_t NS = 8;                          // stretch neighbours of a particle in flight
     constexpr uint32_t NE = 12;                         // bend entries of a particle staged in LDS
     __shared__ uint32_t ent[NE * VTX_TILE];
     const TileDev t = tiles[tile_of(d.remap)];
@@ -626,19 +645,7 @@ __global__ __launch_bounds__(VTX_MT, RPT == 1 ? 6 : 3) void k_iterate(DevState d
         const float4 p4 = P[g - sg.pbase];
         p = xyz(p4);
         w = p4.w;
-        const float nws = -w * sg.stiffness;
-        for (uint32_t k0 = 0; k0 < t.st_k; k0 += NS) {
-            uint2 c[NS];
-            float4 q[NS];
-#pragma unroll
-            for (uint32_t k = 0; k < NS; k++) c[k] = (d.st + t.st_off + min(k0 + k, t.st_k - 1u) * VTX_TILE)[tid];
-#pragma unroll
-            for (uint32_t k = 0; k < NS; k++) q[k] = P[c[k].x == VTX_INVALID ? g - sg.pbase : c[k].x];
-#pragma unroll
-            for (uint32_t k = 0; k < NS; k++)
-                if (k0 + k < t.st_k && c[k].x != VTX_INVALID)
-                    stretch_term(p, w, nws, q[k], __uint_as_float(c[k].y), delta, cnt);
-        }
+        stretch_terms(d, sg, t, P, tid, g - sg.pbase, p, w, delta, cnt);
         attach_terms(d, sg, t.at_off, t.at_k, tid, g - sg.pbase, p, w, delta, cnt);
     }
 #pragma unroll
@@ -652,6 +659,26 @@ __global__ __launch_bounds__(VTX_MT, RPT == 1 ? 6 : 3) void k_iterate(DevState d
         if (vertex) add(u0);
     }
     if (!vertex) return;
+    if (cnt > 0) p = madd(p, delta, frcp((float)cnt) * sg.omega);
+    epilogue<EPI>(d, sg, g, in, p, w, h);
+}
+
+// The pass of tiles without bending constraints: one thread per particle and no LDS, as the form above keeps
+// two thirds of its threads and 64 KB idle there: 490,000 particles without bending 605 -> 419 us a frame of 32
+// passes, 576 particles 133 -> 127.
+template <int EPI>
+__global__ __launch_bounds__(VTX_TILE) void k_iterate_plain(DevState d, const TileDev* __restrict__ tiles, int in, float h) {
+    const TileDev t = tiles[tile_of(d.remap)];
+    if (threadIdx.x >= t.count) return;
+    const SegDev sg = d.segs[t.seg];
+    const uint32_t g = t.begin + threadIdx.x;
+    const float4* __restrict__ P = d.P[in] + sg.pbase;
+    const float4 p4 = P[g - sg.pbase];
+    V3 p = xyz(p4), delta = v3(0.f, 0.f, 0.f);
+    const float w = p4.w;
+    int cnt = 0;
+    stretch_terms(d, sg, t, P, threadIdx.x, g - sg.pbase, p, w, delta, cnt);
+    attach_terms(d, sg, t.at_off, t.at_k, threadIdx.x, g - sg.pbase, p, w, delta, cnt);
     if (cnt > 0) p = madd(p, delta, frcp((float)cnt) * sg.omega);
     epilogue<EPI>(d, sg, g, in, p, w, h);
 }
@@ -1346,11 +1373,20 @@ static void launch_iterate_split(const DevState& d, int in, float h, int epilogu
 
 template <int RPT>
 static void launch_iterate_mesh(const DevState& d, int in, float h, int epilogue, hipStream_t s) {
-    if (!d.nitiles) return;
-    const dim3 gr(d.nitiles), bl(VTX_MT);
+    if (d.nitiles == d.nptiles) return;
+    const dim3 gr(d.nitiles - d.nptiles), bl(VTX_MT);
     if (epilogue == EPI_NONE) hipLaunchKernelGGL((k_iterate<EPI_NONE, RPT>), gr, bl, 0, s, d, d.itiles, in, h);
     else if (epilogue == EPI_FINALIZE) hipLaunchKernelGGL((k_iterate<EPI_FINALIZE, RPT>), gr, bl, 0, s, d, d.itiles, in, h);
     else hipLaunchKernelGGL((k_iterate<EPI_FINALIZE_PREDICT, RPT>), gr, bl, 0, s, d, d.itiles, in, h);
+}
+
+static void launch_iterate_plain(const DevState& d, int in, float h, int epilogue, hipStream_t s) {
+    if (!d.nptiles) return;
+    const dim3 gr(d.nptiles), bl(VTX_TILE);
+    const TileDev* t = d.itiles + (d.nitiles - d.nptiles);
+    if (epilogue == EPI_NONE) hipLaunchKernelGGL(k_iterate_plain<EPI_NONE>, gr, bl, 0, s, d, t, in, h);
+    else if (epilogue == EPI_FINALIZE) hipLaunchKernelGGL(k_iterate_plain<EPI_FINALIZE>, gr, bl, 0, s, d, t, in, h);
+    else hipLaunchKernelGGL(k_iterate_plain<EPI_FINALIZE_PREDICT>, gr, bl, 0, s, d, t, in, h);
 }
 
 hipError_t launch_iterate(const DevState& d, int in, float h, int epilogue, bool constraints, int lra_batch,
@@ -1370,8 +1406,9 @@ hipError_t launch_iterate(const DevState& d, int in, float h, int epilogue, bool
     // a tile's records in one round while every tile has a CU of its own (8.5 against 11.5 us for 90
     // tiles of 1,334 records), else in rounds of half the LDS and twice the workgroups per CU (625 tiles
     // 28.5 against 33.4 us)
-    if (d.nitiles <= 256) launch_iterate_mesh<2>(d, in, h, epilogue, s);
+    if (d.nitiles - d.nptiles <= 256) launch_iterate_mesh<2>(d, in, h, epilogue, s);
     else launch_iterate_mesh<1>(d, in, h, epilogue, s);
+    launch_iterate_plain(d, in, h, epilogue, s);
     return last_launch();
 }
 

@@ -205,7 +205,8 @@ struct DevState {
     float4* sPX;              // per sorted position, 32 B: the predicted position with w = local
                               // particle index, then the initial position (one cache line holds both)
     uint32_t* nbr;            // neighbour tables per segment, chunks of four entries (16 or 8 bytes)
-    const TileDev* itiles;    // particle tiles of segments on the general (ELL) Jacobi path
+    const TileDev* itiles;    // particle tiles of segments on the general (ELL) Jacobi path; the last nptiles
+                              // have no bending constraints and a launch of their own
     const GridTileDev* gtiles;
     const GridTileDev* ltiles;   // grid tiles whose dense attachments run on four lanes per particle
     const GridTileDev* ftiles;   // fside x fside tiles of the grid segments whose passes are fused
@@ -217,6 +218,7 @@ struct DevState {
     uint32_t ntiles, nstiles, nhist, ncells;
     uint32_t hbase0, nltiles, nhparts;       // hbase0: first histogram entry of this table set
     uint32_t nftiles, nmtiles, fside, live;   // live: VTX_LIVE_* of the table set
+    uint32_t nptiles, pad3;
     uint32_t nparticles, nitiles, ngtiles, remap;   // remap: workgroups -> tiles through xcd_tile
 };
 
