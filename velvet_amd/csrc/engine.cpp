@@ -1459,7 +1459,6 @@ void Engine::rebuild_tables() {
              (total_n > VTX_HASH_PART_FULL ? VTX_LIVE_FULL : 0u);
     d.nstiles = (uint32_t)hst.size();
     d.nhist = hbase;
-    d.ncells = (uint32_t)acell_.cap;
     TableSet ts;
     const size_t k_seg = ts.add(hseg), k_tile = ts.add(htile), k_itile = ts.add(hitile), k_gtile = ts.add(hgtile),
                  k_ltile = ts.add(hltile), k_st = ts.add(hst), k_hs = ts.add(hpart),

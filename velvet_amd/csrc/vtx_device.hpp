@@ -215,10 +215,9 @@ struct DevState {
     const float4* rest4;      // grid: stretch rest lengths owned by a vertex (R, D, X-diag, anti-diag)
     const uint32_t* gflags;   // grid: bending slots present at a cell (VTX_BX | VTX_BR | VTX_BD)
     const float4* brest4;     // grid: bending rest angles of a cell (X, R, D)
-    uint32_t ntiles, nstiles, nhist, ncells;
+    uint32_t ntiles, nstiles, nhist, nptiles;
     uint32_t hbase0, nltiles, nhparts;       // hbase0: first histogram entry of this table set
     uint32_t nftiles, nmtiles, fside, live;   // live: VTX_LIVE_* of the table set
-    uint32_t nptiles, pad3;
     uint32_t nparticles, nitiles, ngtiles, remap;   // remap: workgroups -> tiles through xcd_tile
 };
 
