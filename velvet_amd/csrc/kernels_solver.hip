@@ -610,28 +610,41 @@ __global__ __launch_bounds__(VTX_MT, RPT == 1 ? 6 : 3) void k_iterate(DevState d
             }
         }
     };
-    // the particle's terms among records [u0, u0 + UB): its entries ascend, so the rounds keep the order
+    // four entries from k0 on, those of records [u0, u0 + nu); returns the last one's record from u0 on
+    const auto add4 = [&](uint32_t u0, uint32_t nu, uint32_t k0) {
+        float4 v[4];
+        bool on[4];
+        uint32_t last = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++) {
+            const uint32_t r = min(k0 + k, t.bd_k - 1u) * VTX_TILE + tid;
+            const uint32_t e = k0 < NE ? ent[r] : (d.bd + t.bd_off)[r];
+            const uint32_t j = (e & 0x3FFFFFFFu) - u0;
+            const bool mine = k0 + k < t.bd_k && e != VTX_INVALID && j < nu;
+            v[k] = grad[e >> 30][mine ? j : 0u];
+            on[k] = mine && act[mine ? j : 0u];
+            last = j;
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++) {
+            const V3 sum = madd(delta, xyz(v[k]), -w * v[k].w);
+            delta = v3(on[k] ? sum.x : delta.x, on[k] ? sum.y : delta.y, on[k] ? sum.z : delta.z);
+            cnt += on[k] ? 1 : 0;
+        }
+        return last;
+    };
+    // the particle's terms among the round's records. Its entries ascend, so the rounds keep the order, and a
+    // later round goes on at the first group of four (next) that was not used up: with every round over all
+    // entries, a mesh with a vertex of 20,000 bends took 707 ms a frame of 8 passes (now 87)
+    uint32_t next = 0;
     const auto add = [&](uint32_t u0) {
         const uint32_t nu = min(t.ub_n - u0, (uint32_t)UB);
-        for (uint32_t k0 = 0; k0 < t.bd_k; k0 += 4) {
-            float4 v[4];
-            bool on[4];
-#pragma unroll
-            for (uint32_t k = 0; k < 4; k++) {
-                const uint32_t r = min(k0 + k, t.bd_k - 1u) * VTX_TILE + tid;
-                const uint32_t e = k0 < NE ? ent[r] : (d.bd + t.bd_off)[r];
-                const uint32_t j = (e & 0x3FFFFFFFu) - u0;
-                const bool mine = k0 + k < t.bd_k && e != VTX_INVALID && j < nu;
-                v[k] = grad[e >> 30][mine ? j : 0u];
-                on[k] = mine && act[mine ? j : 0u];
-            }
-#pragma unroll
-            for (uint32_t k = 0; k < 4; k++) {
-                const V3 sum = madd(delta, xyz(v[k]), -w * v[k].w);
-                delta = v3(on[k] ? sum.x : delta.x, on[k] ? sum.y : delta.y, on[k] ? sum.z : delta.z);
-                cnt += on[k] ? 1 : 0;
-            }
+        if (t.ub_n <= UB) {
+            for (uint32_t k0 = 0; k0 < t.bd_k; k0 += 4) add4(u0, nu, k0);
+            return;
         }
+        for (; next < t.bd_k; next += 4)
+            if (add4(u0, nu, next) >= nu) break;
     };
 
     // the first entry rows (contiguous: row k at k * VTX_TILE), loaded while the records are evaluated
