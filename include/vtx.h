@@ -162,8 +162,10 @@ int vtx_stencil_segments(vtx_solver* s, int32_t* count);
 typedef struct vtx_tuning {
     int32_t use_graph;         /* replay frames from a hipGraph */
     int32_t neighbor_order;    /* how the neighbour search takes self-colliding segments of more than
-                                  131072 particles: 0 = whole blocks of cells by particle index, 1 and
-                                  2 = in hash-sorted order (smaller segments always) */
+                                  131072 particles: 0 = whole blocks of cells by particle index, 1 = in
+                                  hash-sorted order (smaller segments always), 2 = by index those grid
+                                  cloths of more than 524288 particles on a tuned hash grid whose cells
+                                  are sparsely filled (fewer than 5.5 particles), sorted the others */
     int32_t lra_batch;         /* dense attachment distances a grid cloth with 32 or more slots loads per
                                   batch: 4 or 16 (64, accepted as before, runs as 16) */
     int32_t xcd_remap;         /* hand each XCD a contiguous run of tiles */

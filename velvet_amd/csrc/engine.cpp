@@ -1639,7 +1639,13 @@ void Engine::hash_build(const DevState& d, int in, hipStream_t s) {
         stage_end(s);
     }
     stage_begin("k_neighbors", "Solver_HashCache", s);
-    VTX_HIP(launch_neighbors(d, in, src, tun_.nbr_order == 0, s));
+    const SearchRule rule = search_rule(tun_.nbr_order);
+    bool by_index = false;
+    for (int32_t k : table_seg_) {
+        const SegDev& g = segs_[(size_t)k]->dev;
+        by_index = by_index || ((g.flags & VTX_SEG_SELFCOL) && search_by_index(rule, g.n, g.flags));
+    }
+    VTX_HIP(launch_neighbors(d, in, src, by_index, rule, s));
     stage_end(s);
     sorted_src_ = src;
 }
@@ -1944,7 +1950,7 @@ Tuning Engine::autotune(int frames, float frame_dt, bool use_cache, double* fram
                 if (knob == 8 && v > 3) t.nbr_order = 0;
                 if (knob == 8 ? t.hash_grid == base.hash_grid && t.nbr_order == base.nbr_order
                     : knob == 0 ? t.graph == base.graph
-                    : knob == 1 ? (t.nbr_order == 0) == (base.nbr_order == 0)
+                    : knob == 1 ? t.nbr_order == base.nbr_order
                                 : knob == 2 ? t.lra_batch == base.lra_batch
                                 : knob == 3 ? t.remap == base.remap
                                 : knob == 4 ? t.gather_block == base.gather_block

@@ -133,7 +133,7 @@ struct Segment {
 // replayed from a graph, never the arithmetic.
 struct Tuning {
     bool graph = true;        // replay frames from a hipGraph
-    int nbr_order = 2;        // 0: the search takes large segments by particle index; 1, 2: in sorted order
+    int nbr_order = 2;        // search of large segments: 0 by particle index, 1 in sorted order, 2 see search_rule
     int lra_batch = 16;       // distances of 32 or more dense slots loaded per batch: 4 or 16 (64 runs as 16)
     bool remap = true;        // XCD-aware workgroup -> tile remap
     int gather_block = 256;   // threads per workgroup of the contact pass

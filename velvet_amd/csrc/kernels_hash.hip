@@ -267,7 +267,8 @@ __global__ __launch_bounds__(VTX_TILE) void k_clear_cells(DevState d) {
 // FindCellStart_Kernel (Velvet/SpatialHashGPU.cu:44-77) per segment with local sorted
 // positions (cells were filled with ~0u: empty), plus the inverse permutation (particle ->
 // sorted position) in the sort's free key buffer, from which k_sorted_records writes the
-// sorted records in particle order.
+// sorted records in particle order, and the number of cells in a sample (SearchRule), left in the sort's free
+// value buffer.
 __global__ __launch_bounds__(VTX_TILE) void k_cell_bounds(DevState d, int in, int src) {
     const TileDev t = d.tiles[tile_of(d.remap)];
     if (threadIdx.x >= t.count) return;
@@ -289,6 +290,21 @@ __global__ __launch_bounds__(VTX_TILE) void k_cell_bounds(DevState d, int in, in
     }
     if (local == sg.n - 1) cells[key].y = sg.n;
     d.keys[src ^ 1][sg.pbase + d.vals[src][g]] = local;
+    if (t.begin == sg.pbase && sg.n > VTX_SEARCH_SAMPLED) {   // the first tile, full: cells of the sample
+        constexpr uint32_t R = VTX_SEARCH_SAMPLE / VTX_TILE;
+        __shared__ uint32_t wsum[VTX_TILE / 64];
+        uint32_t k[R], next[R], count = 0;
+#pragma unroll
+        for (uint32_t r = 0; r < R; r++) {
+            k[r] = sk[sg.pbase + r * VTX_TILE + local];
+            next[r] = sk[sg.pbase + r * VTX_TILE + local + 1];
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < R; r++) count += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(k[r] != next[r]));
+        if ((local & 63u) == 0) wsum[local >> 6] = count;
+        __syncthreads();
+        if (local == 0) d.vals[src ^ 1][sg.pbase] = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+    }
 }
 
 // The sorted copies for the neighbour search, written from particle order: coalesced reads of the
@@ -905,7 +921,8 @@ __device__ __forceinline__ void neighbor_blocks(const NbSet& a, const uint32_t* 
 // The search over the segments' particle tiles (a tile's sorted positions): 4 PW particles per
 // workgroup of four waves.
 template <int PW, bool BY_INDEX>
-__global__ __launch_bounds__(256) void k_neighbors(DevState d, int in, const uint32_t* __restrict__ inv) {
+__global__ __launch_bounds__(256) void k_neighbors(DevState d, int in, const uint32_t* __restrict__ inv,
+                                                   const uint32_t* __restrict__ sample, SearchRule rule) {
     __shared__ NbLds<PW> lds[4];
     const uint32_t b = tile_of(d.remap), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     constexpr uint32_t S = VTX_TILE / (4 * PW);                 // workgroups per tile
@@ -927,7 +944,7 @@ __global__ __launch_bounds__(256) void k_neighbors(DevState d, int in, const uin
     a.diam2 = sg.diam2;
     a.n16 = sg.flags & VTX_SEG_NBR16;
     const uint32_t i = t.begin - sg.pbase + first, cnt = min((uint32_t)PW, t.count - first);
-    if (BY_INDEX && sg.n > VTX_SEARCH_BY_INDEX && !(sg.flags & VTX_SEG_HASH_PART))
+    if (BY_INDEX && search_by_index(rule, sg.n, sg.flags) && (!rule.cells || sample[sg.pbase] >= rule.cells))
         neighbor_blocks<PW>(a, inv + sg.pbase, d.P[in] + sg.pbase, i, cnt, lds[wave]);
     else
         neighbor_wave<PW, true>(a, i, cnt, lds[wave]);
@@ -1264,10 +1281,10 @@ hipError_t launch_cell_bounds(const DevState& d, int in, int src, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_neighbors(const DevState& d, int in, int src, bool by_index, hipStream_t s) {
+hipError_t launch_neighbors(const DevState& d, int in, int src, bool by_index, SearchRule rule, hipStream_t s) {
     const auto nb = [&](auto kernel, uint32_t pw) {
         hipLaunchKernelGGL(kernel, dim3(d.ntiles * (VTX_TILE / (4 * pw))), dim3(256), 0, s, d, in,
-                           (const uint32_t*)d.keys[src ^ 1]);   // the inverse permutations k_cell_bounds leaves
+                           (const uint32_t*)d.keys[src ^ 1], (const uint32_t*)d.vals[src ^ 1], rule);   // k_cell_bounds' output
     };
     if (search_small(d.nparticles)) nb(k_neighbors<8, false>, 8);
     else if (by_index) nb(k_neighbors<32, true>, 32);

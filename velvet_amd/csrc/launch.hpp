@@ -31,9 +31,9 @@ hipError_t launch_fill_u32(uint32_t* a, uint32_t n, uint32_t v, hipStream_t s);
 hipError_t launch_clear_cells(const DevState& d, hipStream_t s);
 hipError_t launch_hash_parts(const DevState& d, int in, int dst, hipStream_t s);
 hipError_t launch_cell_bounds(const DevState& d, int in, int src, hipStream_t s);
-// by_index: segments of more than VTX_SEARCH_BY_INDEX particles on the device-wide build by particle index
-// (src: the side its sort ended on); same results
-hipError_t launch_neighbors(const DevState& d, int in, int src, bool by_index, hipStream_t s);
+// by_index: some segment is searched by particle index under `rule` (src: the side its sort ended on); same
+// results either way
+hipError_t launch_neighbors(const DevState& d, int in, int src, bool by_index, SearchRule rule, hipStream_t s);
 
 // HashObjects of the kernel-launch tier (Velvet/SpatialHashGPU.cuh:7-25) on raw device arrays.
 struct HashObjectsArgs {

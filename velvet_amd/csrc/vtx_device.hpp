@@ -57,8 +57,6 @@
 #define VTX_HASH_HEAVY 128u
 #define VTX_COLLIDE_SMALL 81920u   // live particles up to which the contact pass reads ahead
 
-#define VTX_SEARCH_BY_INDEX 131072u   // particles of a segment whose records (32 B each) outgrow an L2
-
 // floor(2^32 / M), for the remainder by M (hash_coords).
 static inline uint32_t mod_constant(uint32_t M) { return M > 1 ? (uint32_t)((1ull << 32) / M) : ~0u; }
 
@@ -86,6 +84,28 @@ static inline uint32_t hash_part_width(uint32_t n, uint32_t M, uint32_t share) {
 // mirror image; shifted coordinates have no such partner nearby.
 #define VTX_SEG_HASH_SHIFT 2048u
 #define VTX_HASH_SHIFT 1000003u
+// Which segments of the device-wide build the neighbour search takes by particle index (neighbor_blocks):
+// those of more than `above` particles that have the flags `need`, where the first VTX_SEARCH_SAMPLE
+// sorted particles, a random sample of the cells, lie in more than `cells` of them (k_cell_bounds counts).
+#define VTX_SEARCH_BY_INDEX 131072u   // particles of a segment whose records (32 B each) outgrow an L2
+#define VTX_SEARCH_SAMPLED 524288u    // ... whose cells are sampled
+#define VTX_SEARCH_SAMPLE 2048u
+struct SearchRule {
+    uint32_t above, need, cells;
+};
+static inline __host__ __device__ bool search_by_index(const SearchRule& r, uint32_t n, uint32_t flags) {
+    return n > r.above && (flags & r.need) == r.need && !(flags & VTX_SEG_HASH_PART);
+}
+// neighbor_order 0: every such segment; 1: none; 2, the default: grid cloths of more than 2^19 particles on a
+// tuned hash grid while their cells hold fewer than 5.5 particles on average. Crowded cells make uneven
+// blocks, on the reference grid mirrored cells share buckets, and smaller segments gain little (us a search,
+// sorted / by index: 1,048,576 particles at rest on grid 1 243 / 155, on grid 2 249 / 150, in a pile on grid 1
+// 318 / 497; 360,000 at rest 76 / 76 and 84 / 72, in a pile 110 / 126).
+static inline SearchRule search_rule(int order) {
+    if (order == 0) return SearchRule{VTX_SEARCH_BY_INDEX, 0u, 0u};
+    if (order == 2) return SearchRule{VTX_SEARCH_SAMPLED, VTX_SEG_GRID | VTX_SEG_HASH_SHIFT, VTX_SEARCH_SAMPLE * 2 / 11};
+    return SearchRule{~0u, 0u, 0u};
+}
 // The segment's neighbour table holds 16-bit entries (0xffff the sentinel): self-collision
 // segments of at most VTX_NBR16_N particles, whose indices and sentinel fit in 16 bits. Chunks
 // of four entries are then 8 bytes: half the table traffic of the search's stores and of the
