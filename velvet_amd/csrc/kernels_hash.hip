@@ -1100,7 +1100,7 @@ __global__ __launch_bounds__(VTX_TILE) void k_raw_split_cells(const uint2* __res
     }
 }
 
-// Particles per wave of the neighbour search. Up to 2^17 particles a wave takes 8: the chip's 8,192
+// Particles per wave of the neighbour search. Up to 2^17 particles in a launch a wave takes 8: the chip's 8,192
 // waves are not all busy, and a wave's particles go one after the other (measured, us per search, 8 /
 // 32 particles a wave: 16,384 particles 11.8 / 27.9, 65,536 17.1 / 29.7). Above, 32: the lookups of a
 // run and its candidates' loads serve more particles (963,130 particles in 256 cloths 164.9 / 129.9;

@@ -1358,7 +1358,10 @@ hipError_t launch_collide(const DevState& d, int in, float h, int block, hipStre
     // few particles with neighbours: the pass is the chain of its loads, so eight neighbours and their start positions at a
     // time, on many CUs; many: the lines it touches and the registers (102 for 72) count, so four, and start
     // positions of contacts only. Folded cloths, us a frame of ten contact passes, 4 / 8: 4,096 particles
-    // 158 / 137, 40,000 190 / 175, 65,536 242 / 232, 131,044 302 / 313, 1,048,576 1109 / 1280.
+    // 158 / 137, 40,000 190 / 175, 65,536 242 / 232, 131,044 302 / 313, 1,048,576 1109 / 1280. With segments on
+    // several streams the launch's own particles count, for the search too (search_small): three folded cloths
+    // of 230 x 230 on two / three streams 354 / 366 us a frame, with the live set's count 377 / 393; of
+    // 350 x 350 579 / 591 and 580 / 600.
     if ((d.live & VTX_LIVE_SELFCOL) && d.nparticles <= VTX_COLLIDE_SMALL) launch(k_collide<64, 8>, 64);
     else if (block == 64) launch(k_collide<64, 4>, 64);
     else if (block == 128) launch(k_collide<128, 4>, 128);
