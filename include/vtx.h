@@ -171,7 +171,9 @@ typedef struct vtx_tuning {
     int32_t xcd_remap;         /* hand each XCD a contiguous run of tiles */
     float frame_ms;            /* vtx_autotune: the chosen variant's frame time (0 from the cache) */
     int32_t gather_block;      /* threads per workgroup of the contact pass: 64, 128 or 256 (each
-                                  256-particle tile split across workgroups) */
+                                  256-particle tile split across workgroups). No effect where segments
+                                  collide with themselves and a stream group has at most 81920
+                                  particles: 64 there */
     int32_t streams;           /* k = 1..4: the segments split into k particle-balanced groups
                                   whose frames run concurrently on k streams */
     int32_t lra_split;         /* no effect: once four or one threads per particle in the Jacobi pass of

@@ -1,0 +1,27 @@
+"""A tuning knob that does nothing for the live set keeps its value."""
+import numpy as np
+import pytest
+
+from velvet_amd import scenes as S
+from velvet_amd.solver import ClothSolver
+
+pytestmark = pytest.mark.gpu
+
+
+def _solver(sides, substeps=2):
+    s = ClothSolver()
+    for k, n in enumerate(sides):
+        c = S.grid_cloth(n, 0.05, center=(0.0, 1.0, 0.0), jitter=2e-3, seed=k, stream=18)
+        c.x[:, 1] += (0.04 * np.floor(3.0 * S.uniform(k, 19, c.n))).astype(np.float32)
+        c.x[:, 0] *= np.float32(0.6)
+        p = S.Params(num_substeps=substeps, num_iterations=2, friction=0.3, max_num_neighbors=30)
+        s.load_scene(S.Scene(S.finish_params(p, [c]), [c], [S.sphere((0.1, 0.9, 0.05), 0.08)], 2))
+    return s
+
+
+def test_knob_without_effect_keeps_its_value():
+    for block in (64, 128, 256):
+        with _solver((100, 80), substeps=3) as s:
+            s.set_tuning(gather_block=block)
+            assert s.autotune(frames=1)["gather_block"] == block
+

@@ -1931,7 +1931,7 @@ Tuning Engine::autotune(int frames, float frame_dt, bool use_cache, double* fram
             if (knob == 8 && !any_grid_tunable_) continue;
             if (knob == 1 && !any_large_search_) continue;
             if (knob == 2 && !any_lra_split_) continue;
-            if (knob == 4 && !need_collide_) continue;
+            if (knob == 4 && (!need_collide_ || std::all_of(groups_.begin(), groups_.end(), collide_ahead))) continue;
             if (knob == 5 && table_seg_.size() < 2) continue;
             if (knob == 7 && !any_hash_lds_) continue;
             // the grid decides whether the search by index gains: tried together

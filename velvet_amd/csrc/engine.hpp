@@ -136,7 +136,7 @@ struct Tuning {
     int nbr_order = 2;        // search of large segments: 0 by particle index, 1 in sorted order, 2 see search_rule
     int lra_batch = 16;       // distances of 32 or more dense slots loaded per batch: 4 or 16 (64 runs as 16)
     bool remap = true;        // XCD-aware workgroup -> tile remap
-    int gather_block = 256;   // threads per workgroup of the contact pass
+    int gather_block = 256;   // threads per workgroup of the contact pass (launches of more than 81,920 particles)
     int streams = 1;          // k > 1: segments split into k particle-balanced groups whose frames
                               // run on k streams, overlapping latency- and VALU-bound stages
     bool lra_split = true;    // kept for callers (vtx_tuning.lra_split), no effect

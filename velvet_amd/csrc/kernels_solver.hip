@@ -1362,7 +1362,7 @@ hipError_t launch_collide(const DevState& d, int in, float h, int block, hipStre
     // several streams the launch's own particles count, for the search too (search_small): three folded cloths
     // of 230 x 230 on two / three streams 354 / 366 us a frame, with the live set's count 377 / 393; of
     // 350 x 350 579 / 591 and 580 / 600.
-    if ((d.live & VTX_LIVE_SELFCOL) && d.nparticles <= VTX_COLLIDE_SMALL) launch(k_collide<64, 8>, 64);
+    if (collide_ahead(d)) launch(k_collide<64, 8>, 64);
     else if (block == 64) launch(k_collide<64, 4>, 64);
     else if (block == 128) launch(k_collide<128, 4>, 128);
     else launch(k_collide<256, 4>, 256);

@@ -9,9 +9,13 @@ namespace vtx {
 enum { EPILOGUE_NONE = 0, EPILOGUE_FINALIZE = 1, EPILOGUE_FINALIZE_PREDICT = 2 };
 
 hipError_t launch_frame_begin(const DevState& d, float frame_dt, float h, hipStream_t s);
-// block: threads per workgroup (64, 128 or 256; same results)
+// Whether the contact pass of a launch reads ahead, in workgroups of 64 threads (launch_collide says why)
+inline bool collide_ahead(const DevState& d) {
+    return (d.live & VTX_LIVE_SELFCOL) && d.nparticles <= VTX_COLLIDE_SMALL;
+}
+// block: threads per workgroup where it does not (64, 128 or 256; same results)
 hipError_t launch_collide(const DevState& d, int in, float h, int block, hipStream_t s);
-// lra_batch: dense attachment distances loaded per batch (4, 16 or 64; same results)
+// lra_batch: distances of 32 or more dense slots loaded per batch: below 16 four, else 16; same results
 hipError_t launch_iterate(const DevState& d, int in, float h, int epilogue, bool constraints, int lra_batch,
                           hipStream_t s);
 // Fused passes of the grid segments in d.ftiles: most passes per launch for tiles of side 8, 12, 16
