@@ -1,4 +1,6 @@
-"""A tuning knob that does nothing for the live set keeps its value."""
+"""The tuner's cache tells apart live sets for which a knob acts and for which it does not: the contact pass's
+block on both sides of 81,920 particles, the search order with and without a segment of more than 131,072; and
+a knob that does nothing keeps its value."""
 import numpy as np
 import pytest
 
@@ -17,6 +19,16 @@ def _solver(sides, substeps=2):
         p = S.Params(num_substeps=substeps, num_iterations=2, friction=0.3, max_num_neighbors=30)
         s.load_scene(S.Scene(S.finish_params(p, [c]), [c], [S.sphere((0.1, 0.9, 0.05), 0.08)], 2))
     return s
+
+
+@pytest.mark.parametrize("first,second", [((270,), (300,)), ((316, 316, 316), (450, 220, 220))])
+def test_classes(first, second):
+    """Both of one size class and segment class."""
+    print(f"[gpu] tuned {first}, then {second}", flush=True)
+    with _solver(first) as s:
+        s.autotune(frames=2)
+    with _solver(second) as s:
+        assert s.autotune(frames=2, use_cache=True)["frame_ms"] > 0
 
 
 def test_knob_without_effect_keeps_its_value():

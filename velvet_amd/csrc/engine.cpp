@@ -1831,7 +1831,9 @@ void Engine::set_tuning(const Tuning& t) {
 }
 
 // Shape class of the live set: log2 buckets of particles and segments, whether the hash,
-// the stencil path and dense attachments are present, and the substep / iteration counts.
+// the stencil path and dense attachments are present, whether a segment is large enough for the search by
+// index and the set small enough for the contact pass that reads ahead (the knobs of both act there or not),
+// and the substep / iteration counts.
 std::string Engine::shape_class() {
     ensure_committed();
     uint32_t nseg = 0, ngrid = 0;
@@ -1843,7 +1845,8 @@ std::string Engine::shape_class() {
     std::ostringstream o;
     const uint32_t np = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(1, live_particles_), UINT32_MAX);
     o << "p" << ceil_log2(np) << ".s" << ceil_log2(std::max(1u, nseg))
-      << ".h" << (any_selfcol_ ? (any_grid_tunable_ ? 2 : 1) : 0) << ".g" << (ngrid ? 1 : 0) << ".l"
+      << ".h" << (any_selfcol_ ? (any_grid_tunable_ ? 2 : 1) : 0)
+      << (any_large_search_ ? "i" : "") << (live_particles_ <= VTX_COLLIDE_SMALL ? "a" : "") << ".g" << (ngrid ? 1 : 0) << ".l"
       << (any_lra_split_ ? 2 : any_lra_dense_ ? 1 : 0) << "."
       << substeps_ << "x" << iterations_;
     return o.str();
