@@ -1,6 +1,6 @@
 """The tuner's cache tells apart live sets for which a knob acts and for which it does not: the contact pass's
 block on both sides of 81,920 particles, the search order with and without a segment of more than 131,072; and
-a knob that does nothing keeps its value."""
+a knob that does nothing keeps its value. gather_block in sets where it acts gives the same results."""
 import numpy as np
 import pytest
 
@@ -37,3 +37,23 @@ def test_knob_without_effect_keeps_its_value():
             s.set_tuning(gather_block=block)
             assert s.autotune(frames=1)["gather_block"] == block
 
+
+def test_blocks_of_the_contact_pass_bit_identical():
+    """More than 81,920 particles, so that the block acts; against eight neighbours at a time in smaller sets."""
+    def run(sides, **tuning):
+        with _solver(sides) as s:
+            s.set_tuning(**tuning)
+            for _ in range(2):
+                s.Simulate()
+            s.synchronize()
+            return [(s.positions(k), s.velocities(k)) for k in range(len(sides))]
+
+    sides = (257, 130, 33)
+    want = [run(sides[:1])[0]]
+    assert sum(n * n for n in sides) > 81920
+    for block in (64, 128, 256):
+        print(f"[gpu] contact pass in blocks of {block}", flush=True)
+        got = run(sides, gather_block=block)
+        want += got[len(want):]
+        for (x, v), (xr, vr) in zip(got, want):
+            assert np.isfinite(x).all() and np.array_equal(x, xr) and np.array_equal(v, vr)
