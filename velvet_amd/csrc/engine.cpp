@@ -731,13 +731,20 @@ static void tile_distances(const Segment& sg, Prepared& pr) {
         GridTileDev& t = pr.gtiles[ti];
         t.at_off = (uint32_t)(ti * per_tile);
         const uint32_t h = std::min<uint32_t>(VTX_GT, pr.grows - t.a0), w = std::min<uint32_t>(VTX_GT, pr.gcols - t.b0);
-        for (size_t s = 0; s < L; s++) {
-            const size_t q = s / qs, k = s % qs;
-            float* out = pr.lra.data() + 4 * (ti * per_tile + (q * groups + k / 4) * VTX_TILE) + k % 4;
-            const float* in = sg.at_dist.data() + s * n + (size_t)t.a0 * pr.gcols + t.b0;
-            for (uint32_t a = 0; a < h; a++, in += pr.gcols, out += 4 * VTX_GT)
-                for (uint32_t b = 0; b < w; b++) out[4 * b] = in[b] * lrs;
-        }
+        for (size_t q = 0; q < VTX_LRA_PARTS; q++)
+            for (size_t s = q * qs; s < std::min((q + 1) * qs, L); s += 4) {   // four slots' distances side by side
+                const size_t m = std::min<size_t>(4, std::min((q + 1) * qs, L) - s);
+                const float* in = sg.at_dist.data() + s * n + (size_t)t.a0 * pr.gcols + t.b0;
+                float* out = pr.lra.data() + 4 * (ti * per_tile + (q * groups + (s - q * qs) / 4) * VTX_TILE);
+                for (uint32_t a = 0; a < h; a++, in += pr.gcols, out += 4 * VTX_GT) {
+                    if (m == 4)
+                        for (uint32_t b = 0; b < w; b++)
+                            for (size_t k = 0; k < 4; k++) out[4 * b + k] = in[k * n + b] * lrs;
+                    else
+                        for (uint32_t b = 0; b < w; b++)
+                            for (size_t k = 0; k < m; k++) out[4 * b + k] = in[k * n + b] * lrs;
+                }
+            }
     }
 }
 
@@ -778,11 +785,18 @@ void Engine::prepare_segment(Segment& sg) {
         pr.brest4 = std::move(G.brest4);
     }
 
+    // dense long-range attachments: entry c = slot * n + particle for every slot and particle
+    const size_t A = sg.at_pid.size();
+    pr.lra_dense = n > 0 && L > 0 && A == (size_t)L * n;
+    for (size_t c = 0; c < A && pr.lra_dense; c += n)
+        for (size_t i = 0; i < n && pr.lra_dense; i++)
+            pr.lra_dense = (size_t)sg.at_pid[c + i] == i && (size_t)sg.at_slot[c + i] == c / n;
+
     // incidence lists (CSR over local particles, registration order); the stencil path reads
     // neither stretch / bend lists nor triangle lists (its normals come from the grid), so a grid
     // segment builds only the attachment lists
     std::vector<uint32_t> s_st(n + 1, 0), s_at(n + 1, 0), s_bd(n + 1, 0), s_tr(n + 1, 0);
-    const size_t S = sg.st_rest.size(), A = sg.at_pid.size(), B = sg.bd_rest.size();
+    const size_t S = sg.st_rest.size(), B = sg.bd_rest.size();
     const size_t T = pr.grid ? 0 : sg.tris.size() / 3;
     if (!pr.grid) {
         for (size_t c = 0; c < S; c++) {
@@ -792,7 +806,8 @@ void Engine::prepare_segment(Segment& sg) {
         for (size_t c = 0; c < B; c++)
             for (int r = 0; r < 4; r++) s_bd[(size_t)sg.bd[4 * c + r] + 1]++;
     }
-    for (size_t c = 0; c < A; c++) s_at[(size_t)sg.at_pid[c] + 1]++;
+    if (!pr.lra_dense)
+        for (size_t c = 0; c < A; c++) s_at[(size_t)sg.at_pid[c] + 1]++;
     for (size_t c = 0; c < T; c++)
         for (int r = 0; r < 3; r++) s_tr[(size_t)sg.tris[3 * c + r] + 1]++;
     for (uint32_t i = 0; i < n; i++) {
@@ -839,15 +854,9 @@ void Engine::prepare_segment(Segment& sg) {
                 l_bd[fb[v]++] = (cnt[t] - 1 - ub[t]) | (r << 30);
             }
     }
-    // dense long-range attachments: entry c = slot * n + particle for every slot and particle
-    pr.lra_dense = n > 0 && L > 0 && A == (size_t)L * n;
-    for (size_t c = 0; c < A && pr.lra_dense; c++)
-        pr.lra_dense = (size_t)sg.at_pid[c] == c % n && (size_t)sg.at_slot[c] == c / n;
     if (pr.lra_dense) {
         pr.lra_tiled = tiles_distances(pr, n, L);
         if (!pr.lra_tiled) pr.lra = sg.at_dist;   // already slot-major
-        std::fill(s_at.begin(), s_at.end(), 0u);
-        l_at.clear();
     } else {
         std::vector<uint32_t> f(s_at.begin(), s_at.end() - 1);
         for (size_t c = 0; c < A; c++)
