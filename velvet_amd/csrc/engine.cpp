@@ -709,7 +709,7 @@ static void fill_state(const Segment& sg, Prepared& pr) {
 
 // Tiled dense attachments (VTX_SEG_LRA_TILED): float4 of one tile, and whether a grid segment has them.
 // Whole tiles and groups of four are stored, so a cloth of few columns or rows would take up to 16 times
-// the memory: beyond twice (and 4 MB) the distances stay slot-major.
+// the memory: beyond twice (and 4 MB) the distances stay slot-major, and where a budget asks (Segment::compact).
 static size_t tiled_stride(size_t L) {
     return VTX_LRA_PARTS * (((L + VTX_LRA_PARTS - 1) / VTX_LRA_PARTS + 3) / 4) * VTX_TILE;
 }
@@ -855,7 +855,7 @@ void Engine::prepare_segment(Segment& sg) {
             }
     }
     if (pr.lra_dense) {
-        pr.lra_tiled = tiles_distances(pr, n, L);
+        pr.lra_tiled = !sg.compact && tiles_distances(pr, n, L);
         if (!pr.lra_tiled) pr.lra = sg.at_dist;   // already slot-major
     } else {
         std::vector<uint32_t> f(s_at.begin(), s_at.end() - 1);
@@ -934,11 +934,18 @@ static size_t bytes_of(const Ranges& r) {
            r.n_trec * sizeof(uint4) + r.n_slot * sizeof(float4) + r.n_col * sizeof(ColliderDev) + r.n_lra * 4;
 }
 
-size_t Engine::bytes_estimate(const Segment& sg) { return bytes_of(needs_of(sg)); }
+// A segment's bytes as budgets count them: what it registers. A bend counts once, although every tile that
+// holds one of its particles keeps a record of it (some 6% of a mesh's bytes).
+size_t Engine::bytes_estimate(const Segment& sg) {
+    Ranges r = needs_of(sg);
+    r.n_brec = sg.prep.grid ? 0 : sg.bd_rest.size();
+    r.n_lra = sg.prep.lra.size();
+    return bytes_of(r);
+}
 
 size_t Engine::device_bytes_estimate(int32_t s) {
     prepare(s);
-    return bytes_of(needs_of(seg(s)));
+    return bytes_estimate(seg(s));
 }
 
 size_t Engine::pool_bytes() const {

@@ -109,6 +109,7 @@ struct Segment {
     bool active = true;                      // simulated by the solver's frames
     bool uploaded = false;                   // device ranges hold the current state
     bool prepared = false;                   // `prep` matches the host data
+    bool compact = false;                    // dense distances slot-major, never tiled
     Prepared prep;
     Ranges rg;
     SegDev dev{};                            // absolute bases filled at upload

@@ -60,6 +60,12 @@ void Server::worker_loop() {
         try {
             e_.prepare_segment(*j->sp);
             bytes = Engine::bytes_estimate(*j->sp);
+            if (bytes > limit_ && j->sp->prep.lra_tiled) {   // tiles are stored whole: without them it may fit
+                j->sp->compact = true;
+                j->sp->prepared = false;
+                e_.prepare_segment(*j->sp);
+                bytes = Engine::bytes_estimate(*j->sp);
+            }
             n = j->sp->n();
             work = (uint64_t)n * (uint64_t)j->sp->prm.num_substeps;
             reject = bytes > limit_ || (cfg_.max_live_particles && n > cfg_.max_live_particles);
