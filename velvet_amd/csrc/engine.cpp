@@ -1296,6 +1296,7 @@ void Engine::rebuild_tables() {
     std::vector<HashPartDev> hpart;                  // cell ranges of the segments k_hash_part builds
     std::vector<SortTileDev> hst;
     table_seg_.clear();
+    fused_ranges_.assign(1, {});
     any_selfcol_ = false;
     any_lra_dense_ = false;
     any_lra_split_ = false;
@@ -1357,6 +1358,7 @@ void Engine::rebuild_tables() {
             cuts.push_back(Cut{htile.size(), hitile.size(), hgtile.size(), hltile.size(), hst.size(), hpart.size(),
                                hftile.size(), hmtile.size(), hbase, (uint32_t)cum});
             compact = 0;                       // each group sorts on its own
+            fused_ranges_.emplace_back();
         }
         cum += sg.n();
         const uint32_t ti = (uint32_t)hseg.size();
@@ -1405,6 +1407,7 @@ void Engine::rebuild_tables() {
             if (!sg.prep.grid) hitile.push_back(t);
         }
         const bool fused = fside && fusable(sg) && !single[cuts.size()];
+        if (fused) fused_ranges_.back().emplace_back(d.pbase, d.n);
         for (GridTileDev gt : sg.prep.gtiles) {
             gt.seg = ti;
             gt.at_off += (uint32_t)(sg.prep.lra_tiled ? sg.rg.lra / 4 : sg.rg.at);
@@ -1667,8 +1670,15 @@ void Engine::hash_build(const DevState& d, int in, hipStream_t s) {
 }
 
 // VtClothSolverGPU::Simulate stage order (Velvet/VtClothSolverGPU.hpp:56-111) for one table set.
-// In timing mode every launch group is bracketed by an event pair labelled with its kernel.
-void Engine::record_group(const DevState& d, float frame_dt, hipStream_t s, hipEvent_t after_hash) {
+// In timing mode every launch group is bracketed by an event pair labelled with its kernel. Returns whether
+// the frame leaves the fused segments' predicted positions, as vtx_run_hash hashes them, in P1.
+//
+// One pass per launch leaves in P0 the positions before the last pass of the frame or, where that reads P1,
+// those before the pass ahead of it, and so do fused launches: the frame's last one keeps those positions
+// from its tiles and writes them to the buffer that it does not read. Where that is P1 they are copied when
+// they are asked for (settle_predicted).
+bool Engine::record_group(const DevState& d, float frame_dt, hipStream_t s, hipEvent_t after_hash) {
+    bool in_p1 = false;
     const float h = frame_dt / (float)substeps_;
     stage_begin("k_frame_begin", "Solver_CollideSDFs+Solver_Predict", s);
     VTX_HIP(launch_frame_begin(d, frame_dt, h, s));
@@ -1706,15 +1716,18 @@ void Engine::record_group(const DevState& d, float frame_dt, hipStream_t s, hipE
             int launches = (iterations_ + most - 1) / most;
             // every segment leaves the substep in the same ping-pong buffer
             if (single && (launches ^ iterations_) & 1) launches++;
+            const int toggles = substeps_ * ((need_collide_ ? 1 : 0) + iterations_);   // of one pass per launch
+            const int keep = !last_sub || launches == iterations_ ? 0 : (toggles - 1) & 1 ? 2 : 1;
             for (; launches > 0; launches--) {
-                const int passes = (left + launches - 1) / launches;
+                const int passes = left / launches;         // the last launch has the most
                 left -= passes;
                 const int epi = left ? (int)EPILOGUE_NONE : epi_last;
                 stage_begin("k_iterate", label[epi], s, passes);
-                VTX_HIP(launch_iterate_fused(d, fcur, passes, h, epi, s));
+                VTX_HIP(launch_iterate_fused(d, fcur, passes, left ? 0 : keep, h, epi, s));
                 stage_end(s);
                 fcur ^= 1;
             }
+            in_p1 = keep && fcur == 1;                      // the last launch read P0
         }
         for (int it = 0; single && it < iterations_; it++) {
             const int epi = it == iterations_ - 1 ? epi_last : (int)EPILOGUE_NONE;
@@ -1728,6 +1741,16 @@ void Engine::record_group(const DevState& d, float frame_dt, hipStream_t s, hipE
     stage_begin("k_normals", "Solver_UpdateNormals", s);
     VTX_HIP(launch_normals(d, s));
     stage_end(s);
+    return in_p1;
+}
+
+// The last frame's predicted positions into P0 (record_group).
+void Engine::settle_predicted() {
+    join();
+    if (!predicted_in_p1_) return;
+    for (auto& r : in_p1_)   // a range given to another segment since holds the same in both
+        VTX_HIP(hipMemcpyAsync(pl_.P0 + r.first, pl_.P1 + r.first, sizeof(float4) * r.second, hipMemcpyDeviceToDevice, stream_));
+    predicted_in_p1_ = false;
 }
 
 // One frame: with several table sets, group k > 0 runs on stream k of its own. Joined (graph
@@ -1737,21 +1760,25 @@ void Engine::record_group(const DevState& d, float frame_dt, hipStream_t s, hipE
 // own, and the solver's stream does not wait for them at the end of the frame; join() adds
 // that wait, and every operation other than the next frame that touches device state calls it.
 void Engine::record_frame(float frame_dt, hipStream_t s, bool lazy) {
+    in_p1_.clear();
+    const auto note = [&](size_t k, bool in_p1) {
+        if (in_p1) in_p1_.insert(in_p1_.end(), fused_ranges_[k].begin(), fused_ranges_[k].end());
+    };
     if (groups_.size() < 2) {
-        record_group(groups_.empty() ? ds_ : groups_[0], frame_dt, s);
+        note(0, record_group(groups_.empty() ? ds_ : groups_[0], frame_dt, s));
         return;
     }
     if (lazy) {
-        record_group(groups_[0], frame_dt, s, ev_fork_);
+        note(0, record_group(groups_[0], frame_dt, s, ev_fork_));
     } else {
         VTX_HIP(hipEventRecord(ev_fork_, s));
-        record_group(groups_[0], frame_dt, s);
+        note(0, record_group(groups_[0], frame_dt, s));
     }
     pending_join_ = groups_.size() - 1;
     try {
         for (size_t k = 1; k < groups_.size(); k++) {
             VTX_HIP(hipStreamWaitEvent(xstreams_[k - 1], ev_fork_, 0));
-            record_group(groups_[k], frame_dt, xstreams_[k - 1]);
+            note(k, record_group(groups_[k], frame_dt, xstreams_[k - 1]));
             VTX_HIP(hipEventRecord(ev_join_[k - 1], xstreams_[k - 1]));
         }
     } catch (...) {
@@ -1813,6 +1840,7 @@ void Engine::simulate(float frame_dt) {
         // a caller's stream keeps its order: work queued on it after the frame sees every group
         record_frame(frame_dt, stream_, own_stream_);
     }
+    predicted_in_p1_ = !in_p1_.empty();
 }
 
 void Engine::sync_stream() {
@@ -2124,6 +2152,7 @@ void Engine::write_predicted(int32_t s, const float* xyz) {
     VTX_REQUIRE(xyz, VTX_EINVAL, "positions are NULL");
     ensure_committed();
     VTX_REQUIRE(sg.uploaded, VTX_ESTATE, "segment is not resident on the device");
+    settle_predicted();
     synchronize();
     const uint32_t n = sg.n();
     if (!n) return;
@@ -2141,6 +2170,7 @@ void Engine::run_hash() {
     join();
     ensure_committed();
     VTX_REQUIRE(any_selfcol_, VTX_ESTATE, "no active segment has self collision enabled");
+    settle_predicted();
     for (const DevState& g : groups_) hash_build(g, 0, stream_);
     synchronize();
 }

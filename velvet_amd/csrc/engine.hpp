@@ -269,7 +269,8 @@ private:
     void grow_pools(const Ranges& need);
     void record_frame(float frame_dt, hipStream_t s, bool lazy);
     void hash_build(const DevState& d, int in, hipStream_t s);
-    void record_group(const DevState& d, float frame_dt, hipStream_t s, hipEvent_t after_hash = nullptr);
+    bool record_group(const DevState& d, float frame_dt, hipStream_t s, hipEvent_t after_hash = nullptr);
+    void settle_predicted();
     void stage_begin(const char* kernel, const char* label, hipStream_t s, int passes = 1);
     void stage_end(hipStream_t s);
     void check_seg(int32_t s) const;
@@ -313,6 +314,11 @@ private:
     std::vector<hipEvent_t> ev_join_;        // one per extra stream
     size_t pending_join_ = 0;                // extra streams whose last frame the solver's stream has not joined
     std::vector<int32_t> table_seg_;         // table index -> segment id
+    // ranges (first particle, count) of the fused segments, per group; those whose predicted positions the
+    // recorded frame leaves in P1; whether a frame has left them there since settle_predicted
+    std::vector<std::vector<std::pair<size_t, uint32_t>>> fused_ranges_;
+    std::vector<std::pair<size_t, uint32_t>> in_p1_;
+    bool predicted_in_p1_ = false;
     int passes_ = 1;
     int sorted_src_ = 0;
     bool any_selfcol_ = false;

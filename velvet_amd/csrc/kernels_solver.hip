@@ -1026,11 +1026,12 @@ __device__ __forceinline__ void fuse_stretch(const SegDev& sg, const float4* sp,
     }
 }
 
-// One pass on the region of side R centred on the tile; EPI applies to the last one (R == T).
+// One pass on the region of side R centred on the tile; EPI applies to the last one (R == T). keep 1 or 2: the
+// tile's positions before the last or the next to last pass go to P[in ^ 1] (launch_iterate_fused).
 template <int EPI, int T, int R>
 __device__ __forceinline__ void fuse_pass(const DevState& d, const SegDev& sg, float4* sp, const float4* sr,
                                           const float (*sl)[VTX_FS * VTX_FS], float4 (&corr)[4][FuseTile<T>::NS],
-                                          uint32_t nslots, int a0, int b0, int in, float h, float xpbd) {
+                                          uint32_t nslots, int a0, int b0, int in, int keep, float h, float xpbd) {
     using F = FuseTile<T, R>;
     constexpr uint32_t mark = (VTX_FS - R) / 4;            // one per region size
     const int tid = (int)threadIdx.x, lane = tid & 63;
@@ -1061,6 +1062,10 @@ __device__ __forceinline__ void fuse_pass(const DevState& d, const SegDev& sg, f
         const float4 p4 = sp[sc];
         p = xyz(p4);
         w = p4.w;
+        if (EPI == EPI_FINALIZE && R <= T + 4 && keep == (R - T) / 4 + 1) {
+            constexpr int O = (R - T) / 2;                  // the tile within the region
+            if (y >= O && y < O + T && x >= O && x < O + T) d.P[in ^ 1][sg.pbase + (uint32_t)(a * (int)sg.cols + b)] = p4;
+        }
         fuse_stretch<8>(sg, sp, sr, sc, p, w, delta, cnt);
         for (uint32_t s = 0; s < nslots; s++) {                 // every slot is a part of its own
             V3 part = v3(0.f, 0.f, 0.f);
@@ -1084,7 +1089,7 @@ __device__ __forceinline__ void fuse_pass(const DevState& d, const SegDev& sg, f
 
 template <int EPI, int T>
 __global__ __launch_bounds__(1024) void k_iterate_fused(DevState d, const GridTileDev* __restrict__ tiles, int in,
-                                                        int passes, float h) {
+                                                        int passes, int keep, float h) {
     using F = FuseTile<T>;
     __shared__ float4 sp[VTX_FS * VTX_FS];                    // positions
     __shared__ float4 sr[VTX_FS * VTX_FS];                    // owned stretch rest lengths, NaN off the cloth
@@ -1118,11 +1123,11 @@ __global__ __launch_bounds__(1024) void k_iterate_fused(DevState d, const GridTi
     __syncthreads();
     const float xpbd = sg.bend_compliance * frcp(h) * frcp(h);   // compliance / h^2 (cu:173)
     if constexpr (T <= 8)
-        if (passes > 3) fuse_pass<EPI, T, T + 12>(d, sg, sp, sr, sl, corr, nslots, a0, b0, in, h, xpbd);
+        if (passes > 3) fuse_pass<EPI, T, T + 12>(d, sg, sp, sr, sl, corr, nslots, a0, b0, in, keep, h, xpbd);
     if constexpr (T <= 12)
-        if (passes > 2) fuse_pass<EPI, T, T + 8>(d, sg, sp, sr, sl, corr, nslots, a0, b0, in, h, xpbd);
-    if (passes > 1) fuse_pass<EPI, T, T + 4>(d, sg, sp, sr, sl, corr, nslots, a0, b0, in, h, xpbd);
-    fuse_pass<EPI, T, T>(d, sg, sp, sr, sl, corr, nslots, a0, b0, in, h, xpbd);
+        if (passes > 2) fuse_pass<EPI, T, T + 8>(d, sg, sp, sr, sl, corr, nslots, a0, b0, in, keep, h, xpbd);
+    if (passes > 1) fuse_pass<EPI, T, T + 4>(d, sg, sp, sr, sl, corr, nslots, a0, b0, in, keep, h, xpbd);
+    fuse_pass<EPI, T, T>(d, sg, sp, sr, sl, corr, nslots, a0, b0, in, keep, h, xpbd);
 }
 
 // One pass of a 16 x 16 tile of a cloth with many dense attachments (VTX_SEG_LRA_TILED, at least
@@ -1429,19 +1434,20 @@ hipError_t launch_iterate(const DevState& d, int in, float h, int epilogue, bool
 }
 
 template <int T>
-static void launch_fused(const DevState& d, int in, int passes, float h, int epilogue, hipStream_t s) {
+static void launch_fused(const DevState& d, int in, int passes, int keep, float h, int epilogue, hipStream_t s) {
     const dim3 gr(d.nftiles), bl(1024);
-    if (epilogue == EPI_NONE) hipLaunchKernelGGL((k_iterate_fused<EPI_NONE, T>), gr, bl, 0, s, d, d.ftiles, in, passes, h);
-    else if (epilogue == EPI_FINALIZE) hipLaunchKernelGGL((k_iterate_fused<EPI_FINALIZE, T>), gr, bl, 0, s, d, d.ftiles, in, passes, h);
-    else hipLaunchKernelGGL((k_iterate_fused<EPI_FINALIZE_PREDICT, T>), gr, bl, 0, s, d, d.ftiles, in, passes, h);
+    if (epilogue == EPI_NONE) hipLaunchKernelGGL((k_iterate_fused<EPI_NONE, T>), gr, bl, 0, s, d, d.ftiles, in, passes, keep, h);
+    else if (epilogue == EPI_FINALIZE) hipLaunchKernelGGL((k_iterate_fused<EPI_FINALIZE, T>), gr, bl, 0, s, d, d.ftiles, in, passes, keep, h);
+    else hipLaunchKernelGGL((k_iterate_fused<EPI_FINALIZE_PREDICT, T>), gr, bl, 0, s, d, d.ftiles, in, passes, keep, h);
 }
 
-hipError_t launch_iterate_fused(const DevState& d, int in, int passes, float h, int epilogue, hipStream_t s) {
+hipError_t launch_iterate_fused(const DevState& d, int in, int passes, int keep, float h, int epilogue, hipStream_t s) {
     if (!d.nftiles) return hipSuccess;
     if (passes < 1 || passes > fuse_passes(d.fside)) return hipErrorInvalidValue;   // the staged halo
-    if (d.fside == 8) launch_fused<8>(d, in, passes, h, epilogue, s);
-    else if (d.fside == 12) launch_fused<12>(d, in, passes, h, epilogue, s);
-    else launch_fused<16>(d, in, passes, h, epilogue, s);
+    if (keep && (epilogue != EPI_FINALIZE || keep > passes)) return hipErrorInvalidValue;
+    if (d.fside == 8) launch_fused<8>(d, in, passes, keep, h, epilogue, s);
+    else if (d.fside == 12) launch_fused<12>(d, in, passes, keep, h, epilogue, s);
+    else launch_fused<16>(d, in, passes, keep, h, epilogue, s);
     return last_launch();
 }
 

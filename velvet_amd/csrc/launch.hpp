@@ -20,7 +20,9 @@ hipError_t launch_iterate(const DevState& d, int in, float h, int epilogue, bool
                           hipStream_t s);
 // Fused passes of the grid segments in d.ftiles: most passes per launch for tiles of side 8, 12, 16
 inline int fuse_passes(uint32_t side) { return (VTX_FS - (int)side) / 4; }
-hipError_t launch_iterate_fused(const DevState& d, int in, int passes, float h, int epilogue, hipStream_t s);
+// keep (the frame's last launch): 1 / 2 = the positions before the last / next to last pass go to P[in ^ 1], which
+// the launch itself leaves unwritten; 0 = none
+hipError_t launch_iterate_fused(const DevState& d, int in, int passes, int keep, float h, int epilogue, hipStream_t s);
 hipError_t launch_normals(const DevState& d, hipStream_t s);
 hipError_t launch_check_finite(const DevState& d, uint32_t* flags, uint32_t nseg, hipStream_t s);
 
