@@ -368,8 +368,9 @@ __device__ __forceinline__ void wave_lds_sync() {
 // of c particles costs c^2, so a range with a cell of more than VTX_HASH_HEAVY sorts its list in LDS
 // instead, or, if it holds more than the list, places such cells by two runs over the keys in index order
 // for up to 256 of them at a time (hash_part_runs), so that no input costs quadratic time: 131,072 objects
-// with their search, in cells of 100 / 140 / 300 / 2,000: 66 / 80 / 93 / 101 us, in a table of 1,000 cells
-// 95 us (device-wide sort 113 / 113 / 111 / 109, 97; two runs for each crowded cell 66 / 649 / 455 / 263, 460).
+// with their search, in cells of 100 / 140 / 300 / 2,000 / 6,000: 66 / 80 / 93 / 101 / 166 us, in a table of
+// 1,000 cells 94 us (device-wide sort 112 / 111 / 110 / 107 / 104, 96; two runs for each crowded cell 67 / 652 /
+// 455 / 265 / 167, 461). All in one cell is one workgroup's work: 330 us (77; 441).
 // Bound by latency: a launch's 2.6 us, then the chain range record, keys, LDS counts, scan, placement,
 // gathered records, and from 2^15 particles on the two runs over the keys. No workgroup waits for another,
 // where the dozen launches of a device-wide sort did and one workgroup per segment with a radix sort in
@@ -383,6 +384,11 @@ struct alignas(16) HashPartLds {           // cnt is read and written four words
     uint32_t wsum[16], nheavy, below;
 };
 static_assert(offsetof(HashPartLds, cnt) % 16 == 0, "cnt is accessed in 16-byte units");
+
+// Whether the wave's lanes (all active) have hit and one value: 64 LDS additions to one word go one by one.
+__device__ __forceinline__ bool wave_of(uint32_t k, bool hit) {
+    return __builtin_amdgcn_ballot_w64(hit && k == __builtin_amdgcn_readfirstlane(k)) == ~0ull;
+}
 
 // Ascending bitonic sort of a[0..m), m a power of two of at least 1. Thread t exchanges a pair 2^b apart;
 // for pairs up to 64 apart a wave's threads stay within 128 words of their own, so steps of such pairs
@@ -408,7 +414,7 @@ __device__ __forceinline__ void sort_list(uint32_t* a, uint32_t m) {
 // The cells of more than VTX_HASH_HEAVY particles of a range that holds more than its list, up to 256 (512)
 // of them at a time: wave w takes the w-th part of the particles in order, counts its particles per cell,
 // then places them behind those of the waves before it, 64 at a time ranked by ballots over the cell's number.
-// U times 64 keys are in flight.
+// U times 64 keys are in flight. L.heavy: the cells with their first places.
 template <uint32_t BT, uint32_t U, class S>
 __device__ __forceinline__ void hash_part_runs(const S& s, uint32_t n, uint32_t lo, uint32_t C, uint32_t base,
                                                uint32_t nheavy, HashPartLds& L) {
@@ -417,11 +423,6 @@ __device__ __forceinline__ void hash_part_runs(const S& s, uint32_t n, uint32_t 
     static_assert(HB == 1u << BITS, "a cell's number among HB");
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     __syncthreads();                                        // the cells' bounds are read
-    for (uint32_t h = tid; h < nheavy; h += BT) {           // with the cell's first place (< 2^17)
-        const uint32_t k = L.heavy[h];
-        L.heavy[h] = (k ? L.cnt[k - 1] : 0u) << 12 | k;
-    }
-    __syncthreads();
     for (uint32_t k = tid; k < C; k += BT) L.cnt[k] = VTX_INVALID;
     __syncthreads();
     for (uint32_t h = tid; h < nheavy; h += BT) L.cnt[L.heavy[h] & 0xFFFu] = h;
@@ -447,7 +448,11 @@ __device__ __forceinline__ void hash_part_runs(const S& s, uint32_t n, uint32_t 
             load(i0);
 #pragma unroll
             for (uint32_t u = 0; u < U; u++)
-                if (q[u] < nb) atomicAdd(&hw[q[u]], 1u);
+                if (wave_of(q[u], q[u] < nb)) {
+                    if (lane == 0) atomicAdd(&hw[q[u]], 64u);
+                } else if (q[u] < nb) {
+                    atomicAdd(&hw[q[u]], 1u);
+                }
         }
         __syncthreads();
         for (uint32_t h = tid; h < nb; h += BT) {
@@ -465,13 +470,16 @@ __device__ __forceinline__ void hash_part_runs(const S& s, uint32_t n, uint32_t 
 #pragma unroll
             for (uint32_t u = 0; u < U; u++) {
                 const bool hit = q[u] < nb;
-                uint64_t peers = __builtin_amdgcn_ballot_w64(hit);
-                if (!peers) continue;
+                const uint64_t hits = __builtin_amdgcn_ballot_w64(hit);
+                if (!hits) continue;
+                const uint32_t f = (uint32_t)__builtin_amdgcn_readlane((int)q[u], __builtin_ctzll(hits));
+                uint64_t peers = hits;
+                if (hits & ~__builtin_amdgcn_ballot_w64(q[u] == f))   // more than one cell
 #pragma unroll
-                for (int c = 0; c < BITS; c++) {
-                    const uint32_t m = (uint32_t)((int32_t)(q[u] << (31 - c)) >> 31);   // bit c as 0 / ~0
-                    peers &= ~(__builtin_amdgcn_ballot_w64(m != 0u) ^ ((uint64_t)m << 32 | m));
-                }
+                    for (int c = 0; c < BITS; c++) {
+                        const uint32_t m = (uint32_t)((int32_t)(q[u] << (31 - c)) >> 31);   // bit c as 0 / ~0
+                        peers &= ~(__builtin_amdgcn_ballot_w64(m != 0u) ^ ((uint64_t)m << 32 | m));
+                    }
                 const uint32_t rank = (uint32_t)__popcll(peers & lt);
                 at[u] = hw[hit ? q[u] : 0u] + rank;
                 wave_lds_sync();
@@ -553,6 +561,7 @@ __device__ __forceinline__ void hash_part(const S& s, uint32_t n, uint32_t lo, u
     const uint32_t padded = own <= 1u ? 1u : 1u << (32 - __builtin_clz(own - 1u));   // list entries to sort
     __syncthreads();
     // the range's particles into their cells, in any order; more than fit go through global scratch
+    constexpr uint32_t FLAG = 1u << 31;                     // in cnt: a crowded cell that has its end already
     const auto rest = [&](uint32_t* __restrict__ list, auto clamp) {
         for (uint32_t i0 = 0; i0 < rounds; i0 += U * BT) {
             if (KEYED && n > U * BT) s.template load<BT, U>(i0 + tid, kk);
@@ -561,7 +570,7 @@ __device__ __forceinline__ void hash_part(const S& s, uint32_t n, uint32_t lo, u
                 if (i0 + u * BT >= n) break;
                 const uint32_t i = i0 + u * BT + tid;
                 const uint32_t k = KEYED && n > U * BT ? (i < n ? kk[u] - lo : VTX_INVALID) : kk[u];
-                if (k < C) list[atomicAdd(&L.cnt[k], 1u)] = k << 20 | i;
+                if (k < C && !(clamp.value && L.cnt[k] >> 31)) list[atomicAdd(&L.cnt[k], 1u)] = k << 20 | i;
             }
         }
         __syncthreads();
@@ -573,19 +582,26 @@ __device__ __forceinline__ void hash_part(const S& s, uint32_t n, uint32_t lo, u
             }
             return;
         }
-        for (uint32_t g = tid; g < own; g += BT) {
-            const uint32_t e = list[g], k = e >> 20;
-            const uint32_t begin = k ? L.cnt[k - 1] : 0u, end = L.cnt[k];
-            if (end - begin > VTX_HASH_HEAVY) continue;
-            uint32_t at = begin;
-            for (uint32_t j = begin; j < end; j += 4) {   // what follows the cell in the list is larger than e
-                uint32_t o[4];
+        constexpr uint32_t V = clamp.value ? 4 : 1;         // entries of the list in flight
+        for (uint32_t g0 = tid; g0 < own; g0 += V * BT) {
+            uint32_t ev[V];
 #pragma unroll
-                for (uint32_t u = 0; u < 4; u++) o[u] = list[clamp.value ? min(j + u, own - 1u) : j + u];
+            for (uint32_t v = 0; v < V; v++) ev[v] = list[V > 1 ? min(g0 + v * BT, own - 1u) : g0];
 #pragma unroll
-                for (uint32_t u = 0; u < 4; u++) at += (!clamp.value || j + u < own) && o[u] < e;
+            for (uint32_t v = 0; v < V; v++) {
+                const uint32_t e = ev[v], k = e >> 20;
+                if (V > 1 && (g0 + v * BT >= own || e == VTX_INVALID)) continue;
+                const uint32_t begin = k ? L.cnt[k - 1] & ~FLAG : 0u, end = L.cnt[k];
+                uint32_t at = begin;
+                for (uint32_t j = begin; j < end; j += 4) {   // what follows the cell in the list is larger than e
+                    uint32_t o[4];
+#pragma unroll
+                    for (uint32_t u = 0; u < 4; u++) o[u] = list[clamp.value ? min(j + u, own - 1u) : j + u];
+#pragma unroll
+                    for (uint32_t u = 0; u < 4; u++) at += (!clamp.value || j + u < end) && o[u] < e;
+                }
+                s.put(base + at, lo + k, e & 0xFFFFFu);
             }
-            s.put(base + at, lo + k, e & 0xFFFFFu);
         }
     };
     if (own <= VTX_HASH_PART_LIST) {
@@ -594,10 +610,33 @@ __device__ __forceinline__ void hash_part(const S& s, uint32_t n, uint32_t lo, u
             for (uint32_t g = own + tid; g < padded; g += BT) L.list[g] = VTX_INVALID;
         rest(L.list, std::false_type{});
     } else {
+        // crowded cells stay out of the list: their places are marked empty
+        constexpr uint32_t NH = (VTX_HASH_PART_N / VTX_HASH_HEAVY + BT - 1) / BT;
+        uint32_t end[NH];
+#pragma unroll
+        for (uint32_t r = 0; r < NH; r++) {
+            const uint32_t h = r * BT + tid, k = h < nheavy ? L.heavy[h] : 0u;
+            end[r] = k + 1u < C ? L.cnt[k + 1u] : own;
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t r = 0; r < NH; r++) {
+            const uint32_t h = r * BT + tid;
+            if (h < nheavy) {
+                const uint32_t k = L.heavy[h];
+                L.heavy[h] = L.cnt[k] << 12 | k;            // with the cell's first place (< 2^17)
+                L.cnt[k] = end[r] | FLAG;
+            }
+        }
+        __syncthreads();
+        for (uint32_t h = 0; h < nheavy; h++) {
+            const uint32_t b = L.heavy[h] >> 12, e = L.cnt[L.heavy[h] & 0xFFFu] & ~FLAG;
+            for (uint32_t g = b + tid; g < e; g += BT) (spill + base)[g] = VTX_INVALID;
+        }
         rest(spill + base, std::true_type{});
     }
     for (uint32_t k = tid; k < C; k += BT) {
-        const uint32_t begin = k ? L.cnt[k - 1] : 0u, end = L.cnt[k];
+        const uint32_t begin = k ? L.cnt[k - 1] & ~FLAG : 0u, end = L.cnt[k] & ~FLAG;
         s.cell(lo + k, end > begin ? base + begin : VTX_INVALID, end > begin ? base + end : VTX_INVALID);
     }
     if (nheavy && own > VTX_HASH_PART_LIST) hash_part_runs<BT, KEYED ? 4 : 1>(s, n, lo, C, base, nheavy, L);
