@@ -136,6 +136,17 @@ static void pack_tile(std::vector<E>& out, const std::vector<uint32_t>& start, c
     }
 }
 
+// Entries that pack_tile makes of n particles' lists.
+static size_t packed_size(const std::vector<uint32_t>& start, uint32_t n) {
+    size_t size = 0;
+    for (uint32_t first = 0; first < n; first += VTX_TILE) {
+        uint32_t K = 0;
+        for (uint32_t i = first; i < std::min<uint32_t>(first + VTX_TILE, n); i++) K = std::max(K, start[i + 1] - start[i]);
+        size += (size_t)K * VTX_TILE;
+    }
+    return size;
+}
+
 // Sliced-ELL packing with an explicit lane -> particle map (-1: lane has no particle).
 template <class E>
 static void pack_lanes(std::vector<E>& out, const std::vector<uint32_t>& start, const std::vector<E>& items,
@@ -875,8 +886,15 @@ void Engine::prepare_segment(Segment& sg) {
         std::vector<uint32_t> f(s_tr.begin(), s_tr.end() - 1);
         for (size_t c = 0; c < T; c++)
             for (int r = 0; r < 3; r++) l_tr[f[sg.tris[3 * c + r]]++] = (uint32_t)c;
+        pr.trec.reserve(T);
         for (size_t c = 0; c < T; c++)
             pr.trec.push_back(make_uint4(sg.tris[3 * c], sg.tris[3 * c + 1], sg.tris[3 * c + 2], 0));
+    }
+    if (!pr.grid) {
+        pr.est.reserve(packed_size(s_st, n));
+        pr.eat.reserve(packed_size(s_at, n));
+        pr.ebd.reserve(packed_size(s_bd, n));
+        pr.etr.reserve(packed_size(s_tr, n));
     }
     for (uint32_t first = 0; first < n; first += VTX_TILE) {
         TileDev t{};
