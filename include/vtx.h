@@ -179,8 +179,9 @@ typedef struct vtx_tuning {
     int32_t lra_split;         /* no effect: once four or one threads per particle in the Jacobi pass of
                                   grid cloths with 32 or more dense attachment slots; now always four */
     int32_t hash_lds;          /* 1: self-colliding segments of at most 131072 particles (table of
-                                  at most 2^19 cells) build their spatial hash by cell ranges, a
-                                  workgroup each; 0: every segment takes the device-wide sort */
+                                  at most 2^19 cells and at least one per 2048 particles) build
+                                  their spatial hash by cell ranges, a workgroup each; 0: every
+                                  segment takes the device-wide sort */
     int32_t hash_grid;         /* hash-grid resolution of segments with tune_hash_grid = 1 (others
                                   keep the reference grid): 0 = the reference grid (table of
                                   hash_table_size cells, cell coordinates hashed as they are);

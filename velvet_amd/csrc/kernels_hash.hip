@@ -735,8 +735,9 @@ __global__ __launch_bounds__(BT, 8) void k_hash_part(DevState d, int in, int dst
 // 88 -> 11.8 us, 65,536 particles 54.6 -> 16.9 us, 963,130 in 256 draped cloths 204.8 -> 106.7 us (a
 // particle tests some 150 candidates at 15 VALU instructions per 64, and 6 more where one is accepted:
 // 85% of its VALU issue time). A segment whose records outgrow the L2 is bound by fetching each cell's
-// records some 27 times, as neighbours in the sorted order are no neighbours in space: a folded pile of
-// 1,048,576 759 -> 267 us, 874 MB (by particle index instead: neighbor_blocks).
+// records again and again, as neighbours in the sorted order are no neighbours in space: 1,048,576 particles,
+// 33.5 MB of records, fetch 1,605 MB a search at rest (242 us) and 1,083 MB in a pile (286 us; one particle
+// per lane 759) (by particle index instead: neighbor_blocks).
 struct NbSet {
     const float4* rec;    // sorted records: position with w = index at 2i, initial position at 2i + 1
     const uint2* cells;   // (start, end) per hash cell
@@ -920,16 +921,15 @@ __device__ __forceinline__ void neighbor_wave(const NbSet& a, uint32_t i0, uint3
     else neighbor_wave_as<PW, CHUNK ? NB_CHUNK32 : NB_COLUMN, false, LISTED>(a, i0, cnt, L);
 }
 
-// The search by particle index (neighbor_order 0), for segments whose records outgrow the L2. In sorted order
+// The search by particle index (search_rule), for segments whose records outgrow the L2. In sorted order
 // the waves that run at one time have no cells in common, as neighbouring hashes are no neighbours in space.
 // Here a wave takes whole blocks of cells by index: neighbours in a cloth's index order are neighbours in
 // space, and a tile's wave and those beside it (on one XCD) share cells. A block is what a bucket holds of an
 // aligned run of PW sorted positions; the one of its particles that leads it is drawn by a hash of its first
 // position, so that of several layers not the lowest does all the work. inv: particle -> sorted position.
-// A draped 1,048,576-particle cloth on grid 1: 244 -> 162 us a search, 1.74 -> 1.58 ms a frame; on the
-// reference grid, whose mirrored cells share buckets, no gain; and a pile whose frames overlap with two
-// other solvers' loses, 2.89 -> 3.03 ms, as the waves are uneven and fetches are not what bounds it. So the
-// caller (neighbor_order) or the tuner chooses.
+// A draped 1,048,576-particle cloth on grid 1 fetches 440 MB instead of 1,605: 243 -> 154 us a search, 1.78 ->
+// 1.61 ms a frame; on the reference grid, whose mirrored cells share buckets, 245 -> 198 us. A pile loses,
+// 319 -> 497 us, as the waves are uneven and fetches are not what bounds it.
 template <int PW>
 __device__ __forceinline__ void neighbor_blocks(const NbSet& a, const uint32_t* __restrict__ inv,
                                                 const float4* __restrict__ P, uint32_t first, uint32_t cnt, NbLds<PW>& L) {

@@ -704,9 +704,8 @@ __global__ __launch_bounds__(VTX_TILE) void k_iterate_plain(DevState d, const Ti
 // LDS, and each vertex gathers its 8 stretch terms, its attachments and its 12 bending terms in
 // a fixed order. The three slot types are evaluated one after another through the same LDS
 // area (X, then R, then D), which keeps the workgroup at ~18 KB of LDS (8 workgroups per CU). A large live
-// set is bound by VALU issue (1024 x 1024: 99% of the 24 us in which the CUs are busy, of 28.2 us a pass;
-// the LDS is busy half of the time): of 869 instructions a wave, 430 are the slots' arithmetic, 180 the
-// stretch terms. Cell indices by 24-bit products with the division shared between types, and staging
+// set is bound by VALU issue (1024 x 1024: 99% of the 24 us in which the CUs are busy, of 28.2 us a pass):
+// of 869 instructions a wave, 430 are the slots' arithmetic, 180 the stretch terms. Cell indices by 24-bit products with the division shared between types, and staging
 // without divisions took it from 28.7 to 28.2 us (512 cloths of 963,130 particles 3174 -> 3129 us a frame
 // pair). Vectors of four per role instead of the planes take 21 KB, one workgroup less per CU: 31.5 us.
 // Slot owner ranges relative to the tile origin (a0, b0): X rows/cols [-1, 15] (17 x 17),

@@ -189,7 +189,6 @@ struct alignas(16) ColliderDev {
 #define VTX_LIVE_KEYED 2u     // k_hash_part's segments of several ranges have VTX_SEG_HASH_KEYED
 #define VTX_LIVE_FULL 4u      // more than VTX_HASH_PART_FULL particles
 
-// Pointers and sizes every kernel may need; passed by value (kernel-argument segment).
 // A range of a segment's hash cells (k_hash_part), with what its workgroup needs of the segment.
 struct HashPartDev {
     uint32_t pbase, n, tbase, M, lo, cells, mod, shift, keyed;
@@ -197,6 +196,7 @@ struct HashPartDev {
     uint32_t pad[2];
 };
 
+// Pointers and sizes every kernel may need; passed by value (kernel-argument segment).
 struct DevState {
     const SegDev* segs;
     const TileDev* tiles;
