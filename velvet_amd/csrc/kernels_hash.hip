@@ -366,7 +366,8 @@ __device__ __forceinline__ void wave_lds_sync() {
 // into their cells in any order and finds each one's place inside its cell by counting the cell's smaller
 // indices: a stable sort by key, so the same table and records as the device-wide path. Counting a cell
 // of c particles costs c^2, so a range with a cell of more than VTX_HASH_HEAVY sorts its list in LDS
-// instead, or, if it holds more than the list, places such cells by two runs over the keys in index order
+// instead, or, if it holds more than the list or few keys are to be run over (VTX_HASH_SORT_MIN: a sort takes
+// 13 us, two runs over 1,600 keys 1, over 24,100 3), places such cells by two runs over the keys in index order
 // for up to 256 of them at a time (hash_part_runs), so that no input costs quadratic time: 131,072 objects
 // with their search, in cells of 100 / 140 / 300 / 2,000 / 6,000: 66 / 80 / 93 / 101 / 166 us, in a table of
 // 1,000 cells 94 us (device-wide sort 112 / 111 / 110 / 107 / 104, 96; two runs for each crowded cell 67 / 652 /
@@ -560,57 +561,11 @@ __device__ __forceinline__ void hash_part(const S& s, uint32_t n, uint32_t lo, u
     const uint32_t base = L.below, nheavy = L.nheavy;
     const uint32_t padded = own <= 1u ? 1u : 1u << (32 - __builtin_clz(own - 1u));   // list entries to sort
     __syncthreads();
-    // the range's particles into their cells, in any order; more than fit go through global scratch
+    // the range's particles into their cells, in any order; more than fit go through global scratch. Crowded
+    // cells are sorted with the list, or stay out of it (their places marked empty) and are placed afterwards
     constexpr uint32_t FLAG = 1u << 31;                     // in cnt: a crowded cell that has its end already
-    const auto rest = [&](uint32_t* __restrict__ list, auto clamp) {
-        for (uint32_t i0 = 0; i0 < rounds; i0 += U * BT) {
-            if (KEYED && n > U * BT) s.template load<BT, U>(i0 + tid, kk);
-#pragma unroll
-            for (uint32_t u = 0; u < U; u++) {
-                if (i0 + u * BT >= n) break;
-                const uint32_t i = i0 + u * BT + tid;
-                const uint32_t k = KEYED && n > U * BT ? (i < n ? kk[u] - lo : VTX_INVALID) : kk[u];
-                if (k < C && !(clamp.value && L.cnt[k] >> 31)) list[atomicAdd(&L.cnt[k], 1u)] = k << 20 | i;
-            }
-        }
-        __syncthreads();
-        if (!clamp.value && nheavy) {
-            sort_list<BT>(list, padded);
-            for (uint32_t g = tid; g < own; g += BT) {
-                const uint32_t e = list[g];
-                s.put(base + g, lo + (e >> 20), e & 0xFFFFFu);
-            }
-            return;
-        }
-        constexpr uint32_t V = clamp.value ? 4 : 1;         // entries of the list in flight
-        for (uint32_t g0 = tid; g0 < own; g0 += V * BT) {
-            uint32_t ev[V];
-#pragma unroll
-            for (uint32_t v = 0; v < V; v++) ev[v] = list[V > 1 ? min(g0 + v * BT, own - 1u) : g0];
-#pragma unroll
-            for (uint32_t v = 0; v < V; v++) {
-                const uint32_t e = ev[v], k = e >> 20;
-                if (V > 1 && (g0 + v * BT >= own || e == VTX_INVALID)) continue;
-                const uint32_t begin = k ? L.cnt[k - 1] & ~FLAG : 0u, end = L.cnt[k];
-                uint32_t at = begin;
-                for (uint32_t j = begin; j < end; j += 4) {   // what follows the cell in the list is larger than e
-                    uint32_t o[4];
-#pragma unroll
-                    for (uint32_t u = 0; u < 4; u++) o[u] = list[clamp.value ? min(j + u, own - 1u) : j + u];
-#pragma unroll
-                    for (uint32_t u = 0; u < 4; u++) at += (!clamp.value || j + u < end) && o[u] < e;
-                }
-                s.put(base + at, lo + k, e & 0xFFFFFu);
-            }
-        }
-    };
-    if (own <= VTX_HASH_PART_LIST) {
-        if (tid < 3) L.list[own + tid] = VTX_INVALID;
-        if (nheavy)
-            for (uint32_t g = own + tid; g < padded; g += BT) L.list[g] = VTX_INVALID;
-        rest(L.list, std::false_type{});
-    } else {
-        // crowded cells stay out of the list: their places are marked empty
+    const bool fits = own <= VTX_HASH_PART_LIST, runs = nheavy && (!fits || n <= VTX_HASH_SORT_MIN);
+    const auto keep_out = [&](uint32_t* __restrict__ list) {
         constexpr uint32_t NH = (VTX_HASH_PART_N / VTX_HASH_HEAVY + BT - 1) / BT;
         uint32_t end[NH];
 #pragma unroll
@@ -631,15 +586,76 @@ __device__ __forceinline__ void hash_part(const S& s, uint32_t n, uint32_t lo, u
         __syncthreads();
         for (uint32_t h = 0; h < nheavy; h++) {
             const uint32_t b = L.heavy[h] >> 12, e = L.cnt[L.heavy[h] & 0xFFFu] & ~FLAG;
-            for (uint32_t g = b + tid; g < e; g += BT) (spill + base)[g] = VTX_INVALID;
+            for (uint32_t g = b + tid; g < e; g += BT) list[g] = VTX_INVALID;
         }
-        rest(spill + base, std::true_type{});
+    };
+    const auto fill = [&](uint32_t* __restrict__ list, auto crowded) {
+        for (uint32_t i0 = 0; i0 < rounds; i0 += U * BT) {
+            if (KEYED && n > U * BT) s.template load<BT, U>(i0 + tid, kk);
+#pragma unroll
+            for (uint32_t u = 0; u < U; u++) {
+                if (i0 + u * BT >= n) break;
+                const uint32_t i = i0 + u * BT + tid;
+                const uint32_t k = KEYED && n > U * BT ? (i < n ? kk[u] - lo : VTX_INVALID) : kk[u];
+                if (k < C && !(crowded.value && L.cnt[k] >> 31)) list[atomicAdd(&L.cnt[k], 1u)] = k << 20 | i;
+            }
+        }
+        __syncthreads();
+    };
+    // every particle behind the smaller ones of its cell; V entries of the list in flight
+    const auto place = [&](const uint32_t* __restrict__ list, auto crowded, auto v_, auto clamp) {
+        constexpr uint32_t V = v_.value;
+        for (uint32_t g0 = tid; g0 < own; g0 += V * BT) {
+            uint32_t ev[V];
+#pragma unroll
+            for (uint32_t v = 0; v < V; v++) ev[v] = list[V > 1 ? min(g0 + v * BT, own - 1u) : g0];
+#pragma unroll
+            for (uint32_t v = 0; v < V; v++) {
+                const uint32_t e = ev[v], k = e >> 20;
+                if ((V > 1 && g0 + v * BT >= own) || (crowded.value && e == VTX_INVALID)) continue;
+                const uint32_t begin = k ? L.cnt[k - 1] & (crowded.value ? ~FLAG : ~0u) : 0u, end = L.cnt[k];
+                uint32_t at = begin;
+                for (uint32_t j = begin; j < end; j += 4) {   // what follows the cell in the list is larger than e
+                    uint32_t o[4];
+#pragma unroll
+                    for (uint32_t u = 0; u < 4; u++) o[u] = list[clamp.value ? min(j + u, own - 1u) : j + u];
+#pragma unroll
+                    for (uint32_t u = 0; u < 4; u++) at += (!(clamp.value || crowded.value) || j + u < end) && o[u] < e;
+                }
+                s.put(base + at, lo + k, e & 0xFFFFFu);
+            }
+        }
+    };
+    constexpr std::integral_constant<uint32_t, 1> one{};
+    constexpr std::integral_constant<uint32_t, 4> four{};
+    constexpr std::true_type yes{};
+    constexpr std::false_type no{};
+    if (fits && tid < 3) L.list[own + tid] = VTX_INVALID;
+    if (!fits) {
+        keep_out(spill + base);
+        fill(spill + base, yes);
+        place(spill + base, yes, four, yes);
+    } else if (!nheavy) {
+        fill(L.list, no);
+        place(L.list, no, one, no);
+    } else if (runs) {
+        keep_out(L.list);
+        fill(L.list, yes);
+        place(L.list, yes, one, no);
+    } else {
+        for (uint32_t g = own + tid; g < padded; g += BT) L.list[g] = VTX_INVALID;
+        fill(L.list, no);
+        sort_list<BT>(L.list, padded);
+        for (uint32_t g = tid; g < own; g += BT) {
+            const uint32_t e = L.list[g];
+            s.put(base + g, lo + (e >> 20), e & 0xFFFFFu);
+        }
     }
     for (uint32_t k = tid; k < C; k += BT) {
         const uint32_t begin = k ? L.cnt[k - 1] & ~FLAG : 0u, end = L.cnt[k] & ~FLAG;
         s.cell(lo + k, end > begin ? base + begin : VTX_INVALID, end > begin ? base + end : VTX_INVALID);
     }
-    if (nheavy && own > VTX_HASH_PART_LIST) hash_part_runs<BT, KEYED ? 4 : 1>(s, n, lo, C, base, nheavy, L);
+    if (runs) hash_part_runs<BT, KEYED ? 4 : 2>(s, n, lo, C, base, nheavy, L);
 }
 
 // A segment's particles: float4 positions, keys from k_hash_keys or worked out here.

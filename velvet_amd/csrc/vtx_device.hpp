@@ -55,6 +55,7 @@
 #define VTX_HASH_PART_CELLS 4096u    // cells of a range at most
 #define VTX_HASH_PART_LIST 4096u     // particles of a range held in LDS
 #define VTX_HASH_HEAVY 128u
+#define VTX_HASH_SORT_MIN 32768u     // particles beyond which a range of crowded cells sorts its list
 #define VTX_COLLIDE_SMALL 81920u   // particles of a launch (a stream group's) up to which the contact pass reads ahead
 
 // floor(2^32 / M), for the remainder by M (hash_coords).
