@@ -32,7 +32,7 @@ def _run(scenes, streams=1):
         return [(s.positions(k), s.velocities(k), s.normals(k)) for k in segs]
 
 
-@pytest.mark.parametrize("sides,streams", [((2, 20), 1), ((16, 17), 1), ((255, 20), 1), ((257, 20), 1), ((300, 40, 33), 2)])
+@pytest.mark.parametrize("sides,streams", [((2, 20), 1), ((16, 17), 1), ((255, 20), 1), ((257, 20), 1), ((300, 40, 33), 2), ((1027, 30), 1)])
 def test_plain_tiles_beside_bent_ones(sides, streams):
     print(f"[gpu] plain tiles {sides} streams={streams}", flush=True)
     scenes = [_scene(n, "none" if k != 1 else "pairs", (2, 0, 3)[k], k) for k, n in enumerate(sides)]
