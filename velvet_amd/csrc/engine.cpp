@@ -1463,15 +1463,13 @@ void Engine::rebuild_tables() {
         hbase += 256u * nst;
         if (!in_lds) compact += d.n;
     }
-    // tiles without bending constraints behind the others of their group, for the launch of their own: where
-    // all are, or where they fill the chip several times over; fewer go along with the others' launch, as one
-    // more costs some 8 us (490,000 particles in 1,914 tiles gain 6 us a pass)
+    // tiles without bending constraints behind the others of their group
     std::vector<uint32_t> plain(cuts.size() + 1, 0);
     for (size_t k = 0; k <= cuts.size(); k++) {
         const auto b = hitile.begin() + (ptrdiff_t)(k ? cuts[k - 1].i : 0);
         const auto e = k < cuts.size() ? hitile.begin() + (ptrdiff_t)cuts[k].i : hitile.end();
         const auto m = std::stable_partition(b, e, [](const TileDev& t) { return t.ub_n != 0; });
-        if (m == b || e - m > 4096) plain[k] = (uint32_t)(e - m);
+        plain[k] = (uint32_t)(e - m);
     }
     passes_ = std::max(1, (int)((maxbits + 7) / 8));
     VTX_REQUIRE((hbase + VTX_SCAN_BLOCK - 1) / VTX_SCAN_BLOCK <= 65536u, VTX_ECAPACITY, "histogram too large");

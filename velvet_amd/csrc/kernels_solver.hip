@@ -543,6 +543,23 @@ __device__ __forceinline__ void stretch_terms(const DevState& d, const SegDev& s
     }
 }
 
+// One pass of a particle (lane of its tile) that has no bending constraints.
+template <int EPI>
+__device__ __forceinline__ void plain_particle(const DevState& d, const TileDev& t, uint32_t lane, int in, float h) {
+    if (lane >= t.count) return;
+    const SegDev sg = d.segs[t.seg];
+    const uint32_t g = t.begin + lane;
+    const float4* __restrict__ P = d.P[in] + sg.pbase;
+    const float4 p4 = P[g - sg.pbase];
+    V3 p = xyz(p4), delta = v3(0.f, 0.f, 0.f);
+    const float w = p4.w;
+    int cnt = 0;
+    stretch_terms(d, sg, t, P, lane, g - sg.pbase, p, w, delta, cnt);
+    attach_terms(d, sg, t.at_off, t.at_k, lane, g - sg.pbase, p, w, delta, cnt);
+    if (cnt > 0) p = madd(p, delta, frcp((float)cnt) * sg.omega);
+    epilogue<EPI>(d, sg, g, in, p, w, h);
+}
+
 // One Jacobi pass on the general path: SolveStretch (cu:65-102) + SolveAttachment
 // (cu:205-235) + SolveBending (cu:117-189) gathered per particle over its incident
 // constraints (sliced ELL), then ApplyDeltas (cu:253-264) and the epilogue.
@@ -555,17 +572,29 @@ __device__ __forceinline__ void stretch_terms(const DevState& d, const SegDev& s
 // dozen dependent gathers and evaluations: 20.7 us a pass for 22,801 particles in 90 tiles, now 8.5 us;
 // 4,608 particles 15.4 -> 7.1, 90,000 19.0 -> 15.4, 490,000 63.5 -> 57.8 us, where the halves even out:
 // a tile of consecutive particles of a mesh meets 1.7 times the bends it owns.
+//
+// The last nptiles of the tiles have no bends; MIXED, a workgroup takes three of them, a thread per
+// particle (one each kept two thirds of the threads idle: 490,000 particles without bends beside 90,000 with
+// them 2,067 -> 1,000 us a frame of 32 passes). The branch costs a pass 2 to 4%, so sets without such tiles, and
+// those of no more tiles than CUs, do without it.
 #define VTX_MT 768             // threads of the workgroup
-template <int EPI, int RPT>
+template <int EPI, int RPT, bool MIXED>
 __global__ __launch_bounds__(VTX_MT, RPT == 1 ? 6 : 3) void k_iterate(DevState d, const TileDev* __restrict__ tiles, int in, float h) {
     constexpr uint32_t UB = RPT * VTX_MT;               // records of a round
     __shared__ float4 grad[4][UB];
     __shared__ uint32_t act[UB];
     constexpr uint32_t NE = 12;                         // bend entries of a particle staged in LDS
     __shared__ uint32_t ent[NE * VTX_TILE];
-    const TileDev t = tiles[tile_of(d.remap)];
+    const uint32_t tid = threadIdx.x, wg = tile_of(d.remap);
+    const uint32_t nbent = d.nitiles - d.nptiles;
+    if (MIXED && wg >= nbent) {
+        constexpr uint32_t PT = VTX_MT / VTX_TILE;
+        const uint32_t i = nbent + PT * (wg - nbent) + __builtin_amdgcn_readfirstlane(tid / VTX_TILE);
+        if (i < d.nitiles) plain_particle<EPI>(d, tiles[i], tid % VTX_TILE, in, h);
+        return;
+    }
+    const TileDev t = tiles[wg];
     const SegDev sg = d.segs[t.seg];
-    const uint32_t tid = threadIdx.x;
     const bool vertex = tid < t.count;
     const uint32_t g = t.begin + tid;
     const float4* __restrict__ P = d.P[in] + sg.pbase;
@@ -676,24 +705,11 @@ __global__ __launch_bounds__(VTX_MT, RPT == 1 ? 6 : 3) void k_iterate(DevState d
     epilogue<EPI>(d, sg, g, in, p, w, h);
 }
 
-// The pass of tiles without bending constraints: one thread per particle and no LDS, as the form above keeps
-// two thirds of its threads and 64 KB idle there: 490,000 particles without bending 605 -> 419 us a frame of 32
-// passes, 576 particles 133 -> 127.
+// Tiles without bending constraints in a set that has no others: one thread per particle and no LDS, of which
+// k_iterate holds 64 KB (490,000 particles 605 -> 419 us a frame of 32 passes, 576 particles 133 -> 127).
 template <int EPI>
 __global__ __launch_bounds__(VTX_TILE) void k_iterate_plain(DevState d, const TileDev* __restrict__ tiles, int in, float h) {
-    const TileDev t = tiles[tile_of(d.remap)];
-    if (threadIdx.x >= t.count) return;
-    const SegDev sg = d.segs[t.seg];
-    const uint32_t g = t.begin + threadIdx.x;
-    const float4* __restrict__ P = d.P[in] + sg.pbase;
-    const float4 p4 = P[g - sg.pbase];
-    V3 p = xyz(p4), delta = v3(0.f, 0.f, 0.f);
-    const float w = p4.w;
-    int cnt = 0;
-    stretch_terms(d, sg, t, P, threadIdx.x, g - sg.pbase, p, w, delta, cnt);
-    attach_terms(d, sg, t.at_off, t.at_k, threadIdx.x, g - sg.pbase, p, w, delta, cnt);
-    if (cnt > 0) p = madd(p, delta, frcp((float)cnt) * sg.omega);
-    epilogue<EPI>(d, sg, g, in, p, w, h);
+    plain_particle<EPI>(d, tiles[tile_of(d.remap)], threadIdx.x, in, h);
 }
 
 // ---------------------------------------------------------------- grid stencil path
@@ -1391,22 +1407,23 @@ static void launch_iterate_split(const DevState& d, int in, float h, int epilogu
     else hipLaunchKernelGGL((k_iterate_split<EPI_FINALIZE_PREDICT, B>), gr, bl, 0, s, d, d.ltiles, in, h);
 }
 
-template <int RPT>
+template <int RPT, bool MIXED>
 static void launch_iterate_mesh(const DevState& d, int in, float h, int epilogue, hipStream_t s) {
-    if (d.nitiles == d.nptiles) return;
-    const dim3 gr(d.nitiles - d.nptiles), bl(VTX_MT);
-    if (epilogue == EPI_NONE) hipLaunchKernelGGL((k_iterate<EPI_NONE, RPT>), gr, bl, 0, s, d, d.itiles, in, h);
-    else if (epilogue == EPI_FINALIZE) hipLaunchKernelGGL((k_iterate<EPI_FINALIZE, RPT>), gr, bl, 0, s, d, d.itiles, in, h);
-    else hipLaunchKernelGGL((k_iterate<EPI_FINALIZE_PREDICT, RPT>), gr, bl, 0, s, d, d.itiles, in, h);
+    constexpr uint32_t PT = VTX_MT / VTX_TILE;
+    const uint32_t plain = MIXED ? d.nptiles : 0u;
+    const dim3 gr(d.nitiles - plain + (plain + PT - 1) / PT), bl(VTX_MT);
+    const auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, gr, bl, 0, s, d, d.itiles, in, h); };
+    if (epilogue == EPI_NONE) launch(k_iterate<EPI_NONE, RPT, MIXED>);
+    else if (epilogue == EPI_FINALIZE) launch(k_iterate<EPI_FINALIZE, RPT, MIXED>);
+    else launch(k_iterate<EPI_FINALIZE_PREDICT, RPT, MIXED>);
 }
 
 static void launch_iterate_plain(const DevState& d, int in, float h, int epilogue, hipStream_t s) {
-    if (!d.nptiles) return;
     const dim3 gr(d.nptiles), bl(VTX_TILE);
-    const TileDev* t = d.itiles + (d.nitiles - d.nptiles);
-    if (epilogue == EPI_NONE) hipLaunchKernelGGL(k_iterate_plain<EPI_NONE>, gr, bl, 0, s, d, t, in, h);
-    else if (epilogue == EPI_FINALIZE) hipLaunchKernelGGL(k_iterate_plain<EPI_FINALIZE>, gr, bl, 0, s, d, t, in, h);
-    else hipLaunchKernelGGL(k_iterate_plain<EPI_FINALIZE_PREDICT>, gr, bl, 0, s, d, t, in, h);
+    const auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, gr, bl, 0, s, d, d.itiles, in, h); };
+    if (epilogue == EPI_NONE) launch(k_iterate_plain<EPI_NONE>);
+    else if (epilogue == EPI_FINALIZE) launch(k_iterate_plain<EPI_FINALIZE>);
+    else launch(k_iterate_plain<EPI_FINALIZE_PREDICT>);
 }
 
 hipError_t launch_iterate(const DevState& d, int in, float h, int epilogue, bool constraints, int lra_batch,
@@ -1426,9 +1443,15 @@ hipError_t launch_iterate(const DevState& d, int in, float h, int epilogue, bool
     // a tile's records in one round while every tile has a CU of its own (8.5 against 11.5 us for 90
     // tiles of 1,334 records), else in rounds of half the LDS and twice the workgroups per CU (625 tiles
     // 28.5 against 33.4 us)
-    if (d.nitiles - d.nptiles <= 256) launch_iterate_mesh<2>(d, in, h, epilogue, s);
-    else launch_iterate_mesh<1>(d, in, h, epilogue, s);
-    launch_iterate_plain(d, in, h, epilogue, s);
+    if (d.nptiles == d.nitiles) {
+        if (d.nitiles) launch_iterate_plain(d, in, h, epilogue, s);
+    } else if (d.nitiles <= 256) {
+        launch_iterate_mesh<2, false>(d, in, h, epilogue, s);
+    } else if (d.nptiles) {
+        launch_iterate_mesh<1, true>(d, in, h, epilogue, s);
+    } else {
+        launch_iterate_mesh<1, false>(d, in, h, epilogue, s);
+    }
     return last_launch();
 }
 

@@ -227,7 +227,7 @@ struct DevState {
                               // particle index, then the initial position (one cache line holds both)
     uint32_t* nbr;            // neighbour tables per segment, chunks of four entries (16 or 8 bytes)
     const TileDev* itiles;    // particle tiles of segments on the general (ELL) Jacobi path; the last nptiles
-                              // have no bending constraints and a launch of their own
+                              // have no bending constraints
     const GridTileDev* gtiles;
     const GridTileDev* ltiles;   // grid tiles whose dense attachments run on four lanes per particle
     const GridTileDev* ftiles;   // fside x fside tiles of the grid segments whose passes are fused
