@@ -1,6 +1,7 @@
 """The general Jacobi path with a vertex of very many bends (a fan of triangles around it): the rounds over a
 tile's bend records go on where they stopped, so the time grows with the bends (four times as many within six
 times the time; every round over all entries took twelve times), and the particles' numbers don't matter."""
+import dataclasses
 import time
 
 import numpy as np
@@ -29,8 +30,8 @@ def _fan(d, order=None):
     return S.Scene(S.finish_params(p, [c]), [c], [], 2)
 
 
-def _run(scene, frames=2):
-    with ClothSolver() as s:
+def _run(scene, frames=2, **kw):
+    with ClothSolver(**kw) as s:
         s.load_scene(scene)
         s.Simulate()
         s.synchronize()
@@ -47,6 +48,22 @@ def test_renumbered_fan(d):
     to = np.argsort(S.uniform(d, 13, d + 1))
     _, x, v = _run(_fan(d))
     _, xr, vr = _run(_fan(d, to))
+    assert np.isfinite(x).all() and np.array_equal(x, xr[to]) and np.array_equal(v, vr[to])
+
+
+@pytest.mark.parametrize("n,repeat", [(20, 5), (20, 6), (262, 5), (262, 6)])
+def test_renumbered_grid(n, repeat):
+    """60 and 72 entries of a particle, on both sides of the count where rounds keep a particle's place, in sets of
+    no more tiles than CUs and of more."""
+    print(f"[gpu] grid of {n}, bends {repeat} times", flush=True)
+    c = S.grid_cloth(n, 0.05, center=(0.0, 1.0, 0.0), jitter=2e-3, seed=n, stream=11)
+    rest = S.uniform(n, 12, c.bend_rest.size, 0.0, 0.2).astype(np.float32)
+    c.bend, c.bend_rest = np.repeat(c.bend, repeat, axis=0), np.repeat(rest, repeat)
+    to = np.argsort(S.uniform(n, 13, c.n))
+    m = dataclasses.replace(c, x=c.x[np.argsort(to)], tris=to[c.tris].astype(np.uint32), stretch=to[c.stretch].astype(np.int32),
+                            bend=to[c.bend].astype(np.uint32))
+    p = S.Params(num_substeps=2, num_iterations=2, enable_self_collision=False)
+    (_, x, v), (_, xr, vr) = (_run(S.Scene(S.finish_params(p, [k]), [k], [], 2), stencil=False) for k in (c, m))
     assert np.isfinite(x).all() and np.array_equal(x, xr[to]) and np.array_equal(v, vr[to])
 
 

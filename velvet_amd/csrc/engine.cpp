@@ -1464,12 +1464,12 @@ void Engine::rebuild_tables() {
         if (!in_lds) compact += d.n;
     }
     // tiles without bending constraints behind the others of their group
-    std::vector<uint32_t> plain(cuts.size() + 1, 0);
+    std::vector<uint32_t> plain(cuts.size() + 1, 0), many(cuts.size() + 1, 0);
     for (size_t k = 0; k <= cuts.size(); k++) {
         const auto b = hitile.begin() + (ptrdiff_t)(k ? cuts[k - 1].i : 0);
         const auto e = k < cuts.size() ? hitile.begin() + (ptrdiff_t)cuts[k].i : hitile.end();
-        const auto m = std::stable_partition(b, e, [](const TileDev& t) { return t.ub_n != 0; });
-        plain[k] = (uint32_t)(e - m);
+        plain[k] = (uint32_t)(e - std::stable_partition(b, e, [](const TileDev& t) { return t.ub_n != 0; }));
+        if (std::any_of(b, e, [](const TileDev& t) { return t.bd_k > VTX_MANY_BENDS; })) many[k] = VTX_LIVE_MANY_BENDS;
     }
     passes_ = std::max(1, (int)((maxbits + 7) / 8));
     VTX_REQUIRE((hbase + VTX_SCAN_BLOCK - 1) / VTX_SCAN_BLOCK <= 65536u, VTX_ECAPACITY, "histogram too large");
@@ -1570,6 +1570,7 @@ void Engine::rebuild_tables() {
         g.ntiles = (uint32_t)(hi.t - lo.t);
         g.nitiles = (uint32_t)(hi.i - lo.i);
         g.nptiles = plain[k];
+        g.live |= many[k];
         g.ngtiles = (uint32_t)(hi.g - lo.g);
         g.nltiles = (uint32_t)(hi.l - lo.l);
         g.nstiles = (uint32_t)(hi.s - lo.s);

@@ -385,7 +385,7 @@ __device__ __forceinline__ const float4* tiled_part(const DevState& d, const Seg
 // ELL in registration order, where a part ends wherever the slot's part changes -- so attachments
 // registered particle-major in slot order sum exactly as the dense form does. NA listed attachments are in
 // flight: one after another each waits for its entry and then for its slot (general path, frames of 32 passes,
-// 131,769 particles with 8: 1,071 -> 875 us, 360,000 with 16: 2,296 -> 1,720); the stencil tiles have no
+// 131,769 particles with 35: 1,979 -> 1,339 us, 360,000 with 16: 2,296 -> 1,720); the stencil tiles have no
 // registers left for more than one.
 template <uint32_t NA>
 __device__ __forceinline__ void attach_terms(const DevState& d, const SegDev& sg, uint32_t at_off, uint32_t at_k,
@@ -585,12 +585,12 @@ __device__ __forceinline__ void plain_particle(const DevState& d, const TileDev&
 // 4,608 particles 15.4 -> 7.1, 90,000 19.0 -> 15.4, 490,000 63.5 -> 57.8 us, where the halves even out:
 // a tile of consecutive particles of a mesh meets 1.7 times the bends it owns.
 //
-// The last nptiles of the tiles have no bends; MIXED, a workgroup takes three of them, a thread per
-// particle (one each kept two thirds of the threads idle: 490,000 particles without bends beside 90,000 with
-// them 2,067 -> 1,000 us a frame of 32 passes). The branch costs a pass 2 to 4%, so sets without such tiles, and
-// those of no more tiles than CUs, do without it.
+// ANY: sets whose last nptiles tiles have no bends, of which a workgroup takes three, a thread per particle (one
+// each kept two thirds of the threads idle: 490,000 particles without bends beside 90,000 with them 2,067 -> 1,000
+// us a frame of 32 passes), or that have particles of more than VTX_MANY_BENDS bends. Its branches cost a pass 2
+// to 4%, so other sets do without them.
 #define VTX_MT 768             // threads of the workgroup
-template <int EPI, int RPT, bool MIXED>
+template <int EPI, int RPT, bool ANY>
 __global__ __launch_bounds__(VTX_MT, RPT == 1 ? 6 : 3) void k_iterate(DevState d, const TileDev* __restrict__ tiles, int in, float h) {
     constexpr uint32_t UB = RPT * VTX_MT;               // records of a round
     __shared__ float4 grad[4][UB];
@@ -599,7 +599,7 @@ __global__ __launch_bounds__(VTX_MT, RPT == 1 ? 6 : 3) void k_iterate(DevState d
     __shared__ uint32_t ent[NE * VTX_TILE];
     const uint32_t tid = threadIdx.x, wg = tile_of(d.remap);
     const uint32_t nbent = d.nitiles - d.nptiles;
-    if (MIXED && wg >= nbent) {
+    if (ANY && RPT == 1 && wg >= nbent) {
         constexpr uint32_t PT = VTX_MT / VTX_TILE;
         const uint32_t i = nbent + PT * (wg - nbent) + __builtin_amdgcn_readfirstlane(tid / VTX_TILE);
         if (i < d.nitiles) plain_particle<EPI>(d, tiles[i], tid % VTX_TILE, in, h);
@@ -674,13 +674,15 @@ __global__ __launch_bounds__(VTX_MT, RPT == 1 ? 6 : 3) void k_iterate(DevState d
         }
         return last;
     };
-    // the particle's terms among the round's records. Its entries ascend, so the rounds keep the order, and a
-    // later round goes on at the first group of four (next) that was not used up: with every round over all
-    // entries, a mesh with a vertex of 20,000 bends took 707 ms a frame of 8 passes (now 87)
+    // the particle's terms among the round's records. Its entries ascend, so the rounds keep the order, and where
+    // there are many a later round goes on at the first group of four (next) that was not used up: with every
+    // round over all entries, a mesh with a vertex of 20,000 bends took 707 ms a frame of 8 passes (now 87). Few
+    // entries are gone over again in each round, as the lanes' own places cost more (251,001 particles of an
+    // irregular mesh 1,271 us a frame of 32 passes, with them 1,490)
     uint32_t next = 0;
     const auto add = [&](uint32_t u0) {
         const uint32_t nu = min(t.ub_n - u0, (uint32_t)UB);
-        if (t.ub_n <= UB) {
+        if (!ANY || t.ub_n <= UB || t.bd_k <= VTX_MANY_BENDS) {
             for (uint32_t k0 = 0; k0 < t.bd_k; k0 += 4) add4(u0, nu, k0);
             return;
         }
@@ -1419,15 +1421,15 @@ static void launch_iterate_split(const DevState& d, int in, float h, int epilogu
     else hipLaunchKernelGGL((k_iterate_split<EPI_FINALIZE_PREDICT, B>), gr, bl, 0, s, d, d.ltiles, in, h);
 }
 
-template <int RPT, bool MIXED>
+template <int RPT, bool ANY>
 static void launch_iterate_mesh(const DevState& d, int in, float h, int epilogue, hipStream_t s) {
     constexpr uint32_t PT = VTX_MT / VTX_TILE;
-    const uint32_t plain = MIXED ? d.nptiles : 0u;
+    const uint32_t plain = ANY && RPT == 1 ? d.nptiles : 0u;
     const dim3 gr(d.nitiles - plain + (plain + PT - 1) / PT), bl(VTX_MT);
     const auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, gr, bl, 0, s, d, d.itiles, in, h); };
-    if (epilogue == EPI_NONE) launch(k_iterate<EPI_NONE, RPT, MIXED>);
-    else if (epilogue == EPI_FINALIZE) launch(k_iterate<EPI_FINALIZE, RPT, MIXED>);
-    else launch(k_iterate<EPI_FINALIZE_PREDICT, RPT, MIXED>);
+    if (epilogue == EPI_NONE) launch(k_iterate<EPI_NONE, RPT, ANY>);
+    else if (epilogue == EPI_FINALIZE) launch(k_iterate<EPI_FINALIZE, RPT, ANY>);
+    else launch(k_iterate<EPI_FINALIZE_PREDICT, RPT, ANY>);
 }
 
 static void launch_iterate_plain(const DevState& d, int in, float h, int epilogue, hipStream_t s) {
@@ -1452,17 +1454,21 @@ hipError_t launch_iterate(const DevState& d, int in, float h, int epilogue, bool
     // four threads per vertex leave 128 registers a thread: a batch of 64 distances runs as 16
     if (lra_batch >= 16) launch_iterate_split<4>(d, in, h, epilogue, s);
     else launch_iterate_split<1>(d, in, h, epilogue, s);
+    if (!d.nitiles) return last_launch();
+    if (d.nptiles == d.nitiles) {
+        launch_iterate_plain(d, in, h, epilogue, s);
+        return last_launch();
+    }
     // a tile's records in one round while every tile has a CU of its own (8.5 against 11.5 us for 90
     // tiles of 1,334 records), else in rounds of half the LDS and twice the workgroups per CU (625 tiles
     // 28.5 against 33.4 us)
-    if (d.nptiles == d.nitiles) {
-        if (d.nitiles) launch_iterate_plain(d, in, h, epilogue, s);
-    } else if (d.nitiles <= 256) {
-        launch_iterate_mesh<2, false>(d, in, h, epilogue, s);
-    } else if (d.nptiles) {
-        launch_iterate_mesh<1, true>(d, in, h, epilogue, s);
+    const bool many = d.live & VTX_LIVE_MANY_BENDS, any = many || d.nptiles;
+    if (d.nitiles <= 256) {
+        if (many) launch_iterate_mesh<2, true>(d, in, h, epilogue, s);
+        else launch_iterate_mesh<2, false>(d, in, h, epilogue, s);
     } else {
-        launch_iterate_mesh<1, false>(d, in, h, epilogue, s);
+        if (any) launch_iterate_mesh<1, true>(d, in, h, epilogue, s);
+        else launch_iterate_mesh<1, false>(d, in, h, epilogue, s);
     }
     return last_launch();
 }

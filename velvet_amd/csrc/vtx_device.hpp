@@ -189,6 +189,8 @@ struct alignas(16) ColliderDev {
 #define VTX_LIVE_SELFCOL 1u   // a segment that collides with itself
 #define VTX_LIVE_KEYED 2u     // k_hash_part's segments of several ranges have VTX_SEG_HASH_KEYED
 #define VTX_LIVE_FULL 4u      // more than VTX_HASH_PART_FULL particles
+#define VTX_LIVE_MANY_BENDS 8u   // (of a stream group) a particle with more than VTX_MANY_BENDS bend entries
+#define VTX_MANY_BENDS 64u
 
 // A range of a segment's hash cells (k_hash_part), with what its workgroup needs of the segment.
 struct HashPartDev {
