@@ -585,14 +585,14 @@ __device__ __forceinline__ void plain_particle(const DevState& d, const TileDev&
 // 4,608 particles 15.4 -> 7.1, 90,000 19.0 -> 15.4, 490,000 63.5 -> 57.8 us, where the halves even out:
 // a tile of consecutive particles of a mesh meets 1.7 times the bends it owns.
 //
-// ANY: sets whose last nptiles tiles have no bends, of which a workgroup takes three, a thread per particle (one
+// ANY: sets whose last nptiles tiles have no bends, of which a workgroup takes MT / 256, a thread per particle (one
 // each kept two thirds of the threads idle: 490,000 particles without bends beside 90,000 with them 2,067 -> 1,000
 // us a frame of 32 passes), or that have particles of more than VTX_MANY_BENDS bends. Its branches cost a pass 2
 // to 4%, so other sets do without them.
 #define VTX_MT 768             // threads of the workgroup
-template <int EPI, int RPT, bool ANY>
-__global__ __launch_bounds__(VTX_MT, RPT == 1 ? 6 : 3) void k_iterate(DevState d, const TileDev* __restrict__ tiles, int in, float h) {
-    constexpr uint32_t UB = RPT * VTX_MT;               // records of a round
+template <int EPI, int RPT, bool ANY, int MT>
+__global__ __launch_bounds__(MT, RPT == 1 ? 6 : 3) void k_iterate(DevState d, const TileDev* __restrict__ tiles, int in, float h) {
+    constexpr uint32_t UB = RPT * MT;               // records of a round
     __shared__ float4 grad[4][UB];
     __shared__ uint32_t act[UB];
     constexpr uint32_t NE = 12;                         // bend entries of a particle staged in LDS
@@ -600,7 +600,7 @@ __global__ __launch_bounds__(VTX_MT, RPT == 1 ? 6 : 3) void k_iterate(DevState d
     const uint32_t tid = threadIdx.x, wg = tile_of(d.remap);
     const uint32_t nbent = d.nitiles - d.nptiles;
     if (ANY && RPT == 1 && wg >= nbent) {
-        constexpr uint32_t PT = VTX_MT / VTX_TILE;
+        constexpr uint32_t PT = MT / VTX_TILE;
         const uint32_t i = nbent + PT * (wg - nbent) + __builtin_amdgcn_readfirstlane(tid / VTX_TILE);
         if (i < d.nitiles) plain_particle<EPI>(d, tiles[i], tid % VTX_TILE, in, h);
         return;
@@ -616,7 +616,7 @@ __global__ __launch_bounds__(VTX_MT, RPT == 1 ? 6 : 3) void k_iterate(DevState d
     int cnt = 0;
     // records [u0, u0 + UB) of the tile, the last waves first: the first ones hold the particles
     const auto evaluate = [&](uint32_t u0) {
-        const uint32_t u = VTX_MT - 1u - tid;
+        const uint32_t u = MT - 1u - tid;
         if (u0 + u >= t.ub_n) return;
         const uint4* __restrict__ rec = d.brec + t.ub_off + u0;
         uint4 ix[RPT];
@@ -624,7 +624,7 @@ __global__ __launch_bounds__(VTX_MT, RPT == 1 ? 6 : 3) void k_iterate(DevState d
         float4 q[RPT][4];
 #pragma unroll
         for (int r = 0; r < RPT; r++) {                 // a record past the last repeats it, unused
-            const uint32_t v = min(u + r * VTX_MT, t.ub_n - 1u - u0);
+            const uint32_t v = min(u + r * MT, t.ub_n - 1u - u0);
             ix[r] = rec[v];
             rest[r] = (d.brest + t.ub_off + u0)[v];
         }
@@ -637,7 +637,7 @@ __global__ __launch_bounds__(VTX_MT, RPT == 1 ? 6 : 3) void k_iterate(DevState d
         }
 #pragma unroll
         for (int r = 0; r < RPT; r++) {
-            const uint32_t v = u + r * VTX_MT;
+            const uint32_t v = u + r * MT;
             if (r && u0 + v >= t.ub_n) break;
             float lam;
             BendGrad bg;
@@ -691,11 +691,11 @@ __global__ __launch_bounds__(VTX_MT, RPT == 1 ? 6 : 3) void k_iterate(DevState d
     };
 
     // the first entry rows (contiguous: row k at k * VTX_TILE), loaded while the records are evaluated
-    constexpr uint32_t ER = NE * VTX_TILE / VTX_MT;
+    constexpr uint32_t ER = NE * VTX_TILE / MT;
     uint32_t er[ER];
     const uint32_t nent = min(t.bd_k, NE) * VTX_TILE;
 #pragma unroll
-    for (uint32_t k = 0; k < ER; k++) er[k] = k * VTX_MT + tid < nent ? (d.bd + t.bd_off)[k * VTX_MT + tid] : VTX_INVALID;
+    for (uint32_t k = 0; k < ER; k++) er[k] = k * MT + tid < nent ? (d.bd + t.bd_off)[k * MT + tid] : VTX_INVALID;
     evaluate(0);
     if (vertex) {
         const float4 p4 = P[g - sg.pbase];
@@ -705,7 +705,7 @@ __global__ __launch_bounds__(VTX_MT, RPT == 1 ? 6 : 3) void k_iterate(DevState d
         attach_terms<4>(d, sg, t.at_off, t.at_k, tid, g - sg.pbase, p, w, delta, cnt);
     }
 #pragma unroll
-    for (uint32_t k = 0; k < ER; k++) ent[k * VTX_MT + tid] = er[k];
+    for (uint32_t k = 0; k < ER; k++) ent[k * MT + tid] = er[k];
     __syncthreads();
     if (vertex) add(0);
     for (uint32_t u0 = UB; u0 < t.ub_n; u0 += UB) {
@@ -1421,15 +1421,15 @@ static void launch_iterate_split(const DevState& d, int in, float h, int epilogu
     else hipLaunchKernelGGL((k_iterate_split<EPI_FINALIZE_PREDICT, B>), gr, bl, 0, s, d, d.ltiles, in, h);
 }
 
-template <int RPT, bool ANY>
+template <int RPT, bool ANY, int MT>
 static void launch_iterate_mesh(const DevState& d, int in, float h, int epilogue, hipStream_t s) {
-    constexpr uint32_t PT = VTX_MT / VTX_TILE;
+    constexpr uint32_t PT = MT / VTX_TILE;
     const uint32_t plain = ANY && RPT == 1 ? d.nptiles : 0u;
-    const dim3 gr(d.nitiles - plain + (plain + PT - 1) / PT), bl(VTX_MT);
+    const dim3 gr(d.nitiles - plain + (plain + PT - 1) / PT), bl(MT);
     const auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, gr, bl, 0, s, d, d.itiles, in, h); };
-    if (epilogue == EPI_NONE) launch(k_iterate<EPI_NONE, RPT, ANY>);
-    else if (epilogue == EPI_FINALIZE) launch(k_iterate<EPI_FINALIZE, RPT, ANY>);
-    else launch(k_iterate<EPI_FINALIZE_PREDICT, RPT, ANY>);
+    if (epilogue == EPI_NONE) launch(k_iterate<EPI_NONE, RPT, ANY, MT>);
+    else if (epilogue == EPI_FINALIZE) launch(k_iterate<EPI_FINALIZE, RPT, ANY, MT>);
+    else launch(k_iterate<EPI_FINALIZE_PREDICT, RPT, ANY, MT>);
 }
 
 static void launch_iterate_plain(const DevState& d, int in, float h, int epilogue, hipStream_t s) {
@@ -1461,14 +1461,22 @@ hipError_t launch_iterate(const DevState& d, int in, float h, int epilogue, bool
     }
     // a tile's records in one round while every tile has a CU of its own (8.5 against 11.5 us for 90
     // tiles of 1,334 records), else in rounds of half the LDS and twice the workgroups per CU (625 tiles
-    // 28.5 against 33.4 us)
+    // 28.5 against 33.4 us). Then 512 tiles are in flight at a time with 768 threads a tile, 768 with 512
+    // threads, which take 1.3 times as long each: the fewer turns count. Frames of 32 passes, 768 / 512
+    // threads: 352 tiles 459 / 503 us, 515 787 / 622 (one thread per particle 676), 791 925 / 1,013, 1,407
+    // 1,361 / 1,207, 2,823 2,526 / 2,206, 981 of an irregular mesh 1,268 / 1,432 (three plain tiles as one)
     const bool many = d.live & VTX_LIVE_MANY_BENDS, any = many || d.nptiles;
+    const uint32_t wg = d.nitiles - d.nptiles + d.nptiles / 3;
+    const bool narrow = 13 * ((wg + 767) / 768) < 10 * ((wg + 511) / 512);
     if (d.nitiles <= 256) {
-        if (many) launch_iterate_mesh<2, true>(d, in, h, epilogue, s);
-        else launch_iterate_mesh<2, false>(d, in, h, epilogue, s);
+        if (many) launch_iterate_mesh<2, true, VTX_MT>(d, in, h, epilogue, s);
+        else launch_iterate_mesh<2, false, VTX_MT>(d, in, h, epilogue, s);
+    } else if (narrow) {
+        if (any) launch_iterate_mesh<1, true, 512>(d, in, h, epilogue, s);
+        else launch_iterate_mesh<1, false, 512>(d, in, h, epilogue, s);
     } else {
-        if (any) launch_iterate_mesh<1, true>(d, in, h, epilogue, s);
-        else launch_iterate_mesh<1, false>(d, in, h, epilogue, s);
+        if (any) launch_iterate_mesh<1, true, VTX_MT>(d, in, h, epilogue, s);
+        else launch_iterate_mesh<1, false, VTX_MT>(d, in, h, epilogue, s);
     }
     return last_launch();
 }
