@@ -202,7 +202,8 @@ int vtx_set_tuning(vtx_solver* s, const vtx_tuning* t);
 /* Time the variants on the current live set (coordinate descent, `frames` timed frames each,
  * positions and velocities restored after every trial, so the simulation does not advance),
  * apply the fastest and cache it for the live set's shape class (log2 buckets of particles and
- * segments, hash / stencil / dense-attachment presence, substeps x iterations). use_cache = 1
+ * segments, hash / stencil / dense-attachment presence, whether a segment is large enough for the search
+ * by index and the set small enough for the read-ahead contact pass, substeps x iterations). use_cache = 1
  * applies a class tuned earlier in this process without timing. hash_grid is tried only when a
  * live segment has tune_hash_grid = 1. */
 int vtx_autotune(vtx_solver* s, int32_t frames, float frame_dt, int32_t use_cache, vtx_tuning* out);

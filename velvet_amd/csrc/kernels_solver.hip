@@ -586,7 +586,7 @@ __device__ __forceinline__ void plain_particle(const DevState& d, const TileDev&
 // a tile of consecutive particles of a mesh meets 1.7 times the bends it owns.
 //
 // ANY: sets whose last nptiles tiles have no bends, of which a workgroup takes MT / 256, a thread per particle (one
-// each kept two thirds of the threads idle: 490,000 particles without bends beside 90,000 with them 2,067 -> 1,000
+// each kept two thirds of the threads idle: 490,000 particles without bends beside 90,000 with them 2,067 -> 1,017
 // us a frame of 32 passes), or that have particles of more than VTX_MANY_BENDS bends. Its branches cost a pass 2
 // to 4%, so other sets do without them.
 #define VTX_MT 768             // threads of the workgroup
